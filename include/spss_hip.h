@@ -185,7 +185,8 @@ int spss_get_cell_layout(spss_system *sys, int *k, int *xsplit);
  * the kernel's workgroup / j-tile shapes {64,64}, {64,256}, {128,128}, {128,512}, {256,256},
  * {256,512} (particles per workgroup, j per LDS tile) and keeps the fastest for the handle's
  * all-pairs evaluations; ms per evaluation into table_ms (at most table_cap entries), the chosen
- * index into *chosen.  Every shape visits j in ascending order, so results do not depend on it. */
+ * index into *chosen.  Every shape adds a particle's pairs over the same segments of the j's (their
+ * number depends on n alone), j ascending inside each, so results do not depend on the shape. */
 int spss_autotune_all_pairs(spss_system *sys, int probe_evals, double *table_ms, int table_cap, int *chosen);
 int spss_get_all_pairs_config(spss_system *sys, int *block, int *jtile);
 /* selects shape `config` (the index into the list above) by hand */

@@ -88,6 +88,7 @@ struct spss_system {
   // the next sync_master
   bool master_stale = false;
   int resident_kind = 0;
+  AllPairsScratch ap;                // all-pairs records and partial sums
   int ap_config = kAllPairsDefault;  // all-pairs workgroup and j-tile sizes (spss_autotune_all_pairs)
   int xsplit = 1;                    // FP32C cell grid: columns per square cell (spss_set_cell_layout)
   KernelTimer *timer = nullptr;  // around the pair kernel of the RHS
@@ -172,6 +173,14 @@ int ensure_scan(spss_system *h) {
   return dalloc_n(&h->scan_blk, scan_blocks(h->n) + 1);
 }
 
+int ensure_all_pairs(spss_system *h) {
+  if (h->ap.part) return SPSS_OK;
+  h->ap.nseg = all_pairs_segments(h->n);
+  if (!h->ap.rec) TRY(dalloc_n(&h->ap.rec, (size_t)4 * h->n));
+  if (!h->ap.om) TRY(dalloc_n(&h->ap.om, h->n));
+  return dalloc_n(&h->ap.part, (size_t)h->ap.nseg * 5 * h->n);
+}
+
 // EvaluateRhs's dispatch on rho (ParticleSystemFirstOrderPtr.cpp:131-153; model 6:
 // ParticleSystemSecondOrderPtr.cpp:125-138)
 int resolve_method(const spss_system *h, int method) {
@@ -240,13 +249,16 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
   h->P.higher_order = h->higher_order ? 1 : 0;
   const double *nat = h->have_nat ? h->nat : nullptr;
   double *compl_out = h->higher_order ? h->compl_f : nullptr;
-  launch_stage(st, (long)h->s * h->n, d_state, d_kprev, k_coef * dt, h->stage);
+  if (m == SPSS_METHOD_ALL_PAIRS)
+    launch_all_pairs_stage(st, h->P, d_state, d_kprev, k_coef * dt, h->stage, h->ap);
+  else
+    launch_stage(st, (long)h->s * h->n, d_state, d_kprev, k_coef * dt, h->stage);
   switch (m) {
     case SPSS_METHOD_GLOBAL_FIELD:
       launch_global(st, h->P, h->stage, h->partial, h->scal, nat, d_knext, compl_out);
       break;
     case SPSS_METHOD_ALL_PAIRS:
-      launch_all_pairs(st, h->P, h->stage, nat, d_knext, compl_out, h->ap_config);
+      launch_all_pairs(st, h->P, h->ap, h->stage, nat, d_knext, compl_out, h->ap_config);
       break;
     case SPSS_METHOD_LINKED_LIST:
       if (h->p.precision == SPSS_PRECISION_FP32C) {
@@ -539,6 +551,8 @@ int spss_create(const spss_params *p, spss_system **out) {
   step(dalloc_n(&h->noise, (size_t)3 * h->n));
   step(dalloc_n(&h->partial, nb * 4 + 64));
   step(dalloc_n(&h->scal, 64));
+  // with the handle, so that an all-pairs evaluation allocates nothing (a caller may capture it)
+  if (p->precision != SPSS_PRECISION_FP32C) step(ensure_all_pairs(h));
   if (rc != SPSS_OK) {
     spss_destroy(h);
     return rc;
@@ -576,7 +590,7 @@ int spss_destroy(spss_system *h) {
   delete h->timer;
   void *bufs[] = {h->state, h->stage, h->k[0], h->k[1], h->k[2], h->k[3], h->deriv, h->compl_f, h->nat,
                   h->noise, h->partial, h->scal, h->acc, h->io[0], h->io[1], h->io[2], h->vcount, h->vstart,
-                  h->vlist, h->pcount, h->pstart, h->plist, h->scan_blk};
+                  h->vlist, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec, h->ap.om, h->ap.part};
   for (void *b : bufs) hipFree(b);
   for (double *b : h->dp) hipFree(b);
   if (h->dp_host) hipHostFree(h->dp_host);
@@ -910,23 +924,24 @@ int spss_autotune_all_pairs(spss_system *h, int probe_evals, double *table_ms, i
   if (!h) return fail(SPSS_ERR_INVALID, "NULL handle");
   if (probe_evals < 1) return fail(SPSS_ERR_INVALID, "probe_evals >= 1 required");
   TRY(sync_master(h));
+  TRY(ensure_all_pairs(h));
   const size_t m = (size_t)h->s * h->n;
   double *k = nullptr;
   TRY(dalloc_n(&k, m));
   const double *nat = h->have_nat ? h->nat : nullptr;
   double *compl_out = h->higher_order ? h->compl_f : nullptr;
   h->P.higher_order = h->higher_order ? 1 : 0;
-  launch_stage(h->stream, (long)m, h->state, nullptr, 0.0, h->stage);
+  launch_all_pairs_stage(h->stream, h->P, h->state, nullptr, 0.0, h->stage, h->ap);
   double best = 1e300;
   int best_c = h->ap_config;
   int rc = SPSS_OK;
   for (int c = 0; c < kAllPairsConfigCount && rc == SPSS_OK; ++c) {
-    launch_all_pairs(h->stream, h->P, h->stage, nat, k, compl_out, c);  // warm-up
+    launch_all_pairs(h->stream, h->P, h->ap, h->stage, nat, k, compl_out, c);  // warm-up
     EventPair ev;
     hipError_t e = ev.create();
     if (e == hipSuccess) e = hipEventRecord(ev.start, h->stream);
     for (int r = 0; r < probe_evals && e == hipSuccess; ++r)
-      launch_all_pairs(h->stream, h->P, h->stage, nat, k, compl_out, c);
+      launch_all_pairs(h->stream, h->P, h->ap, h->stage, nat, k, compl_out, c);
     if (e == hipSuccess) e = hipEventRecord(ev.stop, h->stream);
     float ms = 0.f;
     if (e == hipSuccess) e = ev.elapsed(&ms);
