@@ -27,8 +27,16 @@ namespace {
 // outside it at all, ClassA is no minimum image there), or a phase without a finite phasor
 constexpr double kExactMark = __builtin_huge_val();
 
+__device__ __forceinline__ void phasor_any(double phi, double ref, double &sn, double &cs) {
+  if (fabs(phi) <= kPhase64)
+    frame_phasor(phi, ref, sn, cs);
+  else
+    sincos(phi - ref, &sn, &cs);
+}
+
 template <int S>
-__global__ __launch_bounds__(256) void ap_stage(DevParams P, const double *__restrict__ state, const double *kprev,
+__global__ __launch_bounds__(256) void ap_stage(DevParams P, const double *__restrict__ state,
+                                                const double *__restrict__ kprev,
                                                 double kc_dt, double *__restrict__ stage, double4 *__restrict__ rec,
                                                 double *__restrict__ om) {
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -44,8 +52,8 @@ __global__ __launch_bounds__(256) void ap_stage(DevParams P, const double *__res
   }
   double x, y, sn, cs;
   apply_pbc(P, st[0], st[1], x, y);
-  sincos(st[kPhi] - ref, &sn, &cs);
-  bool fine = fabs(sn) <= 1.0 && fabs(st[0]) <= kFar64 * P.xs && fabs(st[1]) <= kFar64 * P.ys;
+  phasor_any(st[kPhi], ref, sn, cs);
+  bool fine = fabs(sn) <= 1.5 && fabs(st[0]) <= kFar64 * P.xs && fabs(st[1]) <= kFar64 * P.ys;
   if (S == 6) fine = fine && st[0] >= 0.0 && st[0] < P.xs && st[1] >= 0.0 && st[1] < P.ys;
   if (S == 4 && P.higher_order) {
     const double o = st[kOm] - frame_ref(state[kOm] + (kprev ? kc_dt * kprev[kOm] : 0.0));
@@ -61,57 +69,56 @@ __device__ __forceinline__ void add_pair(PhasorSums &a, double w, double s, doub
   a.card += w;
 }
 
-// one staged tile of cnt j's against the PPL particles of a lane by the cheap test, four j's at a time
-template <int S, bool HO, int PPL, int T, bool OWN>
-__device__ __forceinline__ void tile_pairs(const DevParams &P, double band, const double *__restrict__ stage,
-                                           const double4 *tile, const double *tom, int i0, int j0, int cnt,
-                                           const double (&x_i)[PPL], const double (&y_i)[PPL], PhasorSums (&a)[PPL]) {
-  for (int t0 = 0; t0 < cnt; t0 += 4) {
-    double w[PPL][4], near = 1e300;
-    double4 r[4];
+// four entries from t0 on of a staged tile of cnt j's against the PPL particles of a lane by the
+// cheap test; MASKED: fewer than four are left, or some may be the lane's own particles
+template <int S, bool HO, int PPL, int T, bool MASKED>
+__device__ __forceinline__ void four_j(const DevParams &P, double band, double neg_slope,
+                                       const double *__restrict__ stage, const double4 *tile, const double *tom, int i0,
+                                       int j0, int t0, int cnt, const double (&x_i)[PPL], const double (&y_i)[PPL],
+                                       PhasorSums (&a)[PPL]) {
+  double w[PPL][4], near = 1e300;
+  double4 r[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) r[u] = tile[min(t0 + u, cnt - 1)];
+  for (int u = 0; u < 4; ++u) r[u] = tile[MASKED ? min(t0 + u, cnt - 1) : t0 + u];
 #pragma unroll
-    for (int p = 0; p < PPL; ++p)
+  for (int p = 0; p < PPL; ++p)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        double dx = fabs(r[u].x - x_i[p]), dy = fabs(r[u].y - y_i[p]);
-        dx = fmin(dx, P.xs - dx);
-        dy = fmin(dy, P.ys - dy);
-        const double t = __builtin_fma(dx, dx, __builtin_fma(dy, dy, -P.rho2));
-        near = fmin(near, fabs(t));
-        bool in = t <= 0.0 && t0 + u < cnt;
-        if (OWN) in = in && j0 + t0 + u != i0 + p * T + (int)threadIdx.x;
-        w[p][u] = in ? 1.0 : 0.0;
-      }
-    if (near <= band) {  // rare: the reference's own test decides these pairs
-#pragma unroll
-      for (int p = 0; p < PPL; ++p)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int j = j0 + t0 + u;
-          const bool there = t0 + u < cnt && j != i0 + p * T + (int)threadIdx.x;
-          w[p][u] = there && pair_in_range<S>(P, x_i[p], y_i[p], stage[(long)j * S], stage[(long)j * S + 1]) ? 1.0 : 0.0;
-        }
+    for (int u = 0; u < 4; ++u) {
+      double dx = fabs(r[u].x - x_i[p]), dy = fabs(r[u].y - y_i[p]);
+      dx = fmin(dx, P.xs - dx);
+      dy = fmin(dy, P.ys - dy);
+      const double t = __builtin_fma(dx, dx, __builtin_fma(dy, dy, -P.rho2));
+      near = fmin(near, fabs(t));
+      w[p][u] = pair_weight(t, neg_slope);
+      if (MASKED && (t0 + u >= cnt || j0 + t0 + u == i0 + p * T + (int)threadIdx.x)) w[p][u] = 0.0;
     }
+  if (near <= band) {  // rare: the reference's own test decides these pairs
 #pragma unroll
     for (int p = 0; p < PPL; ++p)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        add_pair(a[p], w[p][u], r[u].z, r[u].w);
-        if (HO) {
-          const double wo = w[p][u] * tom[min(t0 + u, cnt - 1)];
-          a[p].TS = __builtin_fma(wo, r[u].z, a[p].TS);
-          a[p].TC = __builtin_fma(wo, r[u].w, a[p].TC);
-        }
+        const int j = j0 + t0 + u;
+        const bool there = !MASKED || (t0 + u < cnt && j != i0 + p * T + (int)threadIdx.x);
+        w[p][u] = there && pair_in_range<S>(P, x_i[p], y_i[p], stage[(long)j * S], stage[(long)j * S + 1]) ? 1.0 : 0.0;
       }
   }
+#pragma unroll
+  for (int p = 0; p < PPL; ++p)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      add_pair(a[p], w[p][u], r[u].z, r[u].w);
+      if (HO) {
+        const double wo = w[p][u] * tom[MASKED ? min(t0 + u, cnt - 1) : t0 + u];
+        a[p].TS = __builtin_fma(wo, r[u].z, a[p].TS);
+        a[p].TC = __builtin_fma(wo, r[u].w, a[p].TC);
+      }
+    }
 }
 
 // PPL particles per lane (BLOCK / PPL threads): a tile entry read from LDS serves PPL pairs, which
 // halves the LDS reads per pair (at one particle per lane they take as long as the arithmetic)
 template <int S, bool HO, int BLOCK, int JT, int PPL>
-__global__ __launch_bounds__(BLOCK / PPL) void ap_pairs(DevParams P, double band, int seglen,
+__global__ __launch_bounds__(BLOCK / PPL) void ap_pairs(DevParams P, double band, double neg_slope, int seglen,
                                                         const double *__restrict__ stage,
                                                         const double4 *__restrict__ rec, const double *__restrict__ om,
                                                         double *__restrict__ part) {
@@ -150,10 +157,12 @@ __global__ __launch_bounds__(BLOCK / PPL) void ap_pairs(DevParams P, double band
     if (__syncthreads_and(ok)) {
       // only tiles that hold some of the workgroup's own particles compare i with j
       const bool own = j0 < i0 + BLOCK && j0 + cnt > i0;
-      if (own)
-        tile_pairs<S, HO, PPL, T, true>(P, band, stage, tile, tom, i0, j0, cnt, x_i, y_i, a);
-      else
-        tile_pairs<S, HO, PPL, T, false>(P, band, stage, tile, tom, i0, j0, cnt, x_i, y_i, a);
+      int t0 = 0;
+      if (!own)
+        for (; t0 + 4 <= cnt; t0 += 4)
+          four_j<S, HO, PPL, T, false>(P, band, neg_slope, stage, tile, tom, i0, j0, t0, cnt, x_i, y_i, a);
+      for (; t0 < cnt; t0 += 4)
+        four_j<S, HO, PPL, T, true>(P, band, neg_slope, stage, tile, tom, i0, j0, t0, cnt, x_i, y_i, a);
     } else {
       for (int t = 0; t < cnt; ++t) {
         const int j = j0 + t;
@@ -230,7 +239,9 @@ __global__ __launch_bounds__(256) void ap_finish(DevParams P, int nseg, const do
 #pragma unroll
   for (int q = 0; q < S; ++q) st[q] = stage[(long)i * S + q];
   const double om_i = HO ? st[Slots<S>::omega] - frame_ref(stage[Slots<S>::omega]) : 0.0;
-  const PairAcc pa = pair_acc<S>(P, a, st[Slots<S>::phi] - frame_ref(stage[Slots<S>::phi]), om_i);
+  double s_i, c_i;
+  phasor_any(st[Slots<S>::phi], frame_ref(stage[Slots<S>::phi]), s_i, c_i);
+  const PairAcc pa = pair_acc<S>(P, a, s_i, c_i, om_i);
   write_k<S>(P, st, i, pa, nat ? nat[i] : 0.0, k_next, compl_out);
 }
 
@@ -238,8 +249,9 @@ template <int S, bool HO, int BLOCK, int JT>
 void pairs_as(hipStream_t st, const DevParams &P, const AllPairsScratch &W, const double *stage) {
   constexpr int PPL = BLOCK >= 128 ? 2 : 1;
   const dim3 grid((unsigned)((P.n + BLOCK - 1) / BLOCK), (unsigned)W.nseg);
+  const double band = pair_band(P.rho2, P.xs, P.ys);
   ap_pairs<S, HO, BLOCK, JT, PPL><<<grid, dim3(BLOCK / PPL), 0, st>>>(
-      P, pair_band(P.rho2, P.xs, P.ys), (P.n + W.nseg - 1) / W.nseg, stage, (const double4 *)W.rec, W.om, W.part);
+      P, band, pair_neg_slope(band), (P.n + W.nseg - 1) / W.nseg, stage, (const double4 *)W.rec, W.om, W.part);
 }
 
 template <int S, bool HO>
@@ -262,10 +274,10 @@ const int kAllPairsConfigs[kAllPairsConfigCount][2] = {{64, 64}, {64, 256}, {128
                                                         {256, 256}, {256, 512}};
 
 // segments of the j's: 64 fill the chip from some thousand particles on (17 groups x 64 segments x 2
-// waves at n = 4,099); more particles bring their own groups, and 2^20 / n of them keep the
-// partial sums within 2^20 particles' worth
+// waves at n = 4,099); more particles bring their own groups, and 2^19 / n of them keep the
+// partial sums within 2^19 particles' worth (21 MB)
 int all_pairs_segments(int n) {
-  const long by_work = (n + 63) / 64, by_size = (1L << 20) / n;
+  const long by_work = (n + 63) / 64, by_size = (1L << 19) / n;
   long g = by_work < 64 ? by_work : 64;
   if (g > by_size) g = by_size;
   return g < 1 ? 1 : (int)g;

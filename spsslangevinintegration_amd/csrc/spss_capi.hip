@@ -66,6 +66,7 @@ struct spss_system {
   double *partial = nullptr, *scal = nullptr, *acc = nullptr;
   double *io[3] = {nullptr, nullptr, nullptr};
   CellBuffers cells, vcells;
+  Cells64 cells64;
   int *vcount = nullptr, *vstart = nullptr, *vlist = nullptr;
   long vcap = 0;
   int *pcount = nullptr, *pstart = nullptr, *plist = nullptr;
@@ -167,6 +168,24 @@ int ensure_cells(spss_system *h, CellBuffers &cb, int ncx, int ncy) {
   return SPSS_OK;
 }
 
+int ensure_cells64(spss_system *h) {
+  Cells64 &B = h->cells64;
+  if (B.snap) return SPSS_OK;
+  const size_t n = h->n, cells = (size_t)h->ncx * h->ncy;
+  for (int **p : {&B.order[0], &B.order[1], &B.key, &B.slot})
+    if (!*p) TRY(dalloc_n(p, n));
+  if (!B.tmp) TRY(dalloc_n(&B.tmp, 2 * n));
+  if (!B.count) TRY(dalloc_n(&B.count, cells));
+  if (!B.start) TRY(dalloc_n(&B.start, cells + 1));
+  if (!B.local) TRY(dalloc_n(&B.local, cells + 1));
+  if (!B.blocksum) TRY(dalloc_n(&B.blocksum, scan_blocks(cells) + 1));
+  if (!B.bad) TRY(dalloc_n(&B.bad, 1));
+  if (!B.pre) TRY(dalloc_n(&B.pre, n * h->s));
+  launch_iota(h->stream, h->n, B.order[0]);
+  launch_fill_int(h->stream, (long)cells, B.count, 0);
+  return dalloc_n(&B.snap, n * h->s);
+}
+
 // scratch of the scans over n counts
 int ensure_scan(spss_system *h) {
   if (h->scan_blk) return SPSS_OK;
@@ -174,11 +193,13 @@ int ensure_scan(spss_system *h) {
 }
 
 int ensure_all_pairs(spss_system *h) {
-  if (h->ap.part) return SPSS_OK;
+  if (h->ap.rec) return SPSS_OK;
+  const size_t n = h->n;
   h->ap.nseg = all_pairs_segments(h->n);
-  if (!h->ap.rec) TRY(dalloc_n(&h->ap.rec, (size_t)4 * h->n));
-  if (!h->ap.om) TRY(dalloc_n(&h->ap.om, h->n));
-  return dalloc_n(&h->ap.part, (size_t)h->ap.nseg * 5 * h->n);
+  TRY(dalloc_n(&h->ap.rec, (5 + (size_t)h->ap.nseg * 5) * n));  // one allocation for the three arrays
+  h->ap.om = h->ap.rec + 4 * n;
+  h->ap.part = h->ap.om + n;
+  return SPSS_OK;
 }
 
 // EvaluateRhs's dispatch on rho (ParticleSystemFirstOrderPtr.cpp:131-153; model 6:
@@ -241,15 +262,23 @@ int build_verlet(spss_system *h, int m) {
   return SPSS_OK;
 }
 
+// fresh: d_knext counts as zero-filled before the call (the stochastic steppers' derivative,
+// StochasticEulerStepperPtr.hpp:43), whatever it holds
 int rhs_device(spss_system *h, int method, const double *d_state, const double *d_kprev, double *d_knext,
-               double k_coef, double dt) {
+               double k_coef, double dt, bool fresh = false) {
   const int m = resolve_method(h, method);
   TRY(check_method(h, m));
   hipStream_t st = h->stream;
   h->P.higher_order = h->higher_order ? 1 : 0;
+  h->P.fresh_k = fresh ? 1 : 0;
   const double *nat = h->have_nat ? h->nat : nullptr;
   double *compl_out = h->higher_order ? h->compl_f : nullptr;
-  if (m == SPSS_METHOD_ALL_PAIRS)
+  const bool tiled = m == SPSS_METHOD_LINKED_LIST && h->p.precision != SPSS_PRECISION_FP32C &&
+                     cells64_serves(h->P, h->ncx, h->ncy);
+  if (tiled) {
+    TRY(ensure_cells64(h));
+    launch_cells64_build(st, h->P, d_state, d_kprev, k_coef * dt, h->ncx, h->cells64);
+  } else if (m == SPSS_METHOD_ALL_PAIRS)
     launch_all_pairs_stage(st, h->P, d_state, d_kprev, k_coef * dt, h->stage, h->ap);
   else
     launch_stage(st, (long)h->s * h->n, d_state, d_kprev, k_coef * dt, h->stage);
@@ -263,6 +292,10 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
     case SPSS_METHOD_LINKED_LIST:
       if (h->p.precision == SPSS_PRECISION_FP32C) {
         TRY(fast_rhs(h->fast, st, h->P, h->stage, nat, d_knext, compl_out));
+      } else if (tiled) {
+        if (h->timer) h->timer->begin(st);
+        launch_cells64_pairs(st, h->P, h->ncx, h->cells64, nat, d_knext, compl_out);
+        if (h->timer) h->timer->end(st);
       } else {
         TRY(ensure_cells(h, h->cells, h->ncx, h->ncy));
         launch_cell_build(st, h->P, h->stage, h->ncx, h->ncy, h->cells);
@@ -413,9 +446,8 @@ int euler_step(spss_system *h, int method, double dt, int noise_mode, const doub
   if (use_fused(h, method)) return fast_fused_step(h, 0, dt, noise_mode, noise);
   if (use_fused_verlet(h, method)) return verlet_fused_step(h, 0, dt, noise_mode, noise);
   TRY(master_write(h, true));
-  const size_t m = (size_t)h->s * h->n;
-  launch_fill_double(h->stream, (long)m, h->deriv, 0.0);  // std::fill(derivative, 0), :43
-  TRY(rhs_device(h, method, h->state, h->deriv, h->deriv, 0.0, dt));
+  // the derivative is zero-filled and serves as k_prev with coefficient 0 (:43-47): no stage change
+  TRY(rhs_device(h, method, h->state, nullptr, h->deriv, 0.0, dt, true));
   int kmode;
   const double *kptr;
   TRY(noise_source(h, noise_mode, noise, (size_t)(h->s == 6 ? 3 : 1) * h->n, &kmode, &kptr));
@@ -440,10 +472,8 @@ int srk_step(spss_system *h, int method, double dt, int noise_mode, const double
     return verlet_fused_step(h, 1, dt, noise_mode, noise);
   }
   TRY(master_write(h, true));
-  const size_t m = (size_t)h->s * h->n;
-  launch_fill_double(h->stream, (long)m, h->deriv, 0.0);
   h->higher_order = true;  // StochasticRungeKuttaStepperPtr.hpp:44
-  TRY(rhs_device(h, method, h->state, h->deriv, h->deriv, 0.0, dt));
+  TRY(rhs_device(h, method, h->state, nullptr, h->deriv, 0.0, dt, true));
   int kmode;
   const double *kptr;
   TRY(noise_source(h, noise_mode, noise, (size_t)2 * h->n, &kmode, &kptr));
@@ -590,10 +620,15 @@ int spss_destroy(spss_system *h) {
   delete h->timer;
   void *bufs[] = {h->state, h->stage, h->k[0], h->k[1], h->k[2], h->k[3], h->deriv, h->compl_f, h->nat,
                   h->noise, h->partial, h->scal, h->acc, h->io[0], h->io[1], h->io[2], h->vcount, h->vstart,
-                  h->vlist, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec, h->ap.om, h->ap.part};
+                  h->vlist, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec};
   for (void *b : bufs) hipFree(b);
   for (double *b : h->dp) hipFree(b);
   if (h->dp_host) hipHostFree(h->dp_host);
+  Cells64 &c64 = h->cells64;
+  for (int *b : {c64.order[0], c64.order[1], c64.key, c64.slot, c64.count, c64.start, c64.local, c64.blocksum, c64.bad, c64.tmp})
+    hipFree(b);
+  hipFree(c64.pre);
+  hipFree(c64.snap);
   for (CellBuffers *cb : {&h->cells, &h->vcells}) {
     hipFree(cb->key);
     hipFree(cb->slot);

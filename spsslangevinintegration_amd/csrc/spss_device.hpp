@@ -28,6 +28,7 @@ struct DevParams {
   double xrs, yrs; // 1.0 / x_size (the constructor, PeriodicBoundaryConditions.cpp:7-21)
   int natfreq_local;
   int higher_order;
+  int fresh_k;     // the derivative starts from zero: entries the local branches leave alone are written as 0
 };
 
 // ---- periodic boundary conditions (BoundaryConfiguration/PeriodicBoundaryConditions.cpp)
@@ -125,14 +126,16 @@ __device__ __forceinline__ void pair_term(const DevParams &P, double x_i, double
 // ---- output row of the local branches
 // model 4: ParticleSystemFirstOrderPtr.cpp:303-313; model 6: ParticleSystemSecondOrderPtr.cpp:219-227;
 // model 3 (m = 0): k = (v0 cos phi, v0 sin phi, w_i + sigma A / n)
+// (sin_i, cos_i: of the particle's phase)
 template <int S>
 __device__ __forceinline__ void write_k(const DevParams &P, const double *st, int i, const PairAcc &a,
-                                        double nat_i, double *k_next, double *compl_out) {
+                                        double nat_i, double sin_i, double cos_i, double *k_next,
+                                        double *compl_out) {
   const long ii = (long)i * S;
   if (S == 4) {
-    double phi_i = st[2], omega_i = st[3];
-    k_next[ii] = P.v0 * cos(phi_i);
-    k_next[ii + 1] = P.v0 * sin(phi_i);
+    const double omega_i = st[3];
+    k_next[ii] = P.v0 * cos_i;
+    k_next[ii + 1] = P.v0 * sin_i;
     k_next[ii + 2] = omega_i;
     if (P.natfreq_local) {
       if (a.card != 0.0)
@@ -141,6 +144,8 @@ __device__ __forceinline__ void write_k(const DevParams &P, const double *st, in
         k_next[ii + 3] = -P.xi * omega_i + nat_i;
     } else if (a.card != 0.0) {
       k_next[ii + 3] = -P.xi * omega_i + P.sigma * a.align / a.card;
+    } else if (P.fresh_k) {
+      k_next[ii + 3] = 0.0;
     }
     if (P.higher_order && compl_out) {
       double c = a.compl_f;
@@ -148,22 +153,30 @@ __device__ __forceinline__ void write_k(const DevParams &P, const double *st, in
       compl_out[i] = c;
     }
   } else if (S == 6) {
-    double vx = st[2], vy = st[3], phi_i = st[4], omega_i = st[5];
+    const double vx = st[2], vy = st[3], omega_i = st[5];
     k_next[ii] = vx;
     k_next[ii + 1] = vy;
-    k_next[ii + 2] = -P.xi_r * vx + P.v0 * cos(phi_i);
-    k_next[ii + 3] = -P.xi_r * vy + P.v0 * sin(phi_i);
+    k_next[ii + 2] = -P.xi_r * vx + P.v0 * cos_i;
+    k_next[ii + 3] = -P.xi_r * vy + P.v0 * sin_i;
     k_next[ii + 4] = omega_i;
-    if (a.card != 0.0) k_next[ii + 5] = -P.xi * omega_i + P.sigma * a.align / a.card;
+    if (a.card != 0.0)
+      k_next[ii + 5] = -P.xi * omega_i + P.sigma * a.align / a.card;
+    else if (P.fresh_k)
+      k_next[ii + 5] = 0.0;
   } else {
-    double phi_i = st[2];
-    k_next[ii] = P.v0 * cos(phi_i);
-    k_next[ii + 1] = P.v0 * sin(phi_i);
+    k_next[ii] = P.v0 * cos_i;
+    k_next[ii + 1] = P.v0 * sin_i;
     if (a.card != 0.0)
       k_next[ii + 2] = nat_i + P.sigma * a.align / a.card;
     else
       k_next[ii + 2] = nat_i;
   }
+}
+
+template <int S>
+__device__ __forceinline__ void write_k(const DevParams &P, const double *st, int i, const PairAcc &a,
+                                        double nat_i, double *k_next, double *compl_out) {
+  write_k<S>(P, st, i, a, nat_i, sin(st[Slots<S>::phi]), cos(st[Slots<S>::phi]), k_next, compl_out);
 }
 
 // ---- counter-based RNG: Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11) written from the

@@ -580,6 +580,11 @@ __global__ void k_fill_int(long m, int *__restrict__ p, int v) {
   if (k < m) p[k] = v;
 }
 
+__global__ void k_iota(int n, int *__restrict__ p) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) p[k] = k;
+}
+
 // ---------------------------------------------------------------------------
 // host-side launchers
 
@@ -703,6 +708,10 @@ void launch_copy16(hipStream_t st, long n16, const void *src, void *dst) {
 
 void launch_fill_int(hipStream_t st, long m, int *p, int v) {
   if (m > 0) k_fill_int<<<dim3(nblk(m)), dim3(kBlock), 0, st>>>(m, p, v);
+}
+
+void launch_iota(hipStream_t st, int n, int *p) {
+  if (n > 0) k_iota<<<dim3(nblk(n)), dim3(kBlock), 0, st>>>(n, p);
 }
 
 }  // namespace spss

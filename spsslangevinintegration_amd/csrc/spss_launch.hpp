@@ -117,6 +117,23 @@ void launch_all_pairs(hipStream_t st, const DevParams &P, const AllPairsScratch 
 void launch_cell_build(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy, CellBuffers &cb);
 void launch_linked_list(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy,
                         const CellBuffers &cb, const double *nat, double *k_next, double *compl_out);
+// the FP64 linked list on a unit box of 3 x 3 to 1448 x 1448 cells (spss_cells64.hip); other boxes,
+// coarser grids, where the reference visits cells more than once, and finer ones, whose cells are
+// mostly empty below a hundred million particles, take the two calls above
+struct Cells64 {
+  int *order[2] = {nullptr, nullptr};  // [n] particle of each sorted position: the last build's, the next one's
+  int cur = 0;
+  int *key = nullptr, *slot = nullptr, *count = nullptr, *blocksum = nullptr, *bad = nullptr;
+  int *local = nullptr, *start = nullptr;      // [cells + 1] starts inside a scan block, starts
+  int *tmp = nullptr;                          // [2 n]
+  double *pre = nullptr, *snap = nullptr;      // [s n] stage state in the last build's and in this one's order
+};
+bool cells64_serves(const DevParams &P, int ncx, int ncy);
+void launch_cells64_build(hipStream_t st, const DevParams &P, const double *state, const double *kprev, double kc_dt,
+                          int nc, Cells64 &B);
+void launch_cells64_pairs(hipStream_t st, const DevParams &P, int nc, const Cells64 &B, const double *nat,
+                          double *k_next, double *compl_out);
+void launch_iota(hipStream_t st, int n, int *p);
 // exclusive scan of count[0..m) into start[0..m]; count is left zeroed; blocksum: scratch of
 // scan_blocks(m) + 1 ints (spss_scan.hpp)
 void launch_scan(hipStream_t st, int *count, int *start, int m, int *blocksum);

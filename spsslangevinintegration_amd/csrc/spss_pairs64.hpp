@@ -15,6 +15,8 @@
 // expressions on the stored positions (pair_in_range).
 #pragma once
 
+#include <math.h>
+
 #include "spss_device.hpp"
 
 namespace spss {
@@ -24,8 +26,50 @@ struct PhasorSums {
   double S = 0.0, C = 0.0, card = 0.0, TS = 0.0, TC = 0.0;
 };
 
-// a reference phase or phase velocity: any finite value serves
-__device__ __forceinline__ double frame_ref(double v) { return fabs(v) < 1e300 ? v : 0.0; }
+// sin and cos of x + e for |x| <= 2^30 and a correction |e| far below one: reduction to |r| <= pi/4 by
+// multiples of pi/2 (pi/2 in two parts, Cody and Waite, Software Manual for the Elementary Functions;
+// the first difference is exact, the multiples' low bits are 2^-52), then the Taylor polynomials to r^17 and r^16, whose next
+// terms are below 2^-60.  Branch-free and about a fifth of the instructions of the general sincos.
+__device__ __forceinline__ void small_sincos(double x, double e, double &sn, double &cs) {
+  const double k = rint(x * 0x1.45f306dc9c883p-1);  // 2 / pi
+  const double r0 = __builtin_fma(-k, 0x1.921fb54442d18p+0, x);
+  const double r = __builtin_fma(-k, 0x1.1a62633145c07p-54, r0);
+  e = __builtin_fma(-k, 0x1.1a62633145c07p-54, r0 - r) + e;  // what r lacks
+  const double z = r * r;
+  double p = __builtin_fma(z, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
+  p = __builtin_fma(z, p, 1.0 / 6227020800.0);
+  p = __builtin_fma(z, p, -1.0 / 39916800.0);
+  p = __builtin_fma(z, p, 1.0 / 362880.0);
+  p = __builtin_fma(z, p, -1.0 / 5040.0);
+  p = __builtin_fma(z, p, 1.0 / 120.0);
+  p = __builtin_fma(z, p, -1.0 / 6.0);
+  const double h = 0.5 * z, w = 1.0 - h;
+  const double s = r + __builtin_fma(r * z, p, __builtin_fma(-h, e, e));
+  double q = __builtin_fma(z, 1.0 / 20922789888000.0, -1.0 / 87178291200.0);
+  q = __builtin_fma(z, q, 1.0 / 479001600.0);
+  q = __builtin_fma(z, q, -1.0 / 3628800.0);
+  q = __builtin_fma(z, q, 1.0 / 40320.0);
+  q = __builtin_fma(z, q, -1.0 / 720.0);
+  q = __builtin_fma(z, q, 1.0 / 24.0);
+  // 1 - z/2 + z^2 q with the rounding of 1 - z/2 put back
+  const double c = w + __builtin_fma(-e, r, __builtin_fma(z * z, q, (1.0 - w) - h));
+  const int n = (int)k;
+  const double a = (n & 1) ? c : s, b = (n & 1) ? s : c;
+  sn = (n & 2) ? -a : a;
+  cs = ((n + 1) & 2) ? -b : b;
+}
+
+// sin, cos of phi - ref; the difference's rounding error (up to 2^-51 for phases a turn apart) is
+// carried along, which keeps the phasors within an ulp of those of the exact difference
+// (phases and references up to kPhase64)
+constexpr double kPhase64 = 0x1p29;
+__device__ __forceinline__ void frame_phasor(double phi, double ref, double &sn, double &cs) {
+  const double d = phi - ref, b = d - phi;
+  small_sincos(d, (phi - (d - b)) - (ref + b), sn, cs);
+}
+
+// a reference phase or phase velocity: any value of an ordinary size serves
+__device__ __forceinline__ double frame_ref(double v) { return fabs(v) <= kPhase64 ? v : 0.0; }
 
 // |t| of a pair below which its distance test goes to pair_in_range.  Coordinates up to
 // kFar64 boxes from the origin, wrapped and shifted, put |dx| off by at most ~2^-40 of the box;
@@ -34,6 +78,12 @@ constexpr double kFar64 = 4096.0;
 inline double pair_band(double rho2, double xs, double ys) {
   return rho2 * 0x1p-30 + sqrt(rho2) * (xs > ys ? xs : ys) * 0x1p-33;
 }
+
+// the weight of a pair at t = d^2 - rho^2: 1 within the radius, 0 beyond it (and for NaN), one VALU
+// operation with the output clamp.  -slope is a power of two with slope * band > 2, so it is exact
+// outside the guard band.
+__device__ __forceinline__ double pair_weight(double t, double neg_slope) { return fmin(fmax(t * neg_slope, 0.0), 1.0); }
+inline double pair_neg_slope(double band) { return -ldexp(1.0, ilogb(2.0 / band) + 1); }
 
 // the reference's own distance test: models 3 and 4 ClassC on the wrapped x_i and stored x_j
 // (ParticleSystemFirstOrderPtr.cpp:285-289), model 6 ClassA (ParticleSystemSecondOrderPtr.cpp:208-212)
@@ -47,19 +97,25 @@ __device__ __forceinline__ bool pair_in_range(const DevParams &P, double x_i, do
   return dx * dx + dy * dy <= P.rho2;
 }
 
-// the coupling sums of the reference (PairAcc) from the phasor sums: psi_i, om_i relative to the
-// frame's references
+// a b - c d, the rounding of c d put back
+__device__ __forceinline__ double cross(double a, double b, double c, double d) {
+  const double p = c * d;
+  return __builtin_fma(a, b, -p) - __builtin_fma(c, d, -p);
+}
+
+// the coupling sums of the reference (PairAcc) from the phasor sums: s_i, c_i the particle's own
+// phasor, om_i relative to the frame's reference
 template <int S>
-__device__ __forceinline__ PairAcc pair_acc(const DevParams &P, const PhasorSums &q, double psi_i, double om_i) {
+__device__ __forceinline__ PairAcc pair_acc(const DevParams &P, const PhasorSums &q, double s_i, double c_i,
+                                            double om_i) {
   PairAcc a{0.0, 0.0, 0.0};
   if (q.card == 0.0) return a;
-  double s_i, c_i;
-  sincos(psi_i, &s_i, &c_i);
-  const double sn = c_i * q.S - s_i * q.C, cs = c_i * q.C + s_i * q.S;  // sums of sin, cos (phi_j - phi_i)
+  // sums of sin, cos (phi_j - phi_i)
+  const double sn = cross(c_i, q.S, s_i, q.C), cs = __builtin_fma(c_i, q.C, s_i * q.S);
   a.align = sn * P.cos_a - cs * P.sin_a;
   a.card = q.card;
   if (S == 4 && P.higher_order) {
-    const double tsn = c_i * q.TS - s_i * q.TC, tcs = c_i * q.TC + s_i * q.TS;
+    const double tsn = cross(c_i, q.TS, s_i, q.TC), tcs = __builtin_fma(c_i, q.TC, s_i * q.TS);
     a.compl_f = (tcs - om_i * cs) * P.cos_a + (tsn - om_i * sn) * P.sin_a;
   }
   return a;
