@@ -67,8 +67,11 @@ struct spss_system {
   double *io[3] = {nullptr, nullptr, nullptr};
   CellBuffers cells, vcells;
   Cells64 cells64;
-  int *vcount = nullptr, *vstart = nullptr, *vlist = nullptr;
+  int *vcount = nullptr, *vstart = nullptr, *vlist = nullptr, *vslot = nullptr;
+  int *vhuge = nullptr;         // set by phases beyond the pair loop's range, cleared at a build
+  double *vstage = nullptr;     // stage state in the order of the lists' build
   long vcap = 0;
+  const int *vorder = nullptr;  // cell order of the lists' build (null: built over all pairs)
   int *pcount = nullptr, *pstart = nullptr, *plist = nullptr;
   int *scan_blk = nullptr;  // scratch of the scans over n counts (Verlet lists, pair export)
   long pcap = 0;
@@ -236,12 +239,14 @@ int build_verlet(spss_system *h, int m) {
     TRY(dalloc_n(&h->vcount, h->n + 1));
     TRY(dalloc_n(&h->vstart, h->n + 1));
   }
+  h->vorder = nullptr;
   if (m == SPSS_METHOD_VERLET) {
     launch_verlet_count_all(st, h->P, h->stage, rmax2, h->vcount);
   } else {
     TRY(ensure_cells(h, h->vcells, h->ncvx, h->ncvy));
     launch_cell_build(st, h->P, h->stage, h->ncvx, h->ncvy, h->vcells);
     launch_verlet_count_cells(st, h->P, h->stage, h->ncvx, h->ncvy, h->vcells, rmax2, h->vcount);
+    h->vorder = h->vcells.sorted;
   }
   TRY(ensure_scan(h));
   launch_scan(st, h->vcount, h->vstart, h->n, h->scan_blk);
@@ -252,13 +257,21 @@ int build_verlet(spss_system *h, int m) {
   if ((long)total > h->vcap) {
     hipFree(h->vlist);
     h->vlist = nullptr;
-    h->vcap = std::max<long>((long)total + total / 4, 1024);
-    TRY(dalloc_n(&h->vlist, (size_t)h->vcap));
+    hipFree(h->vslot);
+    h->vslot = nullptr;
+    h->vcap = 0;
+    const long cap = std::max<long>((long)total + total / 4, 1024);
+    TRY(dalloc_n(&h->vlist, (size_t)cap));
+    TRY(dalloc_n(&h->vslot, (size_t)cap));
+    h->vcap = cap;
   }
+  if (!h->vhuge) TRY(dalloc_n(&h->vhuge, 1));
+  if (!h->vstage) TRY(dalloc_n(&h->vstage, (size_t)h->s * h->n));
+  launch_fill_int(st, 1, h->vhuge, 0);
   if (m == SPSS_METHOD_VERLET)
-    launch_verlet_fill_all(st, h->P, h->stage, rmax2, h->vstart, h->vlist);
+    launch_verlet_fill_all(st, h->P, h->stage, rmax2, h->vstart, h->vlist, h->vslot);
   else
-    launch_verlet_fill_cells(st, h->P, h->stage, h->ncvx, h->ncvy, h->vcells, rmax2, h->vstart, h->vlist);
+    launch_verlet_fill_cells(st, h->P, h->stage, h->ncvx, h->ncvy, h->vcells, rmax2, h->vstart, h->vlist, h->vslot);
   return SPSS_OK;
 }
 
@@ -273,6 +286,7 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
   h->P.fresh_k = fresh ? 1 : 0;
   const double *nat = h->have_nat ? h->nat : nullptr;
   double *compl_out = h->higher_order ? h->compl_f : nullptr;
+  const bool verlet = m == SPSS_METHOD_VERLET || m == SPSS_METHOD_LINKED_LIST_VERLET;
   const bool tiled = m == SPSS_METHOD_LINKED_LIST && h->p.precision != SPSS_PRECISION_FP32C &&
                      cells64_serves(h->P, h->ncx, h->ncy);
   if (tiled) {
@@ -280,7 +294,7 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
     launch_cells64_build(st, h->P, d_state, d_kprev, k_coef * dt, h->ncx, h->cells64);
   } else if (m == SPSS_METHOD_ALL_PAIRS)
     launch_all_pairs_stage(st, h->P, d_state, d_kprev, k_coef * dt, h->stage, h->ap);
-  else
+  else if (!verlet || h->should_update)  // the Verlet pair sums stage in the order of their lists
     launch_stage(st, (long)h->s * h->n, d_state, d_kprev, k_coef * dt, h->stage);
   switch (m) {
     case SPSS_METHOD_GLOBAL_FIELD:
@@ -310,7 +324,8 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
         TRY(build_verlet(h, m));
         h->should_update = false;
       }
-      launch_verlet_pairs(st, h->P, h->stage, h->vstart, h->vlist, nat, d_knext, compl_out);
+      launch_stage_order(st, h->n, h->s, d_state, d_kprev, k_coef * dt, h->vorder, h->vstage, h->vhuge);
+      launch_verlet_pairs(st, h->P, h->vstage, h->vorder, h->vstart, h->vslot, h->vhuge, nat, d_knext, compl_out);
       h->uses_verlet = true;
       break;
     default:
@@ -620,7 +635,7 @@ int spss_destroy(spss_system *h) {
   delete h->timer;
   void *bufs[] = {h->state, h->stage, h->k[0], h->k[1], h->k[2], h->k[3], h->deriv, h->compl_f, h->nat,
                   h->noise, h->partial, h->scal, h->acc, h->io[0], h->io[1], h->io[2], h->vcount, h->vstart,
-                  h->vlist, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec};
+                  h->vlist, h->vslot, h->vstage, h->vhuge, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec};
   for (void *b : bufs) hipFree(b);
   for (double *b : h->dp) hipFree(b);
   if (h->dp_host) hipHostFree(h->dp_host);
@@ -1143,9 +1158,9 @@ int spss_neighbour_pairs(spss_system *h, int method, const double *host_stage, i
   if (m == SPSS_METHOD_LINKED_LIST && h->p.precision == SPSS_PRECISION_FP32C)
     TRY(fast_pairs_fill(h->fast, st, h->P, h->stage, h->pstart, h->plist));
   else if (m == SPSS_METHOD_LINKED_LIST)
-    launch_verlet_fill_cells(st, h->P, h->stage, h->ncx, h->ncy, h->cells, rho2, h->pstart, h->plist);
+    launch_verlet_fill_cells(st, h->P, h->stage, h->ncx, h->ncy, h->cells, rho2, h->pstart, h->plist, nullptr);
   else
-    launch_verlet_fill_all(st, h->P, h->stage, rho2, h->pstart, h->plist);
+    launch_verlet_fill_all(st, h->P, h->stage, rho2, h->pstart, h->plist, nullptr);
   std::vector<int> start(h->n + 1), js(total > 0 ? total : 1);
   HIPCHECK(hipMemcpyAsync(start.data(), h->pstart, sizeof(int) * (h->n + 1), hipMemcpyDeviceToHost, st));
   if (total > 0) HIPCHECK(hipMemcpyAsync(js.data(), h->plist, sizeof(int) * total, hipMemcpyDeviceToHost, st));

@@ -8,6 +8,7 @@
 
 #include "spss_device.hpp"
 #include "spss_launch.hpp"
+#include "spss_pairs64.hpp"
 #include "spss_scan.hpp"
 
 namespace spss {
@@ -120,85 +121,178 @@ __global__ __launch_bounds__(kBlock) void k_linked_list(DevParams P, const doubl
 // Verlet lists.  Build over all pairs (ParticleSystemFirstOrderPtr.cpp:497-543: x_i as stored)
 // or from the cell stencil (:643-743: x_i wrapped).  Two passes: counts, then lists written in
 // the reference's visiting order after a scan of the counts.
+//
+// Several lanes share a particle (LPP of a wave, a power of two): a list or a cell is read as
+// contiguous runs and thousands of particles fill the chip, where one thread per particle left it to
+// 79 workgroups at n = 20,011 (list build, both passes: 480 -> 53 us).
+
+// position of a lane among those of its group of LPP whose flag is set, and their number
+template <int LPP>
+__device__ __forceinline__ int group_rank(bool flag, int &total) {
+  const int lane = threadIdx.x & 63, g = lane & ~(LPP - 1);
+  unsigned long long m = __ballot(flag) >> g;
+  if (LPP < 64) m &= (1ull << (LPP & 63)) - 1;
+  total = __popcll(m);
+  return __popcll(m & ((1ull << (lane - g)) - 1));
+}
+
+// one run [b, e) of candidates of particle i (ids from `sorted`, or the run itself when null) by a
+// group of LPP lanes, in order; returns how many are within the list radius.  A list holds the ids,
+// and beside them the positions in `sorted`, by which the pair loop reads.  Every lane of the group
+// takes part in every round.
+template <int S, int LPP, bool FILL>
+__device__ __forceinline__ int list_run(const DevParams &P, const double *__restrict__ stage,
+                                        const int *__restrict__ sorted, double rmax2, int i, double x_i, double y_i,
+                                        int b, int e, int w, int *__restrict__ vlist, int *__restrict__ vslot) {
+  int found = 0;
+  for (int u0 = b; u0 < e; u0 += LPP) {
+    const int u = u0 + (threadIdx.x & (LPP - 1));
+    const int j = u < e ? (sorted ? sorted[u] : u) : i;
+    bool in = false;
+    if (j != i) {
+      double dx, dy;
+      class_c_unsigned(P, x_i, y_i, stage[(long)j * S], stage[(long)j * S + 1], dx, dy);
+      in = dx * dx + dy * dy <= rmax2;
+    }
+    int total;
+    const int r = group_rank<LPP>(in, total);
+    if (FILL && in) {
+      vlist[w + found + r] = j;
+      if (vslot) vslot[w + found + r] = u;
+    }
+    found += total;
+  }
+  return found;
+}
+
+constexpr int kBuildLanes = 16;
 
 template <int S, bool FILL>
-__global__ void k_verlet_build_all(DevParams P, const double *__restrict__ stage, double rmax2,
-                                   int *__restrict__ vcount, const int *__restrict__ vstart,
-                                   int *__restrict__ vlist) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(kBlock) void k_verlet_build_all(DevParams P, const double *__restrict__ stage,
+                                                             double rmax2, int *__restrict__ vcount,
+                                                             const int *__restrict__ vstart, int *__restrict__ vlist,
+                                                             int *__restrict__ vslot) {
+  constexpr int LPP = 64;  // a wave per particle: the runs are all n particles
+  const int i = (blockIdx.x * kBlock + threadIdx.x) / LPP;
   if (i >= P.n) return;
-  const double x_i = stage[(long)i * S], y_i = stage[(long)i * S + 1];
-  int c = 0;
-  int w = FILL ? vstart[i] : 0;
-  for (int j = 0; j < P.n; ++j) {
-    if (j == i) continue;
-    double dx, dy;
-    class_c_unsigned(P, x_i, y_i, stage[(long)j * S], stage[(long)j * S + 1], dx, dy);
-    double dr2 = dx * dx + dy * dy;
-    if (dr2 <= rmax2) {
-      if (FILL) vlist[w++] = j;
-      ++c;
-    }
-  }
-  if (!FILL) vcount[i] = c;
+  const int c = list_run<S, LPP, FILL>(P, stage, nullptr, rmax2, i, stage[(long)i * S], stage[(long)i * S + 1], 0, P.n,
+                                       FILL ? vstart[i] : 0, vlist, vslot);
+  if (!FILL && (threadIdx.x & (LPP - 1)) == 0) vcount[i] = c;
 }
 
 template <int S, bool FILL>
-__global__ void k_verlet_build_cells(DevParams P, const double *__restrict__ stage, int ncx, int ncy,
-                                     const int *__restrict__ start, const int *__restrict__ sorted, double rmax2,
-                                     int *__restrict__ vcount, const int *__restrict__ vstart,
-                                     int *__restrict__ vlist) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= P.n) return;
+__global__ __launch_bounds__(kBlock) void k_verlet_build_cells(DevParams P, const double *__restrict__ stage, int ncx,
+                                                               int ncy, const int *__restrict__ start,
+                                                               const int *__restrict__ sorted, double rmax2,
+                                                               int *__restrict__ vcount,
+                                                               const int *__restrict__ vstart,
+                                                               int *__restrict__ vlist, int *__restrict__ vslot) {
+  constexpr int LPP = kBuildLanes;
+  const int t = (blockIdx.x * kBlock + threadIdx.x) / LPP;
+  // the ballots of a wave need all of its lanes: groups past the end repeat the last particle
+  const int i = sorted[min(t, P.n - 1)];  // cell order: neighbouring groups read the same cells
   double x_i, y_i;
   key_wrap<S>(P, stage[(long)i * S], stage[(long)i * S + 1], x_i, y_i);
   const int cx = cell_coord(x_i, ncx), cy = cell_coord(y_i, ncy);
+  const int w = FILL ? vstart[i] : 0;
   int cnt = 0;
-  int w = FILL ? vstart[i] : 0;
   for (int dyc = -1; dyc <= 1; ++dyc) {
     const int jy = adjust_cell(cy + dyc, ncy);
     for (int dxc = -1; dxc <= 1; ++dxc) {
       const int c = jy * ncx + adjust_cell(cx + dxc, ncx);
-      const int e = start[c + 1];
-      for (int u = start[c]; u < e; ++u) {
-        const int j = sorted[u];
-        if (j == i) continue;
-        double dx, dy;
-        class_c_unsigned(P, x_i, y_i, stage[(long)j * S], stage[(long)j * S + 1], dx, dy);
-        double dr2 = dx * dx + dy * dy;
-        if (dr2 <= rmax2) {
-          if (FILL) vlist[w++] = j;
-          ++cnt;
-        }
-      }
+      cnt += list_run<S, LPP, FILL>(P, stage, sorted, rmax2, i, x_i, y_i, start[c], start[c + 1], w + cnt, vlist, vslot);
     }
   }
-  if (!FILL) vcount[i] = cnt;
+  if (!FILL && t < P.n && (threadIdx.x & (LPP - 1)) == 0) vcount[i] = cnt;
 }
 
-// Verlet pair loop, ParticleSystemFirstOrderPtr.cpp:553-613 (x_i as stored, list order)
+// stage state in the order of the lists' build (order null: as it is).  `huge` (cleared at the
+// build) is set by a finite phase beyond kPhase64.
 template <int S>
-__global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, const double *__restrict__ stage,
-                                                         const int *__restrict__ vstart, const int *__restrict__ vlist,
-                                                         const double *__restrict__ nat, double *__restrict__ k_next,
-                                                         double *__restrict__ compl_out) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= P.n) return;
-  double st[S];
+__global__ __launch_bounds__(kBlock) void k_stage_order(int n, const double *__restrict__ state,
+                                                        const double *__restrict__ kprev, double kc_dt,
+                                                        const int *__restrict__ order, double *__restrict__ vstage,
+                                                        int *__restrict__ huge) {
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t >= n) return;
+  const long i = order ? order[t] : t;
+  double v[S];
 #pragma unroll
-  for (int q = 0; q < S; ++q) st[q] = stage[(long)i * S + q];
-  const double phi_i = st[Slots<S>::phi];
-  const double omega_i = (S == 3) ? 0.0 : st[Slots<S>::omega];
-  PairAcc a{0.0, 0.0, 0.0};
-  const int e = vstart[i + 1];
-  for (int u = vstart[i]; u < e; ++u) {
-    const int j = vlist[u];
-    if (j == i) continue;
-    const double *sj = stage + (long)j * S;
-    pair_term<S>(P, st[0], st[1], phi_i, omega_i, sj[0], sj[1], sj[Slots<S>::phi],
-                 (S == 3) ? 0.0 : sj[Slots<S>::omega], a);
+  for (int q = 0; q < S; ++q) v[q] = state[i * S + q] + (kprev ? kc_dt * kprev[i * S + q] : 0.0);
+#pragma unroll
+  for (int q = 0; q < S; ++q) vstage[(long)t * S + q] = v[q];
+  const double phi = fabs(v[Slots<S>::phi]);
+  if (phi > kPhase64 && phi < __builtin_huge_val()) *huge = 1;
+}
+
+// the pair terms of ParticleSystemFirstOrderPtr.cpp:285-299 over every LPP-th entry of a list
+template <int S, int LPP, bool HO, bool HUGE>
+__device__ __forceinline__ void list_terms(const DevParams &P, const double *__restrict__ vstage,
+                                           const int *__restrict__ vslot, int u, int e, const double *st, PairAcc &a) {
+  if (u >= e) return;
+  // the next entry's state and the position of the one after it are read while this one is computed
+  int j = vslot[u], j1 = u + LPP < e ? vslot[u + LPP] : j;
+  double x = vstage[(long)j * S], y = vstage[(long)j * S + 1], phi = vstage[(long)j * S + 2];
+  for (; u < e; u += LPP) {
+    const int j2 = u + 2 * LPP < e ? vslot[u + 2 * LPP] : j1;
+    const double x1 = vstage[(long)j1 * S], y1 = vstage[(long)j1 * S + 1], phi1 = vstage[(long)j1 * S + 2];
+    if (pair_in_range<S>(P, st[0], st[1], x, y)) {
+      a.card += 1.0;
+      if (HO || HUGE) {
+        double sn, cs;
+        if (HUGE)
+          sincos(phi - st[2], &sn, &cs);
+        else
+          frame_phasor(phi, st[2], sn, cs);
+        a.align += sn * P.cos_a - cs * P.sin_a;
+        if (HO) a.compl_f += (vstage[(long)j * S + S - 1] - st[S - 1]) * (cs * P.cos_a + sn * P.sin_a);
+      } else {
+        double e1, e2;
+        const double d = two_diff(two_diff(phi, st[2], e1), P.alpha, e2);
+        a.align += small_sin(d, e1 + e2);
+      }
+    }
+    j = j1;
+    j1 = j2;
+    x = x1;
+    y = y1;
+    phi = phi1;
   }
-  write_k<S>(P, st, i, a, nat ? nat[i] : 0.0, k_next, compl_out);
+}
+
+// Verlet pair loop, ParticleSystemFirstOrderPtr.cpp:553-613 (x_i as stored): LPP lanes per particle
+// take every LPP-th entry of its list, their sums are added in a fixed tree.  The stage state lies in
+// the cell order of the lists' build, where the entries of a list are runs of neighbours: a group's
+// reads are a few lines instead of one line per entry.  ~60 instructions per entry bound it (n =
+// 20,011, ~400 entries of which 140 in range: 404 us with one thread per particle, 56 with 16
+// lanes, 41 with the states in list order, 35 with sin(d - alpha) by small_sin, 32 with the next
+// entry read ahead; 8 and 32 lanes: 39 and 31).
+template <int S, int LPP, bool HO>
+__global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, const double *__restrict__ vstage,
+                                                         const int *__restrict__ order,
+                                                         const int *__restrict__ vstart, const int *__restrict__ vslot,
+                                                         const int *__restrict__ huge, const double *__restrict__ nat,
+                                                         double *__restrict__ k_next, double *__restrict__ compl_out) {
+  const int t = (int)(((long)blockIdx.x * kBlock + threadIdx.x) / LPP), l = threadIdx.x & (LPP - 1);
+  const int i = t < P.n ? (order ? order[t] : t) : -1;
+  double st[S] = {};
+  PairAcc a{0.0, 0.0, 0.0};
+  if (i >= 0) {
+#pragma unroll
+    for (int q = 0; q < S; ++q) st[q] = vstage[(long)t * S + q];
+    const int b = vstart[i] + l, e = vstart[i + 1];
+    if (*huge)
+      list_terms<S, LPP, HO, true>(P, vstage, vslot, b, e, st, a);
+    else
+      list_terms<S, LPP, HO, false>(P, vstage, vslot, b, e, st, a);
+  }
+#pragma unroll
+  for (int off = LPP / 2; off > 0; off >>= 1) {
+    a.align += __shfl_down(a.align, off, LPP);
+    a.card += __shfl_down(a.card, off, LPP);
+    if (HO) a.compl_f += __shfl_down(a.compl_f, off, LPP);
+  }
+  if (i >= 0 && l == 0) write_k<S>(P, st, i, a, nat ? nat[i] : 0.0, k_next, compl_out);
 }
 
 // ---------------------------------------------------------------------------
@@ -626,23 +720,51 @@ void launch_scan(hipStream_t st, int *count, int *start, int m, int *blocksum) {
 }
 
 void launch_verlet_count_all(hipStream_t st, const DevParams &P, const double *stage, double rmax2, int *vcount) {
-  SPSS_DISPATCH_S(P.s, k_verlet_build_all<SS, false><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, stage, rmax2, vcount, nullptr, nullptr));
+  SPSS_DISPATCH_S(P.s, k_verlet_build_all<SS, false><<<dim3(nblk(64L * P.n)), dim3(kBlock), 0, st>>>(P, stage, rmax2, vcount, nullptr, nullptr, nullptr));
 }
 void launch_verlet_fill_all(hipStream_t st, const DevParams &P, const double *stage, double rmax2,
-                            const int *vstart, int *vlist) {
-  SPSS_DISPATCH_S(P.s, k_verlet_build_all<SS, true><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, stage, rmax2, nullptr, vstart, vlist));
+                            const int *vstart, int *vlist, int *vslot) {
+  SPSS_DISPATCH_S(P.s, k_verlet_build_all<SS, true><<<dim3(nblk(64L * P.n)), dim3(kBlock), 0, st>>>(P, stage, rmax2, nullptr, vstart, vlist, vslot));
 }
 void launch_verlet_count_cells(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy,
                                const CellBuffers &cb, double rmax2, int *vcount) {
-  SPSS_DISPATCH_S(P.s, k_verlet_build_cells<SS, false><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, stage, ncx, ncy, cb.start, cb.sorted, rmax2, vcount, nullptr, nullptr));
+  SPSS_DISPATCH_S(P.s, k_verlet_build_cells<SS, false><<<dim3(nblk((long)kBuildLanes * P.n)), dim3(kBlock), 0, st>>>(P, stage, ncx, ncy, cb.start, cb.sorted, rmax2, vcount, nullptr, nullptr, nullptr));
 }
 void launch_verlet_fill_cells(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy,
-                              const CellBuffers &cb, double rmax2, const int *vstart, int *vlist) {
-  SPSS_DISPATCH_S(P.s, k_verlet_build_cells<SS, true><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, stage, ncx, ncy, cb.start, cb.sorted, rmax2, nullptr, vstart, vlist));
+                              const CellBuffers &cb, double rmax2, const int *vstart, int *vlist, int *vslot) {
+  SPSS_DISPATCH_S(P.s, k_verlet_build_cells<SS, true><<<dim3(nblk((long)kBuildLanes * P.n)), dim3(kBlock), 0, st>>>(P, stage, ncx, ncy, cb.start, cb.sorted, rmax2, nullptr, vstart, vlist, vslot));
 }
-void launch_verlet_pairs(hipStream_t st, const DevParams &P, const double *stage, const int *vstart,
-                         const int *vlist, const double *nat, double *k_next, double *compl_out) {
-  SPSS_DISPATCH_S(P.s, k_verlet_pairs<SS><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, stage, vstart, vlist, nat, k_next, compl_out));
+void launch_stage_order(hipStream_t st, int n, int s, const double *state, const double *kprev, double kc_dt,
+                        const int *order, double *vstage, int *huge) {
+  if (s == 4)
+    k_stage_order<4><<<dim3(nblk(n)), dim3(kBlock), 0, st>>>(n, state, kprev, kc_dt, order, vstage, huge);
+  else
+    k_stage_order<3><<<dim3(nblk(n)), dim3(kBlock), 0, st>>>(n, state, kprev, kc_dt, order, vstage, huge);
+}
+
+template <int S, bool HO>
+static void verlet_pairs_as(hipStream_t st, const DevParams &P, const double *vstage, const int *order,
+                            const int *vstart, const int *vslot, const int *huge, const double *nat, double *k_next,
+                            double *compl_out) {
+  // 16 lanes read a list in contiguous 64-byte runs; fewer than 16,384 particles need a wave each to
+  // fill the chip
+  if (P.n < 16384)
+    k_verlet_pairs<S, 64, HO><<<dim3(nblk(64L * P.n)), dim3(kBlock), 0, st>>>(P, vstage, order, vstart, vslot, huge, nat,
+                                                                              k_next, compl_out);
+  else
+    k_verlet_pairs<S, 16, HO><<<dim3(nblk(16L * P.n)), dim3(kBlock), 0, st>>>(P, vstage, order, vstart, vslot, huge, nat,
+                                                                              k_next, compl_out);
+}
+
+void launch_verlet_pairs(hipStream_t st, const DevParams &P, const double *vstage, const int *order,
+                         const int *vstart, const int *vslot, const int *huge, const double *nat, double *k_next,
+                         double *compl_out) {
+  if (P.s == 3)
+    verlet_pairs_as<3, false>(st, P, vstage, order, vstart, vslot, huge, nat, k_next, compl_out);
+  else if (P.higher_order)
+    verlet_pairs_as<4, true>(st, P, vstage, order, vstart, vslot, huge, nat, k_next, compl_out);
+  else
+    verlet_pairs_as<4, false>(st, P, vstage, order, vstart, vslot, huge, nat, k_next, compl_out);
 }
 
 void launch_global(hipStream_t st, const DevParams &P, const double *stage, double *partial, double *fields,

@@ -137,15 +137,22 @@ void launch_iota(hipStream_t st, int n, int *p);
 // exclusive scan of count[0..m) into start[0..m]; count is left zeroed; blocksum: scratch of
 // scan_blocks(m) + 1 ints (spss_scan.hpp)
 void launch_scan(hipStream_t st, int *count, int *start, int m, int *blocksum);
+// Verlet lists: counts, then for every particle the ids of its entries (vlist) and their positions
+// in the candidates' order (vslot: in cb.sorted, or the ids again over all pairs; may be null)
 void launch_verlet_count_all(hipStream_t st, const DevParams &P, const double *stage, double rmax2, int *vcount);
 void launch_verlet_fill_all(hipStream_t st, const DevParams &P, const double *stage, double rmax2,
-                            const int *vstart, int *vlist);
+                            const int *vstart, int *vlist, int *vslot);
 void launch_verlet_count_cells(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy,
                                const CellBuffers &cb, double rmax2, int *vcount);
 void launch_verlet_fill_cells(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy,
-                              const CellBuffers &cb, double rmax2, const int *vstart, int *vlist);
-void launch_verlet_pairs(hipStream_t st, const DevParams &P, const double *stage, const int *vstart,
-                         const int *vlist, const double *nat, double *k_next, double *compl_out);
+                              const CellBuffers &cb, double rmax2, const int *vstart, int *vlist, int *vslot);
+// the stage state in the order of the lists' build (null: over all pairs) and the pair sums over it;
+// huge: set by phases that need the general sine, cleared by the caller at a build
+void launch_stage_order(hipStream_t st, int n, int s, const double *state, const double *kprev, double kc_dt,
+                        const int *order, double *vstage, int *huge);
+void launch_verlet_pairs(hipStream_t st, const DevParams &P, const double *vstage, const int *order,
+                         const int *vstart, const int *vslot, const int *huge, const double *nat, double *k_next,
+                         double *compl_out);
 void launch_global(hipStream_t st, const DevParams &P, const double *stage, double *partial, double *fields,
                    const double *nat, double *k_next, double *compl_out);
 void launch_rk4_combine(hipStream_t st, int s, int n, double *state, const double *k1, const double *k2,
