@@ -95,6 +95,8 @@ struct spss_system {
   AllPairsScratch ap;                // all-pairs records and partial sums
   int ap_config = kAllPairsDefault;  // all-pairs workgroup and j-tile sizes (spss_autotune_all_pairs)
   int xsplit = 1;                    // FP32C cell grid: columns per square cell (spss_set_cell_layout)
+  void *scratch = nullptr;  // of the observers (system_scratch)
+  size_t scratch_cap = 0;
   KernelTimer *timer = nullptr;  // around the pair kernel of the RHS
   // Dormand-Prince 5(4) buffers (allocated on first use): two states and derivatives, k2..k6,
   // a stage state and a pinned host copy for observers
@@ -635,7 +637,7 @@ int spss_destroy(spss_system *h) {
   delete h->timer;
   void *bufs[] = {h->state, h->stage, h->k[0], h->k[1], h->k[2], h->k[3], h->deriv, h->compl_f, h->nat,
                   h->noise, h->partial, h->scal, h->acc, h->io[0], h->io[1], h->io[2], h->vcount, h->vstart,
-                  h->vlist, h->vslot, h->vstage, h->vhuge, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec};
+                  h->vlist, h->vslot, h->vstage, h->vhuge, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec, h->scratch};
   for (void *b : bufs) hipFree(b);
   for (double *b : h->dp) hipFree(b);
   if (h->dp_host) hipHostFree(h->dp_host);
@@ -1208,6 +1210,19 @@ int system_view(spss_system *h, SystemView *v) {
   v->y_size = h->P.ys;
   v->x_rsize = h->P.xrs;
   v->y_rsize = h->P.yrs;
+  return SPSS_OK;
+}
+
+int system_scratch(spss_system *h, size_t bytes, void **p) {
+  if (bytes > h->scratch_cap) {
+    HIPCHECK(hipStreamSynchronize(h->stream));
+    hipFree(h->scratch);
+    h->scratch = nullptr;
+    h->scratch_cap = 0;
+    TRY(dalloc(&h->scratch, bytes));
+    h->scratch_cap = bytes;
+  }
+  *p = h->scratch;
   return SPSS_OK;
 }
 }  // namespace spss

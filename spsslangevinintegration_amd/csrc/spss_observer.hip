@@ -11,8 +11,9 @@
 // Summary (BinaryObserverFirstOrderPtr.cpp:126-146, BinaryObserverSecondOrderPtr.cpp:175-193):
 // Z = (1/n) sum_i ((float) cos phi_i + i (float) sin phi_i), accumulated in complex<float> in
 // particle order; the line "t \t |Z| \t arg Z" with the default stream formatting.  The phasors
-// are computed in parallel and summed in particle order by one lane, so the float sums are the
-// reference's; |Z| and arg Z are taken on the host with std::abs / std::arg of complex<float>.
+// are computed in parallel and summed with the rounding of every addition in particle order
+// (spss_seqsum.hpp), so the float sums are the reference's; |Z| and arg Z are taken on the host with
+// std::abs / std::arg of complex<float>.
 //
 // Restart (SimulationEngineFirstOrderPtr.cpp:70-94): the last complete frame of a file, found
 // from the file size, its floats widened to double.
@@ -26,6 +27,7 @@
 
 #include "../../include/spss_hip.h"
 #include "spss_launch.hpp"
+#include "spss_seqsum.hpp"
 
 using namespace spss;
 
@@ -50,25 +52,187 @@ __global__ void ob_frame(const double *__restrict__ state, long m, int s, int wr
   out[k] = v;
 }
 
-__global__ void ob_phasors(const double *__restrict__ state, int n, int s, int slot, float2 *__restrict__ ph) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double phi = state[(long)i * s + slot];
-  ph[i] = make_float2((float)cos(phi), (float)sin(phi));
+// cosines into ph, sines into ph + npad; zeros from n to npad
+__global__ void ob_phasors(const double *__restrict__ state, int n, long npad, int s, int slot,
+                           float *__restrict__ ph) {
+  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
+  if (i >= npad) return;
+  float re = 0.f, im = 0.f;
+  if (i < n) {
+    const double phi = state[i * s + slot];
+    re = (float)cos(phi);
+    im = (float)sin(phi);
+  }
+  ph[i] = re;
+  ph[npad + i] = im;
 }
 
-// the complex<float> accumulation of the reference, in particle order (one lane; every add
-// depends on the previous one)
-__global__ void ob_sequential_sum(const float2 *__restrict__ ph, int n, float *__restrict__ out) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  float re = 0.f, im = 0.f;
-  for (int i = 0; i < n; ++i) {
-    const float2 v = ph[i];
-    re = re + v.x;
-    im = im + v.y;
+// The complex<float> accumulation of the reference, in particle order (spss_seqsum.hpp).  One lane
+// adding term by term waited out a load per addition: 58.9 ms at n = 1,048,576.  Here ob_runs maps
+// runs of L terms for 64 exponents (a wave per run and component, an exponent per lane), ob_long_runs
+// composes 16 of them, and ob_walk goes through the long runs, into their runs where a long one
+// leaves its binade, and term by term where a run does (n = 1,048,576, random phases: about half of
+// the long runs, a tenth to a third of the runs).  106 + 11 us for the maps, 1.1-1.7 ms for the walk:
+// 4.5 cycles per addition left (370,000 at most of the million), 340 per map looked up.
+__global__ __launch_bounds__(256) void ob_runs(const float *__restrict__ ph, long npad, int L, int nruns,
+                                               SeqMap *__restrict__ runs) {
+  const int w = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int run = w >> 1, comp = w & 1;
+  if (run >= nruns) return;
+  const float scale = ldexpf(1.f, 23 - (lane + kSeqExp0));
+  const float limit = fminf(4194304.f, (float)(1 << 30) / (float)L);
+  const float *c = ph + comp * npad + (long)run * L;
+  SeqMap m = seq_identity();
+  for (int i0 = 0; i0 < L; i0 += 64) {
+    const float v = c[i0 + lane];
+    for (int k = 0; k < 64; ++k) {
+      const float t = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k));
+      seq_term(m, t * scale, limit);
+    }
   }
-  out[0] = re;
-  out[1] = im;
+  runs[((long)run * 2 + comp) * 64 + lane] = m;
+}
+
+__global__ __launch_bounds__(256) void ob_long_runs(const SeqMap *__restrict__ runs, int nruns, int nlong, int limit,
+                                                    SeqMap *__restrict__ longs) {
+  const long t = blockIdx.x * 256L + threadIdx.x;  // (long run, component, exponent)
+  if (t >= nlong * 128L) return;
+  const int q = (int)(t >> 7), rest = (int)(t & 127);
+  SeqMap m = seq_identity();
+  for (int r = q * kSeqLevel; r < min(nruns, (q + 1) * kSeqLevel); ++r) m = seq_compose(m, runs[r * 128L + rest], limit);
+  longs[t] = m;
+}
+
+// s through the map in lane k of m: true if it stayed in its binade
+__device__ __forceinline__ bool seq_pass(const SeqMap &m, int k, float &s) {
+  if (s == 0.f) {  // zeros alone leave it (k: the smallest exponent, which bounds every other term out)
+    const int lo = __builtin_amdgcn_readlane(m.lo[0], k), hi = __builtin_amdgcn_readlane(m.hi[0], k);
+    return __builtin_amdgcn_readlane(m.reach, k) <= 2 && lo == 0 && hi == 0;
+  }
+  const int S = seq_units(s), p = S & 1;
+  const int inc = __builtin_amdgcn_readlane(p ? m.inc[1] : m.inc[0], k);
+  const int lo = __builtin_amdgcn_readlane(p ? m.lo[1] : m.lo[0], k);
+  const int hi = __builtin_amdgcn_readlane(p ? m.hi[1] : m.hi[0], k);
+  const int reach = __builtin_amdgcn_readlane(m.reach, k);
+  if (!seq_stays(S, lo, hi, reach)) return false;
+  s = seq_value(S + inc, s);
+  return true;
+}
+
+__device__ __forceinline__ float wave_uniform(float s) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(s)));
+}
+
+// the exponent slot to look s up in (zero: the smallest), or -1
+__device__ __forceinline__ int seq_lookup(float s) { return s == 0.f ? 0 : seq_slot(s); }
+
+// what the walk needs of one long run: its maps (an exponent per lane), its 16 runs' maps for the
+// exponents k0, k0 + 1, k0 - 1, k0 - 2 (lane = run + 16 * exponent), and its terms if L == 256
+struct SeqGroup {
+  SeqMap lm, rm;
+  int k0;
+  float4 t[kSeqLevel];
+};
+
+// WHOLE: runs of 256 terms, whose long run fits the LDS
+template <bool WHOLE>
+struct SeqWalk {
+  const float4 *c;
+  const SeqMap *runs, *longs;
+  int L, nlong, comp, lane;
+
+  __device__ __forceinline__ void run_maps(SeqGroup &g, int q, int k0) const {
+    const int e = lane >> 4, k = k0 + (e == 0 ? 0 : (e == 1 ? 1 : 1 - e));
+    g.k0 = k0;
+    g.rm = runs[(q * kSeqLevel + (lane & 15)) * 128L + comp * 64 + max(0, min(63, k))];
+  }
+
+  // (past the end: the last one again)
+  __device__ __forceinline__ void load(SeqGroup &g, int q, float s) const {
+    q = min(q, nlong - 1);
+    g.lm = longs[q * 128L + comp * 64 + lane];
+    run_maps(g, q, max(0, seq_lookup(wave_uniform(s))));
+    if (WHOLE)
+#pragma unroll
+      for (int t = 0; t < kSeqLevel; ++t) g.t[t] = c[((long)q * kSeqLevel + t) * 64 + lane];
+  }
+
+  // s + the 256 terms at v, one by one: a quarter is read while the one before it is added
+  static __device__ __forceinline__ void add_terms(const float4 *v, float &s) {
+    float4 a[16], b[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) a[t] = v[t];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      if (h < 3)
+#pragma unroll
+        for (int t = 0; t < 16; ++t) b[t] = v[16 * (h + 1) + t];
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < 16; ++t) {
+        s = s + a[t].x;
+        s = s + a[t].y;
+        s = s + a[t].z;
+        s = s + a[t].w;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < 16; ++t) a[t] = b[t];
+    }
+  }
+
+  __device__ __forceinline__ void walk(SeqGroup &g, int q, float4 *terms, float &s) const {
+    if (q >= nlong) return;
+    s = wave_uniform(s);
+    const int kl = seq_lookup(s);
+    if (kl >= 0 && seq_pass(g.lm, kl, s)) return;
+    if (WHOLE) {
+#pragma unroll
+      for (int t = 0; t < kSeqLevel; ++t) terms[64 * t + lane] = g.t[t];
+      __syncthreads();
+    }
+    for (int r = 0; r < kSeqLevel; ++r) {
+      s = wave_uniform(s);
+      const int k = seq_lookup(s);
+      if (k >= 0) {
+        if (k - g.k0 > 1 || k - g.k0 < -2) run_maps(g, q, k);
+        const int d = k - g.k0;
+        if (seq_pass(g.rm, r + 16 * (d >= 0 ? d : 1 - d), s)) continue;
+      }
+      if (WHOLE) {
+        add_terms(terms + r * 64, s);
+        continue;
+      }
+      for (int i0 = 0; i0 < L; i0 += 256) {
+        __syncthreads();
+        terms[lane] = c[(((long)q * kSeqLevel + r) * L + i0) / 4 + lane];
+        __syncthreads();
+        add_terms(terms, s);
+      }
+    }
+    if (WHOLE) __syncthreads();
+  }
+};
+
+// One wave per component (blockIdx.x); the next long run is on its way while one is walked,
+// and the chain of additions is what is left to wait for.
+template <bool WHOLE>
+__global__ __launch_bounds__(64) void ob_walk(const float *__restrict__ ph, long npad, int L, int nlong,
+                                              const SeqMap *__restrict__ runs, const SeqMap *__restrict__ longs,
+                                              float *__restrict__ out) {
+  __shared__ float4 terms[WHOLE ? kSeqLevel * 64 : 64];
+  const int comp = blockIdx.x;
+  const SeqWalk<WHOLE> W{(const float4 *)(ph + comp * npad), runs, longs, L, nlong, comp, (int)threadIdx.x};
+  float s = 0.f;
+  SeqGroup a, b;
+  W.load(a, 0, s);
+  for (int q = 0; q < nlong; q += 2) {
+    W.load(b, q + 1, s);
+    W.walk(a, q, terms, s);
+    W.load(a, q + 2, s);
+    W.walk(b, q + 1, terms, s);
+  }
+  if (threadIdx.x == 0) out[comp] = s;
 }
 
 int check(hipError_t e, const char *what) {
@@ -88,7 +252,7 @@ int frame_to_host(spss_system *sys, double t, float *host) {
   if (rc != SPSS_OK) return rc;
   const long m = (long)v.s * v.n;
   float *d = nullptr;
-  OCHK(hipMalloc(&d, sizeof(float) * (m > 0 ? m : 1)));
+  if ((rc = system_scratch(sys, sizeof(float) * m, (void **)&d)) != SPSS_OK) return rc;
   const unsigned nb = (unsigned)((m + 255) / 256);
   if (m > 0)
     hipLaunchKernelGGL(ob_frame, dim3(nb), dim3(256), 0, v.stream, v.state, m, v.s, v.s == 6 ? 0 : 1, v.x_size,
@@ -96,7 +260,6 @@ int frame_to_host(spss_system *sys, double t, float *host) {
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && m > 0) e = hipMemcpyAsync(host + 1, d, sizeof(float) * m, hipMemcpyDeviceToHost, v.stream);
   if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-  hipFree(d);
   OCHK(e);
   host[0] = (float)t;
   return SPSS_OK;
@@ -108,20 +271,30 @@ int summary_sums(spss_system *sys, float *re, float *im, int *n_out) {
   if (rc != SPSS_OK) return rc;
   if (v.n < 1) return set_error(SPSS_ERR_INVALID, "no particles");
   const int slot = v.s == 6 ? 4 : 2;
-  float2 *ph = nullptr;
-  float *out = nullptr;
-  OCHK(hipMalloc(&ph, sizeof(float2) * v.n));
-  hipError_t e = hipMalloc(&out, 2 * sizeof(float));
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(ob_phasors, dim3((v.n + 255) / 256), dim3(256), 0, v.stream, v.state, v.n, v.s, slot, ph);
-    hipLaunchKernelGGL(ob_sequential_sum, dim3(1), dim3(64), 0, v.stream, ph, v.n, out);
-    e = hipGetLastError();
-  }
+  // runs of 256 terms, longer ones beyond 2^22 particles; whole long runs, filled up with zeros
+  int L = 256;
+  while (v.n / L >= 16384) L *= 2;
+  const int nlong = (int)((v.n + (long)L * kSeqLevel - 1) / ((long)L * kSeqLevel)), nruns = nlong * kSeqLevel;
+  const long npad = (long)nruns * L;
+  SeqMap *runs = nullptr;
+  const size_t maps = ((size_t)nruns + nlong) * 128;
+  if ((rc = system_scratch(sys, maps * sizeof(SeqMap) + sizeof(float) * (2 * npad + 2), (void **)&runs)) != SPSS_OK)
+    return rc;
+  SeqMap *longs = runs + (size_t)nruns * 128;
+  float *ph = (float *)(runs + maps);
+  float *out = ph + 2 * npad;
+  hipLaunchKernelGGL(ob_phasors, dim3((unsigned)(npad / 256)), dim3(256), 0, v.stream, v.state, v.n, npad, v.s, slot, ph);
+  hipLaunchKernelGGL(ob_runs, dim3(nruns / 2), dim3(256), 0, v.stream, ph, npad, L, nruns, runs);
+  hipLaunchKernelGGL(ob_long_runs, dim3((nlong * 128 + 255) / 256), dim3(256), 0, v.stream, runs, nruns, nlong,
+                     (1 << 30) / (L * kSeqLevel), longs);
+  if (L == 256)
+    hipLaunchKernelGGL(ob_walk<true>, dim3(2), dim3(64), 0, v.stream, ph, npad, L, nlong, runs, longs, out);
+  else
+    hipLaunchKernelGGL(ob_walk<false>, dim3(2), dim3(64), 0, v.stream, ph, npad, L, nlong, runs, longs, out);
+  hipError_t e = hipGetLastError();
   float h[2] = {0.f, 0.f};
   if (e == hipSuccess) e = hipMemcpyAsync(h, out, sizeof(h), hipMemcpyDeviceToHost, v.stream);
   if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
-  hipFree(ph);
-  hipFree(out);
   OCHK(e);
   *re = h[0];
   *im = h[1];
