@@ -12,6 +12,8 @@
 //   ml_bwd_weight dW = D^T A, db = sum over the batch of D
 //   ml_bwd_data   D_prev = (D W) * gelu'(Z_prev)
 //   ml_adam       the Adam update of every parameter
+// and for narrow networks (the screen's), all layers in one launch each:
+//   ml_rows       forward and backward of the rows, ml_grad: weight gradients and Adam, ml_predict
 // Parameters are one flat array, layer after layer: W_l [d_{l+1} x d_l] row-major, then b_l.
 #include <hip/hip_runtime.h>
 
@@ -33,6 +35,8 @@ namespace {
 constexpr int kMaxLayers = 8;
 constexpr int kMaxDim = 4096;
 constexpr int kLossCap = 1 << 16;
+constexpr long kPredictPiece = 32768;   // rows copied and launched together
+constexpr long kPredictCap = 1L << 20;  // rows on the device at a time: 4 MB per column
 
 int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
@@ -54,6 +58,11 @@ struct spss_mlp {
   long ndata = 0;
   float *loss = nullptr;  // [kLossCap] per-step losses of one train call
   long adam_t = 0;        // Adam steps taken
+  bool narrow = false;    // all layers in LDS, one launch for all of them (ml_rows, ml_grad, ml_predict)
+  Net net{};
+  float *dzl[kMaxLayers] = {};  // narrow: gradients w.r.t. every Z [max_batch x d_{l+1}]
+  float *px = nullptr, *py = nullptr;  // rows and outputs of one predict call (at most kPredictCap rows)
+  long prows = 0;
 };
 
 namespace {
@@ -71,8 +80,12 @@ void mlp_free(spss_mlp *m) {
     if (*b) hipFree(*b), *b = nullptr;
   for (int l = 0; l <= kMaxLayers; ++l)
     if (m->act[l]) hipFree(m->act[l]), m->act[l] = nullptr;
-  for (int l = 0; l < kMaxLayers; ++l)
+  for (int l = 0; l < kMaxLayers; ++l) {
     if (m->z[l]) hipFree(m->z[l]), m->z[l] = nullptr;
+    if (m->dzl[l]) hipFree(m->dzl[l]), m->dzl[l] = nullptr;
+  }
+  if (m->px) hipFree(m->px), m->px = nullptr;
+  if (m->py) hipFree(m->py), m->py = nullptr;
   if (m->st) hipStreamDestroy(m->st), m->st = nullptr;
 }
 
@@ -108,6 +121,23 @@ int backward(spss_mlp *m, const float *X, long x_off, long x_mod, const float *T
       cur ^= 1;
     }
   }
+  MCHK(hipGetLastError());
+  return SPSS_OK;
+}
+
+int narrow_grid(const spss_mlp *m) {
+  int t = 0;
+  for (int l = 0; l < m->L; ++l) t += narrow_tiles(m->dims[l], m->dims[l + 1]);
+  return t + 1;  // and the loss
+}
+
+// forward, backward and, with g null, the Adam update of one batch on the narrow path
+int narrow_step(spss_mlp *m, const float *X, const float *T, long off, long mod, int B, float *g, const AdamArgs &A,
+                float *loss_dev) {
+  const unsigned lds = narrow_floats(m->dims, m->L) * sizeof(float);
+  hipLaunchKernelGGL(ml_rows, dim3(cdiv(B, kTrainRows)), dim3(kRowsTB), lds, m->st, m->net, m->p, X, T, off, mod, B);
+  hipLaunchKernelGGL(ml_grad, dim3(narrow_grid(m)), dim3(kTB), 0, m->st, m->net, m->p, m->m1, m->m2, g, X, T, off, mod,
+                     B, A, loss_dev);
   MCHK(hipGetLastError());
   return SPSS_OK;
 }
@@ -169,6 +199,28 @@ int spss_mlp_create(spss_mlp **out, const int *dims, int ndims, int max_batch, u
     if (l + 1 < m->L && (e = hipMalloc(&m->act[l + 1], rows * dims[l + 1] * sizeof(float))) != hipSuccess)
       return fail(e, "hipMalloc");
   }
+  m->narrow = narrow_floats(m->dims, m->L) <= kNarrowParams && widest <= kNarrow;
+  if (m->narrow) {
+    for (int l = 0; l < m->L; ++l)
+      if ((e = hipMalloc(&m->dzl[l], rows * dims[l + 1] * sizeof(float))) != hipSuccess) return fail(e, "hipMalloc");
+    m->net.L = m->L;
+    for (int l = 0; l <= m->L; ++l) {
+      m->net.dims[l] = m->dims[l];
+      m->net.act[l] = m->act[l];
+    }
+    for (int l = 0; l < m->L; ++l) {
+      m->net.woff[l] = m->woff[l];
+      m->net.boff[l] = m->boff[l];
+      m->net.dz[l] = m->dzl[l];
+    }
+    m->net.y = m->z[m->L - 1];
+    if ((e = hipFuncSetAttribute((const void *)ml_rows, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 kNarrowParams * (int)sizeof(float))) != hipSuccess)
+      return fail(e, "hipFuncSetAttribute");
+    if ((e = hipFuncSetAttribute((const void *)ml_predict, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 kPredictFloats * (int)sizeof(float))) != hipSuccess)
+      return fail(e, "hipFuncSetAttribute");
+  }
   for (int k = 0; k < 2; ++k)
     if ((e = hipMalloc(&m->dz[k], rows * widest * sizeof(float))) != hipSuccess) return fail(e, "hipMalloc");
   if ((e = hipMalloc(&m->loss, kLossCap * sizeof(float))) != hipSuccess) return fail(e, "hipMalloc");
@@ -226,6 +278,32 @@ int spss_mlp_predict(spss_mlp *m, const float *x, long n, float *y) {
   if (!m || (n > 0 && (!x || !y))) return set_error(SPSS_ERR_INVALID, "NULL argument");
   if (n < 0) return set_error(SPSS_ERR_INVALID, "n must be >= 0");
   const int din = m->dims[0], dout = m->dims[m->L];
+  if (m->narrow) {
+    const long cap = std::min(n, kPredictCap);
+    if (cap > m->prows) {
+      if (m->px) hipFree(m->px), m->px = nullptr;
+      if (m->py) hipFree(m->py), m->py = nullptr;
+      m->prows = 0;
+      MCHK(hipMalloc(&m->px, (size_t)cap * din * sizeof(float)));
+      MCHK(hipMalloc(&m->py, (size_t)cap * dout * sizeof(float)));
+      m->prows = cap;
+    }
+    for (long c0 = 0; c0 < n; c0 += cap) {
+      const long c1 = std::min(n, c0 + cap);
+      // the rows go up in pieces, each piece's launch beside the next one's copy
+      for (long r0 = c0; r0 < c1; r0 += kPredictPiece) {
+        const int B = (int)std::min<long>(kPredictPiece, c1 - r0);
+        MCHK(hipMemcpyAsync(m->px + (r0 - c0) * din, x + r0 * din, (size_t)B * din * sizeof(float),
+                            hipMemcpyHostToDevice, m->st));
+        hipLaunchKernelGGL(ml_predict, dim3(cdiv(B, kPR)), dim3(kTB), kPredictFloats * sizeof(float), m->st, m->net, m->p,
+                           m->px + (r0 - c0) * din, B, m->py + (r0 - c0) * dout);
+        MCHK(hipGetLastError());
+      }
+      MCHK(hipMemcpyAsync(y + c0 * dout, m->py, (size_t)(c1 - c0) * dout * sizeof(float), hipMemcpyDeviceToHost, m->st));
+    }
+    MCHK(hipStreamSynchronize(m->st));
+    return SPSS_OK;
+  }
   for (long r0 = 0; r0 < n; r0 += m->max_batch) {
     const int B = (int)std::min<long>(m->max_batch, n - r0);
     MCHK(hipMemcpyAsync(m->xin, x + r0 * din, (size_t)B * din * sizeof(float), hipMemcpyHostToDevice, m->st));
@@ -245,8 +323,12 @@ int spss_mlp_gradients(spss_mlp *m, const float *x, const float *t, int batch, f
   const int din = m->dims[0], dout = m->dims[m->L];
   MCHK(hipMemcpyAsync(m->xin, x, (size_t)batch * din * sizeof(float), hipMemcpyHostToDevice, m->st));
   MCHK(hipMemcpyAsync(m->tin, t, (size_t)batch * dout * sizeof(float), hipMemcpyHostToDevice, m->st));
-  if ((rc = forward(m, m->xin, 0, batch, batch)) != SPSS_OK) return rc;
-  if ((rc = backward(m, m->xin, 0, batch, m->tin, batch, m->loss)) != SPSS_OK) return rc;
+  if (m->narrow) {
+    if ((rc = narrow_step(m, m->xin, m->tin, 0, batch, batch, m->g, AdamArgs{}, m->loss)) != SPSS_OK) return rc;
+  } else {
+    if ((rc = forward(m, m->xin, 0, batch, batch)) != SPSS_OK) return rc;
+    if ((rc = backward(m, m->xin, 0, batch, m->tin, batch, m->loss)) != SPSS_OK) return rc;
+  }
   MCHK(hipMemcpyAsync(grad, m->g, m->nparam * sizeof(float), hipMemcpyDeviceToHost, m->st));
   float l = 0.f;
   MCHK(hipMemcpyAsync(&l, m->loss, sizeof(float), hipMemcpyDeviceToHost, m->st));
@@ -285,13 +367,20 @@ int spss_mlp_train(spss_mlp *m, int nsteps, int batch, float lr, float beta1, fl
   for (int s = 0; s < nsteps; ++s) {
     // mini-batch: the next `batch` rows of the resident set, wrapping around
     const long off = (m->adam_t * (long)batch) % m->ndata;
+    const double t = (double)(m->adam_t + 1);
+    const double bc1 = 1.0 - std::pow((double)beta1, t), bc2 = 1.0 - std::pow((double)beta2, t);
+    const AdamArgs A{beta1, beta2, (float)(lr / bc1), (float)(1.0 / std::sqrt(bc2)), eps};
+    if (m->narrow) {
+      if ((rc = narrow_step(m, m->data_x, m->data_t, off, m->ndata, batch, nullptr, A, m->loss + s)) != SPSS_OK)
+        return rc;
+      ++m->adam_t;
+      continue;
+    }
     if ((rc = forward(m, m->data_x, off, m->ndata, batch)) != SPSS_OK) return rc;
     if ((rc = backward(m, m->data_x, off, m->ndata, m->data_t, batch, m->loss + s)) != SPSS_OK) return rc;
+    hipLaunchKernelGGL(ml_adam, dim3(adam_grid), dim3(kTB), 0, m->st, m->p, m->g, m->m1, m->m2, m->nparam, A.b1, A.b2,
+                       A.step_size, A.inv_sqrt_bc2, A.eps);
     ++m->adam_t;
-    const double bc1 = 1.0 - std::pow((double)beta1, (double)m->adam_t);
-    const double bc2 = 1.0 - std::pow((double)beta2, (double)m->adam_t);
-    hipLaunchKernelGGL(ml_adam, dim3(adam_grid), dim3(kTB), 0, m->st, m->p, m->g, m->m1, m->m2, m->nparam, beta1,
-                       beta2, (float)(lr / bc1), (float)(1.0 / std::sqrt(bc2)), eps);
   }
   MCHK(hipGetLastError());
   if (losses && nsteps > 0)

@@ -1,6 +1,6 @@
 // spss_mlp_kernels.hpp -- device code of the sweep-screen network (included by spss_mlp.hip).
 //
-// One launch per layer and direction, 256 threads, 32 x 32 output tiles; reductions are staged
+// Networks of any width: one launch per layer and direction, 256 threads, 32 x 32 output tiles; reductions are staged
 // through LDS in chunks of 64 and summed in ascending index order with FMAs, without atomics,
 // so that every result is reproducible bit for bit.  Matrices are row-major FP32.
 #pragma once
@@ -172,6 +172,388 @@ __global__ __launch_bounds__(kTB) void ml_adam(float *p, const float *g, float *
     m[e] = mm;
     v[e] = vv;
     p[e] -= step_size * mm / (sqrtf(vv) * inv_sqrt_bc2 + eps);
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Narrow networks (every width at most kNarrow, parameters within kNarrowParams): the whole
+// network stays in LDS, a launch covers all layers.  Every sum runs over the same terms in the
+// same order as in the kernels above, so the results are the same bits.
+
+constexpr int kNarrow = 128;
+constexpr int kMaxNet = 8;               // layers
+constexpr int kNarrowParams = 35840;     // floats of padded weights and biases in LDS (140 KB)
+
+struct Net {
+  int L;
+  int dims[kMaxNet + 1];
+  long woff[kMaxNet], boff[kMaxNet];
+  float *act[kMaxNet + 1];  // act[l], l >= 1: gelu(Z_{l-1}), batch x dims[l]
+  float *dz[kMaxNet];       // dL/dZ_l, batch x dims[l + 1]
+  float *y;                 // network output, batch x dims[L]
+};
+
+// LDS pitch of a row of W_l: 16-byte aligned, and a 16-byte read of 16 neighbouring rows falls into
+// all 64 banks where in is a multiple of 64
+__host__ __device__ inline int narrow_pitch(int in) { return ((in + 3) & ~3) + 4; }
+__host__ __device__ inline int narrow_floats(const int *dims, int L) {
+  int f = 0;
+  for (int l = 0; l < L; ++l) f += dims[l + 1] * narrow_pitch(dims[l]);
+  return f;
+}
+
+constexpr int kTrainRows = 2;  // rows per workgroup
+constexpr int kRowsTB = 512;   // its threads: as many for the load of the weights as for the rows
+
+// ring index of batch row b (off, b < mod)
+__device__ __forceinline__ long ring(long off, long b, long mod) {
+  const long r = off + b;
+  return r < mod ? r : r - mod;
+}
+
+// a barrier for what the workgroup exchanges through LDS: unlike __syncthreads it does not wait for
+// stores to memory to arrive (1-2 us after every layer)
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// sum over k < n of a[k] w[k], k ascending; a and w 16-byte aligned in LDS.  The reads of 64 terms are
+// issued before the first of them is added.
+__device__ __forceinline__ float dot_row(const float *a, const float *w, int n) {
+  float acc = 0.f;
+  int k = 0;
+  for (; k + 64 <= n; k += 64) {
+    float4 x[16], y[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) x[q] = ((const float4 *)(a + k))[q], y[q] = ((const float4 *)(w + k))[q];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+      acc = __builtin_fmaf(x[q].x, y[q].x, acc);
+      acc = __builtin_fmaf(x[q].y, y[q].y, acc);
+      acc = __builtin_fmaf(x[q].z, y[q].z, acc);
+      acc = __builtin_fmaf(x[q].w, y[q].w, acc);
+    }
+  }
+#pragma unroll 4
+  for (; k < n; ++k) acc = __builtin_fmaf(a[k], w[k], acc);
+  return acc;
+}
+
+// the same down a column of w (pitch step)
+__device__ __forceinline__ float dot_column(const float *a, const float *w, int step, int n) {
+  float acc = 0.f;
+  int k = 0;
+  for (; k + 32 <= n; k += 32) {
+    float4 x[8];
+    float y[32];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) x[q] = ((const float4 *)(a + k))[q];
+#pragma unroll
+    for (int q = 0; q < 32; ++q) y[q] = w[(k + q) * step];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      acc = __builtin_fmaf(x[q].x, y[4 * q], acc);
+      acc = __builtin_fmaf(x[q].y, y[4 * q + 1], acc);
+      acc = __builtin_fmaf(x[q].z, y[4 * q + 2], acc);
+      acc = __builtin_fmaf(x[q].w, y[4 * q + 3], acc);
+    }
+  }
+#pragma unroll 4
+  for (; k < n; ++k) acc = __builtin_fmaf(a[k], w[k * step], acc);
+  return acc;
+}
+
+// One pass of two rows through the network and back, a thread per row and unit: activations, output
+// and the gradients with respect to every Z.  A batch of 256 rows is 128 workgroups; at this size
+// nothing but the chains of FMAs (128 per layer), the load of the weights (137 KB per workgroup from
+// L2) and the launch is left.  Batch 256, 3 x 128 hidden: 14.4 us for what took eight launches
+// (forward 4 x 10.7, backward 3 x 8.4, loss 3.9 us).  What counted on the way: no wait for stores at
+// the barriers, 16-byte LDS reads, a thread per row and unit (a thread for both rows' unit, or loads
+// straight into LDS a word at a time: 24 us).
+__global__ __launch_bounds__(kRowsTB) void ml_rows(Net N, const float *__restrict__ p, const float *__restrict__ X,
+                                                   const float *__restrict__ T, long off, long mod, int B) {
+  extern __shared__ __align__(16) float sh[];
+  __shared__ float zs[kMaxNet][kTrainRows][kNarrow];         // Z of every layer
+  __shared__ __align__(16) float h[2][kTrainRows][kNarrow];  // the layer's input, then gradients
+  const int tid = threadIdx.x, b0 = blockIdx.x * kTrainRows;
+  const int L = N.L, d0 = N.dims[0], m = N.dims[L];
+  const int r = tid / kNarrow, u = tid % kNarrow;  // this thread's row and unit
+  const bool row = r < kTrainRows, there = row && b0 + r < B;
+  float bias[kMaxNet], t = 0.f, x = 0.f;
+#pragma unroll
+  for (int l = 0; l < kMaxNet; ++l) bias[l] = row && l < L && u < N.dims[l + 1] ? p[N.boff[l] + u] : 0.f;
+  if (there && u < d0) x = X[ring(off, b0 + r, mod) * d0 + u];
+  if (there && u < m) t = T[ring(off, b0 + r, mod) * m + u];
+  int at = 0;
+  for (int l = 0; l < L; ++l) {
+    const int in = N.dims[l], out = N.dims[l + 1], pitch = narrow_pitch(in);
+    const float *w = p + N.woff[l];
+    if (in % 4 == 0 && N.woff[l] % 4 == 0) {
+      const int q = in / 4, n4 = out * q;
+#pragma unroll 8
+      for (int e = tid; e < n4; e += kRowsTB) {
+        const int o = e / q;
+        *(float4 *)(sh + at + o * pitch + 4 * (e - o * q)) = ((const float4 *)w)[e];
+      }
+    } else {
+      for (int e = tid; e < out * in; e += kRowsTB) sh[at + (e / in) * pitch + e % in] = w[e];
+    }
+    at += out * pitch;
+  }
+  if (row && u < d0) h[0][r][u] = x;
+  lds_barrier();
+  at = 0;
+  int cur = 0;
+  for (int l = 0; l < L; ++l) {
+    const int in = N.dims[l], out = N.dims[l + 1], pitch = narrow_pitch(in);
+    if (row && u < out) {
+      float bl = 0.f;
+#pragma unroll
+      for (int k = 0; k < kMaxNet; ++k) bl = k == l ? bias[k] : bl;
+      const float z = dot_row(h[cur][r], sh + at + u * pitch, in) + bl;
+      zs[l][r][u] = z;
+      const float g = gelu(z);
+      h[cur ^ 1][r][u] = g;
+      if (there) {
+        if (l + 1 < L)
+          N.act[l + 1][(long)(b0 + r) * out + u] = g;
+        else
+          N.y[(long)(b0 + r) * out + u] = z;
+      }
+    }
+    lds_barrier();
+    at += out * pitch;
+    cur ^= 1;
+  }
+  // dL/dY of the mean squared error, then back through the layers
+  const float scale = 2.f / (float)(B * m);
+  if (row && u < m) {
+    const float g = scale * (zs[L - 1][r][u] - t);
+    h[0][r][u] = g;
+    if (there) N.dz[L - 1][(long)(b0 + r) * m + u] = g;
+  }
+  lds_barrier();
+  cur = 0;
+  for (int l = L - 1; l > 0; --l) {
+    const int in = N.dims[l], out = N.dims[l + 1], pitch = narrow_pitch(in);
+    at -= out * pitch;
+    if (row && u < in) {
+      const float g = dot_column(h[cur][r], sh + at + u, pitch, out) * gelu_grad(zs[l - 1][r][u]);
+      h[cur ^ 1][r][u] = g;
+      if (there) N.dz[l - 1][(long)(b0 + r) * in + u] = g;
+    }
+    lds_barrier();
+    cur ^= 1;
+  }
+}
+
+struct AdamArgs {
+  float b1, b2, step_size, inv_sqrt_bc2, eps;
+};
+
+constexpr int kGT = 16;    // edge of a gradient tile: one output per thread
+constexpr int kGB = 256;   // batch rows in LDS at a time
+
+__host__ __device__ inline int narrow_tiles(int in, int out) {
+  return ((out + kGT - 1) / kGT) * ((in + kGT) / kGT);  // in + 1 columns: the bias is the last
+}
+
+// dW_l = D_l^T A_l with the bias as an extra column, b ascending, for all layers in one launch (a
+// 16 x 16 tile per workgroup: ~160 of them for 3 x 128 hidden, where a layer's 16 tiles of 32 x 32
+// left most of the chip idle: 4 x 20.3 -> 6.6 us at batch 256), then the Adam update of the tile's
+// parameters (g: the gradients alone, no update).  The last workgroup takes the loss.
+__global__ __launch_bounds__(kTB) void ml_grad(Net N, float *__restrict__ p, float *__restrict__ m1,
+                                               float *__restrict__ m2, float *__restrict__ g,
+                                               const float *__restrict__ X, const float *__restrict__ T, long off,
+                                               long mod, int B, AdamArgs A, float *__restrict__ loss) {
+  __shared__ __align__(16) float sd[kGT][kGB + 4], sa[kGT][kGB + 4];
+  const int tid = threadIdx.x, tx = tid % kGT, ty = tid / kGT;
+  int t = blockIdx.x, l = 0;
+  while (l < N.L && t >= narrow_tiles(N.dims[l], N.dims[l + 1])) t -= narrow_tiles(N.dims[l], N.dims[l + 1]), ++l;
+  if (l == N.L) {  // the loss, in the order of ml_mse
+    __shared__ double red[kTB];
+    const int m = N.dims[N.L];
+    double s = 0.0;
+    for (int e = tid; e < B * m; e += kTB) {
+      const float d = N.y[e] - T[ring(off, e / m, mod) * m + e % m];
+      s += (double)d * (double)d;
+    }
+    red[tid] = s;
+    __syncthreads();
+    for (int k = kTB / 2; k > 0; k >>= 1) {
+      if (tid < k) red[tid] += red[tid + k];
+      __syncthreads();
+    }
+    if (tid == 0) *loss = (float)(red[0] / (double)(B * m));
+    return;
+  }
+  const int in = N.dims[l], out = N.dims[l + 1], across = (in + kGT) / kGT;
+  const int o0 = (t / across) * kGT, i0 = (t % across) * kGT;
+  const float *D = N.dz[l], *Al = l == 0 ? X : N.act[l];
+  const int o = o0 + ty, i = i0 + tx;
+  const bool mine = o < out && i <= in;
+  const long e = mine ? (i < in ? N.woff[l] + (long)o * in + i : N.boff[l] + o) : 0;
+  float pe = 0.f, m1e = 0.f, m2e = 0.f;  // on their way while the sums run
+  if (mine && !g) {
+    pe = p[e];
+    m1e = m1[e];
+    m2e = m2[e];
+  }
+  float acc = 0.f;
+  for (int bb = 0; bb < B; bb += kGB) {
+    const int kk = min(kGB, B - bb);
+    if (bb > 0) __syncthreads();
+    const int c = tid % kGT;
+    const bool dc = o0 + c < out, ac = i0 + c < in;
+    float vd[kGB / kGT], va[kGB / kGT];
+#pragma unroll
+    for (int q = 0; q < kGB / kGT; ++q) {
+      const int r = tid / kGT + q * kGT;
+      vd[q] = 0.f;
+      va[q] = i0 + c == in ? 1.f : 0.f;
+      if (r < kk && dc) vd[q] = D[(long)(bb + r) * out + o0 + c];
+      if (r < kk && ac) va[q] = Al[(l == 0 ? ring(off, bb + r, mod) : (long)(bb + r)) * in + i0 + c];
+    }
+#pragma unroll
+    for (int q = 0; q < kGB / kGT; ++q) {
+      sd[c][tid / kGT + q * kGT] = vd[q];
+      sa[c][tid / kGT + q * kGT] = va[q];
+    }
+    __syncthreads();
+    const float4 *d4 = (const float4 *)sd[ty], *a4 = (const float4 *)sa[tx];
+    int r = 0;
+#pragma unroll 4
+    for (; r + 4 <= kk; r += 4) {
+      const float4 d = d4[r / 4], a = a4[r / 4];
+      acc = __builtin_fmaf(d.x, a.x, acc);
+      acc = __builtin_fmaf(d.y, a.y, acc);
+      acc = __builtin_fmaf(d.z, a.z, acc);
+      acc = __builtin_fmaf(d.w, a.w, acc);
+    }
+    for (; r < kk; ++r) acc = __builtin_fmaf(sd[ty][r], sa[tx][r], acc);
+  }
+  if (!mine) return;
+  if (g) {
+    g[e] = acc;
+    return;
+  }
+  const float mm = __builtin_fmaf(A.b1, m1e, (1.f - A.b1) * acc);
+  const float vv = __builtin_fmaf(A.b2, m2e, (1.f - A.b2) * acc * acc);
+  m1[e] = mm;
+  m2[e] = vv;
+  p[e] = pe - A.step_size * mm / (sqrtf(vv) * A.inv_sqrt_bc2 + A.eps);
+}
+
+// Forward pass of 64 rows per workgroup through all layers: the rows' activations and half of a
+// layer's weights in LDS (70 KB: two workgroups per CU, so that one computes while the other waits
+// for weights), 8 rows x 4 outputs per thread, so that three 16-byte reads feed 32 FMAs.  A layer's
+// outputs replace its inputs once every thread has its sums.  100,000 rows of 3 x 128 hidden: 219 us
+// (31 TFLOP/s; half of it are the error functions of the GELUs) for what took 98 x 4 launches of
+// 10.3 us; with a layer's whole weights in LDS, one workgroup per CU, 344 us.
+constexpr int kPR = 64;           // rows
+constexpr int kPP = kPR + 4;      // pitch of the activations [width][rows]
+constexpr int kPW = kNarrow + 4;  // pitch of the weights [in][out]
+constexpr int kPK = 64;           // inputs whose weights are in LDS at a time
+constexpr int kPredictFloats = kNarrow * kPP + kPK * kPW;
+
+// W[0..out) [k0 .. k0 + 64) transposed into w, four rows of W per wave and step
+__device__ __forceinline__ void stage_weights(const float *__restrict__ wl, int in, int out, int k0, float *w) {
+  const int i = k0 + (threadIdx.x & 63);
+#pragma unroll 4
+  for (int o = (threadIdx.x >> 6) * 4; o < out; o += kTB / 16) {
+    if (i >= in) continue;
+    const float *r = wl + (long)o * in + i;
+    float4 v;
+    v.x = r[0];
+    v.y = o + 1 < out ? r[in] : 0.f;
+    v.z = o + 2 < out ? r[2 * in] : 0.f;
+    v.w = o + 3 < out ? r[3 * in] : 0.f;
+    *(float4 *)(w + (i - k0) * kPW + o) = v;
+  }
+}
+
+__global__ __launch_bounds__(kTB, 2) void ml_predict(Net N, const float *__restrict__ p, const float *__restrict__ X,
+                                                     int n, float *__restrict__ Y) {
+  extern __shared__ __align__(16) float sh[];
+  float *a = sh, *w = sh + kNarrow * kPP;
+  const int tid = threadIdx.x, b0 = blockIdx.x * kPR, R = min(kPR, n - b0);
+  const int og = tid & 31, rg = tid >> 5;
+  const int d0 = N.dims[0];
+  for (int e = tid; e < kPR * d0; e += kTB) {
+    const int r = e / d0, i = e - r * d0;
+    a[i * kPP + r] = r < R ? X[(long)(b0 + r) * d0 + i] : 0.f;
+  }
+  for (int l = 0; l < N.L; ++l) {
+    const int in = N.dims[l], out = N.dims[l + 1];
+    const float *wl = p + N.woff[l], *bias = p + N.boff[l];
+    const bool last = l + 1 == N.L;
+    if (out <= 8) {  // a thread per row and output
+      float z[2] = {};
+      for (int k0 = 0; k0 < in; k0 += kPK) {
+        const int k1 = min(in, k0 + kPK);
+        stage_weights(wl, in, out, k0, w);
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int e = tid + q * kTB, r = e % kPR, o = e / kPR;
+          if (o < out)
+#pragma unroll 8
+            for (int i = k0; i < k1; ++i) z[q] = __builtin_fmaf(a[i * kPP + r], w[(i - k0) * kPW + o], z[q]);
+        }
+        __syncthreads();
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int e = tid + q * kTB, r = e % kPR, o = e / kPR;
+        if (o >= out) continue;
+        const float v = z[q] + bias[o];
+        if (!last)
+          a[o * kPP + r] = gelu(v);
+        else if (r < R)
+          Y[(long)(b0 + r) * out + o] = v;
+      }
+    } else {
+      float acc[8][4] = {}, bo[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) bo[q] = og * 4 + q < out ? bias[og * 4 + q] : 0.f;
+      for (int k0 = 0; k0 < in; k0 += kPK) {
+        const int k1 = min(in, k0 + kPK);
+        stage_weights(wl, in, out, k0, w);
+        __syncthreads();
+        if (og * 4 < out) {
+#pragma unroll 2
+          for (int i = k0; i < k1; ++i) {
+            const float4 x0 = *(const float4 *)(a + i * kPP + rg * 8), x1 = *(const float4 *)(a + i * kPP + rg * 8 + 4);
+            const float4 v = *(const float4 *)(w + (i - k0) * kPW + og * 4);
+            const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+              acc[r][0] = __builtin_fmaf(x[r], v.x, acc[r][0]);
+              acc[r][1] = __builtin_fmaf(x[r], v.y, acc[r][1]);
+              acc[r][2] = __builtin_fmaf(x[r], v.z, acc[r][2]);
+              acc[r][3] = __builtin_fmaf(x[r], v.w, acc[r][3]);
+            }
+          }
+        }
+        __syncthreads();
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int o = og * 4 + q;
+        if (o >= out) continue;
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const float z = acc[r][q] + bo[q];
+          if (!last)
+            a[o * kPP + rg * 8 + r] = gelu(z);
+          else if (rg * 8 + r < R)
+            Y[(long)(b0 + rg * 8 + r) * out + o] = z;
+        }
+      }
+    }
+    __syncthreads();
   }
 }
 
