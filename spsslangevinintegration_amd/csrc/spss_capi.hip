@@ -296,11 +296,11 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
     launch_cells64_build(st, h->P, d_state, d_kprev, k_coef * dt, h->ncx, h->cells64);
   } else if (m == SPSS_METHOD_ALL_PAIRS)
     launch_all_pairs_stage(st, h->P, d_state, d_kprev, k_coef * dt, h->stage, h->ap);
-  else if (!verlet || h->should_update)  // the Verlet pair sums stage in the order of their lists
+  else if (m != SPSS_METHOD_GLOBAL_FIELD && (!verlet || h->should_update))  // the Verlet pair sums stage in the order of their lists
     launch_stage(st, (long)h->s * h->n, d_state, d_kprev, k_coef * dt, h->stage);
   switch (m) {
     case SPSS_METHOD_GLOBAL_FIELD:
-      launch_global(st, h->P, h->stage, h->partial, h->scal, nat, d_knext, compl_out);
+      launch_global(st, h->P, d_state, d_kprev, k_coef * dt, h->partial, nat, d_knext, compl_out);
       break;
     case SPSS_METHOD_ALL_PAIRS:
       launch_all_pairs(st, h->P, h->ap, h->stage, nat, d_knext, compl_out, h->ap_config);
@@ -386,7 +386,41 @@ int noise_source(spss_system *h, int mode, const double *noise, size_t count, in
   }
 }
 
+// the global field without the displacements that Verlet lists ask for: whole steps on the device
+bool use_global_steps(const spss_system *h, int method) {
+  return resolve_method(h, method) == SPSS_METHOD_GLOBAL_FIELD && !h->uses_verlet &&
+         check_method(h, SPSS_METHOD_GLOBAL_FIELD) == SPSS_OK;
+}
+
+int global_steps(spss_system *h, int stepper, long nsteps, double dt, int noise_mode, const double *noise) {
+  TRY(master_write(h, true));
+  const bool srk = stepper == SPSS_STEPPER_SRK;
+  const double *nat = h->have_nat ? h->nat : nullptr;
+  if (srk) h->higher_order = true;  // StochasticRungeKuttaStepperPtr.hpp:44
+  h->P.higher_order = h->higher_order ? 1 : 0;
+  h->P.fresh_k = stepper == SPSS_STEPPER_RK4 ? 0 : 1;
+  if (stepper == SPSS_STEPPER_RK4) {
+    launch_global_rk4(h->stream, h->P, nsteps, dt, h->state, h->stage, h->k, h->partial, nat, h->compl_f);
+  } else {
+    GfNoise Z;
+    TRY(noise_source(h, noise_mode, noise, (size_t)(srk ? 2 : 1) * h->n, &Z.mode, &Z.array));
+    Z.seed = h->p.seed;
+    Z.step = (uint64_t)h->step;
+    Z.sqrt_dt = std::sqrt(dt);
+    Z.amp = std::sqrt(2.0 * h->p.D_phi);
+    Z.c15 = 0.5 * std::pow(dt, 1.5);
+    Z.is3 = 1.0 / std::sqrt(3.0);
+    Z.friction = h->p.xi;
+    launch_global_stochastic(h->stream, h->P, srk, nsteps, dt, h->state, h->partial, nat, h->compl_f, Z);
+  }
+  HIPCHECK(hipGetLastError());
+  h->step += nsteps;
+  h->eager_steps += nsteps;
+  return SPSS_OK;
+}
+
 int rk4_step(spss_system *h, int method, double dt) {
+  if (use_global_steps(h, method)) return global_steps(h, SPSS_STEPPER_RK4, 1, dt, SPSS_NOISE_NONE, nullptr);
   TRY(master_write(h, true));
   TRY(rhs_device(h, method, h->state, h->k[0], h->k[0], 0.0, dt));
   TRY(rhs_device(h, method, h->state, h->k[0], h->k[1], 0.5, dt));
@@ -462,6 +496,8 @@ int verlet_fused_step(spss_system *h, int srk, double dt, int noise_mode, const 
 int euler_step(spss_system *h, int method, double dt, int noise_mode, const double *noise) {
   if (use_fused(h, method)) return fast_fused_step(h, 0, dt, noise_mode, noise);
   if (use_fused_verlet(h, method)) return verlet_fused_step(h, 0, dt, noise_mode, noise);
+  if (use_global_steps(h, method) && !h->higher_order)
+    return global_steps(h, SPSS_STEPPER_EULER, 1, dt, noise_mode, noise);
   TRY(master_write(h, true));
   // the derivative is zero-filled and serves as k_prev with coefficient 0 (:43-47): no stage change
   TRY(rhs_device(h, method, h->state, nullptr, h->deriv, 0.0, dt, true));
@@ -488,6 +524,7 @@ int srk_step(spss_system *h, int method, double dt, int noise_mode, const double
     h->higher_order = true;
     return verlet_fused_step(h, 1, dt, noise_mode, noise);
   }
+  if (use_global_steps(h, method)) return global_steps(h, SPSS_STEPPER_SRK, 1, dt, noise_mode, noise);
   TRY(master_write(h, true));
   h->higher_order = true;  // StochasticRungeKuttaStepperPtr.hpp:44
   TRY(rhs_device(h, method, h->state, nullptr, h->deriv, 0.0, dt, true));
@@ -596,7 +633,7 @@ int spss_create(const spss_params *p, spss_system **out) {
   step(dalloc_n(&h->compl_f, h->n));
   step(dalloc_n(&h->nat, h->n));
   step(dalloc_n(&h->noise, (size_t)3 * h->n));
-  step(dalloc_n(&h->partial, nb * 4 + 64));
+  step(dalloc_n(&h->partial, std::max((size_t)(nb * 4 + 64), gf_part_doubles(p->n))));
   step(dalloc_n(&h->scal, 64));
   // with the handle, so that an all-pairs evaluation allocates nothing (a caller may capture it)
   if (p->precision != SPSS_PRECISION_FP32C) step(ensure_all_pairs(h));
@@ -815,6 +852,9 @@ int spss_run(spss_system *h, int stepper, int method, long nsteps, double dt, in
     h->replayed_steps += g;
     k += g;
   }
+  if (k < nsteps && use_global_steps(h, method) &&
+      (stepper == SPSS_STEPPER_RK4 || (stepper == SPSS_STEPPER_EULER && !h->higher_order) || srk))
+    return global_steps(h, stepper, nsteps - k, dt, noise_mode, nullptr);
   for (; k < nsteps; ++k) {
     switch (stepper) {
       case SPSS_STEPPER_RK4: TRY(rk4_step(h, method, dt)); break;
@@ -1425,30 +1465,57 @@ int dp_try_step(DpRun &R, bool *ok) {
   double *const *k = h->dp;
   double *tmp = h->dp[DP_TMP];
   const double dt = R.dt;
-  launch_dp_combine(st, R.m, in, dp_terms({din}, {dt * A.a21}), tmp);
-  TRY(dp_rhs(R, tmp, k[DP_K2]));
-  launch_dp_combine(st, R.m, in, dp_terms({din, k[DP_K2]}, {dt * A.a31, dt * A.a32}), tmp);
-  TRY(dp_rhs(R, tmp, k[DP_K3]));
-  launch_dp_combine(st, R.m, in, dp_terms({din, k[DP_K2], k[DP_K3]}, {dt * A.a41, dt * A.a42, dt * A.a43}), tmp);
-  TRY(dp_rhs(R, tmp, k[DP_K4]));
-  launch_dp_combine(st, R.m, in,
-                    dp_terms({din, k[DP_K2], k[DP_K3], k[DP_K4]}, {dt * A.a51, dt * A.a52, dt * A.a53, dt * A.a54}),
-                    tmp);
-  TRY(dp_rhs(R, tmp, k[DP_K5]));
-  launch_dp_combine(st, R.m, in,
-                    dp_terms({din, k[DP_K2], k[DP_K3], k[DP_K4], k[DP_K5]},
-                             {dt * A.a61, dt * A.a62, dt * A.a63, dt * A.a64, dt * A.a65}),
-                    tmp);
-  TRY(dp_rhs(R, tmp, k[DP_K6]));
-  launch_dp_combine(st, R.m, in,
-                    dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6]},
-                             {dt * A.b1, dt * A.b3, dt * A.b4, dt * A.b5, dt * A.b6}),
-                    out);
-  TRY(dp_rhs(R, out, dout));
-  launch_dp_error(st, h->n, h->s, in, din,
-                  dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6], dout},
-                           {dt * A.d1, dt * A.d3, dt * A.d4, dt * A.d5, dt * A.d6, dt * A.d7}),
-                  dt, R.eps_abs, R.eps_rel, h->partial, h->scal + 24);
+  if (resolve_method(h, R.method) == SPSS_METHOD_GLOBAL_FIELD && !h->higher_order) {
+    // a launch per stage: the derivative and the next stage state with the sums of its field
+    const double *nat = h->have_nat ? h->nat : nullptr;
+    double *p0 = h->partial, *p1 = h->partial + gf_part_doubles(h->n) / 2;
+    h->P.higher_order = 0;
+    h->P.fresh_k = 0;
+    launch_global_first(st, h->P, in, din, dt * A.a21, tmp, p0);
+    launch_global_next(st, h->P, tmp, p0, nat, k[DP_K2], in, dp_terms({din}, {dt * A.a31, dt * A.a32}), tmp, p1);
+    launch_global_next(st, h->P, tmp, p1, nat, k[DP_K3], in,
+                       dp_terms({din, k[DP_K2]}, {dt * A.a41, dt * A.a42, dt * A.a43}), tmp, p0);
+    launch_global_next(st, h->P, tmp, p0, nat, k[DP_K4], in,
+                       dp_terms({din, k[DP_K2], k[DP_K3]}, {dt * A.a51, dt * A.a52, dt * A.a53, dt * A.a54}), tmp, p1);
+    launch_global_next(st, h->P, tmp, p1, nat, k[DP_K5], in,
+                       dp_terms({din, k[DP_K2], k[DP_K3], k[DP_K4]},
+                                {dt * A.a61, dt * A.a62, dt * A.a63, dt * A.a64, dt * A.a65}),
+                       tmp, p0);
+    launch_global_next(st, h->P, tmp, p0, nat, k[DP_K6], in,
+                       dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5]},
+                                {dt * A.b1, dt * A.b3, dt * A.b4, dt * A.b5, dt * A.b6}),
+                       out, p1);
+    const int nb = launch_global_error(st, h->P, out, p1, nat, dout, in,
+                                       dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6]},
+                                                {dt * A.d1, dt * A.d3, dt * A.d4, dt * A.d5, dt * A.d6, dt * A.d7}),
+                                       dt, R.eps_abs, R.eps_rel, p0);
+    launch_max_final(st, nb, p0, h->scal + 24);
+  } else {
+    launch_dp_combine(st, R.m, in, dp_terms({din}, {dt * A.a21}), tmp);
+    TRY(dp_rhs(R, tmp, k[DP_K2]));
+    launch_dp_combine(st, R.m, in, dp_terms({din, k[DP_K2]}, {dt * A.a31, dt * A.a32}), tmp);
+    TRY(dp_rhs(R, tmp, k[DP_K3]));
+    launch_dp_combine(st, R.m, in, dp_terms({din, k[DP_K2], k[DP_K3]}, {dt * A.a41, dt * A.a42, dt * A.a43}), tmp);
+    TRY(dp_rhs(R, tmp, k[DP_K4]));
+    launch_dp_combine(st, R.m, in,
+                      dp_terms({din, k[DP_K2], k[DP_K3], k[DP_K4]}, {dt * A.a51, dt * A.a52, dt * A.a53, dt * A.a54}),
+                      tmp);
+    TRY(dp_rhs(R, tmp, k[DP_K5]));
+    launch_dp_combine(st, R.m, in,
+                      dp_terms({din, k[DP_K2], k[DP_K3], k[DP_K4], k[DP_K5]},
+                               {dt * A.a61, dt * A.a62, dt * A.a63, dt * A.a64, dt * A.a65}),
+                      tmp);
+    TRY(dp_rhs(R, tmp, k[DP_K6]));
+    launch_dp_combine(st, R.m, in,
+                      dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6]},
+                               {dt * A.b1, dt * A.b3, dt * A.b4, dt * A.b5, dt * A.b6}),
+                      out);
+    TRY(dp_rhs(R, out, dout));
+    launch_dp_error(st, h->n, h->s, in, din,
+                    dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6], dout},
+                             {dt * A.d1, dt * A.d3, dt * A.d4, dt * A.d5, dt * A.d6, dt * A.d7}),
+                    dt, R.eps_abs, R.eps_rel, h->partial, h->scal + 24);
+  }
   HIPCHECK(hipGetLastError());
   double err = 0.0;
   HIPCHECK(hipMemcpyAsync(&err, h->scal + 24, sizeof(double), hipMemcpyDeviceToHost, st));
@@ -1568,10 +1635,12 @@ int dp_integrate_const(DpRun &R, double t0, double t1, double dt, DpObserver &ob
   double time = t0 + (double)obs_step * dt;
   while (less_eq_with_sign(time + dt, t1, dt)) {
     while (less_eq_with_sign(time, R.t, dt)) {
-      dp_calc_state(R, time, h->state);
+      const double next = t0 + (double)(obs_step + 1) * dt;
+      // without an observer nothing sees a state that the next one of the same step replaces
+      if (obs.fn || !less_eq_with_sign(next, R.t, dt)) dp_calc_state(R, time, h->state);
       TRY(obs.call(h, h->state, time));
       ++obs_step;
-      time = t0 + (double)obs_step * dt;
+      time = next;
     }
     if (less_with_sign(R.t + R.dt, t1, R.dt)) {  // not at the end yet: real steps past the next observation
       while (less_eq_with_sign(R.t, time, dt)) TRY(dp_do_step(R));

@@ -1,0 +1,778 @@
+// spss_global64.hip -- the FP64 global polar order field, ParticleSystemFirstOrderPtr.cpp:155-223:
+// right-hand side, the three steppers and the stages of the Dormand-Prince integrator on it.
+//
+// An evaluation needs Z = <e^{i phi}> (and W = <omega e^{i phi}> for the complementary force) of its
+// stage state before any particle's derivative.  So a launch takes the block sums that the launch
+// before it left, forms Z, evaluates its particles, and, since a stage state is known where its
+// derivative is, goes on to the next stage state and leaves that one's block sums: one launch per
+// stage, no stage pass, no launch for the reduction.  A small system stays in the registers of one
+// workgroup for whole steps.
+//
+// What bounds it: small systems the chain phasor - sums - derivative (n = 1,000: 1.1 us per stage; a
+// Runge-Kutta step took 55 us in 17 launches and takes 4.4), systems up to about 100,000 the latency of a
+// launch (4 us; a step of 16,384: 56 -> 17 us), large ones memory: a Dormand-Prince trial of 1,048,576 moves
+// 1.5 GB at 6.3 TB/s (470 -> 240 us), an Euler step 75 -> 25 us.
+//
+// |Z| sin(arg Z - phi) is Im(Z e^{-i phi}): no arc tangent, no second pair of sine and cosine.
+#pragma clang fp contract(off)
+
+#include "spss_launch.hpp"
+#include "spss_pairs64.hpp"
+
+namespace spss {
+
+namespace {
+
+constexpr int kMaxBlocks = 1024;  // every workgroup reads the sums of all of them
+
+__device__ __forceinline__ void two_sum(double a, double b, double &s, double &e) {
+  s = a + b;
+  const double bb = s - a;
+  e = (a - (s - bb)) + (b - bb);
+}
+
+__device__ __forceinline__ void phasor_of(double phi, double &sn, double &cs) {
+  if (fabs(phi) <= 0x1p30)
+    small_sincos(phi, 0.0, sn, cs);
+  else
+    sincos(phi, &sn, &cs);
+}
+
+// x of the lane that a DPP control names, 0 where there is none
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp(double x) {
+  union { double d; int w[2]; } u, v;
+  u.d = x;
+  v.w[0] = __builtin_amdgcn_update_dpp(0, u.w[0], CTRL, ROWS, 0xf, false);
+  v.w[1] = __builtin_amdgcn_update_dpp(0, u.w[1], CTRL, ROWS, 0xf, false);
+  return v.d;
+}
+
+// sum over a wave in a fixed tree of register moves (row shifts, then row broadcasts); in lane 63
+__device__ __forceinline__ double wave_sum63(double x) {
+  x += dpp<0x111, 0xf>(x);  // row_shr:1
+  x += dpp<0x112, 0xf>(x);
+  x += dpp<0x114, 0xf>(x);
+  x += dpp<0x118, 0xf>(x);
+  x += dpp<0x142, 0xa>(x);  // row_bcast:15
+  x += dpp<0x143, 0xc>(x);  // row_bcast:31
+  return x;
+}
+
+template <int CTRL>
+__device__ __forceinline__ void pair_level(double &s, double &c) {
+  const double s2 = dpp<CTRL, 0xf>(s), c2 = dpp<CTRL, 0xf>(c);
+  double t, e;
+  two_sum(s, s2, t, e);
+  s = t;
+  c = c + c2 + e;
+}
+
+// sum of the compensated pairs (s, c) of lanes 0..15, for every lane
+__device__ __forceinline__ double row_total(double s, double c) {
+  pair_level<0x111>(s, c);
+  pair_level<0x112>(s, c);
+  pair_level<0x114>(s, c);
+  pair_level<0x118>(s, c);
+  union { double d; int w[2]; } u;
+  u.d = s + c;
+  u.w[0] = __builtin_amdgcn_readlane(u.w[0], 15);
+  u.w[1] = __builtin_amdgcn_readlane(u.w[1], 15);
+  return u.d;
+}
+
+// the field as its users need it
+struct Field {
+  double zx, zy, wx, wy, absz, ux, uy;  // Z, W, |Z|, W / |W|
+};
+
+template <bool HO>
+__device__ __forceinline__ void finish_field(Field &f) {
+  if (!HO) return;
+  f.absz = hypot(f.zx, f.zy);
+  const double w = hypot(f.wx, f.wy);
+  f.ux = w > 0.0 ? f.wx / w : 1.0;  // arg(0) = 0
+  f.uy = w > 0.0 ? f.wy / w : 0.0;
+}
+
+// the derivative of one particle of state st and phasor (c, s), and the complementary force (with
+// arg(W) in its last sine, as the reference has it, :215-219)
+template <int S, bool HO>
+__device__ __forceinline__ void derivative(const DevParams &P, const Field &f, const double *st, double s, double c,
+                                           double nat_i, double *k, double &compl_f) {
+  const double A = f.zy * c - f.zx * s, B = f.zx * c + f.zy * s;  // |Z| sin, cos (arg Z - phi)
+  const double force = P.sigma * (A * P.cos_a - B * P.sin_a);
+  k[0] = P.v0 * c;
+  k[1] = P.v0 * s;
+  compl_f = 0.0;
+  if (S == 4) {
+    k[2] = st[3];
+    k[3] = -P.xi * st[3] + nat_i + force;
+    if (HO) {
+      const double wc = f.wx * c + f.wy * s, ws = f.wy * c - f.wx * s;
+      compl_f = P.sigma * ((wc * P.cos_a + ws * P.sin_a) -
+                           st[3] * (B * P.cos_a + f.absz * (f.uy * c - f.ux * s) * P.sin_a));
+    }
+  } else {
+    k[2] = nat_i + force;
+  }
+}
+
+// the sums a stage state adds to: cos, sin, omega cos, omega sin
+template <int S, bool HO>
+__device__ __forceinline__ void field_terms(const double *st, double *v) {
+  phasor_of(st[2], v[1], v[0]);
+  if (HO) {
+    v[2] = st[S - 1] * v[0];
+    v[3] = st[S - 1] * v[1];
+  }
+}
+
+// sums of one workgroup of 256 threads, a compensated pair per column, to out[column][2]
+template <int COLS>
+__device__ __forceinline__ void block_sums(const double *s, const double *c, double *__restrict__ out) {
+  __shared__ double sh[4][COLS][2];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+  for (int q = 0; q < COLS; ++q) {
+    const double ws = wave_sum63(s[q]), wc = wave_sum63(c[q]);
+    if (lane == 63) {
+      sh[wv][q][0] = ws;
+      sh[wv][q][1] = wc;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < COLS) {
+    double t = 0.0, e = 0.0;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      double r, d;
+      two_sum(t, sh[w][threadIdx.x][0], r, d);
+      t = r;
+      e += d + sh[w][threadIdx.x][1];
+    }
+    out[2 * threadIdx.x] = t;
+    out[2 * threadIdx.x + 1] = e;
+  }
+}
+
+// Z (and W) from the block sums of nb workgroups, by every workgroup for itself: a thread per block,
+// then the compensated pairs in fixed trees.  COLS pairs per block.
+template <bool HO>
+__device__ __forceinline__ void field_of(const double *__restrict__ part, int nb, double n, Field &f) {
+  constexpr int COLS = HO ? 4 : 2;
+  __shared__ double fs[16][COLS][2];
+  double s[COLS] = {}, c[COLS] = {};
+  for (int b = threadIdx.x; b < nb; b += 256)
+#pragma unroll
+    for (int q = 0; q < COLS; ++q) {
+      const double x = part[((long)b * COLS + q) * 2], y = part[((long)b * COLS + q) * 2 + 1];
+      double t, e;
+      two_sum(s[q], x, t, e);
+      s[q] = t;
+      c[q] += e + y;
+    }
+  // rows of 16 lanes first: lane 15 of each holds its pair
+  const int row = threadIdx.x >> 4;
+#pragma unroll
+  for (int q = 0; q < COLS; ++q) {
+    pair_level<0x111>(s[q], c[q]);
+    pair_level<0x112>(s[q], c[q]);
+    pair_level<0x114>(s[q], c[q]);
+    pair_level<0x118>(s[q], c[q]);
+    if ((threadIdx.x & 15) == 15) {
+      fs[row][q][0] = s[q];
+      fs[row][q][1] = c[q];
+    }
+  }
+  __syncthreads();
+  double v[COLS];
+#pragma unroll
+  for (int q = 0; q < COLS; ++q) v[q] = row_total(fs[threadIdx.x & 15][q][0], fs[threadIdx.x & 15][q][1]) / n;
+  f.zx = v[0];
+  f.zy = v[1];
+  if (HO) {
+    f.wx = v[COLS - 2];
+    f.wy = v[COLS - 1];
+  }
+  finish_field<HO>(f);
+}
+
+template <int S>
+__device__ __forceinline__ void load_row(const double *__restrict__ p, long i, double *v) {
+#pragma unroll
+  for (int q = 0; q < S; ++q) v[q] = p[i * S + q];
+}
+template <int S>
+__device__ __forceinline__ void store_row(double *__restrict__ p, long i, const double *v) {
+#pragma unroll
+  for (int q = 0; q < S; ++q) p[i * S + q] = v[q];
+}
+
+// what a thread adds up over its particles, with the rounding errors
+template <int COLS>
+__device__ __forceinline__ void add_terms(const double *w, double *s, double *c) {
+#pragma unroll
+  for (int q = 0; q < COLS; ++q) {
+    double t, e;
+    two_sum(s[q], w[q], t, e);
+    s[q] = t;
+    c[q] += e;
+  }
+}
+
+// the first stage: x + c0 * k0 (k0 may be null), stored if asked, and its block sums
+template <int S, bool HO, int PER>
+__global__ __launch_bounds__(256) void gf_first(int n, const double *__restrict__ x, const double *__restrict__ k0,
+                                                double c0, double *__restrict__ out, double *__restrict__ part) {
+  constexpr int COLS = HO ? 4 : 2, kPart = 256 * PER;
+  double s[COLS] = {}, c[COLS] = {};
+  for (long b = (long)blockIdx.x * kPart; b < n; b += (long)gridDim.x * kPart) {
+    double v[PER][S];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const long i = b + p * 256 + threadIdx.x;
+      if (i >= n) continue;
+      load_row<S>(x, i, v[p]);
+      if (k0) {
+        double k[S];
+        load_row<S>(k0, i, k);
+#pragma unroll
+        for (int q = 0; q < S; ++q) v[p][q] = v[p][q] + c0 * k[q];
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const long i = b + p * 256 + threadIdx.x;
+      if (i >= n) continue;
+      double w[COLS];
+      if (out) store_row<S>(out, i, v[p]);
+      field_terms<S, HO>(v[p], w);
+      add_terms<COLS>(w, s, c);
+    }
+  }
+  block_sums<COLS>(s, c, part + (long)blockIdx.x * COLS * 2);
+}
+
+// what follows the derivative k of a particle
+enum GfThen {
+  kThenNothing,  // a right-hand side
+  kThenNext,     // the next stage state base + sum_j c_j k_j + c_n k, and its block sums
+  kThenRk4,      // the step: state += (k1 + 2 k2 + 2 k3 + k) dt / 6, and its block sums
+  kThenEuler,    // the stochastic steps (StochasticEulerStepperPtr.hpp:40-73,
+  kThenSrk,      // StochasticRungeKuttaStepperPtr.hpp:50-76) and the block sums of the new state
+  kThenError     // the error norm of a Dormand-Prince trial: per block the largest relative error
+};
+
+struct GfStep {
+  const double *x = nullptr, *kprev = nullptr;  // stage state x + kc * kprev (kprev may be null)
+  double kc = 0.0;
+  const double *in = nullptr;  // its block sums
+  int nb = 0;                  // from that many workgroups
+  const double *nat = nullptr;
+  double *k = nullptr, *compl_out = nullptr;  // the derivative, the complementary force (may be null)
+  const double *base = nullptr;
+  DpTerms T{};        // terms of what follows; T.c[T.n] is the coefficient of k itself
+  double *next = nullptr, *out = nullptr;  // the state written and its block sums
+  GfNoise noise{};
+  double dt = 0.0, eps_abs = 0.0, eps_rel = 0.0;
+};
+
+__device__ __forceinline__ double gf_draw(const GfNoise &z, long idx, uint32_t particle, int which) {
+  if (z.mode == 1) return z.array[idx];
+  if (z.mode != 3) return 0.0;
+  double z0, z1;
+  philox_normal2(z.seed, particle, 0, z.step, z0, z1);
+  return which ? z1 : z0;
+}
+
+// the step of a stochastic stepper from the derivative f
+template <int S, bool SRK>
+__device__ __forceinline__ void stochastic_update(const GfNoise &z, double dt, int i, const double *f, double compl_f,
+                                                  double *st) {
+  if (!SRK) {
+    const double dW = z.sqrt_dt * gf_draw(z, i, i, 0);
+#pragma unroll
+    for (int q = 0; q < S - 1; ++q) st[q] += f[q] * dt;
+    st[S - 1] += f[S - 1] * dt + z.amp * dW;
+  } else {
+    double U1 = 0.0, U2 = 0.0;
+    if (z.mode == 1) {
+      U1 = z.array[2L * i];
+      U2 = z.array[2L * i + 1];
+    } else if (z.mode == 3) {
+      philox_normal2(z.seed, (uint32_t)i, 0, z.step, U1, U2);
+    }
+    const double dW = U1 * z.sqrt_dt, dZ = z.c15 * (U1 + z.is3 * U2);
+    const double t0 = f[0] * dt - 0.5 * f[2] * f[1] * dt * dt;
+    const double t1 = f[1] * dt + 0.5 * f[2] * f[0] * dt * dt;
+    const double t2 = f[2] * dt + 0.5 * f[S - 1] * dt * dt + z.amp * dZ;
+    const double t3 = f[S - 1] * dt + 0.5 * (compl_f - z.friction * f[S - 1]) * dt * dt + z.amp * (dW - z.friction * dZ);
+    st[0] += t0;
+    st[1] += t1;
+    st[2] += t2;
+    st[S - 1] += t3;
+  }
+}
+
+// NT: terms of T besides the derivative itself; PER: particles per thread and pass
+template <int S, bool HO, int THEN, int NT, int PER>
+__global__ __launch_bounds__(256) void gf_stage(DevParams P, GfStep G) {
+  constexpr int COLS = HO ? 4 : 2, kPart = 256 * PER;
+  constexpr bool kSums = THEN == kThenNext || THEN == kThenRk4 || THEN == kThenEuler || THEN == kThenSrk;
+  Field F{};
+  double s[COLS] = {}, c[COLS] = {}, worst = 0.0;
+  for (long b = (long)blockIdx.x * kPart; b < P.n; b += (long)gridDim.x * kPart) {
+    double st[PER][S];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const long i = b + p * 256 + threadIdx.x;
+      if (i >= P.n) continue;
+      load_row<S>(G.x, i, st[p]);
+      if (G.kprev) {
+        double kp[S];
+        load_row<S>(G.kprev, i, kp);
+#pragma unroll
+        for (int q = 0; q < S; ++q) st[p][q] = st[p][q] + G.kc * kp[q];
+      }
+    }
+    if (b == (long)blockIdx.x * kPart) field_of<HO>(G.in, G.nb, (double)P.n, F);  // over the first loads
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const long i = b + p * 256 + threadIdx.x;
+      if (i >= P.n) continue;
+      double v[S], d[NT ? NT : 1][S], k[S], cf;
+      if (THEN == kThenNext || THEN == kThenRk4 || THEN == kThenError) load_row<S>(G.base, i, v);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) load_row<S>(G.T.k[j], i, d[j]);
+      double sn, cs;
+      phasor_of(st[p][2], sn, cs);
+      derivative<S, HO>(P, F, st[p], sn, cs, G.nat ? G.nat[i] : 0.0, k, cf);
+      if (G.k) store_row<S>(G.k, i, k);
+      if (HO && G.compl_out) G.compl_out[i] = cf;
+      if (THEN == kThenNext) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j) v[q] = v[q] + G.T.c[j] * d[j][q];
+          v[q] = v[q] + G.T.c[NT] * k[q];
+        }
+      } else if (THEN == kThenRk4) {
+#pragma unroll
+        for (int q = 0; q < S; ++q)
+          v[q] += (d[0][q] + 2.0 * d[NT > 1 ? 1 : 0][q] + 2.0 * d[NT > 2 ? 2 : 0][q] + k[q]) * G.dt / 6.0;
+      } else if (THEN == kThenEuler || THEN == kThenSrk) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) v[q] = st[p][q];
+        stochastic_update<S, THEN == kThenSrk>(G.noise, G.dt, (int)i, k, cf, v);
+      } else if (THEN == kThenError) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+          double err = G.T.c[0] * d[0][q];
+#pragma unroll
+          for (int j = 1; j < NT; ++j) err = err + G.T.c[j] * d[j][q];
+          err = err + G.T.c[NT] * k[q];
+          worst = fmax(worst, fabs(err) / (G.eps_abs + G.eps_rel * (1.0 * fabs(v[q]) + (1.0 * G.dt) * fabs(d[0][q]))));
+        }
+      }
+      if (kSums) {
+        store_row<S>(G.next, i, v);
+        double w[COLS];
+        field_terms<S, HO>(v, w);
+        add_terms<COLS>(w, s, c);
+      }
+    }
+  }
+  if (kSums) block_sums<COLS>(s, c, G.out + (long)blockIdx.x * COLS * 2);
+  if (THEN == kThenError) {
+    __shared__ double red[256];
+    red[threadIdx.x] = worst;
+    __syncthreads();
+    for (int off = 128; off > 0; off >>= 1) {
+      if ((int)threadIdx.x < off) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + off]);
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) G.out[blockIdx.x] = red[0];
+  }
+}
+
+// a's upper half of the wave and b's lower half change places: a + b then holds a's half sums in the
+// lower half and b's in the upper one (ROW: the same for odd and even rows of 16 lanes)
+template <bool ROW>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  union { double d; unsigned w[2]; } u, v;
+  u.d = a;
+  v.d = b;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const auto r = ROW ? __builtin_amdgcn_permlane16_swap(u.w[q], v.w[q], false, false)
+                       : __builtin_amdgcn_permlane32_swap(u.w[q], v.w[q], false, false);
+    u.w[q] = r[0];
+    v.w[q] = r[1];
+  }
+  return u.d + v.d;
+}
+
+__device__ __forceinline__ double row_sum(double x) {  // lane 15 of each row
+  x += dpp<0x111, 0xf>(x);
+  x += dpp<0x112, 0xf>(x);
+  x += dpp<0x114, 0xf>(x);
+  x += dpp<0x118, 0xf>(x);
+  return x;
+}
+
+// Up to 256 * PPT particles: one workgroup, the particles in registers, nsteps steps.  The chain of a
+// stage is a phasor, the sums over the workgroup (register moves, one LDS exchange) and the
+// derivative.  The four waves have a SIMD each, and one wave of independent particles issues nearly
+// every cycle it is given, so the particles are split over registers before they are split over more
+// waves, whose reductions would only add instructions.
+enum GfStepper { kSmallRk4, kSmallEuler, kSmallSrk };
+
+template <int S, int STEPPER, int PPT>
+__global__ __launch_bounds__(256) void gf_small(DevParams P, int nsteps, double dt, double *__restrict__ state,
+                                                const double *__restrict__ nat, double *__restrict__ k1,
+                                                double *__restrict__ k2, double *__restrict__ k3,
+                                                double *__restrict__ k4, double *__restrict__ compl_out, GfNoise Z) {
+  constexpr bool HO = STEPPER == kSmallSrk;
+  constexpr int COLS = HO ? 4 : 2;
+  __shared__ double sh[2][COLS][4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  double y[PPT][S], st[PPT][S], w[PPT], sn[PPT], cs[PPT];
+#pragma unroll
+  for (int p = 0; p < PPT; ++p) {
+    const int i = p * 256 + threadIdx.x;
+    w[p] = i < P.n && nat ? nat[i] : 0.0;
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+      y[p][q] = st[p][q] = i < P.n ? state[(long)i * S + q] : 0.0;
+      // the first stage is the state + 0 * k1 (RungeKutta4StepperPtr.cpp:50), which a k1 that is not
+      // finite turns into NaN; after the first step such a k1 is in the state itself
+      if (STEPPER == kSmallRk4 && i < P.n) st[p][q] = y[p][q] + 0.0 * k1[(long)i * S + q];
+    }
+  }
+  int flip = 0;
+  const auto field = [&](Field &F) {
+    bool far = false;
+#pragma unroll
+    for (int p = 0; p < PPT; ++p) {
+      small_sincos(st[p][2], 0.0, sn[p], cs[p]);
+      far = far || !(fabs(st[p][2]) <= 0x1p30);
+    }
+    if (far) {
+#pragma unroll
+      for (int p = 0; p < PPT; ++p)
+        if (!(fabs(st[p][2]) <= 0x1p30)) sincos(st[p][2], &sn[p], &cs[p]);
+    }
+    double s[COLS] = {};
+#pragma unroll
+    for (int p = 0; p < PPT; ++p) {
+      const bool in = p * 256 + (int)threadIdx.x < P.n;
+      const double c1 = in ? cs[p] : 0.0, s1 = in ? sn[p] : 0.0;
+      s[0] += c1;
+      s[1] += s1;
+      if (HO) {
+        s[COLS - 2] += in ? st[p][S - 1] * c1 : 0.0;
+        s[COLS - 1] += in ? st[p][S - 1] * s1 : 0.0;
+      }
+    }
+    double t = swap_add<false>(s[0], s[1]);
+    if (HO) {
+      t = row_sum(swap_add<true>(t, swap_add<false>(s[COLS - 2], s[COLS - 1])));
+      if ((lane & 15) == 15) sh[flip][((lane >> 4) & 1) * 2 + (lane >> 5)][wv] = t;
+    } else {
+      t = row_sum(t);
+      t += dpp<0x142, 0xa>(t);  // row_bcast:15
+      if ((lane & 31) == 31) sh[flip][lane >> 5][wv] = t;
+    }
+    __syncthreads();
+    double v[COLS];
+#pragma unroll
+    for (int q = 0; q < COLS; ++q)
+      v[q] = ((sh[flip][q][0] + sh[flip][q][1]) + (sh[flip][q][2] + sh[flip][q][3])) / (double)P.n;
+    flip ^= 1;  // the other half is free: every wave had read it before this barrier
+    F.zx = v[0];
+    F.zy = v[1];
+    if (HO) {
+      F.wx = v[COLS - 2];
+      F.wy = v[COLS - 1];
+    }
+    finish_field<HO>(F);
+  };
+  for (int step = 0; step < nsteps; ++step) {
+    const bool last = step + 1 == nsteps;
+    Field F{};
+    if (STEPPER == kSmallRk4) {
+      double tot[PPT][S];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        field(F);
+        double *kb = g == 0 ? k1 : (g == 1 ? k2 : (g == 2 ? k3 : k4));
+#pragma unroll
+        for (int p = 0; p < PPT; ++p) {
+          const int i = p * 256 + threadIdx.x;
+          double k[S], cf;
+          derivative<S, false>(P, F, st[p], sn[p], cs[p], w[p], k, cf);
+          if (last && i < P.n) store_row<S>(kb, i, k);
+          const double kc = (g < 2 ? 0.5 : 1.0) * dt;
+#pragma unroll
+          for (int q = 0; q < S; ++q) {
+            tot[p][q] = g == 0 ? k[q] : (g < 3 ? tot[p][q] + 2.0 * k[q] : tot[p][q] + k[q]);
+            if (g < 3) st[p][q] = y[p][q] + kc * k[q];
+          }
+        }
+      }
+#pragma unroll
+      for (int p = 0; p < PPT; ++p)
+#pragma unroll
+        for (int q = 0; q < S; ++q) st[p][q] = y[p][q] = y[p][q] + tot[p][q] * dt / 6.0;
+    } else {
+      field(F);
+#pragma unroll
+      for (int p = 0; p < PPT; ++p) {
+        const int i = p * 256 + threadIdx.x;
+        if (i >= P.n) continue;
+        double k[S], cf;
+        derivative<S, HO>(P, F, st[p], sn[p], cs[p], w[p], k, cf);
+        if (HO && last) compl_out[i] = cf;
+        stochastic_update<S, HO>(Z, dt, i, k, cf, st[p]);
+      }
+      ++Z.step;
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < PPT; ++p) {
+    const int i = p * 256 + threadIdx.x;
+    if (i < P.n) store_row<S>(state, i, st[p]);
+  }
+}
+
+// One particle per thread shortens the chain of a launch, four at a time share the field and the
+// reductions.  A Runge-Kutta step (one, four): n = 4,096: 17, 24 us; 65,536: 21, 26 us; 262,144: 44, 35 us.
+inline bool gf_wide(int n) { return n > 131072; }
+inline int gf_blocks(int n) {
+  const int part = gf_wide(n) ? 1024 : 256;
+  const int nb = (n + part - 1) / part;
+  return nb < kMaxBlocks ? nb : kMaxBlocks;
+}
+
+template <int S, bool HO>
+void first(hipStream_t st, int n, const double *x, const double *k0, double c0, double *out, double *part) {
+  const auto run = [&](auto kernel) { kernel<<<dim3(gf_blocks(n)), dim3(256), 0, st>>>(n, x, k0, c0, out, part); };
+  gf_wide(n) ? run(gf_first<S, HO, 4>) : run(gf_first<S, HO, 1>);
+}
+
+template <int S, bool HO, int THEN, int NT>
+void stage(hipStream_t st, const DevParams &P, GfStep &G) {
+  G.nb = gf_blocks(P.n);
+  const auto run = [&](auto kernel) { kernel<<<dim3(G.nb), dim3(256), 0, st>>>(P, G); };
+  gf_wide(P.n) ? run(gf_stage<S, HO, THEN, NT, 4>) : run(gf_stage<S, HO, THEN, NT, 1>);
+}
+
+template <int S, bool HO>
+void rhs(hipStream_t st, const DevParams &P, const double *x, const double *kprev, double kc, double *part,
+         const double *nat, double *k, double *compl_out) {
+  first<S, HO>(st, P.n, x, kprev, kc, nullptr, part);
+  GfStep G{};
+  G.x = x;
+  G.kprev = kprev;
+  G.kc = kc;
+  G.in = part;
+  G.nat = nat;
+  G.k = k;
+  G.compl_out = compl_out;
+  stage<S, HO, kThenNothing, 0>(st, P, G);
+}
+
+template <int S, bool HO>
+void rk4(hipStream_t st, const DevParams &P, long nsteps, double dt, double *state, double *tmp, double *const *k,
+         double *part, const double *nat, double *compl_out) {
+  double *in = part, *out = part + gf_part_doubles(P.n) / 2;
+  first<S, HO>(st, P.n, state, k[0], 0.0, nullptr, in);  // state + 0 * k1, RungeKutta4StepperPtr.cpp:50
+  for (long s = 0; s < nsteps; ++s)
+    for (int g = 0; g < 4; ++g) {
+      GfStep G{};
+      G.x = g == 0 ? state : tmp;
+      G.kprev = s == 0 && g == 0 ? k[0] : nullptr;  // later a k1 that is not finite is in the state
+      G.in = in;
+      G.nat = nat;
+      G.k = g < 3 || s + 1 == nsteps ? k[g] : nullptr;
+      G.compl_out = compl_out;
+      G.base = state;
+      G.out = out;
+      G.dt = dt;
+      if (g < 3) {
+        G.T.c[0] = (g < 2 ? 0.5 : 1.0) * dt;
+        G.next = tmp;
+        stage<S, HO, kThenNext, 0>(st, P, G);
+      } else {
+        for (int q = 0; q < 3; ++q) G.T.k[q] = k[q];
+        G.next = state;
+        stage<S, HO, kThenRk4, 3>(st, P, G);
+      }
+      double *t = in;
+      in = out;
+      out = t;
+    }
+}
+
+template <int S, bool SRK>
+void stochastic(hipStream_t st, const DevParams &P, long nsteps, double dt, double *state, double *part,
+                const double *nat, double *compl_out, GfNoise Z) {
+  double *in = part, *out = part + gf_part_doubles(P.n) / 2;
+  first<S, SRK>(st, P.n, state, nullptr, 0.0, nullptr, in);
+  for (long s = 0; s < nsteps; ++s) {
+    GfStep G{};
+    G.x = state;
+    G.in = in;
+    G.nat = nat;
+    G.compl_out = s + 1 == nsteps ? compl_out : nullptr;
+    G.next = state;
+    G.out = out;
+    G.dt = dt;
+    G.noise = Z;
+    stage<S, SRK, SRK ? kThenSrk : kThenEuler, 0>(st, P, G);
+    ++Z.step;
+    double *t = in;
+    in = out;
+    out = t;
+  }
+}
+
+// Largest systems of one workgroup.  A step there, in launches: Runge-Kutta n = 2,048: 8.9, 17 us (twice
+// as many do not fit its registers); Euler n = 1,024: 3.5, 5.4 us, 2,048: 6.6, 5.4 us; stochastic
+// Runge-Kutta 4.3, 6.5 and 7.8, 6.5 us.
+constexpr int kSmallRk4N = 2048, kSmallStochasticN = 1024;
+constexpr int kSmallSteps = 1024;  // steps of one launch
+
+template <int S, int STEPPER>
+void small(hipStream_t st, const DevParams &P, long nsteps, double dt, double *state, const double *nat,
+           double *const *k, double *compl_out, GfNoise Z) {
+  for (long s = 0; s < nsteps; s += kSmallSteps) {
+    const int m = (int)(nsteps - s < kSmallSteps ? nsteps - s : kSmallSteps);
+    const auto run = [&](auto kernel) {
+      kernel<<<dim3(1), dim3(256), 0, st>>>(P, m, dt, state, nat, k[0], k[1], k[2], k[3], compl_out, Z);
+    };
+    if (P.n <= 256)
+      run(gf_small<S, STEPPER, 1>);
+    else if (P.n <= 512)
+      run(gf_small<S, STEPPER, 2>);
+    else if (P.n <= 1024)
+      run(gf_small<S, STEPPER, 4>);
+    else if constexpr (STEPPER == kSmallRk4)
+      run(gf_small<S, STEPPER, 8>);
+    Z.step += m;
+  }
+}
+
+}  // namespace
+
+size_t gf_part_doubles(int n) { return (size_t)2 * gf_blocks(n) * 8; }
+
+void launch_global(hipStream_t st, const DevParams &P, const double *x, const double *kprev, double kc, double *part,
+                   const double *nat, double *k_next, double *compl_out) {
+  if (P.s == 3)
+    rhs<3, false>(st, P, x, kprev, kc, part, nat, k_next, compl_out);
+  else if (P.higher_order)
+    rhs<4, true>(st, P, x, kprev, kc, part, nat, k_next, compl_out);
+  else
+    rhs<4, false>(st, P, x, kprev, kc, part, nat, k_next, compl_out);
+}
+
+void launch_global_rk4(hipStream_t st, const DevParams &P, long nsteps, double dt, double *state, double *tmp,
+                       double *const *k, double *part, const double *nat, double *compl_out) {
+  if (P.s == 3) {
+    if (P.n <= kSmallRk4N)
+      small<3, kSmallRk4>(st, P, nsteps, dt, state, nat, k, nullptr, GfNoise{});
+    else
+      rk4<3, false>(st, P, nsteps, dt, state, tmp, k, part, nat, nullptr);
+  } else if (P.higher_order) {
+    rk4<4, true>(st, P, nsteps, dt, state, tmp, k, part, nat, compl_out);
+  } else if (P.n <= kSmallRk4N) {
+    small<4, kSmallRk4>(st, P, nsteps, dt, state, nat, k, nullptr, GfNoise{});
+  } else {
+    rk4<4, false>(st, P, nsteps, dt, state, tmp, k, part, nat, nullptr);
+  }
+}
+
+void launch_global_stochastic(hipStream_t st, const DevParams &P, bool srk, long nsteps, double dt, double *state,
+                              double *part, const double *nat, double *compl_out, const GfNoise &Z) {
+  double *none[4] = {nullptr, nullptr, nullptr, nullptr};
+  const bool one = P.n <= kSmallStochasticN;
+  if (srk) {
+    if (one)
+      small<4, kSmallSrk>(st, P, nsteps, dt, state, nat, none, compl_out, Z);
+    else
+      stochastic<4, true>(st, P, nsteps, dt, state, part, nat, compl_out, Z);
+  } else if (P.s == 4) {
+    if (one)
+      small<4, kSmallEuler>(st, P, nsteps, dt, state, nat, none, nullptr, Z);
+    else
+      stochastic<4, false>(st, P, nsteps, dt, state, part, nat, nullptr, Z);
+  } else {
+    if (one)
+      small<3, kSmallEuler>(st, P, nsteps, dt, state, nat, none, nullptr, Z);
+    else
+      stochastic<3, false>(st, P, nsteps, dt, state, part, nat, nullptr, Z);
+  }
+}
+
+void launch_global_first(hipStream_t st, const DevParams &P, const double *x, const double *k0, double c0, double *out,
+                         double *part) {
+  if (P.s == 4)
+    first<4, false>(st, P.n, x, k0, c0, out, part);
+  else
+    first<3, false>(st, P.n, x, k0, c0, out, part);
+}
+
+namespace {
+template <int S, int THEN>
+void dp_stage(hipStream_t st, const DevParams &P, GfStep &G) {
+  switch (G.T.n) {
+    case 1: stage<S, false, THEN, 1>(st, P, G); break;
+    case 2: stage<S, false, THEN, 2>(st, P, G); break;
+    case 3: stage<S, false, THEN, 3>(st, P, G); break;
+    case 4: stage<S, false, THEN, 4>(st, P, G); break;
+    default: stage<S, false, THEN, 5>(st, P, G);
+  }
+}
+}  // namespace
+
+void launch_global_next(hipStream_t st, const DevParams &P, const double *x, const double *in, const double *nat,
+                        double *k, const double *base, const DpTerms &T, double *next, double *out) {
+  GfStep G{};
+  G.x = x;
+  G.in = in;
+  G.nat = nat;
+  G.k = k;
+  G.base = base;
+  G.T = T;
+  G.next = next;
+  G.out = out;
+  if (P.s == 4)
+    dp_stage<4, kThenNext>(st, P, G);
+  else
+    dp_stage<3, kThenNext>(st, P, G);
+}
+
+int launch_global_error(hipStream_t st, const DevParams &P, const double *x, const double *in, const double *nat,
+                        double *k, const double *x_old, const DpTerms &T, double dt, double eps_abs, double eps_rel,
+                        double *out) {
+  GfStep G{};
+  G.x = x;
+  G.in = in;
+  G.nat = nat;
+  G.k = k;
+  G.base = x_old;
+  G.T = T;
+  G.out = out;
+  G.dt = dt;
+  G.eps_abs = eps_abs;
+  G.eps_rel = eps_rel;
+  if (P.s == 4)
+    stage<4, false, kThenError, 5>(st, P, G);
+  else
+    stage<3, false, kThenError, 5>(st, P, G);
+  return gf_blocks(P.n);
+}
+
+}  // namespace spss

@@ -322,107 +322,6 @@ __device__ __forceinline__ double wave_combine(double s, double c) {
   return s + c;
 }
 
-struct Sum4 {
-  double v[4];
-  double c[4];
-};
-
-__global__ __launch_bounds__(kBlock) void k_polar_partial(int n, int s, int slot_phi, int slot_omega,
-                                                          const double *__restrict__ stage,
-                                                          double *__restrict__ partial) {
-  __shared__ double sh[4][kBlock];
-  int i = blockIdx.x * kBlock + threadIdx.x;
-  double v[4] = {0.0, 0.0, 0.0, 0.0};
-  if (i < n) {
-    double phi = stage[(long)i * s + slot_phi];
-    double c = cos(phi), sn = sin(phi);
-    v[0] = c;
-    v[1] = sn;
-    if (slot_omega >= 0) {
-      double om = stage[(long)i * s + slot_omega];
-      v[2] = om * c;
-      v[3] = om * sn;
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < 4; ++q) sh[q][threadIdx.x] = v[q];
-  __syncthreads();
-  for (int off = kBlock / 2; off > 0; off >>= 1) {
-    if (threadIdx.x < off) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) sh[q][threadIdx.x] += sh[q][threadIdx.x + off];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) partial[(long)blockIdx.x * 4 + q] = sh[q][0];
-  }
-}
-
-// the four block-partial columns summed with compensation (two_sum), one wave per column: each
-// lane takes every 64th block in block order, then the wave combines its 64 compensated pairs in
-// a fixed tree; the sums are divided by n (the field Z and W).  The order is fixed, so the result
-// does not vary between runs.
-__global__ __launch_bounds__(256) void k_polar_final(int nblocks, const double *__restrict__ partial,
-                                                     double *__restrict__ sums, double n) {
-  const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  double s = 0.0, c = 0.0;
-  // eight loads in flight per lane, then the sums in block order (the partials were written by
-  // other CUs: one load at a time would wait out that latency once per block)
-  for (int b0 = lane; b0 < nblocks; b0 += 64 * kFinalBatch) {
-    double x[kFinalBatch];
-#pragma unroll
-    for (int k = 0; k < kFinalBatch; ++k) {
-      const int b = b0 + 64 * k;
-      x[k] = b < nblocks ? partial[(long)b * 4 + q] : 0.0;
-    }
-#pragma unroll
-    for (int k = 0; k < kFinalBatch; ++k) {
-      if (b0 + 64 * k < nblocks) {
-        double t, e;
-        two_sum(s, x[k], t, e);
-        s = t;
-        c += e;
-      }
-    }
-  }
-  const double total = wave_combine(s, c);
-  if (lane == 0) sums[q] = total / n;
-}
-
-// k of the global branch; fields = (Re Z, Im Z, Re W, Im W) already divided by N
-template <int S>
-__global__ void k_global_rhs(DevParams P, const double *__restrict__ stage, const double *__restrict__ fields,
-                             const double *__restrict__ nat, double *__restrict__ k_next,
-                             double *__restrict__ compl_out) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= P.n) return;
-  const double absZ = hypot(fields[0], fields[1]), argZ = atan2(fields[1], fields[0]);
-  const long ii = (long)i * S;
-  const double phi_i = stage[ii + 2];
-  const double nat_i = nat ? nat[i] : 0.0;
-  if (S == 4) {
-    const double omega_i = stage[ii + 3];
-    k_next[ii] = P.v0 * cos(phi_i);
-    k_next[ii + 1] = P.v0 * sin(phi_i);
-    k_next[ii + 2] = omega_i;
-    k_next[ii + 3] =
-        -P.xi * omega_i + nat_i + P.sigma * absZ * (sin(argZ - phi_i) * P.cos_a - cos(argZ - phi_i) * P.sin_a);
-    if (P.higher_order) {
-      const double absW = hypot(fields[2], fields[3]), argW = atan2(fields[3], fields[2]);
-      // :215-219, with arg(W) in the last sine as the reference has it
-      compl_out[i] = P.sigma * (absW * (cos(argW - phi_i) * P.cos_a + sin(argW - phi_i) * P.sin_a) -
-                                omega_i * absZ * (cos(argZ - phi_i) * P.cos_a + sin(argW - phi_i) * P.sin_a));
-    }
-  } else {
-    k_next[ii] = P.v0 * cos(phi_i);
-    k_next[ii + 1] = P.v0 * sin(phi_i);
-    k_next[ii + 2] = nat_i + P.sigma * absZ * (sin(argZ - phi_i) * P.cos_a - cos(argZ - phi_i) * P.sin_a);
-  }
-}
-
-
 // ---------------------------------------------------------------------------
 // steppers.  Each writes the step's total displacement only as the per-block
 // max of dx^2 + dy^2 that CalculateMaxDisplacement needs (:841-850).
@@ -765,18 +664,6 @@ void launch_verlet_pairs(hipStream_t st, const DevParams &P, const double *vstag
     verlet_pairs_as<4, true>(st, P, vstage, order, vstart, vslot, huge, nat, k_next, compl_out);
   else
     verlet_pairs_as<4, false>(st, P, vstage, order, vstart, vslot, huge, nat, k_next, compl_out);
-}
-
-void launch_global(hipStream_t st, const DevParams &P, const double *stage, double *partial, double *fields,
-                   const double *nat, double *k_next, double *compl_out) {
-  const int s = P.s;
-  const int nb = (int)nblk(P.n);
-  k_polar_partial<<<dim3(nb), dim3(kBlock), 0, st>>>(P.n, s, Slots<4>::phi, (s == 4) ? 3 : -1, stage, partial);
-  k_polar_final<<<dim3(1), dim3(256), 0, st>>>(nb, partial, fields, (double)P.n);
-  if (s == 4)
-    k_global_rhs<4><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, stage, fields, nat, k_next, compl_out);
-  else
-    k_global_rhs<3><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, stage, fields, nat, k_next, compl_out);
 }
 
 void launch_rk4_combine(hipStream_t st, int s, int n, double *state, const double *k1, const double *k2,

@@ -155,8 +155,23 @@ void launch_stage_order(hipStream_t st, int n, int s, const double *state, const
 void launch_verlet_pairs(hipStream_t st, const DevParams &P, const double *vstage, const int *order,
                          const int *vstart, const int *vslot, const int *huge, const double *nat, double *k_next,
                          double *compl_out);
-void launch_global(hipStream_t st, const DevParams &P, const double *stage, double *partial, double *fields,
+// the global field (spss_global64.hip).  part: gf_part_doubles(n) doubles of scratch in two halves of
+// block sums; kprev may be null
+size_t gf_part_doubles(int n);
+void launch_global(hipStream_t st, const DevParams &P, const double *x, const double *kprev, double kc, double *part,
                    const double *nat, double *k_next, double *compl_out);
+// nsteps of the Runge-Kutta stepper; k: k1..k4 (left with those of the last step), tmp: a stage state
+void launch_global_rk4(hipStream_t st, const DevParams &P, long nsteps, double dt, double *state, double *tmp,
+                       double *const *k, double *part, const double *nat, double *compl_out);
+struct GfNoise {
+  int mode = 0;  // 0 none, 1 array, 3 Philox
+  const double *array = nullptr;
+  uint64_t seed = 0, step = 0;
+  double sqrt_dt = 0.0, amp = 0.0, c15 = 0.0, is3 = 0.0, friction = 0.0;
+};
+// nsteps of the stochastic Euler (not with the complementary force) or Runge-Kutta stepper
+void launch_global_stochastic(hipStream_t st, const DevParams &P, bool srk, long nsteps, double dt, double *state,
+                              double *part, const double *nat, double *compl_out, const GfNoise &Z);
 void launch_rk4_combine(hipStream_t st, int s, int n, double *state, const double *k1, const double *k2,
                         const double *k3, const double *k4, double dt, double *max_partial);
 void launch_euler(hipStream_t st, int s, int n, double *state, const double *f, double dt, double sqrt_dt,
@@ -180,6 +195,17 @@ void launch_dp_combine(hipStream_t st, long m, const double *x, const DpTerms &T
 // into out[0] (partial: one double per 256 particles); returns the number of partials
 int launch_dp_error(hipStream_t st, int n, int s, const double *x_old, const double *dxdt_old, const DpTerms &T,
                     double dt, double eps_abs, double eps_rel, double *partial, double *out);
+// the same over the global field, from one launch to the next: a stage state out = x + c0 k0 with its
+// block sums; the derivative k at x from the block sums `in` with next = base + sum_j c_j k_j + c k (T.n
+// pointers, T.n + 1 coefficients) and its block sums; the last derivative with the
+// error norm's block maxima (their number is returned)
+void launch_global_first(hipStream_t st, const DevParams &P, const double *x, const double *k0, double c0, double *out,
+                         double *part);
+void launch_global_next(hipStream_t st, const DevParams &P, const double *x, const double *in, const double *nat,
+                        double *k, const double *base, const DpTerms &T, double *next, double *out);
+int launch_global_error(hipStream_t st, const DevParams &P, const double *x, const double *in, const double *nat,
+                        double *k, const double *x_old, const DpTerms &T, double dt, double eps_abs, double eps_rel,
+                        double *out);
 void launch_disp_max(hipStream_t st, int n, int s, const double *tot, double *partial);
 void launch_order_parameter(hipStream_t st, int n, int s, int slot, const double *state, double *partial,
                             double *out);
