@@ -1133,7 +1133,7 @@ int spss_get_verlet_lists(spss_system *h, int *counts, int *flat, long cap, long
   if (!h || !counts || !total) return fail(SPSS_ERR_INVALID, "NULL argument");
   if (h->vfast && h->resident_kind == 2) {  // FP32C: the lists of the last rebuild, by particle id
     std::vector<int> c, f;
-    int rc = vf_lists(h->vfast, h->stream, &c, &f);
+    int rc = vf_lists(h->vfast, h->stream, h->P, &c, &f);
     if (rc != SPSS_OK) return fail(rc, vf_last_error());
     std::copy(c.begin(), c.end(), counts);
     *total = (long)f.size();

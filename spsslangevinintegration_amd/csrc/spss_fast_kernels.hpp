@@ -150,7 +150,7 @@ __device__ __forceinline__ float4 snap_entry(const DevParams &P, const double *s
   double xw, yw;
   apply_pbc(P, st[0], st[1], xw, yw);
   double sn, cn;
-  sincos(st[2], &sn, &cn);
+  phasor_of(st[2], sn, cn);
   return make_float4((float)(xw - (double)cx * Hx), (float)(yw - (double)cy * Hy), (float)cn, (float)sn);
 }
 
@@ -196,7 +196,7 @@ __device__ __forceinline__ void finish_particle(const DevParams &P, const PairBu
   // e^{-i theta}, theta = phi_i + alpha, from the FP64 phase
   double sn = 0.0, cn = 0.0, A64 = 0.0, C64 = 0.0;
   if (MODE == 0) {
-    sincos(pi[2], &sn, &cn);
+    phasor_of(pi[2], sn, cn);
     const double st = sn * P.cos_a + cn * P.sin_a;
     const double ct = cn * P.cos_a - sn * P.sin_a;
     A64 = ct * sy - st * sx;
@@ -748,7 +748,7 @@ __global__ __launch_bounds__(256) void fr_move(DevParams P, Layout L, int n, int
   const double *pi = valid ? rstate + (long)p * S : rstate;
   double sn = 0.0, cn = 1.0, xw = 0.0, yw = 0.0;
   if (valid) {
-    sincos(pi[2], &sn, &cn);
+    phasor_of(pi[2], sn, cn);
     apply_pbc(P, pi[0], pi[1], xw, yw);
   }
   move_and_count<S, SRK>(P, L, ncx, ncy, pi, sn, cn, xw, yw, U, p, valid, mv, farcnt, farslot, cnt9, newcnt,
@@ -1028,7 +1028,7 @@ __global__ __launch_bounds__(256) void fr_scatter(
       if (rnat) nnat[pos] = nat_i;
       // the snapshot (as snap_entry), keeping the phase's sine and cosine and the wrapped
       // position for the next move
-      sincos(out[2], &sn2, &cn2);
+      phasor_of(out[2], sn2, cn2);
       apply_pbc(P, out[0], out[1], xw2, yw2);
       const int ld = cd - base;
       snap[pos] = make_float4((float)(xw2 - (double)(ld % ncx) * Hx), (float)(yw2 - (double)(ld / ncx) * Hy),

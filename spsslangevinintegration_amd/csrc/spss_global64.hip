@@ -31,13 +31,6 @@ __device__ __forceinline__ void two_sum(double a, double b, double &s, double &e
   e = (a - (s - bb)) + (b - bb);
 }
 
-__device__ __forceinline__ void phasor_of(double phi, double &sn, double &cs) {
-  if (fabs(phi) <= 0x1p30)
-    small_sincos(phi, 0.0, sn, cs);
-  else
-    sincos(phi, &sn, &cs);
-}
-
 // x of the lane that a DPP control names, 0 where there is none
 template <int CTRL, int ROWS>
 __device__ __forceinline__ double dpp(double x) {

@@ -59,6 +59,14 @@ __device__ __forceinline__ void small_sincos(double x, double e, double &sn, dou
   cs = ((n + 1) & 2) ? -b : b;
 }
 
+// sin and cos of any phase
+__device__ __forceinline__ void phasor_of(double phi, double &sn, double &cs) {
+  if (fabs(phi) <= 0x1p30)
+    small_sincos(phi, 0.0, sn, cs);
+  else
+    sincos(phi, &sn, &cs);
+}
+
 // sin(x + e) the same way, reduced to |r| <= pi/2 by multiples of pi and a Taylor polynomial to r^21:
 // half the instructions of sine and cosine together
 __device__ __forceinline__ double small_sin(double x, double e) {

@@ -7,6 +7,7 @@
 
 #include "spss_device.hpp"
 #include "spss_fast.hpp"
+#include "spss_pairs64.hpp"
 
 namespace spss {
 
@@ -60,7 +61,7 @@ __device__ __forceinline__ void position_from(const DevParams &P, const double *
 template <int S, bool SRK>
 __device__ __forceinline__ void step_position(const DevParams &P, const double *pi, const StepArgs &U, double &sn,
                                               double &cn, double &x1, double &y1) {
-  sincos(pi[2], &sn, &cn);
+  phasor_of(pi[2], sn, cn);
   position_from<S, SRK>(P, pi, U, sn, cn, x1, y1);
 }
 
@@ -69,7 +70,7 @@ __device__ __forceinline__ void step_particle(const DevParams &P, const Coef &K,
                                               double nat_i, double2 sm, double2 tm, int nnb, const StepArgs &U,
                                               uint64_t step, double *out, double &C, double *disp2 = nullptr) {
   double sn, cn, ddx, ddy;
-  sincos(pi[2], &sn, &cn);
+  phasor_of(pi[2], sn, cn);
   displacement_from<S, SRK>(P, pi, U, sn, cn, ddx, ddy);
   out[0] = pi[0] + ddx;
   out[1] = pi[1] + ddy;

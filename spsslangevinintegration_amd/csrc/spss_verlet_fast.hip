@@ -10,28 +10,32 @@
 //
 // Layout (the resident copy): particles in the cell order of the last rebuild on a grid of
 // side Hv = 1/int(1/r_max); between rebuilds they keep their slots.  Per slot: FP64 state
-// (double-buffered by step), id, natural frequency, FP32 snapshot {x, y wrapped into the box,
-// cos phi, sin phi} and FP32 omega (double-buffered with the state), and an ELL list of width K
-// with its length, in blocks of 256 slots and chunks of four entries (lslot).  Grids of at most
-// kRowTileCols columns also have row tiles of the rebuild's cell order (spans of whole cells of
-// one row, as for the cell-list pair kernel) and a 16-bit copy of every list: the entries' LDS
-// positions in the tile's stage, tile-local in the same chunked form (l16chunk).  Either way a
-// wave's loads of one chunk are contiguous and a particle's entries are not on pages of their own.
+// (double-buffered by step), id, natural frequency, cell, FP32 snapshot {x, y, cos phi, sin phi} and
+// FP32 omega (double-buffered with the state).
+//
+// Grids of at most kRowTileCols columns have row tiles of the rebuild's cell order (spans of whole
+// cells of one row, as for the cell-list pair kernel).  The step is one workgroup per tile: the 3 x (W + 2)
+// cells around its W cells go into LDS and the sums over the particles within rho come from the matrix
+// cores (spss_mfma_pairs.hpp).  The cells of the last rebuild hold every candidate until the next one,
+// so no list is read; lists are built for the few tiles that overflow the stage or a workgroup, and
+// for vf_lists, from the state that the last rebuild left in the scratch arrays.  Snapshots of tiled
+// grids hold positions from the centre of the particle's cell.  At N = 1M, 53 neighbours, skin
+// 0.2 rho, stochastic Runge-Kutta: 107 us per step (a third each: staging, sums, update), where walking
+// 16-bit lists from LDS took 125, bound by LDS reads, and building them 190 per rebuild.
+//
+// Wider grids keep an ELL list of width K per slot with its length, in blocks of 256 slots and chunks of
+// four entries (lslot), and walk it through global memory (vr_lists, vs_step): FP32 distances as
+// x_j - x_i minus its nearest integer, sixteen entries per pass, phasor sums in four FP32 partials
+// flushed into FP64.  Either way a guard band around rho^2 is decided with the reference's FP64 ClassC
+// formula on the stored positions, so neighbour sets are exact.
 //
 // One step is a rebuild -- launches that return at once unless the device flag asks for one:
 // cell keys and histogram, the two-level scan, bucket fill, stable rank and gather into scratch,
-// back into the resident arrays with the new snapshot, the row tiles, the lists -- and the step:
-// one workgroup per row tile stages the snapshots (and omega) of the 3 x (W + 2) cells around its
-// W cells into LDS; each lane walks its list from LDS, sixteen entries per pass (the next pass's
-// entries loaded meanwhile): FP32 distance (the stage holds each position as its periodic image
-// nearest its staged cell, so separations are plain differences; the walks through global memory
-// take x_j - x_i minus its nearest integer), a guard band around rho^2 decided
-// with the reference's FP64 ClassC formula on the stored positions (so neighbour sets are exact),
-// phasor sums in four FP32 partials flushed into FP64 every 16 entries; then the Euler/SRK update
-// of step_particle, the new snapshot and the step's largest squared displacement (maxima by
-// group of workgroups); a one-wave launch after the step (vc_flag) turns it into the next step's
-// flag on the device.  No host synchronisation: steps replay from HIP graphs.  Without tiles
-// (wider grids), vr_lists and vs_step do the same per particle through global memory.
+// back into the resident arrays with the new snapshot, the row tiles, the lists -- and the step,
+// which ends with the Euler/SRK update of step_particle, the new snapshot and the step's largest
+// squared displacement (maxima by group of workgroups); a one-wave launch after the step (vc_flag)
+// turns it into the next step's flag on the device.  No host synchronisation: steps replay from HIP
+// graphs.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -43,6 +47,7 @@
 
 #include "../../include/spss_hip.h"
 #include "spss_launch.hpp"
+#include "spss_mfma_pairs.hpp"
 #include "spss_scan.hpp"
 #include "spss_step.hpp"
 #include "spss_tiles.hpp"
@@ -76,12 +81,17 @@ struct VArgs {
   int n, ncv, cells, K;
   double rmax2;           // FP64 list radius squared
   double half_skin;       // (r_max - rho) / 2
+  double h;               // the cells' side, 1 / ncv
   float r2c, r2h, r2k;    // guard band around rho^2: |d^2 - r2c| <= r2h is decided in FP64
   float m2c, m2h;         // guard band around r_max^2 (list build)
+  float unit, rho_u, r2_u, drift;  // tiled grids: kMUnit per cell side; rho, rho^2 and 1 + half the skin in units
   VCtl *ctl;
 };
 
 __device__ __forceinline__ bool gate_off(const VArgs &A) { return A.ctl->flag == 0; }
+
+// a row or column at most one outside the grid
+__device__ __forceinline__ int wrap_row(int c, int nc) { return c < 0 ? c + nc : (c >= nc ? c - nc : c); }
 
 // device addresses of fields of the control block, formed on the host without dereferencing it
 static int *ctl_flag(VCtl *c) { return reinterpret_cast<int *>(reinterpret_cast<char *>(c) + offsetof(VCtl, flag)); }
@@ -93,7 +103,20 @@ static unsigned long long *ctl_step(VCtl *c) {
 __device__ __forceinline__ float4 vsnap_of(const DevParams &P, const double *st) {
   double xw, yw, sn, cn;
   apply_pbc(P, st[0], st[1], xw, yw);
-  sincos(st[2], &sn, &cn);
+  phasor_of(st[2], sn, cn);
+  return make_float4((float)xw, (float)yw, (float)cn, (float)sn);
+}
+
+// the snapshot of a tiled grid: the position from the centre of the particle's cell of the last rebuild
+// (nearest image), which FP32 holds to 2^-24 of the cell instead of the box
+__device__ __forceinline__ float4 vsnap_cell(const DevParams &P, const double *st, int cx, int cy, double h) {
+  double xw, yw, sn, cn;
+  apply_pbc(P, st[0], st[1], xw, yw);
+  xw -= ((double)cx + 0.5) * h;
+  yw -= ((double)cy + 0.5) * h;
+  xw -= rint(xw);
+  yw -= rint(yw);
+  phasor_of(st[2], sn, cn);
   return make_float4((float)xw, (float)yw, (float)cn, (float)sn);
 }
 
@@ -114,9 +137,6 @@ __device__ __forceinline__ float dd_of(float4 o, float xi, float yi, float c2) {
 __host__ __device__ __forceinline__ long lslot(long p, long t, int K) {
   return ((((p >> 8) * (K >> 2) + (t >> 2)) * 256 + (p & 255)) << 2) + (t & 3);
 }
-// the 16-bit copy, tile-local in the same chunked form: chunk c of the tile's lane u at
-// (tile * K / 4 + c) * 256 + u, four 16-bit entries (uint2) each
-__device__ __forceinline__ long l16chunk(long tile, int u, int c, int K) { return (tile * (K >> 2) + c) * 256 + u; }
 
 // ---------------------------------------------------------------------------
 // rebuild (every launch returns at once when the flag is clear)
@@ -219,8 +239,9 @@ __global__ __launch_bounds__(kVB) void vr_settle(DevParams P, VArgs A, const dou
     }
     id[q] = sid[q];
     if (nat) nat[q] = snat[q];
-    cell[q] = scell[q];
-    snap[q] = vsnap_of(P, st);
+    const int c = scell[q];
+    cell[q] = c;
+    snap[q] = tiles ? vsnap_cell(P, st, c % A.ncv, c / A.ncv, A.h) : vsnap_of(P, st);
     omega[q] = S == 4 ? (float)st[3] : 0.f;
   }
 }
@@ -229,16 +250,16 @@ __global__ __launch_bounds__(kVB) void vr_settle(DevParams P, VArgs A, const dou
 // ParticleSystemFirstOrderPtr.cpp:83-88, ascending slot inside a cell; j is listed when its
 // distance from the wrapped x_i to the stored x_j is within r_max (:694-739).  FP32 test outside a
 // guard band, the reference's FP64 ClassC formula inside it.
-// The list of slot q read from global memory (lists of a grid too wide for row tiles, and of tiles
-// whose stencil cells overflow the LDS stage).
-template <int S>
+// The list of slot q read from global memory.
+// EXACT: every pair by the FP64 formula (tiled grids, whose snapshots are relative to the cells).
+template <int S, bool EXACT>
 __device__ __forceinline__ void list_of_slot(const DevParams &P, const VArgs &A, const int *__restrict__ start,
                                              const int *__restrict__ cell, const double *__restrict__ state,
                                              const float4 *__restrict__ snap, int *__restrict__ list,
                                              int *__restrict__ len, int q) {
   const int c = cell[q];
   const int cx = c % A.ncv, cy = c / A.ncv;
-  const float4 me = snap[q];
+  const float4 me = EXACT ? make_float4(0.f, 0.f, 0.f, 0.f) : snap[q];
   double xi, yi;
   apply_pbc(P, state[(long)q * S], state[(long)q * S + 1], xi, yi);
   int w = 0;
@@ -249,9 +270,9 @@ __device__ __forceinline__ void list_of_slot(const DevParams &P, const VArgs &A,
       const int e = start[cj + 1];
       for (int u = start[cj]; u < e; ++u) {
         if (u == q) continue;
-        const float dd = dd_of(snap[u], me.x, me.y, A.m2c);
+        const float dd = EXACT ? 0.f : dd_of(snap[u], me.x, me.y, A.m2c);
         bool in = dd < 0.f;
-        if (__builtin_fabsf(dd) <= A.m2h) {
+        if (EXACT || __builtin_fabsf(dd) <= A.m2h) {
           double dx, dy;
           class_c_unsigned(P, xi, yi, state[(long)u * S], state[(long)u * S + 1], dx, dy);
           in = dx * dx + dy * dy <= A.rmax2;
@@ -275,7 +296,7 @@ __global__ __launch_bounds__(kVB) void vr_lists(DevParams P, VArgs A, const int 
                                                 int *__restrict__ len) {
   if (gate_off(A)) return;
   const int q = blockIdx.x * kVB + threadIdx.x;
-  if (q < A.n) list_of_slot<S>(P, A, start, cell, state, snap, list, len, q);
+  if (q < A.n) list_of_slot<S, false>(P, A, start, cell, state, snap, list, len, q);
 }
 
 // ---------------------------------------------------------------------------
@@ -505,327 +526,256 @@ __global__ __launch_bounds__(kVB) void vs_step(DevParams P, VArgs A, StepArgs U,
 // ---------------------------------------------------------------------------
 // Row tiles of the rebuild's cell order (grids of at most kRowTileCols columns).  One workgroup
 // per tile -- a span of whole cells of one row, as for the cell-list pair kernel -- stages the
-// snapshots (and omega) of the 3 x (W + 2) cells around its W cells into LDS.  A list entry is
-// then also kept as the candidate's LDS position in its tile's stage (16 bits), and a step reads
-// its candidates from LDS instead of gathering them from global memory: the same values in the
-// same order, so the sums equal the global walk's bit for bit.  A tile whose stencil cells
-// overflow the stage builds and walks its lists through global memory as before.
+// snapshots (and omega) of the 3 x (W + 2) cells around its W cells, which hold every candidate until
+// the next rebuild, and takes the sums over them on the matrix cores (spss_mfma_pairs.hpp): a
+// superset of the lists, whose pairs beyond rho count for nothing, with no list read.  So lists are
+// built only for tiles whose cells overflow the stage or whose particles outnumber the workgroup.
 
-constexpr int kVStage = 1024;     // staged snapshots per tile
-constexpr int kVFar = kVStage;    // one more stage slot, far from everything: the lists' padding
-constexpr int kVCols = 48;     // staged columns W + 2
+constexpr int kVCols = 48;  // staged columns W + 2
 
-template <bool SRK>
-struct VtLds {
-  float4 sdat[kVStage + 1];  // [kVFar]: x, y far away, phasor 0
-  float somega[SRK ? kVStage + 1 : 1];
-  int cglob[3 * kVCols];     // first slot of staged cell (r, q), at r * (W + 2) + q
-  int ccnt[3 * kVCols];      // its particle count
-  int cpos[3 * kVCols + 1];  // its LDS start; [cells] = the staged total
-  double wmax[kVB / 64];
+struct VtPlan {
+  int cglob[3 * kVCols];  // first slot of staged cell (r, q), at r * (W + 2) + q
+  int ccnt[3 * kVCols];   // its particle count
+  int cpos[3 * kVCols];   // its start in staged row r
+  int len[3];             // particles of the staged rows
 };
 
 // the staging plan of tile (row, ca, cb): rows row-1 .. row+1, columns ca-1 .. cb (each wrapped
-// once); returns the staged total (the same for every thread)
-__device__ int vt_plan(const VArgs &A, const int *__restrict__ start, int row, int ca, int cb, int *cglob, int *ccnt,
-                       int *cpos) {
-  const int ncols = cb - ca + 2, ncells = 3 * ncols;
-  for (int e = threadIdx.x; e < ncells; e += kVB) {
-    const int r = e / ncols, q = e - r * ncols;
-    int rr = row + r - 1, cc = ca - 1 + q;
-    rr += rr < 0 ? A.ncv : (rr >= A.ncv ? -A.ncv : 0);
-    cc += cc < 0 ? A.ncv : (cc >= A.ncv ? -A.ncv : 0);
-    const int c = rr * A.ncv + cc;
-    const int g0 = start[c];
-    cglob[e] = g0;
-    ccnt[e] = start[c + 1] - g0;
-  }
-  __syncthreads();
-  if (threadIdx.x < 64) {  // one wave: exclusive prefix of the counts, 64 cells per pass
-    const int lane = threadIdx.x;
-    int run = 0;
-    for (int e0 = 0; e0 < ncells; e0 += 64) {
-      const int e = e0 + lane;
-      const int v = e < ncells ? ccnt[e] : 0;
-      const int incl = wave_incl_scan(v, lane);
-      if (e < ncells) cpos[e] = run + incl - v;
-      run += __shfl(incl, 63, 64);
+// once); returns the staged total of whole units per row (the same for every thread)
+__device__ __forceinline__ int vt_plan(const VArgs &A, const int *__restrict__ start, int row, int ca, int cb,
+                                       VtPlan &L) {
+  const int ncols = cb - ca + 2, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (w < 3) {  // a wave per row, a lane per cell (at most kVCols): exclusive prefix of the counts
+    int g0 = 0, v = 0;
+    if (lane < ncols) {
+      const int c = wrap_row(row + w - 1, A.ncv) * A.ncv + wrap_row(ca - 1 + lane, A.ncv);
+      g0 = start[c];
+      v = start[c + 1] - g0;
     }
-    if (lane == 0) cpos[ncells] = run;
-  }
-  __syncthreads();
-  return cpos[ncells];
-}
-
-// the staged cells' snapshots (and omega) into LDS, G lanes per cell, each position taken as its
-// periodic image nearest the centre of its staged cell (the cells are those of the last rebuild,
-// which the particles may have left by up to half the skin, across the box's edge too) and re-based
-// to the stage's corner (col0, row0 in cells of side 1/ncv): within a stage the separations are
-// then plain differences, with no nearest-image correction per candidate.  Each staged coordinate
-// takes at most two more FP32 roundings (<= 2^-24 each, coordinates below 1), within what the
-// guard bands allow for.
-template <bool SRK>
-__device__ void vt_stage(const VArgs &A, int ncols, int col0, int row0, const float4 *__restrict__ snap,
-                         const float *__restrict__ omega, VtLds<SRK> &L) {
-  const int ncells = 3 * ncols;
-  const float h = 1.f / (float)A.ncv;
-  const float x0 = (float)col0 * h, y0 = (float)row0 * h;
-  const int G = ncells <= kVB / 8 ? 8 : (ncells <= kVB / 4 ? 4 : (ncells <= kVB / 2 ? 2 : 1));
-  const int sub = (int)threadIdx.x % G;
-  for (int c = (int)threadIdx.x / G; c < ncells; c += kVB / G) {
-    const int r = c / ncols, q = c - r * ncols;
-    // centre of the staged cell, unwrapped (its column and row may lie one cell past the edges)
-    const float xc = ((float)(col0 + q) + 0.5f) * h, yc = ((float)(row0 + r) + 0.5f) * h;
-    const int e0 = L.cpos[c], n0 = L.ccnt[c], g0 = L.cglob[c];
-    for (int j = sub; j < n0; j += G) {
-      const float4 v = snap[g0 + j];
-      const float xu = v.x - __builtin_rintf(v.x - xc), yu = v.y - __builtin_rintf(v.y - yc);
-      L.sdat[e0 + j] = make_float4(xu - x0, yu - y0, v.z, v.w);
-      if (SRK) L.somega[e0 + j] = omega[g0 + j];
+    const int incl = wave_incl_scan(v, lane);
+    if (lane < ncols) {
+      const int e = w * ncols + lane;
+      L.cglob[e] = g0;
+      L.ccnt[e] = v;
+      L.cpos[e] = incl - v;
     }
-  }
-  if (threadIdx.x == 0) {  // d^2 of the far slot is ~1e36: out of range, never in a guard band
-    L.sdat[kVFar] = make_float4(1e18f, 1e18f, 0.f, 0.f);
-    if (SRK) L.somega[kVFar] = 0.f;
+    if (lane == 63) L.len[w] = incl;
   }
   __syncthreads();
+  return ((L.len[0] + 15) & ~15) + ((L.len[1] + 15) & ~15) + ((L.len[2] + 15) & ~15);
 }
 
-// d^2 - c2 of two staged entries (plain differences: see vt_stage)
-__device__ __forceinline__ float dd_staged(float4 o, float xi, float yi, float c2) {
-  const float dx = o.x - xi, dy = o.y - yi;
-  return __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, -c2));
-}
-
-// global slot of staged entry t: the last staged cell starting at or before t (an empty cell
-// starts where the next one does, so the cell found holds t)
-__device__ __forceinline__ int vt_slot(const int *cglob, const int *cpos, int ncells, int t) {
-  int lo = 0, hi = ncells - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (cpos[mid] <= t) lo = mid; else hi = mid - 1;
-  }
-  return cglob[lo] + (t - cpos[lo]);
-}
-
-// The lists of a tile's particles, in list_of_slot's order (stencil cells in order, ascending slot
-// inside a cell) and with its decisions, from the staged snapshots; each entry is written twice:
-// as a slot (list, slot-major over all particles) and as its LDS position in the tile's stage
-// (list16, tile-local chunks of four, l16chunk); both written a chunk at a time.
+// The lists of the tiles that walk theirs: in list_of_slot's order (stencil cells in order, ascending
+// slot inside a cell).
 template <int S>
 __global__ __launch_bounds__(kVB) void vt_lists(DevParams P, VArgs A, const int4 *__restrict__ tiles, int ntiles,
                                                 const int *__restrict__ start, const int *__restrict__ cell,
-                                                const double *__restrict__ state, const float4 *__restrict__ snap,
-                                                int *__restrict__ list, uint2 *__restrict__ list16,
+                                                const double *__restrict__ state, int *__restrict__ list,
                                                 int *__restrict__ len) {
   if (gate_off(A)) return;
-  __shared__ VtLds<false> L;
+  __shared__ VtPlan L;
   for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {  // (the same for the whole workgroup)
     const int4 td = tiles[tile];
     const int row = td.y, ca = td.z, cb = td.w;
     if (ca >= cb) continue;  // an unused tile slot
-    const int ncols = cb - ca + 2, ncells = 3 * ncols;
-    __syncthreads();  // the previous tile's stage is consumed
-    const int total = vt_plan(A, start, row, ca, cb, L.cglob, L.ccnt, L.cpos);
-    const int gtb = L.cglob[ncols + 1];
-    const int ntile = start[row * A.ncv + cb] - gtb;
+    __syncthreads();  // the previous tile's plan is consumed
+    const int total = vt_plan(A, start, row, ca, cb, L);
+    const int gtb = start[row * A.ncv + ca], ntile = start[row * A.ncv + cb] - gtb;
     if (ntile > kVB && threadIdx.x == 0) atomicAdd(&A.ctl->big_tiles, 1);
-    if (total > kVStage) {
-      for (int u = threadIdx.x; u < ntile; u += kVB) list_of_slot<S>(P, A, start, cell, state, snap, list, len, gtb + u);
-      continue;
-    }
-    vt_stage<false>(A, ncols, ca - 1, row - 1, snap, nullptr, L);
-    const int ltb = L.cpos[ncols + 1];
-    for (int u = threadIdx.x; u < ntile; u += kVB) {
-      const int q = gtb + u, li = ltb + u;
-      // entries go out four at a time (a chunk of each list): c32 / c16 collect the current chunk
-      int4 c32 = make_int4(0, 0, 0, 0);
-      unsigned int c16lo = 0u, c16hi = 0u;
-      auto flush = [&](int w) {  // the chunk holding entries 4 * (w >> 2) ..
-        *reinterpret_cast<int4 *>(list + lslot(q, w & ~3, A.K)) = c32;
-        if (u < kVB) list16[l16chunk(tile, u, w >> 2, A.K)] = make_uint2(c16lo, c16hi);
-      };
-      const float4 me = L.sdat[li];
-      double xi, yi;
-      apply_pbc(P, state[(long)q * S], state[(long)q * S + 1], xi, yi);
-      const int qi = 1 + cell[q] % A.ncv - ca;  // staged column of the particle's cell
-      int w = 0;
-      for (int r = 0; r < 3; ++r)
-        for (int dq = -1; dq <= 1; ++dq) {
-          const int e = r * ncols + qi + dq;
-          const int t0 = L.cpos[e], t1 = t0 + L.ccnt[e], g0 = L.cglob[e];
-          for (int t = t0; t < t1; ++t) {
-            if (t == li) continue;
-            const float dd = dd_staged(L.sdat[t], me.x, me.y, A.m2c);
-            bool in = dd < 0.f;
-            if (__builtin_fabsf(dd) <= A.m2h) {
-              const long g = g0 + (t - t0);
-              double dx, dy;
-              class_c_unsigned(P, xi, yi, state[g * S], state[g * S + 1], dx, dy);
-              in = dx * dx + dy * dy <= A.rmax2;
-            }
-            if (in) {
-              if (w < A.K) {
-                const int g = g0 + (t - t0), k = w & 3;
-                c32.x = k == 0 ? g : c32.x;
-                c32.y = k == 1 ? g : c32.y;
-                c32.z = k == 2 ? g : c32.z;
-                c32.w = k == 3 ? g : c32.w;
-                const unsigned int h = (unsigned int)t << ((k & 1) * 16);
-                if (k < 2) c16lo = (k == 0 ? 0u : c16lo) | h;
-                else c16hi = (k == 2 ? 0u : c16hi) | h;
-                if (k == 3) flush(w);
-              }
-              ++w;
-            }
-          }
-        }
-      if (w < A.K) {  // the 16-bit list padded with the far slot to a whole pass of 16 (K is a multiple of 16)
-        for (int t = w; t < ((w + 15) & ~15); ++t) {
-          const int k = t & 3;
-          const unsigned int h = (unsigned int)kVFar << ((k & 1) * 16);
-          if (k < 2) c16lo = (k == 0 ? 0u : c16lo) | h;
-          else c16hi = (k == 2 ? 0u : c16hi) | h;
-          if (k == 3) flush(t);
-        }
-      }
-      len[q] = w <= A.K ? w : -1;
-      if (w > A.K) atomicAdd(&A.ctl->overflow, 1ull);
-    }
+    if (total <= kMStage && ntile <= kVB) continue;
+    for (int u = threadIdx.x; u < ntile; u += kVB) list_of_slot<S, true>(P, A, start, cell, state, nullptr, list, len, gtb + u);
   }
 }
 
-// walk_list with the candidates read from the tile's stage (l16: the lane's first chunk of the
-// tile-local 16-bit list, chunk c at l16[c * kVB]; the entries past L up to the pass's end are the
-// far slot, weight 0, so no entry needs a mask): the pass's sixteen list entries are loaded first
-// (global memory, four chunks), the candidates four at a time from LDS, in walk_list's order and
-// grouping
+template <int W>
+struct VtLds {
+  MStage<W> M;
+  VtPlan plan;
+  unsigned short col[kVB];  // staged column of the tile's particles
+  float most[kVB / 64];
+  double wmax[kVB / 64];
+};
+
+// The sums of the tile's particles (the workgroup's first kVB) over the staged cells.  Positions are
+// taken from the tile's centre.  False: a staged value is not finite (the same for every thread).
+template <int S, int W>
+__device__ __forceinline__ bool vt_sums(const DevParams &P, const VArgs &A, int row, int ca, int cb, int gtb, int ntile,
+                                        int total, const int *__restrict__ cell, const double *__restrict__ state,
+                                        const float4 *__restrict__ snap, const float *__restrict__ omega,
+                                        VtLds<W> &Ls, MSums &sum) {
+  constexpr int kPasses = 5;  // chunks of 64 entries per wave: at most kMStage / 64 and two for the rows' rests
+  const VtPlan &L = Ls.plan;
+  const int ncols = cb - ca + 2, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l0 = __builtin_amdgcn_readfirstlane(L.len[0]), l1 = __builtin_amdgcn_readfirstlane(L.len[1]);
+  const int l2 = __builtin_amdgcn_readfirstlane(L.len[2]);
+  const int b1 = (l0 + 15) & ~15, b2 = b1 + ((l1 + 15) & ~15);
+  // positions from the tile's centre, the cell's side kMUnit; |x| <= xm with the particles within half the
+  // skin of their cells.  A coordinate is rounded to 22 bits, so separations up to rho err by 2^-22 xm:
+  // `tight` is twice what d^2 errs by.  The product's roundings are at most 96 of 2^-24 of |x|^2 on top.
+  const float unit = A.unit, r2 = A.r2_u;
+  const float xm = 0.5f * kMUnit * (float)(cb - ca) + A.drift, ym = 0.5f * kMUnit + A.drift;
+  const float tight = 0x1p-20f * A.rho_u * (xm + ym + A.rho_u), band = tight + 96.f * 0x1p-24f * (xm * xm + ym * ym);
+
+  // the staged particles: a row's cells are one run of slots, but for a first column left of the box
+  // and a last one right of it
+  const bool lw = ca == 0, rw = cb == A.ncv;
+  const int s0 = __builtin_amdgcn_readfirstlane(L.cglob[0]), s1 = __builtin_amdgcn_readfirstlane(L.cglob[ncols]);
+  const int s2 = __builtin_amdgcn_readfirstlane(L.cglob[2 * ncols]);
+  // the number of a cell of staged column 0 (of any row's extension to the left)
+  const int f0 = wrap_row(row - 1, A.ncv) * A.ncv + ca - 1, f1 = row * A.ncv + ca - 1;
+  const int f2 = wrap_row(row + 1, A.ncv) * A.ncv + ca - 1;
+  const int c0 = (l0 + 63) >> 6, c1 = c0 + ((l1 + 63) >> 6), c2 = c1 + ((l2 + 63) >> 6);
+  float4 v[kPasses];
+  float om[kPasses], most = 0.f;
+  int at[kPasses], to[kPasses];  // first entry of the wave's chunk; entries of its row from there
+#pragma unroll
+  for (int p = 0; p < kPasses; ++p) {
+    const int ch = 4 * p + wave;
+    const int r = ch < c0 ? 0 : (ch < c1 ? 1 : 2), t0 = 64 * (ch - (r == 0 ? 0 : (r == 1 ? c0 : c1)));
+    at[p] = (r == 0 ? 0 : (r == 1 ? b1 : b2)) + t0;
+    to[p] = ch < c2 ? (r == 0 ? l0 : (r == 1 ? l1 : l2)) - t0 : 0;
+    v[p] = make_float4(0.f, 0.f, 0.f, 0.f);
+    om[p] = 0.f;
+    if (lane < to[p]) {
+      const int t = t0 + lane;
+      int g = (r == 0 ? s0 : (r == 1 ? s1 : s2)) + t;
+      int q;  // staged column
+      if (lw || rw) {
+        const int e = r * ncols;
+        const bool left = lw && t < L.cpos[e + 1], right = rw && t >= L.cpos[e + ncols - 1];
+        const int c = left ? e : (right ? e + ncols - 1 : e + (lw ? 1 : 0));
+        g = L.cglob[c] + (t - L.cpos[c]);
+        q = left ? 0 : (right ? ncols - 1 : cell[g] - (r == 0 ? f0 : (r == 1 ? f1 : f2)));
+      } else {
+        q = cell[g] - (r == 0 ? f0 : (r == 1 ? f1 : f2));
+      }
+      v[p] = snap[g];
+      if (W == 5) om[p] = omega[g];
+      v[p].x = __builtin_fmaf(v[p].x, unit, kMUnit * ((float)q - 0.5f * (float)(cb - ca + 1)));
+      v[p].y = __builtin_fmaf(v[p].y, unit, kMUnit * (float)(r - 1));
+      const float big = __builtin_fabsf(v[p].x) + __builtin_fabsf(v[p].y) + __builtin_fabsf(v[p].z) +
+                        __builtin_fabsf(v[p].w) + __builtin_fabsf(om[p]);
+      most = __builtin_fmaxf(most, big < 0x1p100f ? __builtin_fabsf(om[p]) : __builtin_inff());
+    }
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) most = __builtin_fmaxf(most, __shfl_xor(most, o, 64));
+  if (lane == 0) Ls.most[wave] = most;
+  if ((int)threadIdx.x < ntile) Ls.col[threadIdx.x] = (unsigned short)(cell[gtb + threadIdx.x] - row * A.ncv - ca + 1);
+  m_init(Ls.M);
+  __syncthreads();
+  most = __builtin_fmaxf(__builtin_fmaxf(Ls.most[0], Ls.most[1]), __builtin_fmaxf(Ls.most[2], Ls.most[3]));
+  if (!(most < 0x1p100f)) return false;
+  const int scale = most > 0x1p-90f ? ilogbf(most) + 1 : -89;
+  const float s30 = ldexpf(1.f, 30 - scale);
+#pragma unroll
+  for (int p = 0; p < kPasses; ++p)
+    if (lane < ((to[p] + 15) & ~15))
+      m_write<W>(Ls.M, at[p] + lane, lane < to[p], v[p].x, v[p].y, v[p].z, v[p].w, om[p] * s30);
+  __syncthreads();
+  const int first = b1 + L.cpos[ncols + 1] + 64 * wave, count = min(max(ntile - 64 * wave, 0), 64);
+  if (count == 0) return true;
+  const int p = gtb + 64 * wave + lane;
+  const float4 me = lane < count ? snap[p] : make_float4(0.f, 0.f, 0.f, 0.f);
+  const float mo = W == 5 && lane < count ? omega[p] : 0.f;
+  sum = m_sums<W>(
+      Ls.M, first, count, 3, r2, band, me.z, me.w, mo * s30, scale,
+      [&](int i, int r, int &a, int &b) {
+        const int q0 = r * ncols + Ls.col[64 * wave + i] - 1;
+        const int q1 = r * ncols + Ls.col[64 * wave + min(i + 15, count - 1)] + 1;
+        const int base = r == 0 ? 0 : (r == 1 ? b1 : b2);
+        a = base + L.cpos[q0];
+        b = base + L.cpos[q1] + L.ccnt[q1];
+      },
+      [&](int i, int e) {
+        // differences of the staged positions first: their band is narrower
+        const uint2 pe = m_pos(Ls.M, e), po = m_pos(Ls.M, first + i);
+        const float dx = m_value(pe.x) - m_value(po.x), dy = m_value(pe.y) - m_value(po.y);
+        const float dd = __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, -r2));
+        if (__builtin_fabsf(dd) > tight) return dd < 0.f;
+        // the reference's FP64 test (x_i as stored, rhs_verlet's :566-581)
+        const int r = e < b1 ? 0 : (e < b2 ? 1 : 2), t = e - (r == 0 ? 0 : (r == 1 ? b1 : b2));
+        int q = r * ncols, hi = q + ncols - 1;  // the last cell that starts at or before t holds it
+        while (q < hi) {
+          const int mid = (q + hi + 1) >> 1;
+          if (L.cpos[mid] <= t) q = mid; else hi = mid - 1;
+        }
+        const double *pi = state + (long)(gtb + 64 * wave + i) * S, *pj = state + (long)(L.cglob[q] + t - L.cpos[q]) * S;
+        double ddx, ddy;
+        class_c_unsigned(P, pi[0], pi[1], pj[0], pj[1], ddx, ddy);
+        return ddx * ddx + ddy * ddy <= P.rho2;
+      });
+  return true;
+}
+
+// The sums of slot p of a tiled grid through global memory, over its list (L >= 0) or over the cells of
+// the last rebuild, every pair by the reference's FP64 test (x_i as stored, rhs_verlet's :566-581).
 template <int S, bool SRK>
-__device__ __forceinline__ void walk_list_lds(const DevParams &P, const VArgs &A, const uint2 *__restrict__ l16,
-                                              const VtLds<SRK> &Ls, int ncells, const double *__restrict__ state,
-                                              int p, int li, int L, float xi, float yi, const double *pi, double &sx,
-                                              double &sy, double &tx, double &ty, int &nnb, const uint2 *first) {
-  uint2 nxt[4];  // the next pass's four chunks, loaded while the current pass computes
+__device__ __forceinline__ MSums vt_walk(const DevParams &P, const VArgs &A, const int *__restrict__ list,
+                                         const int *__restrict__ start, const int *__restrict__ cell,
+                                         const double *__restrict__ state, const float4 *__restrict__ snap,
+                                         const float *__restrict__ omega, int p, int L) {
+  MSums m;
+  const double xi = state[(long)p * S], yi = state[(long)p * S + 1];
+  const auto range = [&](int a, int b, auto slot) {  // entries [a, b), four at a time
+    for (int t0 = a; t0 < b; t0 += 4) {
+      double x[4], y[4];
+      float4 o[4];
+      float om[4];
+      int j[4];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) nxt[c] = first[c];  // the first pass's, loaded with the list's length
-  for (int t0 = 0; t0 < L; t0 += 16) {
-    float ax[4] = {0.f, 0.f, 0.f, 0.f}, ay[4] = {0.f, 0.f, 0.f, 0.f}, an = 0.f;
-    float bx[4] = {0.f, 0.f, 0.f, 0.f}, by[4] = {0.f, 0.f, 0.f, 0.f};
-    uint2 cur[4];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) cur[c] = nxt[c];
-    if (t0 + 16 < L) {  // within the list's whole passes (at most K entries)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) nxt[c] = l16[(long)(((t0 + 16) >> 2) + c) * kVB];
-    }
-    int j[16];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {  // four chunks of four 16-bit entries (K is a multiple of 16)
-      const uint2 w = cur[c];
-      const int e[4] = {(int)(w.x & 0xffffu), (int)(w.x >> 16), (int)(w.y & 0xffffu), (int)(w.y >> 16)};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) j[4 * c + k] = e[k];  // past L: the far slot (weight 0)
-    }
-#pragma unroll
-    for (int g8 = 0; g8 < 16; g8 += 8) {  // two groups' candidates read from LDS together
-      float4 o8[8];
-      float om8[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        o8[k] = Ls.sdat[j[g8 + k]];
-        om8[k] = SRK ? Ls.somega[j[g8 + k]] : 0.f;
+      for (int k = 0; k < 4; ++k) {
+        j[k] = slot(min(t0 + k, b - 1));
+        x[k] = state[(long)j[k] * S];
+        y[k] = state[(long)j[k] * S + 1];
+        o[k] = snap[j[k]];
+        if (SRK) om[k] = omega[j[k]];
       }
 #pragma unroll
-      for (int h = 0; h < 8; h += 4) {
-        const int g = g8 + h;
-        const float4 *o = o8 + h;
-        float dd[4], m[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          dd[k] = dd_staged(o[k], xi, yi, A.r2c);
-          m[k] = __builtin_amdgcn_fmed3f(-A.r2k * dd[k], 0.f, 1.f);
-        }
-        const float dmin = __builtin_fminf(__builtin_fminf(__builtin_fabsf(dd[0]), __builtin_fabsf(dd[1])),
-                                           __builtin_fminf(__builtin_fabsf(dd[2]), __builtin_fabsf(dd[3])));
-        if (dmin <= A.r2h) {  // rare: the reference's FP64 test, as in walk4
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if (__builtin_fabsf(dd[k]) <= A.r2h) {
-              const long g2 = vt_slot(Ls.cglob, Ls.cpos, ncells, j[g + k]);
-              double dx, dy;
-              class_c_unsigned(P, pi[0], pi[1], state[g2 * S], state[g2 * S + 1], dx, dy);
-              m[k] = dx * dx + dy * dy <= P.rho2 ? 1.f : 0.f;
-            }
-        }
-        an += (m[0] + m[1]) + (m[2] + m[3]);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          ax[k] = __builtin_fmaf(m[k], o[k].z, ax[k]);
-          ay[k] = __builtin_fmaf(m[k], o[k].w, ay[k]);
+      for (int k = 0; k < 4; ++k) {
+        double dx, dy;
+        class_c_unsigned(P, xi, yi, x[k], y[k], dx, dy);
+        if (t0 + k < b && j[k] != p && dx * dx + dy * dy <= P.rho2) {
+          m.sx += (double)o[k].z;
+          m.sy += (double)o[k].w;
+          ++m.n;
           if (SRK) {
-            const float mo = m[k] * om8[h + k];
-            bx[k] = __builtin_fmaf(mo, o[k].z, bx[k]);
-            by[k] = __builtin_fmaf(mo, o[k].w, by[k]);
+            m.tx += (double)om[k] * (double)o[k].z;
+            m.ty += (double)om[k] * (double)o[k].w;
           }
         }
       }
     }
-    sx += ((double)ax[0] + (double)ax[1]) + ((double)ax[2] + (double)ax[3]);
-    sy += ((double)ay[0] + (double)ay[1]) + ((double)ay[2] + (double)ay[3]);
-    nnb += (int)an;
-    if (SRK) {
-      tx += ((double)bx[0] + (double)bx[1]) + ((double)bx[2] + (double)bx[3]);
-      ty += ((double)by[0] + (double)by[1]) + ((double)by[2] + (double)by[3]);
-    }
+  };
+  if (L >= 0) {
+    range(0, L, [&](int t) { return list[lslot(p, t, A.K)]; });
+    return m;
   }
+  const int c = cell[p];
+  const int cx = c % A.ncv, cy = c / A.ncv;
+  for (int dyc = -1; dyc <= 1; ++dyc)
+    for (int dxc = -1; dxc <= 1; ++dxc) {
+      const int cj = adjust_cell(cy + dyc, A.ncv) * A.ncv + adjust_cell(cx + dxc, A.ncv);
+      range(start[cj], start[cj + 1], [](int t) { return t; });
+    }
+  return m;
 }
 
-// The step of slot p (vs_step's per-particle work); candidates from the tile's stage when
-// `staged` (li: p's LDS position, list16: p's tile-local 16-bit list), else through global
-// memory.  Returns |dr|^2.
+// The step of slot p (vs_step's per-particle work) from its sums.  Returns |dr|^2.
 template <int S, bool SRK>
 __device__ __forceinline__ double vt_particle(const DevParams &P, const VArgs &A, const StepArgs &U, const Coef &K,
-                                              uint64_t step, const int *__restrict__ list,
-                                              const uint2 *__restrict__ list16, const int *__restrict__ len,
-                                              const int *__restrict__ start, const int *__restrict__ cell,
-                                              const double *__restrict__ state, const int *__restrict__ id,
-                                              const double *__restrict__ nat, const float4 *__restrict__ snap,
-                                              const float *__restrict__ omega, double *__restrict__ nstate,
-                                              float4 *__restrict__ nsnap, float *__restrict__ nomega,
-                                              double *__restrict__ compl_out, const VtLds<SRK> *Ls, bool staged,
-                                              int ncells, int p, int li) {
-  const double *pi = state + (long)p * S;
-  uint2 first[4];  // the first pass of the 16-bit list (allocated for every lane of a tile)
-  if (staged) {
-#pragma unroll
-    for (int c = 0; c < 4; ++c) first[c] = list16[(long)c * kVB];
-  }
-  const float4 me = snap[p];
-  const int Lp = len[p];
-  double sx = 0.0, sy = 0.0, tx = 0.0, ty = 0.0;
-  int nnb = 0;
-  if (Lp >= 0 && staged) {
-    const float4 ms = Ls->sdat[li];  // the particle in the stage's coordinates
-    walk_list_lds<S, SRK>(P, A, list16, *Ls, ncells, state, p, li, Lp, ms.x, ms.y, pi, sx, sy, tx, ty, nnb, first);
-  } else if (Lp >= 0) {
-    walk_list<S, SRK>(P, A, list, snap, omega, state, p, Lp, me.x, me.y, pi, sx, sy, tx, ty, nnb);
-  } else {  // (rare) the list outgrew the width: the 3 x 3 cells of the last rebuild hold every candidate
-    const int c = cell[p];
-    const int cx = c % A.ncv, cy = c / A.ncv;
-    for (int dyc = -1; dyc <= 1; ++dyc)
-      for (int dxc = -1; dxc <= 1; ++dxc) {
-        const int cj = adjust_cell(cy + dyc, A.ncv) * A.ncv + adjust_cell(cx + dxc, A.ncv);
-        walk_range<S, SRK, true>(P, A, list, snap, omega, state, p, start[cj], start[cj + 1], me.x, me.y, pi, sx,
-                                 sy, tx, ty, nnb);
-      }
-  }
+                                              uint64_t step, const double *__restrict__ state,
+                                              const int *__restrict__ id, const double *__restrict__ nat,
+                                              double *__restrict__ nstate, float4 *__restrict__ nsnap,
+                                              float *__restrict__ nomega, double *__restrict__ compl_out,
+                                              const MSums &m, int p, int cx, int cy) {
   const int i = id[p];
   double out[S], C, dp2;
-  step_particle<S, SRK>(P, K, pi, i, nat ? nat[p] : 0.0, make_double2(sx, sy), make_double2(tx, ty), nnb, U,
-                        step, out, C, &dp2);
+  step_particle<S, SRK>(P, K, state + (long)p * S, i, nat ? nat[p] : 0.0, make_double2(m.sx, m.sy),
+                        make_double2(m.tx, m.ty), m.n, U, step, out, C, &dp2);
 #pragma unroll
   for (int k = 0; k < S; ++k) nstate[(long)p * S + k] = out[k];
-  nsnap[p] = vsnap_of(P, out);
+  nsnap[p] = vsnap_cell(P, out, cx, cy, A.h);
   nomega[p] = S == 4 ? (float)out[3] : 0.f;
   if (SRK && compl_out) compl_out[i] = C;
   return dp2;
@@ -863,42 +813,49 @@ __global__ __launch_bounds__(kVB) void vt_rest(DevParams P, VArgs A, StepArgs U,
     const int4 td = tiles[t];
     if (td.z >= td.w) continue;
     const int g0 = start[td.y * A.ncv + td.z], ntile = start[td.y * A.ncv + td.w] - g0;
-    for (int u = kVB + threadIdx.x; u < ntile; u += kVB)
-      d2 = fmax(d2, vt_particle<S, SRK>(P, A, U, K, step, list, nullptr, len, start, cell, state, id, nat, snap,
-                                        omega, nstate, nsnap, nomega, compl_out, nullptr, false, 0, g0 + u, 0));
+    for (int u = kVB + threadIdx.x; u < ntile; u += kVB) {
+      const int p = g0 + u;
+      const MSums m = vt_walk<S, SRK>(P, A, list, start, cell, state, snap, omega, p, len[p]);
+      d2 = fmax(d2, vt_particle<S, SRK>(P, A, U, K, step, state, id, nat, nstate, nsnap, nomega, compl_out, m, p,
+                                        cell[p] - td.y * A.ncv, td.y));
+    }
   }
   step_max(A, d2, wmax);
 }
 
 // The step of a tile's first kVB particles, one per lane (vt_rest has the others), and the step's
 // largest displacement as in vs_step.
+// (three workgroups per CU: no more registers than the vector ones, so that the products' results need
+// not be moved out of the accumulation registers)
 template <int S, bool SRK>
-__global__ __launch_bounds__(kVB) void vt_step(DevParams P, VArgs A, StepArgs U, const int4 *__restrict__ tiles,
-                                               int ntiles, const int *__restrict__ list,
-                                               const uint2 *__restrict__ list16, const int *__restrict__ len,
+__global__ __launch_bounds__(kVB, 3) void vt_step(DevParams P, VArgs A, StepArgs U, const int4 *__restrict__ tiles,
+                                               int ntiles, const int *__restrict__ list, const int *__restrict__ len,
                                                const int *__restrict__ start, const int *__restrict__ cell,
                                                const double *__restrict__ state, const int *__restrict__ id,
                                                const double *__restrict__ nat, const float4 *__restrict__ snap,
                                                const float *__restrict__ omega, double *__restrict__ nstate,
                                                float4 *__restrict__ nsnap, float *__restrict__ nomega,
                                                double *__restrict__ compl_out) {
-  __shared__ VtLds<SRK> Ls;
+  constexpr int W = SRK ? 5 : 2;
+  __shared__ VtLds<W> Ls;
   const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
   const int4 td = tile < ntiles ? tiles[tile] : make_int4(0, 0, 0, 0);
   double d2 = 0.0;
   if (td.z < td.w) {  // the same for the whole workgroup
     const int row = td.y, ca = td.z, cb = td.w;
-    const int ncols = cb - ca + 2, ncells = 3 * ncols;
-    const bool staged = vt_plan(A, start, row, ca, cb, Ls.cglob, Ls.ccnt, Ls.cpos) <= kVStage;
-    if (staged) vt_stage<SRK>(A, ncols, ca - 1, row - 1, snap, omega, Ls);
-    const int gtb = Ls.cglob[ncols + 1];
+    const int total = vt_plan(A, start, row, ca, cb, Ls.plan);
+    const int gtb = Ls.plan.cglob[cb - ca + 3];
     const int ntile = start[row * A.ncv + cb] - gtb;
-    const int u = threadIdx.x;
-    if (u < ntile)
-      d2 = vt_particle<S, SRK>(P, A, U, vt_coef(P, U), U.step_dev ? (uint64_t)*U.step_dev : U.step, list,
-                               list16 + l16chunk(tile, u, 0, A.K), len,
-                               start, cell, state, id, nat, snap, omega, nstate, nsnap, nomega, compl_out, &Ls, staged,
-                               ncells, gtb + u, Ls.cpos[ncols + 1] + u);
+    const bool staged = total <= kMStage;
+    MSums sum;
+    const bool have = staged && vt_sums<S, W>(P, A, row, ca, cb, gtb, ntile, total, cell, state, snap, omega, Ls, sum);
+    const int u = threadIdx.x, p = gtb + u;
+    if (u < ntile) {
+      // (rare) staged values that are not finite: the cells; an overflowing stage: the list
+      if (!have) sum = vt_walk<S, SRK>(P, A, list, start, cell, state, snap, omega, p, staged ? -1 : len[p]);
+      d2 = vt_particle<S, SRK>(P, A, U, vt_coef(P, U), U.step_dev ? (uint64_t)*U.step_dev : U.step, state, id, nat,
+                               nstate, nsnap, nomega, compl_out, sum, p, cell[p] - row * A.ncv, row);
+    }
   }
   step_max(A, d2, Ls.wmax);
 }
@@ -952,6 +909,15 @@ __global__ __launch_bounds__(kVB) void vc_iota(int n, int *__restrict__ id) {
   if (p < n) id[p] = p;
 }
 
+// the lists of the last rebuild from the state that it left in the scratch arrays
+template <int S>
+__global__ __launch_bounds__(kVB) void vc_lists(DevParams P, VArgs A, const int *__restrict__ start,
+                                                const int *__restrict__ cell, const double *__restrict__ state,
+                                                int *__restrict__ list, int *__restrict__ len) {
+  const int q = blockIdx.x * kVB + threadIdx.x;
+  if (q < A.n) list_of_slot<S, true>(P, A, start, cell, state, nullptr, list, len, q);
+}
+
 template <int S>
 __global__ __launch_bounds__(kVB) void vc_unpermute(int n, const double *__restrict__ vstate, const int *__restrict__ id,
                                                     double *__restrict__ state) {
@@ -975,19 +941,16 @@ struct VerletFast {
   int *vid = nullptr, *vcell = nullptr;
   double *vnat = nullptr;
   int *list = nullptr, *len = nullptr;
-  // row tiles of the rebuild's cell order (grids of at most kRowTileCols columns): ncv rows of
-  // vt_cmax slots, and the lists as LDS positions in the tiles' stages
+  // row tiles of the rebuild's cell order (grids of at most kRowTileCols columns): ncv rows of vt_cmax slots
   bool tiled = false;
   int vt_wcap = 0, vt_cmax = 0;
   int4 *vtiles = nullptr;
-  uint2 *list16 = nullptr;  // chunks of four 16-bit entries
   int *key = nullptr, *slotc = nullptr, *count = nullptr, *start = nullptr, *tmp = nullptr, *blocksum = nullptr;
   double *sstate = nullptr, *snat = nullptr;
   int *sid = nullptr, *scell = nullptr;
   VCtl *ctl = nullptr;
   int *bmax = nullptr;
   size_t list_cap = 0;    // ints allocated for the lists
-  size_t list16_cap = 0;  // entries allocated for the tile-local 16-bit lists
   bool resident = false, resident_nat = false;
   int cur = 0;
   struct StepGraph {
@@ -1033,7 +996,7 @@ void vf_destroy(VerletFast *v) {
   void *b[] = {v->vstate[0], v->vstate[1], v->vsnap[0], v->vsnap[1], v->vomega[0], v->vomega[1], v->vid,
                v->vcell,     v->vnat,      v->list,     v->len,      v->key,       v->slotc,     v->count,
                v->start,     v->tmp,       v->blocksum, v->sstate,   v->snat,      v->sid,       v->scell,
-               v->ctl,       v->bmax,      v->vtiles,   v->list16};
+               v->ctl,       v->bmax,      v->vtiles};
   for (void *p : b) hipFree(p);
   delete v;
 }
@@ -1109,10 +1072,15 @@ int vf_create(VerletFast **out, hipStream_t st, const DevParams &P, double rho, 
   a.cells = v->cells;
   a.rmax2 = r_max * r_max;
   a.half_skin = 0.5 * (r_max - rho);
+  a.h = 1.0 / (double)ncv;
   a.r2c = (float)(rho * rho);
   a.r2h = (float)band(rho);
   a.r2k = (float)std::ldexp(1.0, std::ilogb(4.0 / (double)a.r2h) + 1);  // power of two, r2k * r2h > 4
   a.m2c = (float)(r_max * r_max);
+  a.unit = (float)(kMUnit * (double)ncv);
+  a.rho_u = (float)(rho * (double)a.unit);
+  a.r2_u = (float)(rho * rho * (double)a.unit * (double)a.unit);
+  a.drift = (float)(kMUnit * (1.0 + a.half_skin * ncv));
   a.m2h = (float)band(r_max);
   a.ctl = v->ctl;
   *out = v;
@@ -1164,19 +1132,13 @@ int vf_enter(VerletFast *v, hipStream_t st, const DevParams &P, int srk, const d
   if (const char *cap = std::getenv("SPSS_VERLET_WIDTH_CAP")) K = std::max(4, std::min(K, std::atoi(cap)));
   K = (K + 15) / 16 * 16;  // whole chunks of four entries, whole passes of sixteen
   const size_t need = ((size_t)v->n + 255) / 256 * 256 * (size_t)K;  // lslot's blocks of 256 slots
-  const size_t need16 = v->tiled ? (size_t)v->ncv * v->vt_cmax * (size_t)K * kVB : 0;  // tile-local
-  if (need > v->list_cap || need16 > v->list16_cap) {
+  if (need > v->list_cap) {
     drop_graphs(v);  // captured launches hold the old list pointer
     hipFree(v->list);
-    hipFree(v->list16);
     v->list = nullptr;
-    v->list16 = nullptr;
     v->list_cap = 0;
-    v->list16_cap = 0;
     VCHK(hipMalloc(&v->list, sizeof(int) * need));
-    if (v->tiled) VCHK(hipMalloc(&v->list16, sizeof(unsigned short) * need16));  // need16 entries
     v->list_cap = need;
-    v->list16_cap = need16;
   }
   if (K != v->K) drop_graphs(v);  // the width is a launch argument of the captured steps
   v->K = K;
@@ -1215,12 +1177,11 @@ static void launch_step(VerletFast *v, hipStream_t st, const DevParams &P, const
     const int ntiles = v->ncv * v->vt_cmax;
     const unsigned tg = (unsigned)((ntiles + 7) / 8 * 8);  // a multiple of 8 for xcd_block
     const unsigned gt = std::min(tg, (unsigned)kGateGrid);
-    vt_lists<S><<<gt, kVB, 0, st>>>(P, A, v->vtiles, ntiles, v->start, v->vcell, v->vstate[c], v->vsnap[c], v->list,
-                                    v->list16, v->len);
+    vt_lists<S><<<gt, kVB, 0, st>>>(P, A, v->vtiles, ntiles, v->start, v->vcell, v->vstate[c], v->list, v->len);
     vt_rest<S, SRK><<<gt, kVB, 0, st>>>(P, A, U, v->vtiles, ntiles, v->list, v->len, v->start, v->vcell, v->vstate[c],
                                         v->vid, nat, v->vsnap[c], v->vomega[c], v->vstate[o], v->vsnap[o],
                                         v->vomega[o], SRK ? compl_out : nullptr);
-    vt_step<S, SRK><<<tg, kVB, 0, st>>>(P, A, U, v->vtiles, ntiles, v->list, v->list16, v->len, v->start, v->vcell,
+    vt_step<S, SRK><<<tg, kVB, 0, st>>>(P, A, U, v->vtiles, ntiles, v->list, v->len, v->start, v->vcell,
                                         v->vstate[c], v->vid, nat, v->vsnap[c], v->vomega[c], v->vstate[o],
                                         v->vsnap[o], v->vomega[o], SRK ? compl_out : nullptr);
   } else {
@@ -1410,11 +1371,19 @@ int vf_status(VerletFast *v, hipStream_t st, int *should_update, double *acc, lo
   return SPSS_OK;
 }
 
-int vf_lists(VerletFast *v, hipStream_t st, std::vector<int> *counts, std::vector<int> *flat) {
+int vf_lists(VerletFast *v, hipStream_t st, const DevParams &P, std::vector<int> *counts, std::vector<int> *flat) {
   const int n = v->n;
   counts->assign(n, 0);
   flat->clear();
   if (!v->resident) return SPSS_OK;
+  if (v->tiled) {  // the tiles' steps need no lists
+    const unsigned nb = vblocks(n);
+    if (v->s == 4)
+      vc_lists<4><<<nb, kVB, 0, st>>>(P, v->A, v->start, v->vcell, v->sstate, v->list, v->len);
+    else
+      vc_lists<3><<<nb, kVB, 0, st>>>(P, v->A, v->start, v->vcell, v->sstate, v->list, v->len);
+    VCHK(hipGetLastError());
+  }
   std::vector<int> id(n), len(n), list(((size_t)n + 255) / 256 * 256 * (size_t)v->K);
   VCHK(hipMemcpyAsync(id.data(), v->vid, sizeof(int) * n, hipMemcpyDeviceToHost, st));
   VCHK(hipMemcpyAsync(len.data(), v->len, sizeof(int) * n, hipMemcpyDeviceToHost, st));

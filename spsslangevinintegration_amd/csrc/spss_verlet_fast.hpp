@@ -46,7 +46,7 @@ void vf_drop(VerletFast *v);
 int vf_status(VerletFast *v, hipStream_t st, int *should_update, double *acc, long *overflow);
 // the lists of the last rebuild in original particle ids: counts[n] by id, then each id's
 // neighbours in list order (stencil order of the build) into flat
-int vf_lists(VerletFast *v, hipStream_t st, std::vector<int> *counts, std::vector<int> *flat);
+int vf_lists(VerletFast *v, hipStream_t st, const DevParams &P, std::vector<int> *counts, std::vector<int> *flat);
 int vf_list_width(const VerletFast *v);
 
 }  // namespace spss
