@@ -30,18 +30,19 @@
 // formula on the stored positions, so neighbour sets are exact.
 //
 // One step is a rebuild -- launches that return at once unless the device flag asks for one:
-// cell keys and histogram, the two-level scan, bucket fill, stable rank and gather into scratch,
-// back into the resident arrays with the new snapshot, the row tiles, the lists -- and the step,
+// the flag, cell keys and histogram; the scan's blocks; starts and bucket fill; stable rank and gather into
+// scratch with the row tiles; back into the resident arrays with the new snapshot and the lists -- and the step,
 // which ends with the Euler/SRK update of step_particle, the new snapshot and the step's largest
-// squared displacement (maxima by group of workgroups); a one-wave launch after the step (vc_flag)
-// turns it into the next step's flag on the device.  No host synchronisation: steps replay from HIP
-// graphs.
+// squared displacement (maxima by group of workgroups), which the next step's first launch turns into its
+// flag on the device.  No host synchronisation: steps replay from HIP graphs.  Seven launches (tiled
+// grids): at N = 16,384 they are the step's time, 29 us, where ten took 34.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <cstddef>
 #include <cstdlib>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -59,20 +60,20 @@ namespace {
 thread_local std::string g_verr;
 constexpr int kVB = 256;         // threads per workgroup
 constexpr int kVGraphSteps = 10;  // steps of the bulk graph (even: the state buffers end where they started)
-constexpr int kGateGrid = 1024;   // workgroups of the launches that run on rebuilds (and vt_rest) only
+constexpr int kGateGrid = 1024;   // workgroups of the launches that run on rebuilds only
 }  // namespace
 
 // device control block
 constexpr int kGroups = 64, kLineU64 = 16;  // workgroup groups of the displacement maximum, a 128-byte line each
 struct VCtl {
-  int flag;                     // rebuild before the next step (should_update_lists_)
-  int pad0;
-  double acc;                   // accumulated_displacement_
+  int flag;                     // rebuild before this step (should_update_lists_), set by vr_keys
+  int force;                    // the resident copy was just entered: rebuild
+  double acc[2];                // accumulated_displacement_, by the parity of the step that reads it
   unsigned long long overflow;  // lists longer than the width K since entry (walked through their cells)
   unsigned long long step;      // Philox step of graph-replayed steps
   int big_tiles;                // tiles of the last rebuild holding more particles than a workgroup
-  int pad1;
-  // the step's largest |dr|^2 by group of workgroups (workgroup b in group b % kGroups), as the
+  int pad;
+  // the last step's largest |dr|^2 by group of workgroups (workgroup b in group b % kGroups), as the
   // bits of a non-negative double, one word per cache line so that the groups' atomics run apart
   unsigned long long gmax[kGroups * kLineU64];
 };
@@ -141,12 +142,27 @@ __host__ __device__ __forceinline__ long lslot(long p, long t, int K) {
 // ---------------------------------------------------------------------------
 // rebuild (every launch returns at once when the flag is clear)
 
+// Before the rest: CalculateMaxDisplacement's bookkeeping (ParticleSystemFirstOrderPtr.cpp:851-860) in
+// the exact mode (one step of margin) from the last step's group maxima, by every wave for itself; the
+// first workgroup leaves the result for the launches after this one, and advances the graph's Philox step.
 template <int S>
-__global__ __launch_bounds__(kVB) void vr_keys(DevParams P, VArgs A, const double *__restrict__ state,
-                                               int *__restrict__ key, int *__restrict__ slotc,
-                                               int *__restrict__ count) {
-  if (gate_off(A)) return;
-  if (blockIdx.x == 0 && threadIdx.x == 0) A.ctl->big_tiles = 0;  // counted again by vt_lists
+__global__ __launch_bounds__(kVB) void vr_keys(DevParams P, VArgs A, int parity, unsigned long long *step_inc,
+                                               const double *__restrict__ state, int *__restrict__ key,
+                                               int *__restrict__ slotc, int *__restrict__ count) {
+  {
+    double m = __longlong_as_double((long long)A.ctl->gmax[(threadIdx.x & 63) * kLineU64]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    const double stepd = sqrt(m), acc = A.ctl->acc[parity] + stepd;
+    const int flag = A.ctl->force || acc + stepd > A.half_skin;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      A.ctl->flag = flag;
+      if (flag) A.ctl->big_tiles = 0;  // counted again by vr_settle
+      A.ctl->acc[1 - parity] = flag ? 0.0 : acc;
+      if (step_inc) *step_inc += 1ull;
+    }
+    if (!flag) return;
+  }
   // the particles are in the last rebuild's cell order and have moved less than half the skin
   // since, so a wave holds a few runs of equal keys: one atomic per run, the run's lanes take
   // consecutive places after it (the order inside a cell is settled by vr_gather)
@@ -176,10 +192,44 @@ __global__ __launch_bounds__(kVB) void vr_keys(DevParams P, VArgs A, const doubl
   }
 }
 
+// the maxima cleared for this step, and the bucket fill.  local (grids of at most kScanLds scan blocks): the
+// starts inside the scan blocks, completed here with the blocks' totals; the counts cleared for their
+// next use
+constexpr int kScanLds = 512;
 __global__ __launch_bounds__(kVB) void vr_scatter(VArgs A, const int *__restrict__ key, const int *__restrict__ slotc,
-                                                  const int *__restrict__ start, int *__restrict__ tmp) {
+                                                  const int *__restrict__ local, const int *__restrict__ blocksum,
+                                                  int nsb, int *__restrict__ count, int *__restrict__ start,
+                                                  int *__restrict__ tmp) {
+  if (blockIdx.x == 0 && threadIdx.x < kGroups) {
+    A.ctl->gmax[threadIdx.x * kLineU64] = 0ull;
+    if (threadIdx.x == 0) A.ctl->force = 0;
+  }
   if (gate_off(A)) return;
-  for (int p = blockIdx.x * kVB + threadIdx.x; p < A.n; p += gridDim.x * kVB) tmp[start[key[p]] + slotc[p]] = p;
+  if (!local) {
+    for (int p = blockIdx.x * kVB + threadIdx.x; p < A.n; p += gridDim.x * kVB) tmp[start[key[p]] + slotc[p]] = p;
+    return;
+  }
+  __shared__ int off[kScanLds];
+  if (threadIdx.x < 64) {
+    int run = 0;
+    for (int b = threadIdx.x; b - (int)threadIdx.x < nsb; b += 64) {
+      const int v = b < nsb ? blocksum[b] : 0, incl = wave_incl_scan(v, threadIdx.x);
+      if (b < nsb) off[b] = run + incl - v;
+      run += __shfl(incl, 63, 64);
+    }
+  }
+  __syncthreads();
+  for (int t = blockIdx.x * kVB + threadIdx.x; t < max(A.n, A.cells); t += gridDim.x * kVB) {
+    if (t < A.n) {
+      const int c = key[t];
+      tmp[local[c] + off[c / (256 * kScanItems)] + slotc[t]] = t;
+    }
+    if (t < A.cells) {
+      start[t] = local[t] + off[t / (256 * kScanItems)];
+      count[t] = 0;
+    }
+    if (t == 0) start[A.cells] = A.n;
+  }
 }
 
 // each cell's particles in ascending previous slot, gathered into the new order in scratch: cells
@@ -191,8 +241,12 @@ __global__ __launch_bounds__(kVB) void vr_gather(VArgs A, const int *__restrict_
                                                  const int *__restrict__ tmp, const double *__restrict__ state,
                                                  const int *__restrict__ id, const double *__restrict__ nat,
                                                  double *__restrict__ sstate, int *__restrict__ sid,
-                                                 double *__restrict__ snat, int *__restrict__ scell) {
+                                                 double *__restrict__ snat, int *__restrict__ scell,
+                                                 int4 *__restrict__ tiles, int wcap, int cmax) {
   if (gate_off(A)) return;
+  // the row tiles of the new order (tiled grids), one wave per row in the first workgroups: they
+  // need only the final cell starts
+  if (tiles && (int)blockIdx.x * 4 < A.ncv) rows_to_tiles([&](int c) { return start[c]; }, A.ncv, wcap, cmax, tiles);
   const int lane = threadIdx.x & 63;
   auto move = [&](int p, int q, int c) {
 #pragma unroll
@@ -214,35 +268,6 @@ __global__ __launch_bounds__(kVB) void vr_gather(VArgs A, const int *__restrict_
     int r = 0;
     for (int t = b; t < e; ++t) r += tmp[t] < p ? 1 : 0;
     move(p, b + r, c);
-  }
-}
-
-// back into the resident arrays, with the snapshot of the new order
-template <int S>
-__global__ __launch_bounds__(kVB) void vr_settle(DevParams P, VArgs A, const double *__restrict__ sstate,
-                                                 const int *__restrict__ sid, const double *__restrict__ snat,
-                                                 const int *__restrict__ scell, double *__restrict__ state,
-                                                 int *__restrict__ id, double *__restrict__ nat,
-                                                 int *__restrict__ cell, float4 *__restrict__ snap,
-                                                 float *__restrict__ omega, const int *__restrict__ start,
-                                                 int4 *__restrict__ tiles, int wcap, int cmax) {
-  if (gate_off(A)) return;
-  // the row tiles of the new order (tiled grids), one wave per row in the first workgroups: they
-  // need only the final cell starts
-  if (tiles && (int)blockIdx.x * 4 < A.ncv) rows_to_tiles([&](int c) { return start[c]; }, A.ncv, wcap, cmax, tiles);
-  for (int q = blockIdx.x * kVB + threadIdx.x; q < A.n; q += gridDim.x * kVB) {
-    double st[S];
-#pragma unroll
-    for (int k = 0; k < S; ++k) {
-      st[k] = sstate[(long)q * S + k];
-      state[(long)q * S + k] = st[k];
-    }
-    id[q] = sid[q];
-    if (nat) nat[q] = snat[q];
-    const int c = scell[q];
-    cell[q] = c;
-    snap[q] = tiles ? vsnap_cell(P, st, c % A.ncv, c / A.ncv, A.h) : vsnap_of(P, st);
-    omega[q] = S == 4 ? (float)st[3] : 0.f;
   }
 }
 
@@ -457,7 +482,7 @@ __device__ __forceinline__ int xcd_block(int b, int nblocks) {
   return (b & 7) * per + (b >> 3);
 }
 
-// The step's largest squared displacement, for vc_flag: wave, workgroup, then one atomic per
+// The step's largest squared displacement, for the next step's vr_keys: wave, workgroup, then one atomic per
 // workgroup on the maximum of its group (kGroups words on their own cache lines).  (A last-workgroup
 // count in the step kernel needs a release fence per workgroup, which writes the XCD's L2 back:
 // 0.45 ms per step at N = 1M with 7,000 workgroups.)
@@ -565,25 +590,44 @@ __device__ __forceinline__ int vt_plan(const VArgs &A, const int *__restrict__ s
   return ((L.len[0] + 15) & ~15) + ((L.len[1] + 15) & ~15) + ((L.len[2] + 15) & ~15);
 }
 
-// The lists of the tiles that walk theirs: in list_of_slot's order (stencil cells in order, ascending
-// slot inside a cell).
+// back into the resident arrays, with the snapshot of the new order
 template <int S>
-__global__ __launch_bounds__(kVB) void vt_lists(DevParams P, VArgs A, const int4 *__restrict__ tiles, int ntiles,
-                                                const int *__restrict__ start, const int *__restrict__ cell,
-                                                const double *__restrict__ state, int *__restrict__ list,
-                                                int *__restrict__ len) {
+__global__ __launch_bounds__(kVB) void vr_settle(DevParams P, VArgs A, const double *__restrict__ sstate,
+                                                 const int *__restrict__ sid, const double *__restrict__ snat,
+                                                 const int *__restrict__ scell, double *__restrict__ state,
+                                                 int *__restrict__ id, double *__restrict__ nat,
+                                                 int *__restrict__ cell, float4 *__restrict__ snap,
+                                                 float *__restrict__ omega, const int *__restrict__ start,
+                                                 const int4 *__restrict__ tiles, int ntiles, int *__restrict__ list,
+                                                 int *__restrict__ len) {
   if (gate_off(A)) return;
+  for (int q = blockIdx.x * kVB + threadIdx.x; q < A.n; q += gridDim.x * kVB) {
+    double st[S];
+#pragma unroll
+    for (int k = 0; k < S; ++k) {
+      st[k] = sstate[(long)q * S + k];
+      state[(long)q * S + k] = st[k];
+    }
+    id[q] = sid[q];
+    if (nat) nat[q] = snat[q];
+    const int c = scell[q];
+    cell[q] = c;
+    snap[q] = tiles ? vsnap_cell(P, st, c % A.ncv, c / A.ncv, A.h) : vsnap_of(P, st);
+    omega[q] = S == 4 ? (float)st[3] : 0.f;
+  }  // tiled grids: the lists of the tiles that walk theirs, from the scratch copy of the state, in
+  // list_of_slot's order
   __shared__ VtPlan L;
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {  // (the same for the whole workgroup)
+  for (int tile = tiles ? blockIdx.x : ntiles; tile < ntiles; tile += gridDim.x) {  // (the same for the whole workgroup)
     const int4 td = tiles[tile];
     const int row = td.y, ca = td.z, cb = td.w;
     if (ca >= cb) continue;  // an unused tile slot
     __syncthreads();  // the previous tile's plan is consumed
     const int total = vt_plan(A, start, row, ca, cb, L);
-    const int gtb = start[row * A.ncv + ca], ntile = start[row * A.ncv + cb] - gtb;
-    if (ntile > kVB && threadIdx.x == 0) atomicAdd(&A.ctl->big_tiles, 1);
-    if (total <= kMStage && ntile <= kVB) continue;
-    for (int u = threadIdx.x; u < ntile; u += kVB) list_of_slot<S, true>(P, A, start, cell, state, nullptr, list, len, gtb + u);
+    const int gtb = start[row * A.ncv + ca], nt = start[row * A.ncv + cb] - gtb;
+    if (nt > kVB && threadIdx.x == 0) atomicAdd(&A.ctl->big_tiles, 1);
+    if (total <= kMStage && nt <= kVB) continue;
+    for (int u = threadIdx.x; u < nt; u += kVB)
+      list_of_slot<S, true>(P, A, start, scell, sstate, nullptr, list, len, gtb + u);
   }
 }
 
@@ -600,7 +644,7 @@ struct VtLds {
 // taken from the tile's centre.  False: a staged value is not finite (the same for every thread).
 template <int S, int W>
 __device__ __forceinline__ bool vt_sums(const DevParams &P, const VArgs &A, int row, int ca, int cb, int gtb, int ntile,
-                                        int total, const int *__restrict__ cell, const double *__restrict__ state,
+                                        const int *__restrict__ cell, const double *__restrict__ state,
                                         const float4 *__restrict__ snap, const float *__restrict__ omega,
                                         VtLds<W> &Ls, MSums &sum) {
   constexpr int kPasses = 5;  // chunks of 64 entries per wave: at most kMStage / 64 and two for the rows' rests
@@ -848,7 +892,7 @@ __global__ __launch_bounds__(kVB, 3) void vt_step(DevParams P, VArgs A, StepArgs
     const int ntile = start[row * A.ncv + cb] - gtb;
     const bool staged = total <= kMStage;
     MSums sum;
-    const bool have = staged && vt_sums<S, W>(P, A, row, ca, cb, gtb, ntile, total, cell, state, snap, omega, Ls, sum);
+    const bool have = staged && vt_sums<S, W>(P, A, row, ca, cb, gtb, ntile, cell, state, snap, omega, Ls, sum);
     const int u = threadIdx.x, p = gtb + u;
     if (u < ntile) {
       // (rare) staged values that are not finite: the cells; an overflowing stage: the list
@@ -873,31 +917,11 @@ __global__ __launch_bounds__(kVB) void vc_block_max(VArgs A, const int *__restri
 
 __global__ void vc_enter(VCtl *c) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
-    c->flag = 1;  // should_update_lists_ starts true (ParticleSystemFirstOrderPtr.cpp:99)
-    c->acc = 0.0;
+    c->flag = c->force = 1;  // should_update_lists_ starts true (ParticleSystemFirstOrderPtr.cpp:99)
+    c->acc[0] = c->acc[1] = 0.0;
     c->overflow = 0ull;
   }
   for (int g = threadIdx.x; g < kGroups; g += blockDim.x) c->gmax[g * kLineU64] = 0ull;
-}
-
-// After the step: CalculateMaxDisplacement's bookkeeping (ParticleSystemFirstOrderPtr.cpp:851-860)
-// in the exact mode (one step of margin) from the group maxima, which are cleared for the next
-// step; the graph's Philox step counter advances (the step kernel has read it).  One wave.
-__global__ void vc_flag(VCtl *c, double half_skin, unsigned long long *step_inc) {
-  const int lane = threadIdx.x;
-  double m = __longlong_as_double((long long)c->gmax[lane * kLineU64]);
-  c->gmax[lane * kLineU64] = 0ull;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
-  if (lane == 0) {
-    const double stepd = sqrt(m);
-    double acc = c->acc + stepd;
-    const int flag = acc + stepd > half_skin ? 1 : 0;
-    if (flag) acc = 0.0;
-    c->acc = acc;
-    c->flag = flag;
-    if (step_inc) *step_inc += 1ull;
-  }
 }
 
 __global__ void vc_set_step(VCtl *c, unsigned long long v) {
@@ -945,7 +969,7 @@ struct VerletFast {
   bool tiled = false;
   int vt_wcap = 0, vt_cmax = 0;
   int4 *vtiles = nullptr;
-  int *key = nullptr, *slotc = nullptr, *count = nullptr, *start = nullptr, *tmp = nullptr, *blocksum = nullptr;
+  int *local = nullptr, *key = nullptr, *slotc = nullptr, *count = nullptr, *start = nullptr, *tmp = nullptr, *blocksum = nullptr;
   double *sstate = nullptr, *snat = nullptr;
   int *sid = nullptr, *scell = nullptr;
   VCtl *ctl = nullptr;
@@ -996,7 +1020,7 @@ void vf_destroy(VerletFast *v) {
   void *b[] = {v->vstate[0], v->vstate[1], v->vsnap[0], v->vsnap[1], v->vomega[0], v->vomega[1], v->vid,
                v->vcell,     v->vnat,      v->list,     v->len,      v->key,       v->slotc,     v->count,
                v->start,     v->tmp,       v->blocksum, v->sstate,   v->snat,      v->sid,       v->scell,
-               v->ctl,       v->bmax,      v->vtiles};
+               v->ctl,       v->bmax,      v->vtiles,   v->local};
   for (void *p : b) hipFree(p);
   delete v;
 }
@@ -1053,6 +1077,7 @@ int vf_create(VerletFast **out, hipStream_t st, const DevParams &P, double rho, 
     const double row_mean = (double)n / (double)ncv;
     v->vt_cmax = std::max((ncv + v->vt_wcap - 1) / v->vt_wcap,
                           std::min(ncv, (int)std::ceil(1.5 * row_mean / (0.94 * kTileCap)) + 2));
+    A(hipMalloc(&v->local, sizeof(int) * (size_t)v->cells));
     A(hipMalloc(&v->vtiles, sizeof(int4) * (size_t)ncv * v->vt_cmax));
   }
   if (e != hipSuccess) {
@@ -1115,9 +1140,9 @@ int vf_enter(VerletFast *v, hipStream_t st, const DevParams &P, int srk, const d
   // block, and the counts cleared again for the first rebuild
   launch_fill_int(st, 1, v->bmax, 0);
   if (v->s == 4)
-    vr_keys<4><<<nb, kVB, 0, st>>>(P, v->A, v->vstate[0], v->key, v->slotc, v->count);
+    vr_keys<4><<<nb, kVB, 0, st>>>(P, v->A, 0, nullptr, v->vstate[0], v->key, v->slotc, v->count);
   else
-    vr_keys<3><<<nb, kVB, 0, st>>>(P, v->A, v->vstate[0], v->key, v->slotc, v->count);
+    vr_keys<3><<<nb, kVB, 0, st>>>(P, v->A, 0, nullptr, v->vstate[0], v->key, v->slotc, v->count);
   vc_block_max<<<vblocks(v->cells), kVB, 0, st>>>(v->A, v->count, v->bmax);
   int bmax = 0;
   VCHK(hipMemcpyAsync(&bmax, v->bmax, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -1160,30 +1185,30 @@ static void launch_step(VerletFast *v, hipStream_t st, const DevParams &P, const
   // the rebuild launches return at once on most steps: a fixed grid of at most kGateGrid
   // workgroups (grid-stride loops) keeps what they cost then down to a dispatch
   const unsigned gg = std::min(nb, (unsigned)kGateGrid);
-  vr_keys<S><<<gg, kVB, 0, st>>>(P, A, v->vstate[c], v->key, v->slotc, v->count);
-  scan_local<<<v->nsb, 256, 0, st>>>(v->count, nullptr, v->cells, v->start, v->blocksum, ctl_flag(A.ctl));
-  scan_add<<<v->nsb, 256, 0, st>>>(v->count, nullptr, v->cells, v->start, v->blocksum, v->nsb, nullptr,
-                                   ctl_flag(A.ctl));
-  vr_scatter<<<gg, kVB, 0, st>>>(A, v->key, v->slotc, v->start, v->tmp);
-  vr_gather<S><<<gg, kVB, 0, st>>>(A, v->key, v->start, v->tmp, v->vstate[c], v->vid, nat, v->sstate, v->sid, v->snat,
-                                   v->scell);
-  // tiled grids: the row tiles of the new order are built by vr_settle's first workgroups, so its
+  vr_keys<S><<<gg, kVB, 0, st>>>(P, A, c, U.step_inc, v->vstate[c], v->key, v->slotc, v->count);
+  scan_local<<<v->nsb, 256, 0, st>>>(v->count, nullptr, v->cells, v->tiled ? v->local : v->start, v->blocksum,
+                                     ctl_flag(A.ctl));
+  if (!v->tiled)
+    scan_add<<<v->nsb, 256, 0, st>>>(v->count, nullptr, v->cells, v->start, v->blocksum, v->nsb, nullptr,
+                                     ctl_flag(A.ctl));
+  vr_scatter<<<gg, kVB, 0, st>>>(A, v->key, v->slotc, v->local, v->blocksum, v->nsb, v->count, v->start, v->tmp);
+  // tiled grids: the row tiles of the new order are built by vr_gather's first workgroups, so its
   // grid covers a wave per row as well
   const unsigned sg = v->tiled ? std::max(gg, (unsigned)((v->ncv + 3) / 4)) : gg;
-  vr_settle<S><<<sg, kVB, 0, st>>>(P, A, v->sstate, v->sid, v->snat, v->scell, v->vstate[c], v->vid,
+  vr_gather<S><<<sg, kVB, 0, st>>>(A, v->key, v->start, v->tmp, v->vstate[c], v->vid, nat, v->sstate, v->sid, v->snat,
+                                   v->scell, v->tiled ? v->vtiles : nullptr, v->vt_wcap, v->vt_cmax);
+  const int ntiles = v->tiled ? v->ncv * v->vt_cmax : 0;
+  vr_settle<S><<<gg, kVB, 0, st>>>(P, A, v->sstate, v->sid, v->snat, v->scell, v->vstate[c], v->vid,
                                    nat ? v->vnat : nullptr, v->vcell, v->vsnap[c], v->vomega[c], v->start,
-                                   v->tiled ? v->vtiles : nullptr, v->vt_wcap, v->vt_cmax);
+                                   v->tiled ? v->vtiles : nullptr, ntiles, v->list, v->len);
   if (v->tiled) {
-    const int ntiles = v->ncv * v->vt_cmax;
     const unsigned tg = (unsigned)((ntiles + 7) / 8 * 8);  // a multiple of 8 for xcd_block
-    const unsigned gt = std::min(tg, (unsigned)kGateGrid);
-    vt_lists<S><<<gt, kVB, 0, st>>>(P, A, v->vtiles, ntiles, v->start, v->vcell, v->vstate[c], v->list, v->len);
-    vt_rest<S, SRK><<<gt, kVB, 0, st>>>(P, A, U, v->vtiles, ntiles, v->list, v->len, v->start, v->vcell, v->vstate[c],
+    vt_rest<S, SRK><<<std::min(tg, (unsigned)kGateGrid), kVB, 0, st>>>(
+        P, A, U, v->vtiles, ntiles, v->list, v->len, v->start, v->vcell, v->vstate[c], v->vid, nat, v->vsnap[c],
+        v->vomega[c], v->vstate[o], v->vsnap[o], v->vomega[o], SRK ? compl_out : nullptr);
+    vt_step<S, SRK><<<tg, kVB, 0, st>>>(P, A, U, v->vtiles, ntiles, v->list, v->len, v->start, v->vcell, v->vstate[c],
                                         v->vid, nat, v->vsnap[c], v->vomega[c], v->vstate[o], v->vsnap[o],
                                         v->vomega[o], SRK ? compl_out : nullptr);
-    vt_step<S, SRK><<<tg, kVB, 0, st>>>(P, A, U, v->vtiles, ntiles, v->list, v->len, v->start, v->vcell,
-                                        v->vstate[c], v->vid, nat, v->vsnap[c], v->vomega[c], v->vstate[o],
-                                        v->vsnap[o], v->vomega[o], SRK ? compl_out : nullptr);
   } else {
     vr_lists<S><<<nb, kVB, 0, st>>>(P, A, v->start, v->vcell, v->vstate[c], v->vsnap[c], v->list, v->len);
     const unsigned nb8 = (nb + 7u) & ~7u;  // a multiple of 8 for xcd_block
@@ -1191,7 +1216,6 @@ static void launch_step(VerletFast *v, hipStream_t st, const DevParams &P, const
                                          v->vsnap[c], v->vomega[c], v->vstate[o], v->vsnap[o], v->vomega[o],
                                          SRK ? compl_out : nullptr);
   }
-  vc_flag<<<1, kGroups, 0, st>>>(A.ctl, A.half_skin, U.step_inc);
 }
 
 static StepArgs vstep_args(double dt, double D_phi, double friction, int noise_mode, const double *noise,
@@ -1325,7 +1349,7 @@ long vf_run_graph(VerletFast *v, hipStream_t st, const DevParams &P, int srk, co
     if (side) v->cur = 1 - v->cur;
   }
   if (rc != SPSS_OK) return -1;
-  vc_set_step<<<1, 64, 0, st>>>(v->ctl, (unsigned long long)step);
+  vc_set_step<<<1, 64, 0, st>>>(v->ctl, (unsigned long long)step - 1ull);  // vr_keys advances it first
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
     g_verr = std::string("vc_set_step: ") + hipGetErrorString(e);
@@ -1363,10 +1387,19 @@ int vf_status(VerletFast *v, hipStream_t st, int *should_update, double *acc, lo
     VCHK(hipMemcpyAsync(&c, v->ctl, sizeof(VCtl), hipMemcpyDeviceToHost, st));
     VCHK(hipStreamSynchronize(st));
   } else {
-    c.flag = 1;  // the next step enters and rebuilds
+    c.force = 1;  // the next step enters and rebuilds
   }
-  if (should_update) *should_update = c.flag;
-  if (acc) *acc = c.acc;
+  // what the next vr_keys will find
+  double m = 0.0;
+  for (int g = 0; g < kGroups; ++g) {
+    double d;
+    std::memcpy(&d, &c.gmax[g * kLineU64], sizeof(d));
+    m = std::max(m, d);
+  }
+  const double stepd = std::sqrt(m), a = c.acc[v->cur] + stepd;
+  const int flag = c.force || a + stepd > v->A.half_skin;
+  if (should_update) *should_update = flag;
+  if (acc) *acc = flag ? 0.0 : a;
   if (overflow) *overflow = (long)c.overflow;
   return SPSS_OK;
 }
