@@ -30,7 +30,8 @@ namespace spss {
 
 namespace {
 constexpr int kFB = kTileCap;   // threads per pair workgroup (one particle of a row tile each)
-constexpr int kStageMax = 1024; // staged entries per workgroup (particles + row padding)
+constexpr int kStageMax = 1120; // staged entries per workgroup (particles + row padding): 1,024 left a step of
+                                // 1M particles a few tiles to redo (fr_far 10.9, now 4.7 us; fr_pairs +0.4)
 constexpr int kPad = 4;         // padding entries after each staged row (>= the unroll - 1)
 constexpr int kMaxCells = 336;  // staged cells (2ky+1) x (W+2kx) of one workgroup
 constexpr int kMaxSpan = 25;    // stencil columns 2kx+1 (kx = k * xsplit <= 12)
@@ -973,7 +974,8 @@ __global__ __launch_bounds__(256) void fr_scatter(
   double sn2 = 0.0, cn2 = 1.0, xw2 = 0.0, yw2 = 0.0;
   if (valid) {
     const int cpr = L.cpr;
-    const int r = L.nrep == 1 ? 0 : cs / cpr, base = r * cpr;
+    int ls = cs;  // the old cell inside its replica
+    const int r = L.nrep == 1 ? 0 : div_small(cs, cpr, ls), base = r * cpr;
     Coef K;
     if (U.coef) {
       K = U.coef[r];
@@ -992,9 +994,11 @@ __global__ __launch_bounds__(256) void fr_scatter(
     step_particle<S, SRK>(P, K, rstate + (long)p * S, id - L.rep_first[r], nat_i, ssum[p],
                           SRK ? tsum[p] : make_double2(0.0, 0.0), scnt[p], U, step, out, C);
     if (SRK && compl_out) compl_out[id] = C;
-    int cd;
+    int cd, tx, ty;
     if (d == kFar) {
-      cd = base + cell_of_position<S>(P, out[0], out[1], ncx, ncy);
+      const int ld = cell_of_position<S>(P, out[0], out[1], ncx, ncy);
+      cd = base + ld;
+      ty = div_small(ld, ncx, tx);
       const int b = nstart[cd] + new_count_of(cnt9, cd, ncx, ncy, cpr);
       const int e = nstart[cd + 1];
       int rank = 0;
@@ -1003,9 +1007,10 @@ __global__ __launch_bounds__(256) void fr_scatter(
     } else {
       // destination cell, then the arrivals ordered before move d: the counts of the moves e
       // with move_order(e) < move_order(d) out of their source cells (ncx, ncy >= 3: one wrap each)
-      const int ls = cs - base;
-      const int cx = ls % ncx, cy = ls / ncx;
-      const int tx = wrap_cell(cx + d % 3 - 1, ncx), ty = wrap_cell(cy + d / 3 - 1, ncy);
+      int cx;
+      const int cy = div_small(ls, ncx, cx);
+      tx = wrap_cell(cx + d % 3 - 1, ncx);
+      ty = wrap_cell(cy + d / 3 - 1, ncy);
       cd = base + ty * ncx + tx;
       int b0 = 0;
       const int od = move_order(d);
@@ -1030,8 +1035,7 @@ __global__ __launch_bounds__(256) void fr_scatter(
       // position for the next move
       phasor_of(out[2], sn2, cn2);
       apply_pbc(P, out[0], out[1], xw2, yw2);
-      const int ld = cd - base;
-      snap[pos] = make_float4((float)(xw2 - (double)(ld % ncx) * Hx), (float)(yw2 - (double)(ld / ncx) * Hy),
+      snap[pos] = make_float4((float)(xw2 - (double)tx * Hx), (float)(yw2 - (double)ty * Hy),
                               (float)cn2, (float)sn2);
       if (omega_f) omega_f[pos] = (S == 4) ? (float)out[3] : 0.f;
     }
@@ -1041,13 +1045,8 @@ __global__ __launch_bounds__(256) void fr_scatter(
                            newcnt, farlist, farlist_n);
 }
 
-// advance the device step counter of graph-replayed runs
-__global__ void fb_step_inc(unsigned long long *step) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1ull;
-}
-
 // per replica: the phase order parameter Z = (1/N) sum e^{i phi} of the resident snapshot,
-// summed in FP64 in a fixed tree; when the step counter has reached `from`, |Z| and |Z|^2 are
+// summed in FP64 in a fixed tree; when `from` steps are done (the counter is the last one's), |Z| and |Z|^2 are
 // added to the replica's running sums (one block per replica)
 __global__ __launch_bounds__(256) void fb_order_stats(Layout L, const float4 *__restrict__ snap,
                                                       const unsigned long long *__restrict__ step,
@@ -1077,7 +1076,7 @@ __global__ __launch_bounds__(256) void fb_order_stats(Layout L, const float4 *__
     const double zr = sc[0] * inv, zi = ss[0] * inv;
     zlast[2 * r] = zr;
     zlast[2 * r + 1] = zi;
-    if (*step >= from) {
+    if (*step + 1ull >= from) {
       const double R2 = zr * zr + zi * zi;
       racc[3 * r] += sqrt(R2);
       racc[3 * r + 1] += R2;

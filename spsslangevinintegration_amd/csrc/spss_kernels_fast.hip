@@ -905,11 +905,8 @@ int fast_batch_step(FastPath *f, hipStream_t st, const DevParams &P, const doubl
   StepArgs U = step_args(dt, 0.0, 0.0, 3, nullptr, 0, 0);
   U.coef = f->coef;
   U.step_dev = f->step_dev;
-  int rc = step_impl(f, st, P, false, state, nat, nullptr, U);
-  if (rc != SPSS_OK) return rc;
-  fb_step_inc<<<1, 64, 0, st>>>(f->step_dev);
-  FCHK(hipGetLastError());
-  return SPSS_OK;
+  U.step_inc = f->step_dev;  // the counter is one behind the step to come, advanced by its fr_pairs
+  return step_impl(f, st, P, false, state, nat, nullptr, U);
 }
 
 int fast_prepare_moves(FastPath *f, hipStream_t st, const DevParams &P, double dt) {
@@ -928,7 +925,7 @@ int fast_batch_observe(FastPath *f, hipStream_t st, uint64_t from) {
 
 int fast_batch_reset(FastPath *f, hipStream_t st, uint64_t step) {
   launch_fill_double(st, 3L * f->R, f->racc, 0.0);
-  const unsigned long long v = step;
+  const unsigned long long v = (unsigned long long)step - 1ull;  // advanced before use
   FCHK(hipMemcpyAsync(f->step_dev, &v, sizeof(v), hipMemcpyHostToDevice, st));
   FCHK(hipStreamSynchronize(st));
   return SPSS_OK;
@@ -940,7 +937,7 @@ int fast_batch_stats(FastPath *f, hipStream_t st, double *racc, double *zlast, u
   if (zlast) FCHK(hipMemcpyAsync(zlast, f->zlast, sizeof(double) * 2 * f->R, hipMemcpyDeviceToHost, st));
   FCHK(hipMemcpyAsync(&v, f->step_dev, sizeof(v), hipMemcpyDeviceToHost, st));
   FCHK(hipStreamSynchronize(st));
-  if (step) *step = v;
+  if (step) *step = v + 1ull;
   return SPSS_OK;
 }
 
