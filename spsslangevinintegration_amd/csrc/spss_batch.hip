@@ -16,6 +16,7 @@
 
 #include "../../include/spss_hip.h"
 #include "spss_fast.hpp"
+#include "spss_hostcopy.hpp"
 #include "spss_launch.hpp"
 
 using namespace spss;
@@ -29,6 +30,7 @@ struct spss_batch {
   double *state = nullptr, *nat = nullptr;  // master state and natural frequencies, replica order
   bool have_nat = false;
   bool master_stale = false;  // the resident copy is ahead of `state`
+  HostCopy copy;
   std::vector<int> rep_n;
   std::vector<Coef> coef;  // per-replica coefficients (to rebuild the cell path at another cell size)
   int nc = 1, k = 1;       // int(1/rho) and the cell subdivision of the current cell path
@@ -264,8 +266,7 @@ int spss_batch_set_state(spss_batch *b, const double *host_state) {
 int spss_batch_get_state(spss_batch *b, double *host_state) {
   if (!b || !host_state) return set_error(SPSS_ERR_INVALID, "NULL argument");
   BTRY(sync_master(b));
-  BCHK(hipMemcpyAsync(host_state, b->state, sizeof(double) * (size_t)b->s * b->n, hipMemcpyDeviceToHost, b->st));
-  BCHK(hipStreamSynchronize(b->st));
+  BCHK(b->copy.to_host(host_state, b->state, sizeof(double) * (size_t)b->s * b->n, b->st));
   return SPSS_OK;
 }
 

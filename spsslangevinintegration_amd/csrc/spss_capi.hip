@@ -18,6 +18,7 @@
 
 #include "../../include/spss_hip.h"
 #include "spss_fast.hpp"
+#include "spss_hostcopy.hpp"
 #include "spss_launch.hpp"
 #include "spss_scan.hpp"
 #include "spss_verlet_fast.hpp"
@@ -96,6 +97,7 @@ struct spss_system {
   int ap_config = kAllPairsDefault;  // all-pairs workgroup and j-tile sizes (spss_autotune_all_pairs)
   int xsplit = 1;                    // FP32C cell grid: columns per square cell (spss_set_cell_layout)
   void *scratch = nullptr;  // of the observers (system_scratch)
+  HostCopy copy;
   size_t scratch_cap = 0;
   KernelTimer *timer = nullptr;  // around the pair kernel of the RHS
   // Dormand-Prince 5(4) buffers (allocated on first use): two states and derivatives, k2..k6,
@@ -729,8 +731,7 @@ int spss_set_state(spss_system *h, const double *host_state) {
 int spss_get_state(spss_system *h, double *host_state) {
   if (!h || !host_state) return fail(SPSS_ERR_INVALID, "NULL argument");
   TRY(sync_master(h));
-  HIPCHECK(hipMemcpyAsync(host_state, h->state, sizeof(double) * h->s * h->n, hipMemcpyDeviceToHost, h->stream));
-  HIPCHECK(hipStreamSynchronize(h->stream));
+  HIPCHECK(h->copy.to_host(host_state, h->state, sizeof(double) * h->s * h->n, h->stream));
   return SPSS_OK;
 }
 
@@ -1252,6 +1253,8 @@ int system_view(spss_system *h, SystemView *v) {
   v->y_rsize = h->P.yrs;
   return SPSS_OK;
 }
+
+HostCopy &system_copy(spss_system *h) { return h->copy; }
 
 int system_scratch(spss_system *h, size_t bytes, void **p) {
   if (bytes > h->scratch_cap) {

@@ -26,6 +26,8 @@ namespace spss {
 int system_view(spss_system *h, SystemView *v);
 // device scratch of at least `bytes` bytes, kept by the handle; what it holds is lost at the next call
 int system_scratch(spss_system *h, size_t bytes, void **p);
+class HostCopy;
+HostCopy &system_copy(spss_system *h);
 
 // two HIP events timing a stretch of one stream, destroyed with the object (also on the early
 // returns of an error path)

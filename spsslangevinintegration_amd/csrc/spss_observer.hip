@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "../../include/spss_hip.h"
+#include "spss_hostcopy.hpp"
 #include "spss_launch.hpp"
 #include "spss_seqsum.hpp"
 
@@ -258,8 +259,7 @@ int frame_to_host(spss_system *sys, double t, float *host) {
     hipLaunchKernelGGL(ob_frame, dim3(nb), dim3(256), 0, v.stream, v.state, m, v.s, v.s == 6 ? 0 : 1, v.x_size,
                        v.y_size, v.x_rsize, v.y_rsize, d);
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess && m > 0) e = hipMemcpyAsync(host + 1, d, sizeof(float) * m, hipMemcpyDeviceToHost, v.stream);
-  if (e == hipSuccess) e = hipStreamSynchronize(v.stream);
+  if (e == hipSuccess) e = system_copy(sys).to_host(host + 1, d, sizeof(float) * m, v.stream);
   OCHK(e);
   host[0] = (float)t;
   return SPSS_OK;
