@@ -69,8 +69,7 @@ struct spss_system {
   CellBuffers cells, vcells;
   Cells64 cells64;
   int *vcount = nullptr, *vstart = nullptr, *vlist = nullptr, *vslot = nullptr;
-  int *vhuge = nullptr;         // set by phases beyond the pair loop's range, cleared at a build
-  double *vstage = nullptr;     // stage state in the order of the lists' build
+  VerletStage vstage;           // stage state in the order of the lists' build
   long vcap = 0;
   const int *vorder = nullptr;  // cell order of the lists' build (null: built over all pairs)
   int *pcount = nullptr, *pstart = nullptr, *plist = nullptr;
@@ -269,9 +268,11 @@ int build_verlet(spss_system *h, int m) {
     TRY(dalloc_n(&h->vslot, (size_t)cap));
     h->vcap = cap;
   }
-  if (!h->vhuge) TRY(dalloc_n(&h->vhuge, 1));
-  if (!h->vstage) TRY(dalloc_n(&h->vstage, (size_t)h->s * h->n));
-  launch_fill_int(st, 1, h->vhuge, 0);
+  if (!h->vstage.stage) {
+    TRY(dalloc_n(&h->vstage.rec, (size_t)4 * h->n));
+    TRY(dalloc_n(&h->vstage.om, (size_t)h->n));
+    TRY(dalloc_n(&h->vstage.stage, (size_t)h->s * h->n));
+  }
   if (m == SPSS_METHOD_VERLET)
     launch_verlet_fill_all(st, h->P, h->stage, rmax2, h->vstart, h->vlist, h->vslot);
   else
@@ -328,8 +329,8 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
         TRY(build_verlet(h, m));
         h->should_update = false;
       }
-      launch_stage_order(st, h->n, h->s, d_state, d_kprev, k_coef * dt, h->vorder, h->vstage, h->vhuge);
-      launch_verlet_pairs(st, h->P, h->vstage, h->vorder, h->vstart, h->vslot, h->vhuge, nat, d_knext, compl_out);
+      launch_stage_order(st, h->P, d_state, d_kprev, k_coef * dt, h->vorder, h->vstage);
+      launch_verlet_pairs(st, h->P, h->vstage, h->vorder, h->vstart, h->vslot, nat, d_knext, compl_out);
       h->uses_verlet = true;
       break;
     default:
@@ -676,7 +677,7 @@ int spss_destroy(spss_system *h) {
   delete h->timer;
   void *bufs[] = {h->state, h->stage, h->k[0], h->k[1], h->k[2], h->k[3], h->deriv, h->compl_f, h->nat,
                   h->noise, h->partial, h->scal, h->acc, h->io[0], h->io[1], h->io[2], h->vcount, h->vstart,
-                  h->vlist, h->vslot, h->vstage, h->vhuge, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec, h->scratch};
+                  h->vlist, h->vslot, h->vstage.stage, h->vstage.rec, h->vstage.om, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec, h->scratch};
   for (void *b : bufs) hipFree(b);
   for (double *b : h->dp) hipFree(b);
   if (h->dp_host) hipHostFree(h->dp_host);

@@ -206,93 +206,106 @@ __global__ __launch_bounds__(kBlock) void k_verlet_build_cells(DevParams P, cons
   if (!FILL && t < P.n && (threadIdx.x & (LPP - 1)) == 0) vcount[i] = cnt;
 }
 
-// stage state in the order of the lists' build (order null: as it is).  `huge` (cleared at the
-// build) is set by a finite phase beyond kPhase64.
+// stage state in the order of the lists' build (order null: as it is), and what the pair sums read of
+// it: x, y wrapped into the box (NaN farther out than the guard band covers) and the phasor in the frame
+// of particle 0's phase; om: omega from particle 0's (may be null)
 template <int S>
-__global__ __launch_bounds__(kBlock) void k_stage_order(int n, const double *__restrict__ state,
+__global__ __launch_bounds__(kBlock) void k_stage_order(DevParams P, const double *__restrict__ state,
                                                         const double *__restrict__ kprev, double kc_dt,
                                                         const int *__restrict__ order, double *__restrict__ vstage,
-                                                        int *__restrict__ huge) {
+                                                        double4 *__restrict__ rec, double *__restrict__ om) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= n) return;
+  if (t >= P.n) return;
   const long i = order ? order[t] : t;
-  double v[S];
+  double v[S], first[S];
 #pragma unroll
-  for (int q = 0; q < S; ++q) v[q] = state[i * S + q] + (kprev ? kc_dt * kprev[i * S + q] : 0.0);
+  for (int q = 0; q < S; ++q) {
+    v[q] = state[i * S + q] + (kprev ? kc_dt * kprev[i * S + q] : 0.0);
+    first[q] = state[q] + (kprev ? kc_dt * kprev[q] : 0.0);
+  }
 #pragma unroll
   for (int q = 0; q < S; ++q) vstage[(long)t * S + q] = v[q];
-  const double phi = fabs(v[Slots<S>::phi]);
-  if (phi > kPhase64 && phi < __builtin_huge_val()) *huge = 1;
+  double sn, cs;
+  frame_phasor_any(v[2], frame_ref(first[2]), sn, cs);
+  double xw, yw;
+  apply_pbc(P, v[0], v[1], xw, yw);
+  const bool near = fabs(v[0]) <= kFar64 * P.xs && fabs(v[1]) <= kFar64 * P.ys;
+  rec[t] = make_double4(near ? xw : __builtin_nan(""), yw, sn, cs);
+  if (S == 4 && om) om[t] = v[S - 1] - frame_ref(first[S - 1]);
 }
 
-// the pair terms of ParticleSystemFirstOrderPtr.cpp:285-299 over every LPP-th entry of a list
-template <int S, int LPP, bool HO, bool HUGE>
-__device__ __forceinline__ void list_terms(const DevParams &P, const double *__restrict__ vstage,
-                                           const int *__restrict__ vslot, int u, int e, const double *st, PairAcc &a) {
-  if (u >= e) return;
-  // the next entry's state and the position of the one after it are read while this one is computed
-  int j = vslot[u], j1 = u + LPP < e ? vslot[u + LPP] : j;
-  double x = vstage[(long)j * S], y = vstage[(long)j * S + 1], phi = vstage[(long)j * S + 2];
-  for (; u < e; u += LPP) {
-    const int j2 = u + 2 * LPP < e ? vslot[u + 2 * LPP] : j1;
-    const double x1 = vstage[(long)j1 * S], y1 = vstage[(long)j1 * S + 1], phi1 = vstage[(long)j1 * S + 2];
-    if (pair_in_range<S>(P, st[0], st[1], x, y)) {
-      a.card += 1.0;
-      if (HO || HUGE) {
-        double sn, cs;
-        if (HUGE)
-          sincos(phi - st[2], &sn, &cs);
-        else
-          frame_phasor(phi, st[2], sn, cs);
-        a.align += sn * P.cos_a - cs * P.sin_a;
-        if (HO) a.compl_f += (vstage[(long)j * S + S - 1] - st[S - 1]) * (cs * P.cos_a + sn * P.sin_a);
-      } else {
-        double e1, e2;
-        const double d = two_diff(two_diff(phi, st[2], e1), P.alpha, e2);
-        a.align += small_sin(d, e1 + e2);
-      }
-    }
-    j = j1;
-    j1 = j2;
-    x = x1;
-    y = y1;
-    phi = phi1;
-  }
-}
-
-// Verlet pair loop, ParticleSystemFirstOrderPtr.cpp:553-613 (x_i as stored): LPP lanes per particle
-// take every LPP-th entry of its list, their sums are added in a fixed tree.  The stage state lies in
-// the cell order of the lists' build, where the entries of a list are runs of neighbours: a group's
-// reads are a few lines instead of one line per entry.  ~60 instructions per entry bound it (n =
-// 20,011, ~400 entries of which 140 in range: 404 us with one thread per particle, 56 with 16
-// lanes, 41 with the states in list order, 35 with sin(d - alpha) by small_sin, 32 with the next
-// entry read ahead; 8 and 32 lanes: 39 and 31).
+// Verlet pair loop, ParticleSystemFirstOrderPtr.cpp:553-613 (x_i as stored), through the phasors
+// (spss_pairs64.hpp): LPP lanes per particle take every LPP-th entry of its list, their sums are added in
+// a fixed tree.  The records lie in the cell order of the lists' build, where the entries of a list are
+// runs of neighbours: a group's reads are a few lines instead of one line per entry.  n = 20,011, ~600
+// entries of which 140 in range: 404 us with one thread per particle and a sine per pair, 32 with 16
+// lanes, records in list order and sin(d - alpha), 18.5 through the phasors (8, 32, 64 lanes: 27, 22, 24),
+// bound by the 32 bytes per entry from the caches (20 TB/s).
 template <int S, int LPP, bool HO>
-__global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, const double *__restrict__ vstage,
+__global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double band, const double *__restrict__ vstage,
+                                                         const double4 *__restrict__ rec,
+                                                         const double *__restrict__ om,
                                                          const int *__restrict__ order,
                                                          const int *__restrict__ vstart, const int *__restrict__ vslot,
-                                                         const int *__restrict__ huge, const double *__restrict__ nat,
-                                                         double *__restrict__ k_next, double *__restrict__ compl_out) {
+                                                         const double *__restrict__ nat, double *__restrict__ k_next,
+                                                         double *__restrict__ compl_out) {
   const int t = (int)(((long)blockIdx.x * kBlock + threadIdx.x) / LPP), l = threadIdx.x & (LPP - 1);
   const int i = t < P.n ? (order ? order[t] : t) : -1;
-  double st[S] = {};
-  PairAcc a{0.0, 0.0, 0.0};
+  PhasorSums q;
+  double4 own{};
   if (i >= 0) {
-#pragma unroll
-    for (int q = 0; q < S; ++q) st[q] = vstage[(long)t * S + q];
-    const int b = vstart[i] + l, e = vstart[i + 1];
-    if (*huge)
-      list_terms<S, LPP, HO, true>(P, vstage, vslot, b, e, st, a);
-    else
-      list_terms<S, LPP, HO, false>(P, vstage, vslot, b, e, st, a);
+    own = rec[t];
+    int u = vstart[i] + l;
+    const int e = vstart[i + 1];
+    if (u < e) {
+      // the next entry's record and the position of the one after it are read while this one is added
+      int j = vslot[u], j1 = u + LPP < e ? vslot[u + LPP] : j;
+      double4 r = rec[j];
+      for (; u < e; u += LPP) {
+        const int j2 = u + 2 * LPP < e ? vslot[u + 2 * LPP] : j1;
+        const double4 r1 = rec[j1];
+        const double ax = fabs(own.x - r.x), ay = fabs(own.y - r.y);
+        const double dx = fmin(ax, P.xs - ax), dy = fmin(ay, P.ys - ay);
+        const double d = __builtin_fma(dx, dx, __builtin_fma(dy, dy, -P.rho2));
+        bool in = d < 0.0;
+        if (!(fabs(d) > band)) {  // rare: the reference's own test on the stored positions
+          const long a = (long)t * S, b = (long)j * S;
+          in = pair_in_range<S>(P, vstage[a], vstage[a + 1], vstage[b], vstage[b + 1]);
+        }
+        if (in) {
+          q.S += r.z;
+          q.C += r.w;
+          q.card += 1.0;
+          if (HO) {
+            const double o = om[j];
+            q.TS += o * r.z;
+            q.TC += o * r.w;
+          }
+        }
+        j = j1;
+        j1 = j2;
+        r = r1;
+      }
+    }
   }
 #pragma unroll
   for (int off = LPP / 2; off > 0; off >>= 1) {
-    a.align += __shfl_down(a.align, off, LPP);
-    a.card += __shfl_down(a.card, off, LPP);
-    if (HO) a.compl_f += __shfl_down(a.compl_f, off, LPP);
+    q.S += __shfl_down(q.S, off, LPP);
+    q.C += __shfl_down(q.C, off, LPP);
+    q.card += __shfl_down(q.card, off, LPP);
+    if (HO) {
+      q.TS += __shfl_down(q.TS, off, LPP);
+      q.TC += __shfl_down(q.TC, off, LPP);
+    }
   }
-  if (i >= 0 && l == 0) write_k<S>(P, st, i, a, nat ? nat[i] : 0.0, k_next, compl_out);
+  if (i >= 0 && l == 0) {
+    double st[S], sn, cs;
+#pragma unroll
+    for (int k = 0; k < S; ++k) st[k] = vstage[(long)t * S + k];
+    phasor_of(st[2], sn, cs);
+    write_k<S>(P, st, i, pair_acc<S>(P, q, own.z, own.w, HO ? om[t] : 0.0), nat ? nat[i] : 0.0, sn, cs, k_next,
+               compl_out);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -633,37 +646,39 @@ void launch_verlet_fill_cells(hipStream_t st, const DevParams &P, const double *
                               const CellBuffers &cb, double rmax2, const int *vstart, int *vlist, int *vslot) {
   SPSS_DISPATCH_S(P.s, k_verlet_build_cells<SS, true><<<dim3(nblk((long)kBuildLanes * P.n)), dim3(kBlock), 0, st>>>(P, stage, ncx, ncy, cb.start, cb.sorted, rmax2, nullptr, vstart, vlist, vslot));
 }
-void launch_stage_order(hipStream_t st, int n, int s, const double *state, const double *kprev, double kc_dt,
-                        const int *order, double *vstage, int *huge) {
-  if (s == 4)
-    k_stage_order<4><<<dim3(nblk(n)), dim3(kBlock), 0, st>>>(n, state, kprev, kc_dt, order, vstage, huge);
+void launch_stage_order(hipStream_t st, const DevParams &P, const double *state, const double *kprev, double kc_dt,
+                        const int *order, const VerletStage &V) {
+  double4 *rec = reinterpret_cast<double4 *>(V.rec);
+  if (P.s == 4)
+    k_stage_order<4><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, state, kprev, kc_dt, order, V.stage, rec, V.om);
   else
-    k_stage_order<3><<<dim3(nblk(n)), dim3(kBlock), 0, st>>>(n, state, kprev, kc_dt, order, vstage, huge);
+    k_stage_order<3><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, state, kprev, kc_dt, order, V.stage, rec, nullptr);
 }
 
 template <int S, bool HO>
-static void verlet_pairs_as(hipStream_t st, const DevParams &P, const double *vstage, const int *order,
-                            const int *vstart, const int *vslot, const int *huge, const double *nat, double *k_next,
+static void verlet_pairs_as(hipStream_t st, const DevParams &P, const VerletStage &V, const int *order,
+                            const int *vstart, const int *vslot, const double *nat, double *k_next,
                             double *compl_out) {
   // 16 lanes read a list in contiguous 64-byte runs; fewer than 16,384 particles need a wave each to
   // fill the chip
+  const double4 *rec = reinterpret_cast<const double4 *>(V.rec);
+  const double band = pair_band(P.rho2, P.xs, P.ys);
   if (P.n < 16384)
-    k_verlet_pairs<S, 64, HO><<<dim3(nblk(64L * P.n)), dim3(kBlock), 0, st>>>(P, vstage, order, vstart, vslot, huge, nat,
-                                                                              k_next, compl_out);
+    k_verlet_pairs<S, 64, HO><<<dim3(nblk(64L * P.n)), dim3(kBlock), 0, st>>>(P, band, V.stage, rec, V.om, order, vstart,
+                                                                              vslot, nat, k_next, compl_out);
   else
-    k_verlet_pairs<S, 16, HO><<<dim3(nblk(16L * P.n)), dim3(kBlock), 0, st>>>(P, vstage, order, vstart, vslot, huge, nat,
-                                                                              k_next, compl_out);
+    k_verlet_pairs<S, 16, HO><<<dim3(nblk(16L * P.n)), dim3(kBlock), 0, st>>>(P, band, V.stage, rec, V.om, order, vstart,
+                                                                              vslot, nat, k_next, compl_out);
 }
 
-void launch_verlet_pairs(hipStream_t st, const DevParams &P, const double *vstage, const int *order,
-                         const int *vstart, const int *vslot, const int *huge, const double *nat, double *k_next,
-                         double *compl_out) {
+void launch_verlet_pairs(hipStream_t st, const DevParams &P, const VerletStage &V, const int *order,
+                         const int *vstart, const int *vslot, const double *nat, double *k_next, double *compl_out) {
   if (P.s == 3)
-    verlet_pairs_as<3, false>(st, P, vstage, order, vstart, vslot, huge, nat, k_next, compl_out);
+    verlet_pairs_as<3, false>(st, P, V, order, vstart, vslot, nat, k_next, compl_out);
   else if (P.higher_order)
-    verlet_pairs_as<4, true>(st, P, vstage, order, vstart, vslot, huge, nat, k_next, compl_out);
+    verlet_pairs_as<4, true>(st, P, V, order, vstart, vslot, nat, k_next, compl_out);
   else
-    verlet_pairs_as<4, false>(st, P, vstage, order, vstart, vslot, huge, nat, k_next, compl_out);
+    verlet_pairs_as<4, false>(st, P, V, order, vstart, vslot, nat, k_next, compl_out);
 }
 
 void launch_rk4_combine(hipStream_t st, int s, int n, double *state, const double *k1, const double *k2,

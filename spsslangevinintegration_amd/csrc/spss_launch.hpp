@@ -150,13 +150,17 @@ void launch_verlet_count_cells(hipStream_t st, const DevParams &P, const double 
                                const CellBuffers &cb, double rmax2, int *vcount);
 void launch_verlet_fill_cells(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy,
                               const CellBuffers &cb, double rmax2, const int *vstart, int *vlist, int *vslot);
-// the stage state in the order of the lists' build (null: over all pairs) and the pair sums over it;
-// huge: set by phases that need the general sine, cleared by the caller at a build
-void launch_stage_order(hipStream_t st, int n, int s, const double *state, const double *kprev, double kc_dt,
-                        const int *order, double *vstage, int *huge);
-void launch_verlet_pairs(hipStream_t st, const DevParams &P, const double *vstage, const int *order,
-                         const int *vstart, const int *vslot, const int *huge, const double *nat, double *k_next,
-                         double *compl_out);
+// the stage state in the order of the lists' build (null: over all pairs), with the records and relative
+// omegas (for the complementary force, else null) that the pair sums over it read
+struct VerletStage {
+  double *stage = nullptr;  // [s n]
+  double *rec = nullptr;    // [4 n] {x, y, sin psi, cos psi}
+  double *om = nullptr;     // [n]
+};
+void launch_stage_order(hipStream_t st, const DevParams &P, const double *state, const double *kprev, double kc_dt,
+                        const int *order, const VerletStage &V);
+void launch_verlet_pairs(hipStream_t st, const DevParams &P, const VerletStage &V, const int *order,
+                         const int *vstart, const int *vslot, const double *nat, double *k_next, double *compl_out);
 // the global field (spss_global64.hip).  part: gf_part_doubles(n) doubles of scratch in two halves of
 // block sums; kprev may be null
 size_t gf_part_doubles(int n);

@@ -67,27 +67,6 @@ __device__ __forceinline__ void phasor_of(double phi, double &sn, double &cs) {
     sincos(phi, &sn, &cs);
 }
 
-// sin(x + e) the same way, reduced to |r| <= pi/2 by multiples of pi and a Taylor polynomial to r^21:
-// half the instructions of sine and cosine together
-__device__ __forceinline__ double small_sin(double x, double e) {
-  const double k = rint(x * 0x1.45f306dc9c883p-2);  // 1 / pi
-  const double r0 = __builtin_fma(-k, 0x1.921fb54442d18p+1, x);
-  const double r = __builtin_fma(-k, 0x1.1a62633145c07p-53, r0);
-  e = __builtin_fma(-k, 0x1.1a62633145c07p-53, r0 - r) + e;
-  const double z = r * r;
-  double p = __builtin_fma(z, 1.0 / 51090942171709440000.0, -1.0 / 121645100408832000.0);
-  p = __builtin_fma(z, p, 1.0 / 355687428096000.0);
-  p = __builtin_fma(z, p, -1.0 / 1307674368000.0);
-  p = __builtin_fma(z, p, 1.0 / 6227020800.0);
-  p = __builtin_fma(z, p, -1.0 / 39916800.0);
-  p = __builtin_fma(z, p, 1.0 / 362880.0);
-  p = __builtin_fma(z, p, -1.0 / 5040.0);
-  p = __builtin_fma(z, p, 1.0 / 120.0);
-  p = __builtin_fma(z, p, -1.0 / 6.0);
-  const double s = r + __builtin_fma(r * z, p, __builtin_fma(-0.5 * z, e, e));
-  return ((int)k & 1) ? -s : s;
-}
-
 // a - b and its rounding error
 __device__ __forceinline__ double two_diff(double a, double b, double &err) {
   const double d = a - b, c = d - a;
@@ -103,6 +82,20 @@ __device__ __forceinline__ void frame_phasor(double phi, double ref, double &sn,
   double err;
   const double d = two_diff(phi, ref, err);
   small_sincos(d, err, sn, cs);
+}
+
+// the same for any phase
+__device__ __forceinline__ void frame_phasor_any(double phi, double ref, double &sn, double &cs) {
+  double err;
+  const double d = two_diff(phi, ref, err);
+  if (fabs(d) <= 0x1p30) {
+    small_sincos(d, err, sn, cs);
+  } else {
+    double s, c;
+    sincos(d, &s, &c);
+    sn = __builtin_fma(err, c, s);
+    cs = __builtin_fma(-err, s, c);
+  }
 }
 
 // a reference phase or phase velocity: any value of an ordinary size serves
