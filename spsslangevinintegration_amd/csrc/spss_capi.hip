@@ -102,6 +102,7 @@ struct spss_system {
   // Dormand-Prince 5(4) buffers (allocated on first use): two states and derivatives, k2..k6,
   // a stage state and a pinned host copy for observers
   double *dp[10] = {};
+  bool dp_planes = false;  // the derivatives among them are in planes (spss_global64.hip)
   double *dp_host = nullptr;
 };
 
@@ -1438,6 +1439,7 @@ struct DpRun {
   int cur = 0;  // which of the two state/derivative buffers holds the current point
   double t = 0.0, t_old = 0.0, dt = 0.0;
   bool deriv_init = false;
+  bool planes = false;  // the global field, with the derivatives in planes
   long steps = 0, rejected = 0;
   double *x(int q) const { return h->dp[q ? DP_X1 : DP_X0]; }
   double *dx(int q) const { return h->dp[q ? DP_D1 : DP_D0]; }
@@ -1469,31 +1471,31 @@ int dp_try_step(DpRun &R, bool *ok) {
   double *const *k = h->dp;
   double *tmp = h->dp[DP_TMP];
   const double dt = R.dt;
-  if (resolve_method(h, R.method) == SPSS_METHOD_GLOBAL_FIELD && !h->higher_order) {
-    // a launch per stage: the derivative and the next stage state with the sums of its field
+  if (R.planes) {
     const double *nat = h->have_nat ? h->nat : nullptr;
-    double *p0 = h->partial, *p1 = h->partial + gf_part_doubles(h->n) / 2;
+    DpTrial D;
+    D.x = in;
+    D.out = out;
+    D.tmp = tmp;
+    D.dt = dt;
+    D.eps_abs = R.eps_abs;
+    D.eps_rel = R.eps_rel;
+    double *const ks[7] = {R.dx(R.cur), k[DP_K2], k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6], dout};
+    std::copy(ks, ks + 7, D.k);
+    D.first = dt * A.a21;
+    D.terms[0] = dp_terms({din}, {dt * A.a31, dt * A.a32});
+    D.terms[1] = dp_terms({din, k[DP_K2]}, {dt * A.a41, dt * A.a42, dt * A.a43});
+    D.terms[2] = dp_terms({din, k[DP_K2], k[DP_K3]}, {dt * A.a51, dt * A.a52, dt * A.a53, dt * A.a54});
+    D.terms[3] = dp_terms({din, k[DP_K2], k[DP_K3], k[DP_K4]},
+                          {dt * A.a61, dt * A.a62, dt * A.a63, dt * A.a64, dt * A.a65});
+    D.terms[4] = dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5]},
+                          {dt * A.b1, dt * A.b3, dt * A.b4, dt * A.b5, dt * A.b6});
+    D.terms[5] = dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6]},
+                          {dt * A.d1, dt * A.d3, dt * A.d4, dt * A.d5, dt * A.d6, dt * A.d7});
     h->P.higher_order = 0;
     h->P.fresh_k = 0;
-    launch_global_first(st, h->P, in, din, dt * A.a21, tmp, p0);
-    launch_global_next(st, h->P, tmp, p0, nat, k[DP_K2], in, dp_terms({din}, {dt * A.a31, dt * A.a32}), tmp, p1);
-    launch_global_next(st, h->P, tmp, p1, nat, k[DP_K3], in,
-                       dp_terms({din, k[DP_K2]}, {dt * A.a41, dt * A.a42, dt * A.a43}), tmp, p0);
-    launch_global_next(st, h->P, tmp, p0, nat, k[DP_K4], in,
-                       dp_terms({din, k[DP_K2], k[DP_K3]}, {dt * A.a51, dt * A.a52, dt * A.a53, dt * A.a54}), tmp, p1);
-    launch_global_next(st, h->P, tmp, p1, nat, k[DP_K5], in,
-                       dp_terms({din, k[DP_K2], k[DP_K3], k[DP_K4]},
-                                {dt * A.a61, dt * A.a62, dt * A.a63, dt * A.a64, dt * A.a65}),
-                       tmp, p0);
-    launch_global_next(st, h->P, tmp, p0, nat, k[DP_K6], in,
-                       dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5]},
-                                {dt * A.b1, dt * A.b3, dt * A.b4, dt * A.b5, dt * A.b6}),
-                       out, p1);
-    const int nb = launch_global_error(st, h->P, out, p1, nat, dout, in,
-                                       dp_terms({din, k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6]},
-                                                {dt * A.d1, dt * A.d3, dt * A.d4, dt * A.d5, dt * A.d6, dt * A.d7}),
-                                       dt, R.eps_abs, R.eps_rel, p0);
-    launch_max_final(st, nb, p0, h->scal + 24);
+    const int nb = launch_dp_global_trial(st, h->P, D, nat, h->partial);
+    launch_max_final(st, nb, h->partial, h->scal + 24);
   } else {
     launch_dp_combine(st, R.m, in, dp_terms({din}, {dt * A.a21}), tmp);
     TRY(dp_rhs(R, tmp, k[DP_K2]));
@@ -1551,7 +1553,15 @@ int dp_initialize(DpRun &R, const double *x0, double t0, double dt0) {
 // dense_output_runge_kutta::do_step (FSAL): trial steps until one is accepted (at most 500)
 int dp_do_step(DpRun &R) {
   if (!R.deriv_init) {
-    TRY(dp_rhs(R, R.x(R.cur), R.dx(R.cur)));
+    if (R.planes) {
+      spss_system *h = R.h;
+      h->P.higher_order = 0;
+      h->P.fresh_k = 0;
+      launch_dp_global_start(h->stream, h->P, R.x(R.cur), h->partial, h->have_nat ? h->nat : nullptr, R.dx(R.cur));
+      HIPCHECK(hipGetLastError());
+    } else {
+      TRY(dp_rhs(R, R.x(R.cur), R.dx(R.cur)));
+    }
     R.deriv_init = true;
   }
   R.t_old = R.t;
@@ -1593,10 +1603,12 @@ void dp_calc_state(DpRun &R, double t, double *out) {
   const double b5t = Aq * A.b5 + Cq * X5;
   const double b6t = Aq * A.b6 - Cq * X6;
   const double b7t = Bq + Cq * X7;
-  launch_dp_combine(R.h->stream, R.m, R.x(1 - R.cur),
-                    dp_terms({R.dx(1 - R.cur), k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6], R.dx(R.cur)},
-                             {dt * b1t, dt * b3t, dt * b4t, dt * b5t, dt * b6t, dt * b7t}),
-                    out);
+  const DpTerms T = dp_terms({R.dx(1 - R.cur), k[DP_K3], k[DP_K4], k[DP_K5], k[DP_K6], R.dx(R.cur)},
+                             {dt * b1t, dt * b3t, dt * b4t, dt * b5t, dt * b6t, dt * b7t});
+  if (R.planes)
+    launch_dp_global_combine(R.h->stream, R.h->s, R.h->n, R.x(1 - R.cur), T, out);
+  else
+    launch_dp_combine(R.h->stream, R.m, R.x(1 - R.cur), T, out);
 }
 
 // odeint's comparisons of times with the sign of the step and a tolerance of one machine epsilon
@@ -1706,6 +1718,14 @@ int spss_dopri5_integrate(spss_system *h, int method, int mode, double t0, doubl
   DpRun R;
   R.h = h;
   R.method = method;
+  R.planes = resolve_method(h, method) == SPSS_METHOD_GLOBAL_FIELD && !h->higher_order;
+  if (h->dp_planes && !R.planes) {  // what the buffers hold matters to such a right-hand side (above): rows again
+    for (int q : {DP_D0, DP_D1, DP_K2, DP_K3, DP_K4, DP_K5, DP_K6}) {
+      launch_dp_global_rows(h->stream, h->s, h->n, h->dp[q], h->dp[DP_TMP]);
+      HIPCHECK(hipMemcpyAsync(h->dp[q], h->dp[DP_TMP], sizeof(double) * m, hipMemcpyDeviceToDevice, h->stream));
+    }
+  }
+  h->dp_planes = R.planes;
   R.m = m;
   R.eps_abs = eps_abs;
   R.eps_rel = eps_rel;

@@ -10,8 +10,8 @@
 //
 // What bounds it: small systems the chain phasor - sums - derivative (n = 1,000: 1.1 us per stage; a
 // Runge-Kutta step took 55 us in 17 launches and takes 4.4), systems up to about 100,000 the latency of a
-// launch (4 us; a step of 16,384: 56 -> 17 us), large ones memory: a Dormand-Prince trial of 1,048,576 moves
-// 1.5 GB at 6.3 TB/s (470 -> 240 us), an Euler step 75 -> 25 us.
+// launch (4 us; a step of 16,384: 56 -> 17 us), large ones memory: a Dormand-Prince trial of 1,048,576 470 ->
+// 214 us, an Euler step 75 -> 25 us.
 //
 // |Z| sin(arg Z - phi) is Im(Z e^{-i phi}): no arc tangent, no second pair of sine and cosine.
 #pragma clang fp contract(off)
@@ -214,10 +214,10 @@ __device__ __forceinline__ void add_terms(const double *w, double *s, double *c)
   }
 }
 
-// the first stage: x + c0 * k0 (k0 may be null), stored if asked, and its block sums
+// the block sums of a first stage x + c0 * k0 (k0 may be null)
 template <int S, bool HO, int PER>
 __global__ __launch_bounds__(256) void gf_first(int n, const double *__restrict__ x, const double *__restrict__ k0,
-                                                double c0, double *__restrict__ out, double *__restrict__ part) {
+                                                double c0, double *__restrict__ part) {
   constexpr int COLS = HO ? 4 : 2, kPart = 256 * PER;
   double s[COLS] = {}, c[COLS] = {};
   for (long b = (long)blockIdx.x * kPart; b < n; b += (long)gridDim.x * kPart) {
@@ -239,7 +239,6 @@ __global__ __launch_bounds__(256) void gf_first(int n, const double *__restrict_
       const long i = b + p * 256 + threadIdx.x;
       if (i >= n) continue;
       double w[COLS];
-      if (out) store_row<S>(out, i, v[p]);
       field_terms<S, HO>(v[p], w);
       add_terms<COLS>(w, s, c);
     }
@@ -250,11 +249,10 @@ __global__ __launch_bounds__(256) void gf_first(int n, const double *__restrict_
 // what follows the derivative k of a particle
 enum GfThen {
   kThenNothing,  // a right-hand side
-  kThenNext,     // the next stage state base + sum_j c_j k_j + c_n k, and its block sums
+  kThenNext,     // the next stage state base + c k, and its block sums
   kThenRk4,      // the step: state += (k1 + 2 k2 + 2 k3 + k) dt / 6, and its block sums
   kThenEuler,    // the stochastic steps (StochasticEulerStepperPtr.hpp:40-73,
-  kThenSrk,      // StochasticRungeKuttaStepperPtr.hpp:50-76) and the block sums of the new state
-  kThenError     // the error norm of a Dormand-Prince trial: per block the largest relative error
+  kThenSrk       // StochasticRungeKuttaStepperPtr.hpp:50-76) and the block sums of the new state
 };
 
 struct GfStep {
@@ -265,10 +263,11 @@ struct GfStep {
   const double *nat = nullptr;
   double *k = nullptr, *compl_out = nullptr;  // the derivative, the complementary force (may be null)
   const double *base = nullptr;
-  DpTerms T{};        // terms of what follows; T.c[T.n] is the coefficient of k itself
+  double c = 0.0;                  // the coefficient of k in the next stage state
+  const double *k1 = nullptr, *k2 = nullptr, *k3 = nullptr;
   double *next = nullptr, *out = nullptr;  // the state written and its block sums
   GfNoise noise{};
-  double dt = 0.0, eps_abs = 0.0, eps_rel = 0.0;
+  double dt = 0.0;
 };
 
 __device__ __forceinline__ double gf_draw(const GfNoise &z, long idx, uint32_t particle, int which) {
@@ -308,13 +307,13 @@ __device__ __forceinline__ void stochastic_update(const GfNoise &z, double dt, i
   }
 }
 
-// NT: terms of T besides the derivative itself; PER: particles per thread and pass
-template <int S, bool HO, int THEN, int NT, int PER>
+// PER: particles per thread and pass
+template <int S, bool HO, int THEN, int PER>
 __global__ __launch_bounds__(256) void gf_stage(DevParams P, GfStep G) {
   constexpr int COLS = HO ? 4 : 2, kPart = 256 * PER;
-  constexpr bool kSums = THEN == kThenNext || THEN == kThenRk4 || THEN == kThenEuler || THEN == kThenSrk;
+  constexpr bool kSums = THEN != kThenNothing;
   Field F{};
-  double s[COLS] = {}, c[COLS] = {}, worst = 0.0;
+  double s[COLS] = {}, c[COLS] = {};
   for (long b = (long)blockIdx.x * kPart; b < P.n; b += (long)gridDim.x * kPart) {
     double st[PER][S];
 #pragma unroll
@@ -334,10 +333,13 @@ __global__ __launch_bounds__(256) void gf_stage(DevParams P, GfStep G) {
     for (int p = 0; p < PER; ++p) {
       const long i = b + p * 256 + threadIdx.x;
       if (i >= P.n) continue;
-      double v[S], d[NT ? NT : 1][S], k[S], cf;
-      if (THEN == kThenNext || THEN == kThenRk4 || THEN == kThenError) load_row<S>(G.base, i, v);
-#pragma unroll
-      for (int j = 0; j < NT; ++j) load_row<S>(G.T.k[j], i, d[j]);
+      double v[S], d[3][S], k[S], cf;
+      if (THEN == kThenNext || THEN == kThenRk4) load_row<S>(G.base, i, v);
+      if (THEN == kThenRk4) {
+        load_row<S>(G.k1, i, d[0]);
+        load_row<S>(G.k2, i, d[1]);
+        load_row<S>(G.k3, i, d[2]);
+      }
       double sn, cs;
       phasor_of(st[p][2], sn, cs);
       derivative<S, HO>(P, F, st[p], sn, cs, G.nat ? G.nat[i] : 0.0, k, cf);
@@ -345,28 +347,14 @@ __global__ __launch_bounds__(256) void gf_stage(DevParams P, GfStep G) {
       if (HO && G.compl_out) G.compl_out[i] = cf;
       if (THEN == kThenNext) {
 #pragma unroll
-        for (int q = 0; q < S; ++q) {
-#pragma unroll
-          for (int j = 0; j < NT; ++j) v[q] = v[q] + G.T.c[j] * d[j][q];
-          v[q] = v[q] + G.T.c[NT] * k[q];
-        }
+        for (int q = 0; q < S; ++q) v[q] = v[q] + G.c * k[q];
       } else if (THEN == kThenRk4) {
 #pragma unroll
-        for (int q = 0; q < S; ++q)
-          v[q] += (d[0][q] + 2.0 * d[NT > 1 ? 1 : 0][q] + 2.0 * d[NT > 2 ? 2 : 0][q] + k[q]) * G.dt / 6.0;
+        for (int q = 0; q < S; ++q) v[q] += (d[0][q] + 2.0 * d[1][q] + 2.0 * d[2][q] + k[q]) * G.dt / 6.0;
       } else if (THEN == kThenEuler || THEN == kThenSrk) {
 #pragma unroll
         for (int q = 0; q < S; ++q) v[q] = st[p][q];
         stochastic_update<S, THEN == kThenSrk>(G.noise, G.dt, (int)i, k, cf, v);
-      } else if (THEN == kThenError) {
-#pragma unroll
-        for (int q = 0; q < S; ++q) {
-          double err = G.T.c[0] * d[0][q];
-#pragma unroll
-          for (int j = 1; j < NT; ++j) err = err + G.T.c[j] * d[j][q];
-          err = err + G.T.c[NT] * k[q];
-          worst = fmax(worst, fabs(err) / (G.eps_abs + G.eps_rel * (1.0 * fabs(v[q]) + (1.0 * G.dt) * fabs(d[0][q]))));
-        }
       }
       if (kSums) {
         store_row<S>(G.next, i, v);
@@ -377,7 +365,109 @@ __global__ __launch_bounds__(256) void gf_stage(DevParams P, GfStep G) {
     }
   }
   if (kSums) block_sums<COLS>(s, c, G.out + (long)blockIdx.x * COLS * 2);
-  if (THEN == kThenError) {
+}
+
+// ---------------------------------------------------------------------------
+// Dormand-Prince trials.  Positions take no part in the field, so the stages before the last need the
+// phases (and omegas) of the state and of the derivatives alone: the derivatives are kept as two planes,
+// A = {dphi/dt, domega/dt} and B = {dx/dt, dy/dt} behind it, the stages run on a copy of the state's phases
+// and a plane of stage phases.  k2's positions enter nothing and are not kept.  A trial moves 1,040
+// bytes per particle at 5.1 TB/s (1,440 with whole rows at 6.2): 1,048,576 particles 214 us, 240 with rows.
+
+enum GpThen {
+  kGpStart,  // the derivative at a whole state
+  kGpNext,   // the derivative at stage phases; the next stage's phases and their block sums
+  kGpOut,    // ... ; the new state and its block sums
+  kGpError   // the derivative at the new state; per block the largest relative error
+};
+
+struct GpStep {
+  const double *x = nullptr;   // the stage: a plane (kGpNext, kGpOut) or whole rows
+  const double *in = nullptr;  // its block sums
+  int nb = 0;
+  const double *nat = nullptr;
+  double *k = nullptr, *kb = nullptr;  // the derivative's planes (kb may be null)
+  const double *base = nullptr;        // the state: its phases (kGpNext) or rows
+  DpTerms T{};                         // earlier derivatives; T.c[T.n] is the coefficient of this one
+  double *next = nullptr, *out = nullptr;
+  double dt = 0.0, eps_abs = 0.0, eps_rel = 0.0;
+};
+
+template <int S, int THEN, int NT, int PER>
+__global__ __launch_bounds__(256) void gp_stage(DevParams P, GpStep G) {
+  constexpr int NA = S - 2, kPart = 256 * PER;
+  constexpr bool kRows = THEN == kGpStart || THEN == kGpError, kWhole = THEN == kGpOut || THEN == kGpError;
+  Field F{};
+  double s[2] = {}, c[2] = {}, worst = 0.0;
+  for (long b = (long)blockIdx.x * kPart; b < P.n; b += (long)gridDim.x * kPart) {
+    double st[PER][4];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const long i = b + p * 256 + threadIdx.x;
+      if (i >= P.n) continue;
+#pragma unroll
+      for (int q = 0; q < NA; ++q) st[p][2 + q] = kRows ? G.x[i * S + 2 + q] : G.x[i * NA + q];
+    }
+    if (b == (long)blockIdx.x * kPart) field_of<false>(G.in, G.nb, (double)P.n, F);  // over the first loads
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const long i = b + p * 256 + threadIdx.x;
+      if (i >= P.n) continue;
+      double v[S], d[NT ? NT : 1][S], k[S], cf, sn, cs;
+      if (THEN == kGpNext) {
+#pragma unroll
+        for (int q = 0; q < NA; ++q) v[2 + q] = G.base[i * NA + q];
+      } else if (kWhole) {
+        load_row<S>(G.base, i, v);
+      }
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const double *a = G.T.k[j], *xy = a + (long)P.n * NA;
+#pragma unroll
+        for (int q = 0; q < NA; ++q) d[j][2 + q] = a[i * NA + q];
+        if (kWhole) {
+          d[j][0] = xy[2 * i];
+          d[j][1] = xy[2 * i + 1];
+        }
+      }
+      phasor_of(st[p][2], sn, cs);
+      derivative<S, false>(P, F, st[p], sn, cs, G.nat ? G.nat[i] : 0.0, k, cf);
+#pragma unroll
+      for (int q = 0; q < NA; ++q) G.k[i * NA + q] = k[2 + q];
+      if (G.kb) {
+        G.kb[2 * i] = k[0];
+        G.kb[2 * i + 1] = k[1];
+      }
+      if (THEN == kGpNext || THEN == kGpOut) {
+#pragma unroll
+        for (int q = THEN == kGpOut ? 0 : 2; q < S; ++q) {
+#pragma unroll
+          for (int j = 0; j < NT; ++j) v[q] = v[q] + G.T.c[j] * d[j][q];
+          v[q] = v[q] + G.T.c[NT] * k[q];
+        }
+        if (THEN == kGpOut) {
+          store_row<S>(G.next, i, v);
+        } else {
+#pragma unroll
+          for (int q = 0; q < NA; ++q) G.next[i * NA + q] = v[2 + q];
+        }
+        double w[2];
+        phasor_of(v[2], w[1], w[0]);
+        add_terms<2>(w, s, c);
+      } else if (THEN == kGpError) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+          double err = G.T.c[0] * d[0][q];
+#pragma unroll
+          for (int j = 1; j < NT; ++j) err = err + G.T.c[j] * d[j][q];
+          err = err + G.T.c[NT] * k[q];
+          worst = fmax(worst, fabs(err) / (G.eps_abs + G.eps_rel * (1.0 * fabs(v[q]) + (1.0 * G.dt) * fabs(d[0][q]))));
+        }
+      }
+    }
+  }
+  if (THEN == kGpNext || THEN == kGpOut) block_sums<2>(s, c, G.out + (long)blockIdx.x * 4);
+  if (THEN == kGpError) {
     __shared__ double red[256];
     red[threadIdx.x] = worst;
     __syncthreads();
@@ -387,6 +477,78 @@ __global__ __launch_bounds__(256) void gf_stage(DevParams P, GfStep G) {
     }
     if (threadIdx.x == 0) G.out[blockIdx.x] = red[0];
   }
+}
+
+// the first stage's phases x + c0 k (k: plane A), the state's phases beside them, the block sums
+template <int S, int PER>
+__global__ __launch_bounds__(256) void gp_first(int n, const double *__restrict__ x, const double *__restrict__ k,
+                                                double c0, double *__restrict__ xa, double *__restrict__ out,
+                                                double *__restrict__ part) {
+  constexpr int NA = S - 2, kPart = 256 * PER;
+  double s[2] = {}, c[2] = {};
+  for (long b = (long)blockIdx.x * kPart; b < n; b += (long)gridDim.x * kPart) {
+    double v[PER][NA], w[PER][NA];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const long i = b + p * 256 + threadIdx.x;
+      if (i >= n) continue;
+#pragma unroll
+      for (int q = 0; q < NA; ++q) {
+        v[p][q] = x[i * S + 2 + q];
+        w[p][q] = k[i * NA + q];
+      }
+    }
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+      const long i = b + p * 256 + threadIdx.x;
+      if (i >= n) continue;
+#pragma unroll
+      for (int q = 0; q < NA; ++q) {
+        xa[i * NA + q] = v[p][q];
+        w[p][q] = v[p][q] + c0 * w[p][q];
+        out[i * NA + q] = w[p][q];
+      }
+      double t[2];
+      phasor_of(w[p][0], t[1], t[0]);
+      add_terms<2>(t, s, c);
+    }
+  }
+  block_sums<2>(s, c, part + (long)blockIdx.x * 4);
+}
+
+// x + sum_j c_j k_j in whole rows (the dense output)
+template <int S>
+__global__ __launch_bounds__(256) void gp_combine(int n, const double *__restrict__ x, DpTerms T,
+                                                  double *__restrict__ out) {
+  constexpr int NA = S - 2;
+  const long i = blockIdx.x * 256L + threadIdx.x;
+  if (i >= n) return;
+  double v[S], d[kDpMaxTerms][S];
+  load_row<S>(x, i, v);
+#pragma unroll
+  for (int j = 0; j < kDpMaxTerms; ++j) {
+    const double *a = T.k[j], *xy = a + (long)n * NA;
+    d[j][0] = xy[2 * i];
+    d[j][1] = xy[2 * i + 1];
+#pragma unroll
+    for (int q = 0; q < NA; ++q) d[j][2 + q] = a[i * NA + q];
+  }
+#pragma unroll
+  for (int q = 0; q < S; ++q) {
+#pragma unroll
+    for (int j = 0; j < kDpMaxTerms; ++j) v[q] = v[q] + T.c[j] * d[j][q];
+    out[i * S + q] = v[q];
+  }
+}
+
+// planes back to rows
+template <int S>
+__global__ __launch_bounds__(256) void gp_rows(int n, const double *__restrict__ planes, double *__restrict__ rows) {
+  const long i = blockIdx.x * 256L + threadIdx.x;
+  if (i >= n) return;
+#pragma unroll
+  for (int q = 0; q < S; ++q)
+    rows[i * S + q] = q < 2 ? planes[(long)n * (S - 2) + 2 * i + q] : planes[i * (S - 2) + q - 2];
 }
 
 // a's upper half of the wave and b's lower half change places: a + b then holds a's half sums in the
@@ -549,22 +711,22 @@ inline int gf_blocks(int n) {
 }
 
 template <int S, bool HO>
-void first(hipStream_t st, int n, const double *x, const double *k0, double c0, double *out, double *part) {
-  const auto run = [&](auto kernel) { kernel<<<dim3(gf_blocks(n)), dim3(256), 0, st>>>(n, x, k0, c0, out, part); };
+void first(hipStream_t st, int n, const double *x, const double *k0, double c0, double *part) {
+  const auto run = [&](auto kernel) { kernel<<<dim3(gf_blocks(n)), dim3(256), 0, st>>>(n, x, k0, c0, part); };
   gf_wide(n) ? run(gf_first<S, HO, 4>) : run(gf_first<S, HO, 1>);
 }
 
-template <int S, bool HO, int THEN, int NT>
+template <int S, bool HO, int THEN>
 void stage(hipStream_t st, const DevParams &P, GfStep &G) {
   G.nb = gf_blocks(P.n);
   const auto run = [&](auto kernel) { kernel<<<dim3(G.nb), dim3(256), 0, st>>>(P, G); };
-  gf_wide(P.n) ? run(gf_stage<S, HO, THEN, NT, 4>) : run(gf_stage<S, HO, THEN, NT, 1>);
+  gf_wide(P.n) ? run(gf_stage<S, HO, THEN, 4>) : run(gf_stage<S, HO, THEN, 1>);
 }
 
 template <int S, bool HO>
 void rhs(hipStream_t st, const DevParams &P, const double *x, const double *kprev, double kc, double *part,
          const double *nat, double *k, double *compl_out) {
-  first<S, HO>(st, P.n, x, kprev, kc, nullptr, part);
+  first<S, HO>(st, P.n, x, kprev, kc, part);
   GfStep G{};
   G.x = x;
   G.kprev = kprev;
@@ -573,14 +735,14 @@ void rhs(hipStream_t st, const DevParams &P, const double *x, const double *kpre
   G.nat = nat;
   G.k = k;
   G.compl_out = compl_out;
-  stage<S, HO, kThenNothing, 0>(st, P, G);
+  stage<S, HO, kThenNothing>(st, P, G);
 }
 
 template <int S, bool HO>
 void rk4(hipStream_t st, const DevParams &P, long nsteps, double dt, double *state, double *tmp, double *const *k,
          double *part, const double *nat, double *compl_out) {
   double *in = part, *out = part + gf_part_doubles(P.n) / 2;
-  first<S, HO>(st, P.n, state, k[0], 0.0, nullptr, in);  // state + 0 * k1, RungeKutta4StepperPtr.cpp:50
+  first<S, HO>(st, P.n, state, k[0], 0.0, in);  // state + 0 * k1, RungeKutta4StepperPtr.cpp:50
   for (long s = 0; s < nsteps; ++s)
     for (int g = 0; g < 4; ++g) {
       GfStep G{};
@@ -594,13 +756,15 @@ void rk4(hipStream_t st, const DevParams &P, long nsteps, double dt, double *sta
       G.out = out;
       G.dt = dt;
       if (g < 3) {
-        G.T.c[0] = (g < 2 ? 0.5 : 1.0) * dt;
+        G.c = (g < 2 ? 0.5 : 1.0) * dt;
         G.next = tmp;
-        stage<S, HO, kThenNext, 0>(st, P, G);
+        stage<S, HO, kThenNext>(st, P, G);
       } else {
-        for (int q = 0; q < 3; ++q) G.T.k[q] = k[q];
+        G.k1 = k[0];
+        G.k2 = k[1];
+        G.k3 = k[2];
         G.next = state;
-        stage<S, HO, kThenRk4, 3>(st, P, G);
+        stage<S, HO, kThenRk4>(st, P, G);
       }
       double *t = in;
       in = out;
@@ -612,7 +776,7 @@ template <int S, bool SRK>
 void stochastic(hipStream_t st, const DevParams &P, long nsteps, double dt, double *state, double *part,
                 const double *nat, double *compl_out, GfNoise Z) {
   double *in = part, *out = part + gf_part_doubles(P.n) / 2;
-  first<S, SRK>(st, P.n, state, nullptr, 0.0, nullptr, in);
+  first<S, SRK>(st, P.n, state, nullptr, 0.0, in);
   for (long s = 0; s < nsteps; ++s) {
     GfStep G{};
     G.x = state;
@@ -623,7 +787,7 @@ void stochastic(hipStream_t st, const DevParams &P, long nsteps, double dt, doub
     G.out = out;
     G.dt = dt;
     G.noise = Z;
-    stage<S, SRK, SRK ? kThenSrk : kThenEuler, 0>(st, P, G);
+    stage<S, SRK, SRK ? kThenSrk : kThenEuler>(st, P, G);
     ++Z.step;
     double *t = in;
     in = out;
@@ -709,63 +873,93 @@ void launch_global_stochastic(hipStream_t st, const DevParams &P, bool srk, long
   }
 }
 
-void launch_global_first(hipStream_t st, const DevParams &P, const double *x, const double *k0, double c0, double *out,
-                         double *part) {
-  if (P.s == 4)
-    first<4, false>(st, P.n, x, k0, c0, out, part);
-  else
-    first<3, false>(st, P.n, x, k0, c0, out, part);
+namespace {
+template <int S, int THEN, int NT>
+void gp(hipStream_t st, const DevParams &P, GpStep &G) {
+  G.nb = gf_blocks(P.n);
+  const auto run = [&](auto kernel) { kernel<<<dim3(G.nb), dim3(256), 0, st>>>(P, G); };
+  gf_wide(P.n) ? run(gp_stage<S, THEN, NT, 4>) : run(gp_stage<S, THEN, NT, 1>);
 }
 
-namespace {
-template <int S, int THEN>
-void dp_stage(hipStream_t st, const DevParams &P, GfStep &G) {
-  switch (G.T.n) {
-    case 1: stage<S, false, THEN, 1>(st, P, G); break;
-    case 2: stage<S, false, THEN, 2>(st, P, G); break;
-    case 3: stage<S, false, THEN, 3>(st, P, G); break;
-    case 4: stage<S, false, THEN, 4>(st, P, G); break;
-    default: stage<S, false, THEN, 5>(st, P, G);
+template <int S>
+void gp_start(hipStream_t st, const DevParams &P, const double *x, double *part, const double *nat, double *k) {
+  first<S, false>(st, P.n, x, nullptr, 0.0, part);
+  GpStep G{};
+  G.x = x;
+  G.in = part;
+  G.nat = nat;
+  G.k = k;
+  G.kb = k + (long)P.n * (S - 2);
+  gp<S, kGpStart, 0>(st, P, G);
+}
+
+template <int S>
+int gp_trial(hipStream_t st, const DevParams &P, const DpTrial &D, const double *nat, double *part) {
+  const long na = (long)P.n * (S - 2);
+  double *p0 = part, *p1 = part + gf_part_doubles(P.n) / 2;
+  double *tmp = D.tmp, *xa = D.tmp + na;
+  const auto first = [&](auto kernel) {
+    kernel<<<dim3(gf_blocks(P.n)), dim3(256), 0, st>>>(P.n, D.x, D.k[0], D.first, xa, tmp, p0);
+  };
+  gf_wide(P.n) ? first(gp_first<S, 4>) : first(gp_first<S, 1>);
+  GpStep G{};
+  G.nat = nat;
+  G.dt = D.dt;
+  G.eps_abs = D.eps_abs;
+  G.eps_rel = D.eps_rel;
+  // stage g (k2 .. k6) takes the block sums in one half and leaves the next ones in the other
+  for (int g = 1; g <= 5; ++g) {
+    G.x = tmp;
+    G.in = g & 1 ? p0 : p1;
+    G.out = g & 1 ? p1 : p0;
+    G.k = D.k[g];
+    G.kb = g == 1 ? nullptr : D.k[g] + na;
+    G.base = g < 5 ? xa : D.x;
+    G.T = D.terms[g - 1];
+    G.next = g < 5 ? tmp : D.out;
+    switch (g) {
+      case 1: gp<S, kGpNext, 1>(st, P, G); break;
+      case 2: gp<S, kGpNext, 2>(st, P, G); break;
+      case 3: gp<S, kGpNext, 3>(st, P, G); break;
+      case 4: gp<S, kGpNext, 4>(st, P, G); break;
+      default: gp<S, kGpOut, 4>(st, P, G);
+    }
   }
+  G.x = D.out;
+  G.in = p1;
+  G.out = p0;
+  G.k = D.k[6];
+  G.kb = D.k[6] + na;
+  G.base = D.x;
+  G.T = D.terms[5];
+  gp<S, kGpError, 5>(st, P, G);
+  return G.nb;
 }
 }  // namespace
 
-void launch_global_next(hipStream_t st, const DevParams &P, const double *x, const double *in, const double *nat,
-                        double *k, const double *base, const DpTerms &T, double *next, double *out) {
-  GfStep G{};
-  G.x = x;
-  G.in = in;
-  G.nat = nat;
-  G.k = k;
-  G.base = base;
-  G.T = T;
-  G.next = next;
-  G.out = out;
-  if (P.s == 4)
-    dp_stage<4, kThenNext>(st, P, G);
-  else
-    dp_stage<3, kThenNext>(st, P, G);
+void launch_dp_global_start(hipStream_t st, const DevParams &P, const double *x, double *part, const double *nat,
+                            double *k) {
+  P.s == 4 ? gp_start<4>(st, P, x, part, nat, k) : gp_start<3>(st, P, x, part, nat, k);
 }
 
-int launch_global_error(hipStream_t st, const DevParams &P, const double *x, const double *in, const double *nat,
-                        double *k, const double *x_old, const DpTerms &T, double dt, double eps_abs, double eps_rel,
-                        double *out) {
-  GfStep G{};
-  G.x = x;
-  G.in = in;
-  G.nat = nat;
-  G.k = k;
-  G.base = x_old;
-  G.T = T;
-  G.out = out;
-  G.dt = dt;
-  G.eps_abs = eps_abs;
-  G.eps_rel = eps_rel;
-  if (P.s == 4)
-    stage<4, false, kThenError, 5>(st, P, G);
+int launch_dp_global_trial(hipStream_t st, const DevParams &P, const DpTrial &D, const double *nat, double *part) {
+  return P.s == 4 ? gp_trial<4>(st, P, D, nat, part) : gp_trial<3>(st, P, D, nat, part);
+}
+
+void launch_dp_global_combine(hipStream_t st, int s, int n, const double *x, const DpTerms &T, double *out) {
+  const dim3 nb((unsigned)((n + 255L) / 256));
+  if (s == 4)
+    gp_combine<4><<<nb, dim3(256), 0, st>>>(n, x, T, out);
   else
-    stage<3, false, kThenError, 5>(st, P, G);
-  return gf_blocks(P.n);
+    gp_combine<3><<<nb, dim3(256), 0, st>>>(n, x, T, out);
+}
+
+void launch_dp_global_rows(hipStream_t st, int s, int n, const double *planes, double *rows) {
+  const dim3 nb((unsigned)((n + 255L) / 256));
+  if (s == 4)
+    gp_rows<4><<<nb, dim3(256), 0, st>>>(n, planes, rows);
+  else
+    gp_rows<3><<<nb, dim3(256), 0, st>>>(n, planes, rows);
 }
 
 }  // namespace spss

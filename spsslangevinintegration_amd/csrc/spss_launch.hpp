@@ -201,17 +201,24 @@ void launch_dp_combine(hipStream_t st, long m, const double *x, const DpTerms &T
 // into out[0] (partial: one double per 256 particles); returns the number of partials
 int launch_dp_error(hipStream_t st, int n, int s, const double *x_old, const double *dxdt_old, const DpTerms &T,
                     double dt, double eps_abs, double eps_rel, double *partial, double *out);
-// the same over the global field, from one launch to the next: a stage state out = x + c0 k0 with its
-// block sums; the derivative k at x from the block sums `in` with next = base + sum_j c_j k_j + c k (T.n
-// pointers, T.n + 1 coefficients) and its block sums; the last derivative with the
-// error norm's block maxima (their number is returned)
-void launch_global_first(hipStream_t st, const DevParams &P, const double *x, const double *k0, double c0, double *out,
-                         double *part);
-void launch_global_next(hipStream_t st, const DevParams &P, const double *x, const double *in, const double *nat,
-                        double *k, const double *base, const DpTerms &T, double *next, double *out);
-int launch_global_error(hipStream_t st, const DevParams &P, const double *x, const double *in, const double *nat,
-                        double *k, const double *x_old, const DpTerms &T, double dt, double eps_abs, double eps_rel,
-                        double *out);
+// the same over the global field.  Derivatives are two planes: [(s-2) n] of phases (and omegas), then
+// [2 n] of positions.
+struct DpTrial {
+  const double *x = nullptr;  // the state
+  double *out = nullptr;      // the new state
+  double *k[7] = {};          // k1 (given) .. k6, the derivative at `out`
+  double *tmp = nullptr;      // [s n]
+  double first = 0.0;         // the coefficient of k1 in the first stage
+  DpTerms terms[6] = {};      // of the later stages, the new state and the error: n earlier derivatives, and
+                              // as c[n] the coefficient of the one formed there
+  double dt = 0.0, eps_abs = 0.0, eps_rel = 0.0;
+};
+void launch_dp_global_start(hipStream_t st, const DevParams &P, const double *x, double *part, const double *nat,
+                            double *k);
+// the error norm's block maxima go to the front of part; their number is returned
+int launch_dp_global_trial(hipStream_t st, const DevParams &P, const DpTrial &D, const double *nat, double *part);
+void launch_dp_global_combine(hipStream_t st, int s, int n, const double *x, const DpTerms &T, double *out);
+void launch_dp_global_rows(hipStream_t st, int s, int n, const double *planes, double *rows);
 void launch_disp_max(hipStream_t st, int n, int s, const double *tot, double *partial);
 void launch_order_parameter(hipStream_t st, int n, int s, int slot, const double *state, double *partial,
                             double *out);

@@ -155,3 +155,38 @@ def test_field_of_zero_and_nonfinite(spss):
         g.set_state(st.reshape(-1))
         g.rk4_step(spss.METHOD_GLOBAL_FIELD, 0.01)
         assert np.all(np.isnan(g.get_state()[3::4]))
+
+
+@pytest.mark.parametrize("model,n,mode", [(3, 1, 0), (4, 255, 1), (3, 257, 1), (4, 1025, 0), (3, 131073, 0),
+                                          (4, 131072, 0), (4, 131073, 1)])
+def test_dormand_prince(spss, model, n, mode):
+    """the trials on planes of phases and positions: the same steps as the oracle's integration, the states
+    within 1e-10 (right-hand sides that agree to 1e-12 over the same steps), with and without an observer;
+    then lists, whose trials work on whole rows, in the same buffers"""
+    from oracle import dopri5_oracle as D
+    o, g = _systems(spss, model, n)
+    st, zeros = _state(model, n), np.zeros(model * n)
+
+    def rhs(x):
+        out = np.zeros(model * n)
+        o.evaluate_rhs(0, np.ascontiguousarray(x), zeros, out, 0.0, 0.0)
+        return out
+
+    integ = D.integrate_const if mode == 0 else D.integrate_adaptive
+    want, want_seen, ost = integ(rhs, st, 0.0, 0.3, 0.05, 1e-7, 1e-7)
+    seen = []
+    for observer in (lambda t, x: seen.append((t, x)), None):
+        g.set_state(st)
+        steps, rejected = g.integrate_dopri5(0.0, 0.3, 0.05, 1e-7, 1e-7, method=spss.METHOD_GLOBAL_FIELD, mode=mode,
+                                             observer=observer)
+        assert (steps, rejected) == (ost.steps, ost.rejected)
+        _close(g.get_state(), want, 1e-10)
+    assert len(seen) == len(want_seen)
+    for (_, x), (_, xw) in zip(seen, want_seen):
+        _close(x, xw, 1e-10)
+    if 1 < n < 2000:
+        h = _systems(spss, model, n)[1]
+        for s in (g, h):
+            s.set_state(st)
+            s.integrate_dopri5(0.0, 0.1, 0.05, 1e-7, 1e-7, method=spss.METHOD_ALL_PAIRS, mode=mode)
+        assert np.array_equal(g.get_state(), h.get_state())
