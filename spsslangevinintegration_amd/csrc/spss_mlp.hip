@@ -217,9 +217,6 @@ int spss_mlp_create(spss_mlp **out, const int *dims, int ndims, int max_batch, u
     if ((e = hipFuncSetAttribute((const void *)ml_rows, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  kNarrowParams * (int)sizeof(float))) != hipSuccess)
       return fail(e, "hipFuncSetAttribute");
-    if ((e = hipFuncSetAttribute((const void *)ml_predict, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 kPredictFloats * (int)sizeof(float))) != hipSuccess)
-      return fail(e, "hipFuncSetAttribute");
   }
   for (int k = 0; k < 2; ++k)
     if ((e = hipMalloc(&m->dz[k], rows * widest * sizeof(float))) != hipSuccess) return fail(e, "hipMalloc");
@@ -295,7 +292,7 @@ int spss_mlp_predict(spss_mlp *m, const float *x, long n, float *y) {
         const int B = (int)std::min<long>(kPredictPiece, c1 - r0);
         MCHK(hipMemcpyAsync(m->px + (r0 - c0) * din, x + r0 * din, (size_t)B * din * sizeof(float),
                             hipMemcpyHostToDevice, m->st));
-        hipLaunchKernelGGL(ml_predict, dim3(cdiv(B, kPR)), dim3(kTB), kPredictFloats * sizeof(float), m->st, m->net, m->p,
+        hipLaunchKernelGGL(ml_predict, dim3(cdiv(B, kPR)), dim3(kTB), 0, m->st, m->net, m->p,
                            m->px + (r0 - c0) * din, B, m->py + (r0 - c0) * dout);
         MCHK(hipGetLastError());
       }

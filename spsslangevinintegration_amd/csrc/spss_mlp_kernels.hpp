@@ -446,112 +446,86 @@ __global__ __launch_bounds__(kTB) void ml_grad(Net N, float *__restrict__ p, flo
   p[e] = pe - A.step_size * mm / (sqrtf(vv) * A.inv_sqrt_bc2 + A.eps);
 }
 
-// Forward pass of 64 rows per workgroup through all layers: the rows' activations and half of a
-// layer's weights in LDS (70 KB: two workgroups per CU, so that one computes while the other waits
-// for weights), 8 rows x 4 outputs per thread, so that three 16-byte reads feed 32 FMAs.  A layer's
-// outputs replace its inputs once every thread has its sums.  100,000 rows of 3 x 128 hidden: 219 us
-// (31 TFLOP/s; half of it are the error functions of the GELUs) for what took 98 x 4 launches of
-// 10.3 us; with a layer's whole weights in LDS, one workgroup per CU, 344 us.
+// Forward pass of 64 rows per workgroup through all layers, on the matrix cores (v_mfma_f32_16x16x4_f32: an
+// FP32 multiply-add per term, k ascending, so the sums are those of the kernels above bit for bit): the rows'
+// activations in LDS, a wave's up to 32 outputs of all rows in its registers, the weights straight from
+// the caches with the next sixteen inputs' on their way.  A layer's outputs replace its inputs once
+// every wave has its sums.  100,000 rows of 3 x 128 hidden: 201 us (34 TFLOP/s; the products 60, the error
+// functions of the GELUs 75, neither beside the other), 219 for FMAs of the vector units with the weights
+// through LDS.  The call is bound by the rows' way up: 32,768 of them take 54 us.
 constexpr int kPR = 64;           // rows
-constexpr int kPP = kPR + 4;      // pitch of the activations [width][rows]
-constexpr int kPW = kNarrow + 4;  // pitch of the weights [in][out]
-constexpr int kPK = 64;           // inputs whose weights are in LDS at a time
-constexpr int kPredictFloats = kNarrow * kPP + kPK * kPW;
+constexpr int kPP = kNarrow + 4;  // pitch of a row's activations: a product's 16 rows x 4 inputs in 64 banks
 
-// W[0..out) [k0 .. k0 + 64) transposed into w, four rows of W per wave and step
-__device__ __forceinline__ void stage_weights(const float *__restrict__ wl, int in, int out, int k0, float *w) {
-  const int i = k0 + (threadIdx.x & 63);
-#pragma unroll 4
-  for (int o = (threadIdx.x >> 6) * 4; o < out; o += kTB / 16) {
-    if (i >= in) continue;
-    const float *r = wl + (long)o * in + i;
-    float4 v;
-    v.x = r[0];
-    v.y = o + 1 < out ? r[in] : 0.f;
-    v.z = o + 2 < out ? r[2 * in] : 0.f;
-    v.w = o + 3 < out ? r[3 * in] : 0.f;
-    *(float4 *)(w + (i - k0) * kPW + o) = v;
-  }
-}
+typedef float mlp4 __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(kTB, 2) void ml_predict(Net N, const float *__restrict__ p, const float *__restrict__ X,
+__global__ __launch_bounds__(kTB, 4) void ml_predict(Net N, const float *__restrict__ p, const float *__restrict__ X,
                                                      int n, float *__restrict__ Y) {
-  extern __shared__ __align__(16) float sh[];
-  float *a = sh, *w = sh + kNarrow * kPP;
+  __shared__ __align__(16) float a[kPR * kPP];
   const int tid = threadIdx.x, b0 = blockIdx.x * kPR, R = min(kPR, n - b0);
-  const int og = tid & 31, rg = tid >> 5;
-  const int d0 = N.dims[0];
-  for (int e = tid; e < kPR * d0; e += kTB) {
-    const int r = e / d0, i = e - r * d0;
-    a[i * kPP + r] = r < R ? X[(long)(b0 + r) * d0 + i] : 0.f;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
+  const int d0 = N.dims[0], d4 = (d0 + 3) & ~3;
+  for (int e = tid; e < kPR * d4; e += kTB) {
+    const int r = e / d4, i = e - r * d4;
+    a[r * kPP + i] = r < R && i < d0 ? X[(long)(b0 + r) * d0 + i] : 0.f;
   }
+  __syncthreads();
   for (int l = 0; l < N.L; ++l) {
-    const int in = N.dims[l], out = N.dims[l + 1];
+    const int in = N.dims[l], out = N.dims[l + 1], tiles = (out + 15) / 16;
     const float *wl = p + N.woff[l], *bias = p + N.boff[l];
-    const bool last = l + 1 == N.L;
-    if (out <= 8) {  // a thread per row and output
-      float z[2] = {};
-      for (int k0 = 0; k0 < in; k0 += kPK) {
-        const int k1 = min(in, k0 + kPK);
-        stage_weights(wl, in, out, k0, w);
-        __syncthreads();
+    const bool last = l + 1 == N.L, two = wave + 4 < tiles;
+    mlp4 acc[2][4] = {};  // outputs 16 (wave + 4 t) + c of rows 16 q + 4 g ..
+    float bo[2] = {};
+    if (wave < tiles) {
+      const int o0 = 16 * wave + c, o1 = o0 + 64;
+      bo[0] = o0 < out ? bias[o0] : 0.f;
+      bo[1] = o1 < out ? bias[o1] : 0.f;
+      float w[2][4], v[2][4];
+      const auto load = [&](int k0, float (&to)[2][4]) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const int e = tid + q * kTB, r = e % kPR, o = e / kPR;
-          if (o < out)
-#pragma unroll 8
-            for (int i = k0; i < k1; ++i) z[q] = __builtin_fmaf(a[i * kPP + r], w[(i - k0) * kPW + o], z[q]);
+        for (int s = 0; s < 4; ++s) {
+          const int k = k0 + 4 * s + g;
+          to[0][s] = k < in && o0 < out ? wl[o0 * in + k] : 0.f;
+          to[1][s] = two && k < in && o1 < out ? wl[o1 * in + k] : 0.f;
         }
-        __syncthreads();
-      }
+      };
+      load(0, w);
+      for (int k0 = 0; k0 < in; k0 += 16) {
+        load(k0 + 16, v);
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int e = tid + q * kTB, r = e % kPR, o = e / kPR;
-        if (o >= out) continue;
-        const float v = z[q] + bias[o];
-        if (!last)
-          a[o * kPP + r] = gelu(v);
-        else if (r < R)
-          Y[(long)(b0 + r) * out + o] = v;
-      }
-    } else {
-      float acc[8][4] = {}, bo[4];
+        for (int s = 0; s < 4; ++s) {
+          if (k0 + 4 * s >= in) break;
+          float x[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) bo[q] = og * 4 + q < out ? bias[og * 4 + q] : 0.f;
-      for (int k0 = 0; k0 < in; k0 += kPK) {
-        const int k1 = min(in, k0 + kPK);
-        stage_weights(wl, in, out, k0, w);
-        __syncthreads();
-        if (og * 4 < out) {
-#pragma unroll 2
-          for (int i = k0; i < k1; ++i) {
-            const float4 x0 = *(const float4 *)(a + i * kPP + rg * 8), x1 = *(const float4 *)(a + i * kPP + rg * 8 + 4);
-            const float4 v = *(const float4 *)(w + (i - k0) * kPW + og * 4);
-            const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+          for (int q = 0; q < 4; ++q) x[q] = a[(16 * q + c) * kPP + k0 + 4 * s + g];
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
-              acc[r][0] = __builtin_fmaf(x[r], v.x, acc[r][0]);
-              acc[r][1] = __builtin_fmaf(x[r], v.y, acc[r][1]);
-              acc[r][2] = __builtin_fmaf(x[r], v.z, acc[r][2]);
-              acc[r][3] = __builtin_fmaf(x[r], v.w, acc[r][3]);
-            }
-          }
+          for (int q = 0; q < 4; ++q) acc[0][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q], w[0][s], acc[0][q], 0, 0, 0);
+          if (two)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              acc[1][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q], w[1][s], acc[1][q], 0, 0, 0);
         }
-        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) w[t][s] = v[t][s];
       }
+    }
+    __syncthreads();
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int o = og * 4 + q;
-        if (o >= out) continue;
+    for (int t = 0; t < 2; ++t) {
+      if (wave + 4 * t >= tiles) continue;
+      const int o = 16 * (wave + 4 * t) + c;
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
-          const float z = acc[r][q] + bo[q];
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = 16 * q + 4 * g + r;
+          const float z = acc[t][q][r] + bo[t];
           if (!last)
-            a[o * kPP + rg * 8 + r] = gelu(z);
-          else if (rg * 8 + r < R)
-            Y[(long)(b0 + rg * 8 + r) * out + o] = z;
+            a[row * kPP + o] = gelu(z);  // zeros past the last output: the next layer's padding
+          else if (row < R && o < out)
+            Y[(long)(b0 + row) * out + o] = z;
         }
-      }
     }
     __syncthreads();
   }
