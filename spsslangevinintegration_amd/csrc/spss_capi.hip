@@ -69,7 +69,8 @@ struct spss_system {
   CellBuffers cells, vcells;
   Cells64 cells64;
   int *vcount = nullptr, *vstart = nullptr, *vlist = nullptr, *vslot = nullptr;
-  VerletStage vstage;           // stage state in the order of the lists' build
+  VerletStage vstage[2];        // stage states in the order of the lists' build
+  unsigned long long *vmax = nullptr;
   long vcap = 0;
   const int *vorder = nullptr;  // cell order of the lists' build (null: built over all pairs)
   int *pcount = nullptr, *pstart = nullptr, *plist = nullptr;
@@ -269,10 +270,13 @@ int build_verlet(spss_system *h, int m) {
     TRY(dalloc_n(&h->vslot, (size_t)cap));
     h->vcap = cap;
   }
-  if (!h->vstage.stage) {
-    TRY(dalloc_n(&h->vstage.rec, (size_t)4 * h->n));
-    TRY(dalloc_n(&h->vstage.om, (size_t)h->n));
-    TRY(dalloc_n(&h->vstage.stage, (size_t)h->s * h->n));
+  if (!h->vmax) {
+    for (VerletStage &v : h->vstage) {
+      if (!v.rec) TRY(dalloc_n(&v.rec, (size_t)4 * h->n));
+      if (!v.om) TRY(dalloc_n(&v.om, (size_t)h->n));
+      if (!v.stage) TRY(dalloc_n(&v.stage, (size_t)h->s * h->n));
+    }
+    TRY(dalloc_n(&h->vmax, kVerletMax));
   }
   if (m == SPSS_METHOD_VERLET)
     launch_verlet_fill_all(st, h->P, h->stage, rmax2, h->vstart, h->vlist, h->vslot);
@@ -330,8 +334,8 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
         TRY(build_verlet(h, m));
         h->should_update = false;
       }
-      launch_stage_order(st, h->P, d_state, d_kprev, k_coef * dt, h->vorder, h->vstage);
-      launch_verlet_pairs(st, h->P, h->vstage, h->vorder, h->vstart, h->vslot, nat, d_knext, compl_out);
+      launch_stage_order(st, h->P, d_state, d_kprev, k_coef * dt, h->vorder, h->vstage[0]);
+      launch_verlet_pairs(st, h->P, h->vstage[0], h->vorder, h->vstart, h->vslot, nat, d_knext, compl_out);
       h->uses_verlet = true;
       break;
     default:
@@ -423,7 +427,48 @@ int global_steps(spss_system *h, int stepper, long nsteps, double dt, int noise_
   return SPSS_OK;
 }
 
+// a Runge-Kutta step over Verlet lists: each launch goes on from the derivative to the next stage
+int verlet_rk4_step(spss_system *h, int m, double dt) {
+  TRY(master_write(h, true));
+  TRY(check_method(h, m));
+  hipStream_t st = h->stream;
+  h->P.higher_order = h->higher_order ? 1 : 0;
+  h->P.fresh_k = 0;
+  const double *nat = h->have_nat ? h->nat : nullptr;
+  double *compl_out = h->higher_order ? h->compl_f : nullptr;
+  if (h->should_update) {
+    launch_stage(st, (long)h->s * h->n, h->state, h->k[0], 0.0, h->stage);
+    TRY(build_verlet(h, m));
+    h->should_update = false;
+  }
+  launch_stage_order(st, h->P, h->state, h->k[0], 0.0, h->vorder, h->vstage[0], h->vmax);
+  VerletThen N;
+  N.base = h->state;
+  N.dt = dt;
+  N.k1 = h->k[0];
+  N.k2 = h->k[1];
+  N.k3 = h->k[2];
+  N.vmax = h->vmax;
+  for (int g = 0; g < 4; ++g) {
+    N.kc = (g < 2 ? 0.5 : 1.0) * dt;
+    N.next = g < 3 ? h->vstage[(g + 1) & 1] : VerletStage{};
+    launch_verlet_pairs(st, h->P, h->vstage[g & 1], h->vorder, h->vstart, h->vslot, nat, h->k[g], compl_out, &N);
+  }
+  HIPCHECK(hipGetLastError());
+  h->uses_verlet = true;
+  ++h->step;
+  ++h->eager_steps;
+  double max2[kVerletMax];
+  HIPCHECK(hipMemcpyAsync(max2, h->vmax, sizeof(max2), hipMemcpyDeviceToHost, st));
+  HIPCHECK(hipStreamSynchronize(st));
+  update_verlet_flag(h, *std::max_element(max2, max2 + kVerletMax));
+  return SPSS_OK;
+}
+
 int rk4_step(spss_system *h, int method, double dt) {
+  const int m = resolve_method(h, method);
+  if ((m == SPSS_METHOD_VERLET || m == SPSS_METHOD_LINKED_LIST_VERLET) && check_method(h, m) == SPSS_OK)
+    return verlet_rk4_step(h, m, dt);
   if (use_global_steps(h, method)) return global_steps(h, SPSS_STEPPER_RK4, 1, dt, SPSS_NOISE_NONE, nullptr);
   TRY(master_write(h, true));
   TRY(rhs_device(h, method, h->state, h->k[0], h->k[0], 0.0, dt));
@@ -678,7 +723,8 @@ int spss_destroy(spss_system *h) {
   delete h->timer;
   void *bufs[] = {h->state, h->stage, h->k[0], h->k[1], h->k[2], h->k[3], h->deriv, h->compl_f, h->nat,
                   h->noise, h->partial, h->scal, h->acc, h->io[0], h->io[1], h->io[2], h->vcount, h->vstart,
-                  h->vlist, h->vslot, h->vstage.stage, h->vstage.rec, h->vstage.om, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec, h->scratch};
+                  h->vlist, h->vslot, h->vstage[0].stage, h->vstage[0].rec, h->vstage[0].om, h->vstage[1].stage,
+                  h->vstage[1].rec, h->vstage[1].om, h->vmax, h->pcount, h->pstart, h->plist, h->scan_blk, h->ap.rec, h->scratch};
   for (void *b : bufs) hipFree(b);
   for (double *b : h->dp) hipFree(b);
   if (h->dp_host) hipHostFree(h->dp_host);

@@ -11,6 +11,8 @@
 #include "spss_pairs64.hpp"
 #include "spss_scan.hpp"
 
+#include <type_traits>
+
 namespace spss {
 
 // ---------------------------------------------------------------------------
@@ -208,30 +210,34 @@ __global__ __launch_bounds__(kBlock) void k_verlet_build_cells(DevParams P, cons
 
 // stage state in the order of the lists' build (order null: as it is), and what the pair sums read of
 // it: x, y wrapped into the box (NaN farther out than the guard band covers) and the phasor in the frame
-// of particle 0's phase; om: omega from particle 0's (may be null)
+// of the phase that particle 0's state has; om: omega from that state's
+template <int S>
+__device__ __forceinline__ void stage_record(const DevParams &P, const double *v, double ref, double om_ref, int t,
+                                             const VerletStage &V) {
+#pragma unroll
+  for (int q = 0; q < S; ++q) V.stage[(long)t * S + q] = v[q];
+  double sn, cs, xw, yw;
+  frame_phasor_any(v[2], ref, sn, cs);
+  apply_pbc(P, v[0], v[1], xw, yw);
+  const bool near = fabs(v[0]) <= kFar64 * P.xs && fabs(v[1]) <= kFar64 * P.ys;
+  reinterpret_cast<double4 *>(V.rec)[t] = make_double4(near ? xw : __builtin_nan(""), yw, sn, cs);
+  if (S == 4) V.om[t] = v[S - 1] - om_ref;
+}
+
+// vmax: the step's displacement maxima, cleared (may be null)
 template <int S>
 __global__ __launch_bounds__(kBlock) void k_stage_order(DevParams P, const double *__restrict__ state,
                                                         const double *__restrict__ kprev, double kc_dt,
-                                                        const int *__restrict__ order, double *__restrict__ vstage,
-                                                        double4 *__restrict__ rec, double *__restrict__ om) {
+                                                        const int *__restrict__ order, VerletStage V,
+                                                        unsigned long long *__restrict__ vmax) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (vmax && t < kVerletMax) vmax[t] = 0ull;
   if (t >= P.n) return;
   const long i = order ? order[t] : t;
-  double v[S], first[S];
+  double v[S];
 #pragma unroll
-  for (int q = 0; q < S; ++q) {
-    v[q] = state[i * S + q] + (kprev ? kc_dt * kprev[i * S + q] : 0.0);
-    first[q] = state[q] + (kprev ? kc_dt * kprev[q] : 0.0);
-  }
-#pragma unroll
-  for (int q = 0; q < S; ++q) vstage[(long)t * S + q] = v[q];
-  double sn, cs;
-  frame_phasor_any(v[2], frame_ref(first[2]), sn, cs);
-  double xw, yw;
-  apply_pbc(P, v[0], v[1], xw, yw);
-  const bool near = fabs(v[0]) <= kFar64 * P.xs && fabs(v[1]) <= kFar64 * P.ys;
-  rec[t] = make_double4(near ? xw : __builtin_nan(""), yw, sn, cs);
-  if (S == 4 && om) om[t] = v[S - 1] - frame_ref(first[S - 1]);
+  for (int q = 0; q < S; ++q) v[q] = state[i * S + q] + (kprev ? kc_dt * kprev[i * S + q] : 0.0);
+  stage_record<S>(P, v, frame_ref(state[2]), S == 4 ? frame_ref(state[S - 1]) : 0.0, t, V);
 }
 
 // Verlet pair loop, ParticleSystemFirstOrderPtr.cpp:553-613 (x_i as stored), through the phasors
@@ -241,10 +247,14 @@ __global__ __launch_bounds__(kBlock) void k_stage_order(DevParams P, const doubl
 // entries of which 140 in range: 404 us with one thread per particle and a sine per pair, 32 with 16
 // lanes, records in list order and sin(d - alpha), 18.5 through the phasors (8, 32, 64 lanes: 27, 22, 24),
 // bound by the 32 bytes per entry from the caches (20 TB/s).
-template <int S, int LPP, bool HO>
+// THEN: 0 the derivative alone; 1 the next Runge-Kutta stage base + kc k beside it, for the next launch; 2
+// the step, base += (k1 + 2 k2 + 2 k3 + k) dt / 6, and its largest squared displacement.
+// A step was ten launches (four stages, four sums, the combination, the maximum), now five: n = 20,011 of
+// 600 entries, five steps with the state's transfers: 647 us, now 551.
+template <int S, int LPP, bool HO, int THEN>
 __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double band, const double *__restrict__ vstage,
                                                          const double4 *__restrict__ rec,
-                                                         const double *__restrict__ om,
+                                                         const double *__restrict__ om, VerletThen N,
                                                          const int *__restrict__ order,
                                                          const int *__restrict__ vstart, const int *__restrict__ vslot,
                                                          const double *__restrict__ nat, double *__restrict__ k_next,
@@ -253,6 +263,7 @@ __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double ban
   const int i = t < P.n ? (order ? order[t] : t) : -1;
   PhasorSums q;
   double4 own{};
+  double far = 0.0;
   if (i >= 0) {
     own = rec[t];
     int u = vstart[i] + l;
@@ -305,6 +316,26 @@ __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double ban
     phasor_of(st[2], sn, cs);
     write_k<S>(P, st, i, pair_acc<S>(P, q, own.z, own.w, HO ? om[t] : 0.0), nat ? nat[i] : 0.0, sn, cs, k_next,
                compl_out);
+    const long ii = (long)i * S;
+    if (THEN == 1) {
+      double v[S];
+#pragma unroll
+      for (int k = 0; k < S; ++k) v[k] = N.base[ii + k] + N.kc * k_next[ii + k];  // what k_next holds: see write_k
+      stage_record<S>(P, v, frame_ref(N.base[2]), S == 4 ? frame_ref(N.base[S - 1]) : 0.0, t, N.next);
+    } else if (THEN == 2) {
+      double tot[S];
+#pragma unroll
+      for (int k = 0; k < S; ++k) {
+        tot[k] = (N.k1[ii + k] + 2.0 * N.k2[ii + k] + 2.0 * N.k3[ii + k] + k_next[ii + k]) * N.dt / 6.0;
+        N.base[ii + k] += tot[k];
+      }
+      far = tot[0] * tot[0] + tot[1] * tot[1];
+    }
+  }
+  if (THEN == 2) {  // CalculateMaxDisplacement's dist2, one atomic per wave; not a number counts for nothing
+    for (int off = 32; off > 0; off >>= 1) far = fmax(far, __shfl_xor(far, off, 64));
+    if ((threadIdx.x & 63) == 0 && far > 0.0)
+      atomicMax(N.vmax + (blockIdx.x & (kVerletMax - 1)), (unsigned long long)__double_as_longlong(far));
   }
 }
 
@@ -647,38 +678,49 @@ void launch_verlet_fill_cells(hipStream_t st, const DevParams &P, const double *
   SPSS_DISPATCH_S(P.s, k_verlet_build_cells<SS, true><<<dim3(nblk((long)kBuildLanes * P.n)), dim3(kBlock), 0, st>>>(P, stage, ncx, ncy, cb.start, cb.sorted, rmax2, nullptr, vstart, vlist, vslot));
 }
 void launch_stage_order(hipStream_t st, const DevParams &P, const double *state, const double *kprev, double kc_dt,
-                        const int *order, const VerletStage &V) {
-  double4 *rec = reinterpret_cast<double4 *>(V.rec);
+                        const int *order, const VerletStage &V, unsigned long long *vmax) {
   if (P.s == 4)
-    k_stage_order<4><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, state, kprev, kc_dt, order, V.stage, rec, V.om);
+    k_stage_order<4><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, state, kprev, kc_dt, order, V, vmax);
   else
-    k_stage_order<3><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, state, kprev, kc_dt, order, V.stage, rec, nullptr);
+    k_stage_order<3><<<dim3(nblk(P.n)), dim3(kBlock), 0, st>>>(P, state, kprev, kc_dt, order, V, vmax);
 }
 
-template <int S, bool HO>
+template <int S, bool HO, int THEN>
 static void verlet_pairs_as(hipStream_t st, const DevParams &P, const VerletStage &V, const int *order,
                             const int *vstart, const int *vslot, const double *nat, double *k_next,
-                            double *compl_out) {
+                            double *compl_out, const VerletThen &N) {
   // 16 lanes read a list in contiguous 64-byte runs; fewer than 16,384 particles need a wave each to
   // fill the chip
   const double4 *rec = reinterpret_cast<const double4 *>(V.rec);
   const double band = pair_band(P.rho2, P.xs, P.ys);
   if (P.n < 16384)
-    k_verlet_pairs<S, 64, HO><<<dim3(nblk(64L * P.n)), dim3(kBlock), 0, st>>>(P, band, V.stage, rec, V.om, order, vstart,
-                                                                              vslot, nat, k_next, compl_out);
+    k_verlet_pairs<S, 64, HO, THEN><<<dim3(nblk(64L * P.n)), dim3(kBlock), 0, st>>>(
+        P, band, V.stage, rec, V.om, N, order, vstart, vslot, nat, k_next, compl_out);
   else
-    k_verlet_pairs<S, 16, HO><<<dim3(nblk(16L * P.n)), dim3(kBlock), 0, st>>>(P, band, V.stage, rec, V.om, order, vstart,
-                                                                              vslot, nat, k_next, compl_out);
+    k_verlet_pairs<S, 16, HO, THEN><<<dim3(nblk(16L * P.n)), dim3(kBlock), 0, st>>>(
+        P, band, V.stage, rec, V.om, N, order, vstart, vslot, nat, k_next, compl_out);
 }
 
 void launch_verlet_pairs(hipStream_t st, const DevParams &P, const VerletStage &V, const int *order,
-                         const int *vstart, const int *vslot, const double *nat, double *k_next, double *compl_out) {
+                         const int *vstart, const int *vslot, const double *nat, double *k_next, double *compl_out,
+                         const VerletThen *then) {
+  const VerletThen N = then ? *then : VerletThen{};
+  const auto as = [&](auto s, auto ho) {
+    constexpr int S = decltype(s)::value;
+    constexpr bool HO = decltype(ho)::value;
+    if (!then)
+      verlet_pairs_as<S, HO, 0>(st, P, V, order, vstart, vslot, nat, k_next, compl_out, N);
+    else if (N.next.stage)
+      verlet_pairs_as<S, HO, 1>(st, P, V, order, vstart, vslot, nat, k_next, compl_out, N);
+    else
+      verlet_pairs_as<S, HO, 2>(st, P, V, order, vstart, vslot, nat, k_next, compl_out, N);
+  };
   if (P.s == 3)
-    verlet_pairs_as<3, false>(st, P, V, order, vstart, vslot, nat, k_next, compl_out);
+    as(std::integral_constant<int, 3>{}, std::false_type{});
   else if (P.higher_order)
-    verlet_pairs_as<4, true>(st, P, V, order, vstart, vslot, nat, k_next, compl_out);
+    as(std::integral_constant<int, 4>{}, std::true_type{});
   else
-    verlet_pairs_as<4, false>(st, P, V, order, vstart, vslot, nat, k_next, compl_out);
+    as(std::integral_constant<int, 4>{}, std::false_type{});
 }
 
 void launch_rk4_combine(hipStream_t st, int s, int n, double *state, const double *k1, const double *k2,

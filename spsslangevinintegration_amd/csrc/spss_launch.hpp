@@ -151,16 +151,27 @@ void launch_verlet_count_cells(hipStream_t st, const DevParams &P, const double 
 void launch_verlet_fill_cells(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy,
                               const CellBuffers &cb, double rmax2, const int *vstart, int *vlist, int *vslot);
 // the stage state in the order of the lists' build (null: over all pairs), with the records and relative
-// omegas (for the complementary force, else null) that the pair sums over it read
+// omegas that the pair sums over it read
 struct VerletStage {
   double *stage = nullptr;  // [s n]
   double *rec = nullptr;    // [4 n] {x, y, sin psi, cos psi}
   double *om = nullptr;     // [n]
 };
+// what follows a derivative of the Runge-Kutta stepper in the same launch: the next stage (next set), or
+// the end of the step
+constexpr int kVerletMax = 64;
+struct VerletThen {
+  double *base = nullptr;  // the state
+  double kc = 0.0, dt = 0.0;
+  VerletStage next;
+  const double *k1 = nullptr, *k2 = nullptr, *k3 = nullptr;
+  unsigned long long *vmax = nullptr;  // [kVerletMax] bits of the largest squared displacements
+};
 void launch_stage_order(hipStream_t st, const DevParams &P, const double *state, const double *kprev, double kc_dt,
-                        const int *order, const VerletStage &V);
+                        const int *order, const VerletStage &V, unsigned long long *vmax = nullptr);
 void launch_verlet_pairs(hipStream_t st, const DevParams &P, const VerletStage &V, const int *order,
-                         const int *vstart, const int *vslot, const double *nat, double *k_next, double *compl_out);
+                         const int *vstart, const int *vslot, const double *nat, double *k_next, double *compl_out,
+                         const VerletThen *then = nullptr);
 // the global field (spss_global64.hip).  part: gf_part_doubles(n) doubles of scratch in two halves of
 // block sums; kprev may be null
 size_t gf_part_doubles(int n);

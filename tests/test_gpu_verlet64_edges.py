@@ -61,3 +61,33 @@ def test_verlet_bad_phase(spss, bad):
     g.evaluate_rhs(5, st.reshape(-1), z, kg, 0.0, 0.01)
     assert np.array_equal(np.isnan(ko), np.isnan(kg)) and np.isnan(ko).any()
     assert np.nanmax(np.abs(kg - ko) / np.maximum(np.abs(ko), 1.0)) <= 1e-12
+
+
+@pytest.mark.parametrize("model,n,rho,method,order", [
+    (4, 1, 0.1, 5, 0), (3, 65, 0.3, 4, 0), (4, 255, 0.05, 5, 1), (4, 2500, 0.06, 4, 1), (3, 16383, 0.03, 5, 0),
+    (4, 16385, 0.03, 5, 0)])
+def test_verlet_rk4_steps(spss, model, n, rho, method, order):
+    """Runge-Kutta steps, whose launches go on to the next stage: four steps, lists rebuilt on the way.
+    Each derivative is within 1e-12 of the oracle's, so that a step of 0.02 adds less than 1e-13 and the
+    state after four stays within 1e-12; the displacement's sum is one of values near 0.02."""
+    import oracle
+    print(f"[gpu] verlet rk4 model={model} n={n} rho={rho} method={method}", flush=True)
+    rng = np.random.default_rng(3 * n + method)
+    st = rng.random((n, model)) - 0.5
+    st[:, 2] *= 6.0
+    kw = dict(model=model, n=n, v0=1.0, xi=0.7, sigma=1.3, rho=rho, alpha=0.4)
+    o, g = oracle.Oracle(**kw), spss.ParticleSystem(**kw)
+    if model == 4:
+        o.set_higher_order(order)
+        g.set_higher_order(order)
+    so = st.reshape(-1).copy()
+    g.set_state(so)
+    rebuilt = 0
+    for _ in range(4):
+        o.rk4_step(method, so, 0.02)
+        g.rk4_step(method, 0.02)
+        flag, acc, uses = g.verlet_status()
+        assert uses and flag == o.should_update_lists and abs(acc - o.accumulated_displacement) <= 1e-13
+        rebuilt += flag
+        assert np.max(np.abs(g.get_state().reshape(-1) - so) / np.maximum(np.abs(so), 1.0)) <= 1e-12
+    assert rebuilt
