@@ -31,6 +31,23 @@ class HostCopy {
   HostCopy &operator=(const HostCopy &) = delete;
   ~HostCopy() { drop(); }
 
+  // the buffer for copies of that much; false if there is none (they go to the runtime then)
+  bool reserve(size_t bytes) {
+    if (bytes < kCopyMin) return false;
+    const size_t want = std::min(kCopyBuffer, piece_of(bytes) * kCopyPieces);
+    if (cap_ >= want) return true;
+    drop();
+    bool ok = hipHostMalloc(reinterpret_cast<void **>(&pin_), want, hipHostMallocDefault) == hipSuccess;
+    for (hipEvent_t &e : ev_) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+      (void)hipGetLastError();
+      drop();
+      return false;
+    }
+    cap_ = want;
+    return true;
+  }
+
   hipError_t to_host(void *dst, const void *src, size_t bytes, hipStream_t st) {
     if (!staged(dst, bytes)) return direct(dst, src, bytes, hipMemcpyDeviceToHost, st);
     char *d = static_cast<char *>(dst);
@@ -87,18 +104,7 @@ class HostCopy {
     } else {
       (void)hipGetLastError();  // memory that the runtime does not know
     }
-    const size_t want = std::min(kCopyBuffer, piece_of(bytes) * kCopyPieces);
-    if (cap_ >= want) return true;
-    drop();
-    bool ok = hipHostMalloc(reinterpret_cast<void **>(&pin_), want, hipHostMallocDefault) == hipSuccess;
-    for (hipEvent_t &e : ev_) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-    if (!ok) {
-      (void)hipGetLastError();
-      drop();
-      return false;
-    }
-    cap_ = want;
-    return true;
+    return reserve(bytes);
   }
 
   // work(0) .. work(n - 1) on this thread and up to kCopyThreads - 1 others
