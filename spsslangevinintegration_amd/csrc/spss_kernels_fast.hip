@@ -431,25 +431,32 @@ static Layout layout_of(const FastPath *f) {
   return L;
 }
 
-// sorted order, cell starts and snapshot of a stage state (original order)
-static void build(FastPath *f, hipStream_t st, const DevParams &P, const double *stage, int *start, float4 *snap,
-                  float *omega) {
+// sorted order, cell starts and snapshot of a stage state (original order); rstate: the resident arrays too
+template <int S>
+static void build_as(FastPath *f, hipStream_t st, const DevParams &P, const double *stage, int *start, int *sorted,
+                     float4 *snap, float *omega, const double *nat, double *rstate, double *rnat) {
   const int n = f->n;
   const unsigned nb = nblocks(n);
-  const Layout L = layout_of(f);
-  if (P.s == 4)
-    fk_keys<4><<<nb, 256, 0, st>>>(P, L, stage, f->ncx, f->ncy, f->key, f->slot, f->count);
-  else
-    fk_keys<3><<<nb, 256, 0, st>>>(P, L, stage, f->ncx, f->ncy, f->key, f->slot, f->count);
+  fk_keys<S><<<nb, 256, 0, st>>>(P, layout_of(f), stage, f->ncx, f->ncy, f->key, f->slot, f->count);
   scan_local<<<f->nsb, 256, 0, st>>>(f->count, nullptr, f->cells, start, f->blocksum);
   scan_add<<<f->nsb, 256, 0, st>>>(f->count, nullptr, f->cells, start, f->blocksum, f->nsb, f->ovf_count);
   fk_scatter<<<nb, 256, 0, st>>>(n, f->key, f->slot, start, f->tmp);
-  if (P.s == 4)
-    fk_rank<4><<<nb, 256, 0, st>>>(P, stage, f->ncx, f->cpr, f->Hx, f->Hy, f->key, start, f->tmp, f->sorted, snap,
-                                   omega);
+  float *om = S == 4 ? omega : nullptr;
+  if (rstate)
+    fk_rank<S, true><<<nb, 256, 0, st>>>(P, stage, f->ncx, f->cpr, f->Hx, f->Hy, f->key, start, f->tmp, nat, sorted,
+                                         snap, om, rstate, rnat);
   else
-    fk_rank<3><<<nb, 256, 0, st>>>(P, stage, f->ncx, f->cpr, f->Hx, f->Hy, f->key, start, f->tmp, f->sorted, snap,
-                                   nullptr);
+    fk_rank<S, false><<<nb, 256, 0, st>>>(P, stage, f->ncx, f->cpr, f->Hx, f->Hy, f->key, start, f->tmp, nullptr,
+                                          sorted, snap, om, nullptr, nullptr);
+}
+
+static void build(FastPath *f, hipStream_t st, const DevParams &P, const double *stage, int *start, int *sorted,
+                  float4 *snap, float *omega, const double *nat = nullptr, double *rstate = nullptr,
+                  double *rnat = nullptr) {
+  if (P.s == 4)
+    build_as<4>(f, st, P, stage, start, sorted, snap, omega, nat, rstate, rnat);
+  else
+    build_as<3>(f, st, P, stage, start, sorted, snap, omega, nat, rstate, rnat);
 }
 
 // row tiles of the rebuilt cell list (single systems), from the starts build() left in f->start
@@ -485,7 +492,7 @@ static void launch_pairs(const FastPath *f, hipStream_t st, const DevParams &P, 
 int fast_rhs(FastPath *f, hipStream_t st, const DevParams &P, const double *stage, const double *nat,
              double *k_next, double *compl_out) {
   const bool srk = P.higher_order && compl_out && P.s == 4;
-  build(f, st, P, stage, f->start, f->snap, srk ? f->omega_f : nullptr);
+  build(f, st, P, stage, f->start, f->sorted, f->snap, srk ? f->omega_f : nullptr);
   rebuilt_row_tiles(f, st);
   PairBufs B = rebuilt_bufs(f, stage);
   B.nat = nat;
@@ -568,12 +575,7 @@ static void ensure_moves_of(FastPath *f, hipStream_t st, const DevParams &P, boo
 static void resident_enter(FastPath *f, hipStream_t st, const DevParams &P, const double *state,
                            const double *nat, bool srk) {
   const int c = f->cur;
-  build(f, st, P, state, f->rstart[c], f->rsnap, (srk && P.s == 4) ? f->romega : nullptr);
-  const unsigned nb = nblocks(f->n);
-  if (P.s == 4)
-    fr_gather<4><<<nb, 256, 0, st>>>(f->n, state, f->sorted, nat, f->rstate[c], f->rid[c], f->rnat[c]);
-  else
-    fr_gather<3><<<nb, 256, 0, st>>>(f->n, state, f->sorted, nat, f->rstate[c], f->rid[c], f->rnat[c]);
+  build(f, st, P, state, f->rstart[c], f->rid[c], f->rsnap, srk ? f->romega : nullptr, nat, f->rstate[c], f->rnat[c]);
   if (f->rtiles)
     fk_row_tiles<<<(f->ncy + 3) / 4, 256, 0, st>>>(f->rstart[c], f->ncx, f->ncy, f->rt_wcap, f->rt_cmax, f->rtiles);
   drop_moves(f, st);
@@ -944,7 +946,7 @@ int fast_batch_stats(FastPath *f, hipStream_t st, double *racc, double *zlast, u
 int fast_replica_count(const FastPath *f) { return f->R; }
 
 int fast_pairs_count(FastPath *f, hipStream_t st, const DevParams &P, const double *stage, int *count) {
-  build(f, st, P, stage, f->start, f->snap, nullptr);
+  build(f, st, P, stage, f->start, f->sorted, f->snap, nullptr);
   rebuilt_row_tiles(f, st);
   PairBufs B = rebuilt_bufs(f, stage);
   B.pcount = count;
