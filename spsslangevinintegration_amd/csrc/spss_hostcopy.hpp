@@ -3,8 +3,9 @@
 // The runtime stages such a copy through its own pinned memory with one thread: 21 MB take 1.2 ms, of
 // which the transfer is 0.4, and 5.1 ms into memory that has no pages yet.  Here the transfer goes to a
 // pinned buffer of the handle in pieces, and up to kCopyThreads threads move them on as they arrive: 0.68
-// and 1.3 ms (two threads 0.68 and 3.0).  Small copies, where the threads' start (some 60 us) counts, and
-// memory that is pinned already go to the runtime; so do copies to the device, where it is no slower.
+// and 1.3 ms (two threads 0.68 and 3.0).  Below 16 MB the runtime does it: a handle's first copy of 10 MB took
+// 1.3 ms here (new pinned pages, threads) and 0.65 there, a later one 0.55 and 0.62.  So it does for memory that
+// is pinned already, and for copies to the device, where it is no slower.
 // Every call returns with the copy done, as before.
 #pragma once
 
@@ -19,7 +20,7 @@
 
 namespace spss {
 
-constexpr size_t kCopyMin = 4u << 20, kCopyBuffer = 32u << 20;  // bytes
+constexpr size_t kCopyMin = 16u << 20, kCopyBuffer = 32u << 20;  // bytes
 constexpr int kCopyPieces = 16, kCopyThreads = 8;
 
 // the pinned buffer (at most kCopyBuffer bytes) and the pieces' events, kept by a handle and given back

@@ -23,7 +23,7 @@ def _system(spss, n, model=4):
     return g, st
 
 
-@pytest.mark.parametrize("n", [131071, 131072, 131073, 200003, 1048576, 1048577, 2300001])
+@pytest.mark.parametrize("n", [131071, 131072, 131073, 200003, 524287, 524288, 524289, 1048576, 1048577, 2300001])
 def test_state(spss, n):
     g, st = _system(spss, n)
     assert np.array_equal(g.get_state(), st)
