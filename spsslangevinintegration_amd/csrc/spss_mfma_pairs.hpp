@@ -35,7 +35,6 @@ typedef _Float16 mhalf4 __attribute__((ext_vector_type(4)));
 constexpr int kMStage = 1088;         // staged entries: particles, and padding to whole units of 16 per row
 constexpr int kMPlane = kMStage + 16; // and one unit out of every range; digit planes 20 banks apart
 constexpr int kMUnits = 84;           // units of one group's candidates, and sixteen out of every range
-constexpr int kMRows = 16;            // rows of a stencil, at most
 constexpr float kMUnit = 1024.f;      // positions: cells to |x| < 25 in halves, their second halves not denormal
 constexpr float kMSquare = 0x1p-14f;  // squares in halves
 constexpr float kMFar = 3e4f;         // "|x|^2" of padding at x = 0, in squares: beyond every range

@@ -1,11 +1,11 @@
 """States and frames copied to the host in threaded pieces: byte counts at and around the smallest staged
 copy, ragged pieces, more than one turn of the pinned buffer, pinned destinations, several handles from
 several threads.  The copies are exact: compared bit for bit with what was set."""
+import ctypes as C
 import threading
 
 import numpy as np
 import pytest
-import torch
 
 pytestmark = pytest.mark.gpu
 
@@ -29,8 +29,13 @@ def test_state(spss, n):
     assert np.array_equal(g.get_state(), st)
     out = np.zeros(4 * n)
     assert np.array_equal(g.get_state(out), st)  # into memory that has its pages
-    pinned = torch.zeros(4 * n, dtype=torch.float64, pin_memory=True).numpy()
-    assert np.array_equal(g.get_state(pinned), st)
+    p = C.c_void_p()
+    assert g.lib.hipHostMalloc(C.byref(p), C.c_size_t(32 * n), C.c_uint(0)) == 0  # of the library's runtime
+    try:
+        pinned = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_double)), (4 * n,))
+        assert np.array_equal(g.get_state(pinned), st)
+    finally:
+        assert g.lib.hipHostFree(p) == 0
 
 
 @pytest.mark.parametrize("n", [349525, 349526, 1048575])
