@@ -276,7 +276,7 @@ int build_verlet(spss_system *h, int m) {
       if (!v.om) TRY(dalloc_n(&v.om, (size_t)h->n));
       if (!v.stage) TRY(dalloc_n(&v.stage, (size_t)h->s * h->n));
     }
-    TRY(dalloc_n(&h->vmax, kVerletMax));
+    TRY(dalloc_n(&h->vmax, kVerletMax * kVerletMaxStep));
   }
   if (m == SPSS_METHOD_VERLET)
     launch_verlet_fill_all(st, h->P, h->stage, rmax2, h->vstart, h->vlist, h->vslot);
@@ -458,10 +458,11 @@ int verlet_rk4_step(spss_system *h, int m, double dt) {
   h->uses_verlet = true;
   ++h->step;
   ++h->eager_steps;
-  double max2[kVerletMax];
+  double max2[kVerletMax * kVerletMaxStep], most = 0.0;
   HIPCHECK(hipMemcpyAsync(max2, h->vmax, sizeof(max2), hipMemcpyDeviceToHost, st));
   HIPCHECK(hipStreamSynchronize(st));
-  update_verlet_flag(h, *std::max_element(max2, max2 + kVerletMax));
+  for (int g = 0; g < kVerletMax; ++g) most = std::max(most, max2[g * kVerletMaxStep]);
+  update_verlet_flag(h, most);
   return SPSS_OK;
 }
 

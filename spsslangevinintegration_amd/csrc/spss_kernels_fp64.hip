@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kBlock) void k_stage_order(DevParams P, const doubl
                                                         const int *__restrict__ order, VerletStage V,
                                                         unsigned long long *__restrict__ vmax) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (vmax && t < kVerletMax) vmax[t] = 0ull;
+  if (vmax && t < kVerletMax) vmax[t * kVerletMaxStep] = 0ull;
   if (t >= P.n) return;
   const long i = order ? order[t] : t;
   double v[S];
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kBlock) void k_stage_order(DevParams P, const doubl
 // THEN: 0 the derivative alone; 1 the next Runge-Kutta stage base + kc k beside it, for the next launch; 2
 // the step, base += (k1 + 2 k2 + 2 k3 + k) dt / 6, and its largest squared displacement.
 // A step was ten launches (four stages, four sums, the combination, the maximum), now five: n = 20,011 of
-// 600 entries, five steps with the state's transfers: 647 us, now 551.
+// 600 entries, five steps with the state's transfers: 647 us, now 513.
 template <int S, int LPP, bool HO, int THEN>
 __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double band, const double *__restrict__ vstage,
                                                          const double4 *__restrict__ rec,
@@ -263,7 +263,12 @@ __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double ban
   const int i = t < P.n ? (order ? order[t] : t) : -1;
   PhasorSums q;
   double4 own{};
-  double far = 0.0;
+  double pre = 0.0, old = 0.0, k4[S] = {};  // THEN 2: component l of k1 + 2 k2 + 2 k3 and of the state
+  if (THEN == 2 && i >= 0 && l < S) {
+    const long c = (long)i * S + l;
+    pre = N.k1[c] + 2.0 * N.k2[c] + 2.0 * N.k3[c];
+    old = N.base[c];
+  }
   if (i >= 0) {
     own = rec[t];
     int u = vstart[i] + l;
@@ -323,19 +328,35 @@ __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double ban
       for (int k = 0; k < S; ++k) v[k] = N.base[ii + k] + N.kc * k_next[ii + k];  // what k_next holds: see write_k
       stage_record<S>(P, v, frame_ref(N.base[2]), S == 4 ? frame_ref(N.base[S - 1]) : 0.0, t, N.next);
     } else if (THEN == 2) {
-      double tot[S];
 #pragma unroll
-      for (int k = 0; k < S; ++k) {
-        tot[k] = (N.k1[ii + k] + 2.0 * N.k2[ii + k] + 2.0 * N.k3[ii + k] + k_next[ii + k]) * N.dt / 6.0;
-        N.base[ii + k] += tot[k];
-      }
-      far = tot[0] * tot[0] + tot[1] * tot[1];
+      for (int k = 0; k < S; ++k) k4[k] = k_next[ii + k];
     }
   }
-  if (THEN == 2) {  // CalculateMaxDisplacement's dist2, one atomic per wave; not a number counts for nothing
+  // CalculateMaxDisplacement's dist2; not a number counts for nothing.  One atomic per workgroup, where it would
+  // raise what is there, the groups' maxima a cache line each: n = 20,011 1.6 us more than THEN 1; per wave with
+  // sixteen maxima to a line 10.5, per workgroup 8.8
+  if (THEN == 2) {
+    __shared__ double wave[kBlock / 64];
+    double k = 0.0, tot = 0.0;
+#pragma unroll
+    for (int c = 0; c < S; ++c) {
+      const double v = __shfl(k4[c], 0, LPP);
+      if (l == c) k = v;
+    }
+    if (i >= 0 && l < S) {
+      tot = (pre + k) * N.dt / 6.0;
+      N.base[(long)i * S + l] = old + tot;
+    }
+    const double dx = __shfl(tot, 0, LPP), dy = __shfl(tot, 1, LPP);
+    double far = dx * dx + dy * dy;
     for (int off = 32; off > 0; off >>= 1) far = fmax(far, __shfl_xor(far, off, 64));
-    if ((threadIdx.x & 63) == 0 && far > 0.0)
-      atomicMax(N.vmax + (blockIdx.x & (kVerletMax - 1)), (unsigned long long)__double_as_longlong(far));
+    if ((threadIdx.x & 63) == 0) wave[threadIdx.x / 64] = far;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 1; w < kBlock / 64; ++w) far = fmax(far, wave[w]);
+      unsigned long long *m = N.vmax + (blockIdx.x & (kVerletMax - 1)) * kVerletMaxStep, v = __double_as_longlong(far);
+      if (far > 0.0 && v > __hip_atomic_load(m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(m, v);
+    }
   }
 }
 

@@ -159,13 +159,13 @@ struct VerletStage {
 };
 // what follows a derivative of the Runge-Kutta stepper in the same launch: the next stage (next set), or
 // the end of the step
-constexpr int kVerletMax = 64;
+constexpr int kVerletMax = 64, kVerletMaxStep = 16;  // maxima of groups of workgroups, a cache line each
 struct VerletThen {
   double *base = nullptr;  // the state
   double kc = 0.0, dt = 0.0;
   VerletStage next;
   const double *k1 = nullptr, *k2 = nullptr, *k3 = nullptr;
-  unsigned long long *vmax = nullptr;  // [kVerletMax] bits of the largest squared displacements
+  unsigned long long *vmax = nullptr;  // [kVerletMax kVerletMaxStep] bits of the largest squared displacements
 };
 void launch_stage_order(hipStream_t st, const DevParams &P, const double *state, const double *kprev, double kc_dt,
                         const int *order, const VerletStage &V, unsigned long long *vmax = nullptr);
