@@ -408,7 +408,7 @@ def screen_at_scale(spss, n_train=20000, n_screen=100000, n_lines=16, steps=2000
 
 
 def fp64_step_rate(spss, steps=10, warmup=2):
-    """the reference-precision (FP64, the reference's operation order) cell-list Euler step of the
+    """the reference-precision (FP64) cell-list Euler step of the
     headline system: device counting sort and 9-cell pair loop every step"""
     g, kw, _, _ = headline_system(spss, precision=spss.PRECISION_FP64)
     g.run(spss.STEPPER_EULER, spss.METHOD_LINKED_LIST, warmup, 0.002, spss.NOISE_PHILOX)

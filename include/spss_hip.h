@@ -47,13 +47,14 @@ extern "C" {
 #define SPSS_METHOD_LINKED_LIST_VERLET 5 /* EvaluateInteractionsWithLinkedListAndVerletNeighborList, :616-815 */
 
 /* arithmetic of the pair sums */
-#define SPSS_PRECISION_FP64 0  /* FP64, the reference's operation order */
+#define SPSS_PRECISION_FP64 0  /* FP64; neighbour sets are the reference's bit for bit */
 #define SPSS_PRECISION_FP32C 1 /* models 3 and 4, the linked-list method (RHS and fused stochastic
                                   steps) and exact-mode Verlet lists (fused stochastic steps): FP32
                                   distance tests (guard band decided in FP64, so the neighbour sets
                                   equal the FP64 ones), coupling sums through the neighbours' unit
-                                  phasors in FP32 partial sums combined in FP64, FP64 state and
-                                  stage combination */
+                                  phasors in FP32 partial sums combined in FP64 (Verlet: exact
+                                  sums of fixed-point phasors on the matrix cores), FP64 state
+                                  and stage combination */
 
 /* Verlet semantics */
 #define SPSS_VERLET_COMPAT 0 /* reference: r_max = rho + 0.05, candidates from the 9 cells */

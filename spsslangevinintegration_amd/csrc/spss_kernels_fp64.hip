@@ -1,9 +1,10 @@
-// spss_kernels_fp64.hip -- FP64 kernels that follow the reference's operation order.
+// spss_kernels_fp64.hip -- FP64 kernels: the cell list on general boxes and grids, Verlet lists, the steppers'
+// updates and the reductions (all pairs, the cell list on the unit box and the global field have files of
+// their own).
 //
-// Every pair sum is accumulated in the order the reference visits the pairs
-// (j ascending for all-pairs; stencil order then ascending j for cells; list
-// order for Verlet), so results agree with the reference to the last few ulps
-// of the device sin/cos.  Built with -ffp-contract=off.
+// The general cell list's sums are accumulated pair by pair in the order the reference visits the pairs
+// (stencil order, then ascending j), so results agree with it to the last few ulps of the device
+// sin/cos; the Verlet sums go through phasors (spss_pairs64.hpp).  Built with -ffp-contract=off.
 #pragma clang fp contract(off)
 
 #include "spss_device.hpp"
