@@ -125,6 +125,7 @@ void launch_linked_list(hipStream_t st, const DevParams &P, const double *stage,
 // coarser grids, where the reference visits cells more than once, and finer ones, whose cells are
 // mostly empty below a hundred million particles, take the two calls above
 struct Cells64 {
+  char *mem = nullptr;                 // the allocation that holds them all
   int *order[2] = {nullptr, nullptr};  // [n] particle of each sorted position: the last build's, the next one's
   int cur = 0;
   int *key = nullptr, *slot = nullptr, *count = nullptr, *blocksum = nullptr, *bad = nullptr;
