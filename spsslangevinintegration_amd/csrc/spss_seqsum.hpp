@@ -37,13 +37,14 @@ __host__ __device__ __forceinline__ void seq_term(SeqMap &m, float v, float limi
     return;
   }
   if (m.reach == kSeqNever) return;
-  const float w = floorf(v), f = v - w;  // both exact
-  const int k = (int)w, up = f > 0.5f ? 1 : 0, tie = f == 0.5f ? 1 : 0;
+  // d is exact (of v's last place and at most half), which v less its floor is not: -(0.5 - 2^-25) leaves 0.5 there
+  const float w = rintf(v), d = v - w;
+  const int k = (int)w, other = d == 0.5f ? 1 : (d == -0.5f ? -1 : 0);  // a tie's other whole number, from k
   const int need = (int)a + 2;
   m.reach = need > m.reach ? need : m.reach;
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
-    m.inc[p] += k + (tie ? ((p + m.inc[p] + k) & 1) : up);
+    m.inc[p] += k + (((p + m.inc[p] + k) & 1) ? other : 0);
     m.lo[p] = m.inc[p] < m.lo[p] ? m.inc[p] : m.lo[p];
     m.hi[p] = m.inc[p] > m.hi[p] ? m.inc[p] : m.hi[p];
   }
