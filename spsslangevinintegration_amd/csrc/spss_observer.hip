@@ -106,10 +106,7 @@ __global__ __launch_bounds__(256) void ob_long_runs(const SeqMap *__restrict__ r
 
 // s through the map in lane k of m: true if it stayed in its binade
 __device__ __forceinline__ bool seq_pass(const SeqMap &m, int k, float &s) {
-  if (s == 0.f) {  // zeros alone leave it (k: the smallest exponent, which bounds every other term out)
-    const int lo = __builtin_amdgcn_readlane(m.lo[0], k), hi = __builtin_amdgcn_readlane(m.hi[0], k);
-    return __builtin_amdgcn_readlane(m.reach, k) <= 2 && lo == 0 && hi == 0;
-  }
+  if (s == 0.f) return seq_zeros(__builtin_amdgcn_readlane(m.reach, k));
   const int S = seq_units(s), p = S & 1;
   const int inc = __builtin_amdgcn_readlane(p ? m.inc[1] : m.inc[0], k);
   const int lo = __builtin_amdgcn_readlane(p ? m.lo[1] : m.lo[0], k);
@@ -123,9 +120,6 @@ __device__ __forceinline__ bool seq_pass(const SeqMap &m, int k, float &s) {
 __device__ __forceinline__ float wave_uniform(float s) {
   return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(s)));
 }
-
-// the exponent slot to look s up in (zero: the smallest), or -1
-__device__ __forceinline__ int seq_lookup(float s) { return s == 0.f ? 0 : seq_slot(s); }
 
 // what the walk needs of one long run: its maps (an exponent per lane), its 16 runs' maps for the
 // exponents k0, k0 + 1, k0 - 1, k0 - 2 (lane = run + 16 * exponent), and its terms if L == 256

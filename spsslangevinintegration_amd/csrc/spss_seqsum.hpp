@@ -22,7 +22,7 @@ constexpr int kSeqLevel = 16;  // runs composed into a long run
 struct SeqMap {
   int inc[2];       // increment of S by its parity at the start
   int lo[2], hi[2]; // least and largest increment on the way (the start's 0 among them)
-  int reach;        // a bound of |c / u| + 1 of every term; kSeqNever: no statement
+  int reach;        // a bound of |c / u| + 1 of every term, 1 for zeros alone; kSeqNever: no statement
   int pad;
 };
 constexpr int kSeqNever = 0x7fffffff;
@@ -40,7 +40,7 @@ __host__ __device__ __forceinline__ void seq_term(SeqMap &m, float v, float limi
   // d is exact (of v's last place and at most half), which v less its floor is not: -(0.5 - 2^-25) leaves 0.5 there
   const float w = rintf(v), d = v - w;
   const int k = (int)w, other = d == 0.5f ? 1 : (d == -0.5f ? -1 : 0);  // a tie's other whole number, from k
-  const int need = (int)a + 2;
+  const int need = a > 0.f ? (int)a + 2 : 1;
   m.reach = need > m.reach ? need : m.reach;
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
@@ -78,6 +78,13 @@ __host__ __device__ __forceinline__ int seq_slot(float s) {
   const int e = (int)((b.u >> 23) & 0xff) - 127 - kSeqExp0;
   return e >= 0 && e < 64 ? e : -1;
 }
+
+// the slot to look s up in (zero: the smallest), or -1
+__host__ __device__ __forceinline__ int seq_lookup(float s) { return s == 0.f ? 0 : seq_slot(s); }
+
+// whether a run whose map has this reach leaves a zero sum at zero: its terms are all zeros (increments of
+// zero do not tell: every exponent's unit has terms too small for it)
+__host__ __device__ __forceinline__ bool seq_zeros(int reach) { return reach == 1; }
 
 // s as a multiple of its ulp
 __host__ __device__ __forceinline__ int seq_units(float s) {

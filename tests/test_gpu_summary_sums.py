@@ -10,7 +10,10 @@ pytestmark = pytest.mark.gpu
 NEAR_TIES = np.concatenate([np.full(140000, np.arccos(0.95)), np.tile([np.arccos(0.95), 1.5786089058042636], 2000)])
 
 
-@pytest.mark.parametrize("phases", [NEAR_TIES], ids=["near ties"])
+TINY = np.tile([5e-18, -1e-18, 1e-30], 4000)  # the sines' sum starts at zero and stays below 2^-45
+
+
+@pytest.mark.parametrize("phases", [NEAR_TIES, np.full(1000, 1e-18), TINY], ids=["near ties", "1e-18", "tiny"])
 def test_summary(phases):
     import spsslangevinintegration_amd as spss
     n = phases.size

@@ -45,9 +45,10 @@ extern "C" float map_sum(const float *c, long n, int L, float s, long *by_map) {
     }
   }
   const auto pass = [&](const std::vector<SeqMap> &maps, long r) {
-    const int k = seq_slot(s);
-    if (s == 0.f || k < 0) return false;
+    const int k = seq_lookup(s);
+    if (k < 0) return false;
     const SeqMap &m = maps[r * 64 + k];
+    if (s == 0.f) return seq_zeros(m.reach);
     const int S = seq_units(s), p = S & 1;
     if (!seq_stays(S, m.lo[p], m.hi[p], m.reach)) return false;
     s = seq_value(S + m.inc[p], s);
@@ -132,3 +133,17 @@ def test_sums_across_binades(lib, seed):
     c[rng.random(n) < 0.01] *= np.float32(2.0 ** -140)  # subnormals among them
     a, b, _ = sums(lib, c)
     assert a == b
+
+
+@pytest.mark.parametrize("term", [1e-18, -1e-18, 2.0 ** -57, 2.0 ** -58, 1e-30, 1e-42])
+def test_tiny_terms_at_a_zero_sum(lib, term):
+    for n in (1, 256, 1000, 5000):
+        for c in (np.full(n, term), np.concatenate([np.zeros(4096), np.full(n, term)]),
+                  np.tile([0.0, term, -term], n)):
+            a, b, _ = sums(lib, c)
+            assert a == b, (n, a, b)
+
+
+def test_zeros_pass_by_map(lib):
+    a, b, by_map = sums(lib, np.concatenate([np.zeros(4096), -np.zeros(4096), [1.0]]))
+    assert a == b == 1.0 and by_map >= 8192
