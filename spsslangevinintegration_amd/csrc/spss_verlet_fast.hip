@@ -1409,6 +1409,11 @@ int vf_lists(VerletFast *v, hipStream_t st, const DevParams &P, std::vector<int>
   counts->assign(n, 0);
   flat->clear();
   if (!v->resident) return SPSS_OK;
+  int force = 0;
+  VCHK(hipMemcpyAsync(&force, reinterpret_cast<char *>(v->ctl) + offsetof(VCtl, force), sizeof(int),
+                      hipMemcpyDeviceToHost, st));
+  VCHK(hipStreamSynchronize(st));
+  if (force) return SPSS_OK;  // no rebuild since entry: the arrays of the last one are another state's, or unwritten
   if (v->tiled) {  // the tiles' steps need no lists
     const unsigned nb = vblocks(n);
     if (v->s == 4)

@@ -45,7 +45,7 @@ void vf_drop(VerletFast *v);
 // the fixed list width (waits for the stream)
 int vf_status(VerletFast *v, hipStream_t st, int *should_update, double *acc, long *overflow);
 // the lists of the last rebuild in original particle ids: counts[n] by id, then each id's
-// neighbours in list order (stencil order of the build) into flat
+// neighbours in list order (stencil order of the build) into flat; empty before the first rebuild
 int vf_lists(VerletFast *v, hipStream_t st, const DevParams &P, std::vector<int> *counts, std::vector<int> *flat);
 int vf_list_width(const VerletFast *v);
 
