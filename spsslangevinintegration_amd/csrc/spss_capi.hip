@@ -1171,7 +1171,7 @@ int spss_calculate_max_displacement(spss_system *h, const double *tot) {
 int spss_verlet_status(spss_system *h, int *should_update, double *acc, int *uses) {
   if (!h) return fail(SPSS_ERR_INVALID, "NULL handle");
   if (h->vfast && h->resident_kind == 2) {  // FP32C Verlet lists: the flag lives on the device
-    int rc = vf_status(h->vfast, h->stream, should_update, acc, nullptr);
+    int rc = vf_status(h->vfast, h->stream, should_update, acc);
     if (rc != SPSS_OK) return fail(rc, vf_last_error());
     if (uses) *uses = 1;
     return SPSS_OK;

@@ -69,7 +69,6 @@ struct VCtl {
   int flag;                     // rebuild before this step (should_update_lists_), set by vr_keys
   int force;                    // the resident copy was just entered: rebuild
   double acc[2];                // accumulated_displacement_, by the parity of the step that reads it
-  unsigned long long overflow;  // lists longer than the width K since entry (walked through their cells)
   unsigned long long step;      // Philox step of graph-replayed steps
   int big_tiles;                // tiles of the last rebuild holding more particles than a workgroup
   int pad;
@@ -311,7 +310,6 @@ __device__ __forceinline__ void list_of_slot(const DevParams &P, const VArgs &A,
   }
   // a list longer than the width is not stored: the step walks that particle's 3 x 3 cells instead
   len[q] = w <= A.K ? w : -1;
-  if (w > A.K) atomicAdd(&A.ctl->overflow, 1ull);
 }
 
 template <int S>
@@ -919,7 +917,6 @@ __global__ void vc_enter(VCtl *c) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     c->flag = c->force = 1;  // should_update_lists_ starts true (ParticleSystemFirstOrderPtr.cpp:99)
     c->acc[0] = c->acc[1] = 0.0;
-    c->overflow = 0ull;
   }
   for (int g = threadIdx.x; g < kGroups; g += blockDim.x) c->gmax[g * kLineU64] = 0ull;
 }
@@ -1127,8 +1124,8 @@ bool vf_graph_ready(const VerletFast *v, const double *nat, int srk) {
 // Entry into the resident copy.  The list width K is sized here from the state entered: the
 // densest 3 x 3 block of cells holds bmax candidates, i.e. a local density of bmax / (9 Hv^2), so a
 // list holds about lam = bmax pi r_max^2 / (9 Hv^2); K = 1.5 lam + 6 sqrt(lam) + 32 (at most bmax
-// + 16) leaves room for the density to grow.  A list that outgrows K later is counted
-// (vf_status); entering again from a fresh state sizes K anew.
+// + 16) leaves room for the density to grow.  A list that outgrows K later is not stored
+// (vf_lists reports it); entering again from a fresh state sizes K anew.
 int vf_enter(VerletFast *v, hipStream_t st, const DevParams &P, int srk, const double *state, const double *nat) {
   (void)srk;
   const unsigned nb = vblocks(v->n);
@@ -1381,7 +1378,7 @@ int vf_sync(VerletFast *v, hipStream_t st, double *state) {
   return SPSS_OK;
 }
 
-int vf_status(VerletFast *v, hipStream_t st, int *should_update, double *acc, long *overflow) {
+int vf_status(VerletFast *v, hipStream_t st, int *should_update, double *acc) {
   VCtl c{};
   if (v->resident) {
     VCHK(hipMemcpyAsync(&c, v->ctl, sizeof(VCtl), hipMemcpyDeviceToHost, st));
@@ -1400,7 +1397,6 @@ int vf_status(VerletFast *v, hipStream_t st, int *should_update, double *acc, lo
   const int flag = c.force || a + stepd > v->A.half_skin;
   if (should_update) *should_update = flag;
   if (acc) *acc = flag ? 0.0 : a;
-  if (overflow) *overflow = (long)c.overflow;
   return SPSS_OK;
 }
 

@@ -41,9 +41,8 @@ bool vf_is_resident(const VerletFast *v);
 int vf_sync(VerletFast *v, hipStream_t st, double *state);
 // forgets the resident copy (the next step re-enters and rebuilds)
 void vf_drop(VerletFast *v);
-// the device's rebuild flag and accumulated displacement, and the number of lists that overflowed
-// the fixed list width (waits for the stream)
-int vf_status(VerletFast *v, hipStream_t st, int *should_update, double *acc, long *overflow);
+// the device's rebuild flag and accumulated displacement (waits for the stream)
+int vf_status(VerletFast *v, hipStream_t st, int *should_update, double *acc);
 // the lists of the last rebuild in original particle ids: counts[n] by id, then each id's
 // neighbours in list order (stencil order of the build) into flat; empty before the first rebuild
 int vf_lists(VerletFast *v, hipStream_t st, const DevParams &P, std::vector<int> *counts, std::vector<int> *flat);
