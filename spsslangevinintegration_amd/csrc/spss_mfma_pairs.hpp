@@ -8,14 +8,17 @@
 // sign over a byte: -1 within, 0 beyond); the few pairs that rounding could decide are decided one
 // by one.
 //
-// The phasors are staged as 32-bit fixed-point numbers, their four signed bytes in planes, the
-// omega-weighted ones as 46-bit numbers on the scale of the tile's largest |omega|.  The sums over the
-// neighbours are then products of 0/-1 bytes and digit bytes, sixteen particles by sixteen planes by 64
-// candidates in a v_mfma_i32_16x16x64_i8: whole numbers, exact in any order and grouping.  An FP32
-// phasor is a 2^-30 multiple from 2^-6 on, so these sums are closer to the exact ones than FP32 partial
-// sums are.
+// The phasors are staged as 38-bit fixed-point numbers, their five signed bytes in planes, cosines and sines
+// each on the scale of the tile's largest; the omega-weighted ones as 46-bit numbers on the scale of the
+// tile's largest |omega| beside.  The sums over the neighbours are then products of 0/-1 bytes and digit bytes,
+// sixteen particles by sixteen planes by 64 candidates in a v_mfma_i32_16x16x64_i8: whole numbers, exact in
+// any order and grouping.  An FP32 phasor is kept whole from 2^-13 of the scale on, and beside one of 2^-9
+// in range what smaller ones lose (2^-38) is below that one's own rounding to FP32 (2^-34): these sums
+// are closer to the exact ones than FP32 partial sums are.  Marks tell whether there is one in range; where
+// there is none (beside a particle far off its neighbours in the same tile) the caller takes the sums
+// itself.
 //
-// Bound: the vector units, 42 operations per 1,024 pairs where a walk over candidates takes 180, and
+// Bound: the vector units, 46 operations per 1,024 pairs where a walk over candidates takes 180, and
 // what comes before and after.  Cycles of a SIMD per 1,024 pairs, measured alone: this product 71 (by
 // v_mfma_f32_16x16x4_f32 139, and nothing else issues meanwhile), signs to bytes and the band's minimum
 // 85 (by v_cvt_pk_u8_f32, which takes eight cycles, 180), the digit products 34; the loop 244.
@@ -32,24 +35,27 @@ typedef float mfloat4 __attribute__((ext_vector_type(4)));
 typedef _Float16 mhalf2 __attribute__((ext_vector_type(2)));
 typedef _Float16 mhalf4 __attribute__((ext_vector_type(4)));
 
-constexpr int kMStage = 1088;         // staged entries: particles, and padding to whole units of 16 per row
-constexpr int kMPlane = kMStage + 16; // and one unit out of every range; digit planes 20 banks apart
-constexpr int kMUnits = 84;           // units of one group's candidates, and sixteen out of every range
+constexpr int kMStage = 1040;         // staged entries: particles, and padding to whole units of 16 per row (what
+                                      // leaves four workgroups to a CU; three: 16 of 115 us at 1M particles)
+constexpr int kMPlane = kMStage + 16; // and one unit out of every range
+constexpr int kMDigits = kMPlane / 4 + 4;  // words of a digit plane: sixteen planes, 12 banks apart, in 64 banks
+constexpr int kMUnits = kMStage / 16 + 16; // units of one group's candidates, and sixteen out of every range
 constexpr float kMUnit = 1024.f;      // positions: cells to |x| < 25 in halves, their second halves not denormal
 constexpr float kMSquare = 0x1p-14f;  // squares in halves
 constexpr float kMFar = 3e4f;         // "|x|^2" of padding at x = 0, in squares: beyond every range
 
-// W: words of digits per entry: 2 (cos, sin) or 5 (and the first digits of omega cos, omega sin; their
-// last two in one word)
+// W: words of digits per entry: the first four digits of cos and of sin, the last one of both with the marks;
+// the first digits of omega cos and omega sin, their last two in one word
+constexpr int kMPlain = 3, kMOmega = 6;
 template <int W>
 struct MStage {
   // entry 4c + j: x1 x2 y1 y2 at pos[j >> 1][2c + (j & 1)]; the squares' halves of entries 4c, 4c + 2, 4c + 1,
   // 4c + 3 at sq[4c ..]
   alignas(16) uint2 pos[2][kMPlane / 2];
   unsigned sq[kMPlane];
-  unsigned limb[4 * W][kMPlane / 4];
+  unsigned limb[4 * W][kMDigits];
   unsigned ones[4];
-  unsigned short units[4][4][kMUnits];     // per wave and group: first entries of its units
+  unsigned char units[4][4][kMUnits];      // per wave and group: its units
 };
 
 __device__ __forceinline__ unsigned m_pack(_Float16 lo, _Float16 hi) {
@@ -88,56 +94,75 @@ __device__ __forceinline__ unsigned quad_transpose(unsigned w, unsigned s1, unsi
   return __builtin_amdgcn_perm((unsigned)__builtin_amdgcn_mov_dpp((int)t, 0x4e, 0xf, 0xf, true), t, s2);
 }
 
-__device__ __forceinline__ int m_fixed30(float c) { return (int)__builtin_rintf(c * 0x1p30f); }
-// omega c = (hi + 2^-15 lo) 2^(e - 30) with the largest |omega| < 2^e; om: omega 2^(30 - e)
-__device__ __forceinline__ int m_fixed45(float om, float c, int &lo) {
-  const float v = om * c, h = __builtin_rintf(v);
-  lo = (int)__builtin_rintf((v - h) * 0x1p15f);
+// a component's scale: its values in the tile times 2^up are below 2^30
+struct MScale {
+  int up;
+  float mark;  // values from there on are marked
+};
+// most: the tile's largest value (< 2^100)
+__device__ __forceinline__ MScale m_scale(float most, float mark) {
+  const bool none = !(most > 0x1p-90f);  // such values may as well be zeros: they lose 2^-127 at most
+  return {none ? 119 : 29 - ilogbf(most), none ? 0.f : mark};
+}
+constexpr float kMMark = 0x1p21f;
+
+// v = hi + 2^-LOW lo for |v| <= 2^30
+template <int LOW>
+__device__ __forceinline__ int m_fixed(float v, int &lo) {
+  const float h = __builtin_rintf(v);
+  lo = (int)__builtin_rintf((v - h) * (float)(1 << LOW));
   return (int)h;
 }
+__device__ __forceinline__ bool m_marked(float v, MScale k) { return __builtin_fabsf(v) >= k.mark; }
 // signed digits of a 32-bit number, and of a smaller one's two
 __device__ __forceinline__ unsigned m_digits(int q) { return ((unsigned)q + 0x80808080u) ^ 0x80808080u; }
 __device__ __forceinline__ unsigned m_digits16(int q) { return (((unsigned)q + 0x8080u) ^ 0x8080u) & 0xffffu; }
 
 // entry e of the stage (not valid: padding, its values zero); the lanes of a quad have consecutive entries
-// of one unit and come here together; x, y in cells / kMUnit; om: omega 2^(30 - e)
+// of one unit and come here together; x, y in cells / kMUnit; c, s, om: scaled
 template <int W>
 __device__ __forceinline__ void m_write(MStage<W> &L, int e, bool valid, float x, float y, float c, float s,
-                                        float om) {
+                                        float om, MScale kc, MScale ks) {
   const int lane = threadIdx.x & 63;
   const unsigned s1 = lane & 1 ? 0x03070105u : 0x06020400u, s2 = lane & 2 ? 0x03020706u : 0x05040100u;
   const uint2 xy = make_uint2(m_halves(x), m_halves(y));
   const float xr = m_value(xy.x), yr = m_value(xy.y);
   m_place(L, e, xy, valid ? kMSquare * __builtin_fmaf(xr, xr, yr * yr) : kMFar);
   unsigned *const d = L.limb[lane & 3] + (e >> 2);
-  constexpr int kNext = 4 * (kMPlane / 4);  // the same digit of the next word
-  d[0] = quad_transpose(m_digits(m_fixed30(c)), s1, s2);
-  d[kNext] = quad_transpose(m_digits(m_fixed30(s)), s1, s2);
-  if (W == 5) {
-    int lc, ls;
-    const int hc = m_fixed45(om, c, lc), hs = m_fixed45(om, s, ls);
-    d[2 * kNext] = quad_transpose(m_digits(hc), s1, s2);
-    d[3 * kNext] = quad_transpose(m_digits(hs), s1, s2);
-    d[4 * kNext] = quad_transpose(m_digits16(lc) | m_digits16(ls) << 16, s1, s2);
+  constexpr int kNext = 4 * kMDigits;  // the same digit of the next word
+  int lc, ls;
+  const int hc = m_fixed<7>(c, lc), hs = m_fixed<7>(s, ls);
+  const unsigned marks = (m_marked(c, kc) ? 1u : 0u) | (m_marked(s, ks) ? 2u : 0u);
+  d[0] = quad_transpose(m_digits(hc), s1, s2);
+  d[kNext] = quad_transpose(m_digits(hs), s1, s2);
+  d[2 * kNext] = quad_transpose((lc & 0xff) | (ls & 0xff) << 8 | marks << 16, s1, s2);
+  if (W == kMOmega) {
+    const int hx = m_fixed<15>(om * (c * 0x1p-30f), lc), hy = m_fixed<15>(om * (s * 0x1p-30f), ls);
+    d[3 * kNext] = quad_transpose(m_digits(hx), s1, s2);
+    d[4 * kNext] = quad_transpose(m_digits(hy), s1, s2);
+    d[5 * kNext] = quad_transpose(m_digits16(lc) | m_digits16(ls) << 16, s1, s2);
   }
 }
 
 struct MSums {
   double sx = 0.0, sy = 0.0, tx = 0.0, ty = 0.0;  // without the particle itself
-  int n = 0;
+  int n = 0;                                      // kMOpen: nothing marked in range
 };
+constexpr int kMOpen = -1;
 
 // The sums of the wave's `count` particles (one per lane, entries first .. first + count - 1 of the stage
 // in cell order); r2: the squared radius in staged units, band: what rounding may move a squared
 // distance by; range(lane, r, a, b): the entries [a, b) of row r of the stencils of particles [lane,
 // lane + 16); in(lane, e): the exact range test of particle `lane` and entry e.  c, s, om: the lane's own
-// phasor and omega 2^(30 - scale), which its sums are rid of.
+// phasor and omega, scaled, which its sums are rid of.  (Its own mark counts too: with the other component
+// its value weighs by that much in what is made of the sums.)
 template <int W, class RANGE, class IN>
 __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int nrows, float r2, float band, float c,
-                                        float s, float om, int scale, RANGE range, IN in) {
+                                        float s, float om, MScale kc, MScale ks, MScale ko, RANGE range, IN in) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15, g = lane >> 4;
   MSums out;
-  int sx[2] = {0, 0}, sy[2] = {0, 0}, tx[2] = {0, 0}, ty[2] = {0, 0}, lx = 0, ly = 0;
+  int sx[2] = {0, 0}, sy[2] = {0, 0}, kx = 0, ky = 0, tx[2] = {0, 0}, ty[2] = {0, 0}, lx = 0, ly = 0;
+  unsigned marked = 0;
   // the units of each group's candidates, four groups at once, one row per lane
   int total = 0;
   {
@@ -150,10 +175,10 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
       const int t = __shfl_up(total, o, 16);
       if (i >= o) total += t;
     }
-    unsigned short *list = L.units[wave][g];
-    for (int t = 0; t < m; ++t) list[total - m + t] = (unsigned short)(16 * (u0 + t));
+    unsigned char *list = L.units[wave][g];
+    for (int t = 0; t < m; ++t) list[total - m + t] = (unsigned char)(u0 + t);
     total = __shfl(total, 15, 16);
-    list[total + i] = (unsigned short)kMStage;  // the last pass's rest, and what is read ahead
+    list[total + i] = (unsigned char)(kMStage / 16);  // the last pass's rest, and what is read ahead
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
@@ -162,9 +187,11 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
   const char *fb = (g < 2 ? reinterpret_cast<const char *>(L.pos[0]) : reinterpret_cast<const char *>(L.sq)) + 16 * (i & 3);
   constexpr int kSecond = sizeof(L.pos[0]);
   const int second = g < 2 ? kSecond : 0;
-  const char *l1 = i < 8 ? reinterpret_cast<const char *>(L.limb[i]) : reinterpret_cast<const char *>(L.ones);
-  const int m1 = i < 8 ? -1 : 0;
-  const char *l2 = reinterpret_cast<const char *>(L.limb[W == 5 && i < 12 ? 8 + i : 0]);
+  // the planes: the phasors' ten digits, and ones; the weighted ones' twelve; the marks
+  const char *l1 = i < 10 ? reinterpret_cast<const char *>(L.limb[i]) : reinterpret_cast<const char *>(L.ones);
+  const int m1 = i < 10 ? -1 : 0;
+  const char *l2 = reinterpret_cast<const char *>(L.limb[W == kMOmega && i < 12 ? 12 + i : 0]);
+  const char *lm = reinterpret_cast<const char *>(L.limb[10]);
   for (int gr = 0; 16 * gr < count; ++gr) {
     const bool real = 16 * gr + i < count;
     const uint2 own = m_pos(L, real ? first + 16 * gr + i : kMStage);
@@ -182,7 +209,7 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
     const mhalf2 b2 = g < 2 ? hx : none, b3 = g < 2 ? hy : (g == 2 ? sq : none);
     const mhalf4 v0 = {b0[0], b0[1], b1[0], b1[1]}, v1 = {b2[0], b2[1], b3[0], b3[1]};
     mint4 s1 = {0, 0, 0, 0}, s2 = {0, 0, 0, 0};
-    const unsigned short *uf = L.units[wave][gr] + (i >> 2), *ul = L.units[wave][gr] + g;
+    const unsigned char *uf = L.units[wave][gr] + (i >> 2), *ul = L.units[wave][gr] + g;
     const int n = __builtin_amdgcn_readlane(total, 16 * gr);
     struct Entries {
       mint4 a, b;
@@ -204,13 +231,15 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
       return r;  // t[q][r]: entry 4r + q of the lane's unit
     };
     const auto bits = [](float t) { return __builtin_bit_cast(unsigned, t); };
-    int el = ul[0], ef = uf[0];
+    mint4 any = {0, 0, 0, 0};  // marks in range
+    int el = 16 * ul[0], ef = 16 * uf[0];
     for (int u = 0; u < n; u += 4) {
       const Products c = products(features(ef));
       const mint4 d1 = *reinterpret_cast<const mint4 *>(l1 + (el & m1));
+      const mint4 dm = *reinterpret_cast<const mint4 *>(lm + el);
       const int el0 = el;
-      el = ul[u + 4];
-      ef = uf[u + 4];
+      el = 16 * ul[u + 4];
+      ef = 16 * uf[u + 4];
       mint4 w;
       float least = __builtin_fabsf(c.t[0][0]);
 #pragma unroll
@@ -235,18 +264,24 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
         }
       }
       s1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(d1, w, s1, 0, 0, 0);
-      if (W == 5) s2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(*reinterpret_cast<const mint4 *>(l2 + el0), w, s2, 0, 0, 0);
+      any |= w & dm;
+      if (W == kMOmega) s2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(*reinterpret_cast<const mint4 *>(l2 + el0), w, s2, 0, 0, 0);
     }
-    // lanes i and 16 + i hold the digits of the cosines' and the sines' sums, lane 32 + i the count and the
-    // last digits; lane 16 gr + i takes them, in pairs
+    // lanes i and 16 + i hold the first digits of the cosines' and the sines' sums, lane 32 + i the last ones and
+    // the count; lane 16 gr + i takes them, in pairs
     const int p0 = s1[0] + (s1[1] << 8), p1 = s1[2] + (s1[3] << 8);
     const int x0 = __shfl(p0, i), x1 = __shfl(p1, i), y0 = __shfl(p0, 16 + i), y1 = __shfl(p1, 16 + i);
-    const int cn = __shfl(s1[0], 32 + i);
+    const int z0 = __shfl(s1[0], 32 + i), z1 = __shfl(s1[1], 32 + i), cn = __shfl(s1[2], 32 + i);
+    unsigned seen = (unsigned)(any[0] | any[1] | any[2] | any[3]);
+    seen |= __shfl_xor(seen, 16);
+    seen |= __shfl_xor(seen, 32);
     if (g == gr) {
-      sx[0] = x0, sx[1] = x1, sy[0] = y0, sy[1] = y1;
+      sx[0] = x0, sx[1] = x1, sy[0] = y0, sy[1] = y1, kx = z0, ky = z1;
       out.n = -cn;
+      marked = seen | seen >> 16;
+      marked |= marked >> 8;
     }
-    if (W == 5) {
+    if (W == kMOmega) {
       const int q0 = s2[0] + (s2[1] << 8), q1 = s2[2] + (s2[3] << 8);
       const int u0 = __shfl(q0, i), u1 = __shfl(q1, i), v0 = __shfl(q0, 16 + i), v1 = __shfl(q1, 16 + i);
       const int a = __shfl(q0, 32 + i), b = __shfl(q1, 32 + i);
@@ -258,13 +293,18 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
     }
   }
   const auto whole = [](const int *q) { return fma((double)q[1], 65536.0, (double)q[0]); };
-  out.sx = -(whole(sx) + (double)m_fixed30(c)) * 0x1p-30;
-  out.sy = -(whole(sy) + (double)m_fixed30(s)) * 0x1p-30;
-  if (W == 5) {
-    int lc, ls;
-    const int hc = m_fixed45(om, c, lc), hs = m_fixed45(om, s, ls);
-    out.tx = ldexp(-(whole(tx) + (double)hc + 0x1p-15 * (double)(lx + lc)), scale - 30);
-    out.ty = ldexp(-(whole(ty) + (double)hs + 0x1p-15 * (double)(ly + ls)), scale - 30);
+  int lc, ls;
+  const int hc = m_fixed<7>(c, lc), hs = m_fixed<7>(s, ls);
+  out.sx = ldexp(-(whole(sx) + (double)hc + 0x1p-7 * (double)(kx + lc)), -kc.up);
+  out.sy = ldexp(-(whole(sy) + (double)hs + 0x1p-7 * (double)(ky + ls)), -ks.up);
+  if (W == kMOmega) {
+    const int hx = m_fixed<15>(om * (c * 0x1p-30f), lc), hy = m_fixed<15>(om * (s * 0x1p-30f), ls);
+    out.tx = ldexp(-(whole(tx) + (double)hx + 0x1p-15 * (double)(lx + lc)), 30 - ko.up - kc.up);
+    out.ty = ldexp(-(whole(ty) + (double)hy + 0x1p-15 * (double)(ly + ls)), 30 - ko.up - ks.up);
+  }
+  if (out.n > 1 && (marked & 3) != 3) {
+    out.n = kMOpen;
+    return out;
   }
   --out.n;
   return out;

@@ -24,17 +24,19 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 // greedy spans of whole cells, each as wide as possible with at most kTileCap particles and at
 // most wcap (<= 64) columns, span i in slot i of the row's cmax slots, empty spans in the unused
 // slots.  Full spans keep the workgroup's waves full where fixed-width
-// tiles leave the last wave of most tiles part-empty.  With cmax * wcap >= ncx every span stays
+// tiles leave the last wave of most tiles part-empty.  more(a, e): whether a span [a, e) of more than one
+// column may be (true for a leading run of e).  With cmax * wcap >= ncx every span stays
 // within wcap columns: a span is widened past the particle bound (a dense row) only as far as
 // the remaining slots need to cover the rest of the row.
+template <class MORE>
 __device__ __forceinline__ void row_tiles(const int *P, int cbase, int row, int ncx, int wcap, int cmax,
-                                          int4 *__restrict__ slots) {
+                                          int4 *__restrict__ slots, MORE more) {
   const int lane = threadIdx.x & 63;
   int a = 0, i = 0;
   while (a < ncx) {  // invariant: ncx - a <= (cmax - i) * wcap
     const int e = a + 1 + lane;
     // true for a leading run of lanes: P is non-decreasing
-    const bool fits = lane < wcap && e <= ncx && P[e] - P[a] <= kTileCap;
+    const bool fits = lane < wcap && e <= ncx && P[e] - P[a] <= kTileCap && more(a, e);
     const int b = max(a + max(__popcll(__ballot(fits)), 1), ncx - (cmax - i - 1) * wcap);
     if (lane == 0) slots[i] = make_int4(cbase, row, a, b);
     a = b;
@@ -55,13 +57,8 @@ __device__ __forceinline__ void rows_to_tiles(START start, int ncx, int ncy, int
   if (row < ncy)
     for (int c = lane; c <= ncx; c += 64) P[w][c] = start(row * ncx + c);
   __syncthreads();
-  if (row < ncy) row_tiles(P[w], 0, row, ncx, wcap, cmax, tiles + (long)row * cmax);
-}
-
-// square grids (ncf x ncf)
-template <class START>
-__device__ __forceinline__ void rows_to_tiles(START start, int ncf, int wcap, int cmax, int4 *__restrict__ tiles) {
-  rows_to_tiles(start, ncf, ncf, wcap, cmax, tiles);
+  if (row < ncy)
+    row_tiles(P[w], 0, row, ncx, wcap, cmax, tiles + (long)row * cmax, [](int, int) { return true; });
 }
 
 }  // namespace spss

@@ -231,6 +231,34 @@ __global__ __launch_bounds__(kVB) void vr_scatter(VArgs A, const int *__restrict
   }
 }
 
+// The row tiles of rows [4 * blockIdx.x, 4 * blockIdx.x + 4), a wave each.  A tile is no wider than its staged
+// cells fit the stage, where those of a single column do: at 24 particles a cell one tile of a hundred would not
+// by its particles alone, and a few tiles that walk lists hold up every step (1M particles: 8 us).
+__device__ __forceinline__ void vt_tiles(const int *__restrict__ start, int nc, int wcap, int cmax,
+                                         int4 *__restrict__ tiles) {
+  __shared__ int R[6][kRowTileCols + 1];  // starts of the rows, and of those around them
+  const int row0 = blockIdx.x * 4;
+  for (int e = threadIdx.x; e < 6 * (nc + 1); e += kVB) {
+    const int r = e / (nc + 1), row = row0 + r - 1;
+    if (row <= nc) R[r][e - r * (nc + 1)] = start[wrap_row(row, nc) * nc + e - r * (nc + 1)];
+  }
+  __syncthreads();
+  const int w = threadIdx.x >> 6, row = row0 + w;
+  if (row >= nc) return;
+  const auto fits = [&](int a, int e) {
+    int total = 0;
+    for (int r = w; r < w + 3; ++r) {
+      int v = R[r][min(e + 1, nc)] - R[r][max(a - 1, 0)];
+      if (a == 0) v += R[r][nc] - R[r][nc - 1];
+      if (e == nc) v += R[r][1] - R[r][0];
+      total += (v + 15) & ~15;
+    }
+    return total <= kMStage;
+  };
+  row_tiles(R[w + 1], 0, row, nc, wcap, cmax, tiles + (long)row * cmax,
+            [&](int a, int e) { return fits(a, e) || !fits(a, a + 1); });
+}
+
 // each cell's particles in ascending previous slot, gathered into the new order in scratch: cells
 // of at most 64 particles one wave each (wave_sort64), then the particles of denser cells one
 // thread each, ranked by counting (grid-stride over the particles: a dense cluster is spread over
@@ -245,7 +273,7 @@ __global__ __launch_bounds__(kVB) void vr_gather(VArgs A, const int *__restrict_
   if (gate_off(A)) return;
   // the row tiles of the new order (tiled grids), one wave per row in the first workgroups: they
   // need only the final cell starts
-  if (tiles && (int)blockIdx.x * 4 < A.ncv) rows_to_tiles([&](int c) { return start[c]; }, A.ncv, wcap, cmax, tiles);
+  if (tiles && (int)blockIdx.x * 4 < A.ncv) vt_tiles(start, A.ncv, wcap, cmax, tiles);
   const int lane = threadIdx.x & 63;
   auto move = [&](int p, int q, int c) {
 #pragma unroll
@@ -557,10 +585,9 @@ __global__ __launch_bounds__(kVB) void vs_step(DevParams P, VArgs A, StepArgs U,
 constexpr int kVCols = 48;  // staged columns W + 2
 
 struct VtPlan {
-  int cglob[3 * kVCols];  // first slot of staged cell (r, q), at r * (W + 2) + q
-  int ccnt[3 * kVCols];   // its particle count
-  int cpos[3 * kVCols];   // its start in staged row r
-  int len[3];             // particles of the staged rows
+  int cglob[3 * kVCols];                  // first slot of staged cell (r, q), at r * (W + 2) + q
+  unsigned short cpos[3 * (kVCols + 1)];  // its start in staged row r, at r * (W + 3) + q, and behind it the row's end
+  int len[3];                             // particles of the staged rows (cpos: meant for rows that fit the stage)
 };
 
 // the staging plan of tile (row, ca, cb): rows row-1 .. row+1, columns ca-1 .. cb (each wrapped
@@ -576,12 +603,8 @@ __device__ __forceinline__ int vt_plan(const VArgs &A, const int *__restrict__ s
       v = start[c + 1] - g0;
     }
     const int incl = wave_incl_scan(v, lane);
-    if (lane < ncols) {
-      const int e = w * ncols + lane;
-      L.cglob[e] = g0;
-      L.ccnt[e] = v;
-      L.cpos[e] = incl - v;
-    }
+    if (lane < ncols) L.cglob[w * ncols + lane] = g0;
+    if (lane <= ncols) L.cpos[w * (ncols + 1) + lane] = (unsigned short)(incl - v);
     if (lane == 63) L.len[w] = incl;
   }
   __syncthreads();
@@ -633,8 +656,8 @@ template <int W>
 struct VtLds {
   MStage<W> M;
   VtPlan plan;
-  unsigned short col[kVB];  // staged column of the tile's particles
-  float most[kVB / 64];
+  unsigned char col[kVB];  // staged column of the tile's particles
+  float most[kVB / 64][3];  // of the waves' staged values
   double wmax[kVB / 64];
 };
 
@@ -668,7 +691,7 @@ __device__ __forceinline__ bool vt_sums(const DevParams &P, const VArgs &A, int 
   const int f2 = wrap_row(row + 1, A.ncv) * A.ncv + ca - 1;
   const int c0 = (l0 + 63) >> 6, c1 = c0 + ((l1 + 63) >> 6), c2 = c1 + ((l2 + 63) >> 6);
   float4 v[kPasses];
-  float om[kPasses], most = 0.f;
+  float om[kPasses], most[3] = {0.f, 0.f, 0.f};  // the largest |omega|, |cos phi|, |sin phi|; infinite: not all are finite
   int at[kPasses], to[kPasses];  // first entry of the wave's chunk; entries of its row from there
 #pragma unroll
   for (int p = 0; p < kPasses; ++p) {
@@ -683,51 +706,60 @@ __device__ __forceinline__ bool vt_sums(const DevParams &P, const VArgs &A, int 
       int g = (r == 0 ? s0 : (r == 1 ? s1 : s2)) + t;
       int q;  // staged column
       if (lw || rw) {
-        const int e = r * ncols;
+        const int e = r * (ncols + 1);
         const bool left = lw && t < L.cpos[e + 1], right = rw && t >= L.cpos[e + ncols - 1];
-        const int c = left ? e : (right ? e + ncols - 1 : e + (lw ? 1 : 0));
-        g = L.cglob[c] + (t - L.cpos[c]);
+        const int c = left ? 0 : (right ? ncols - 1 : (lw ? 1 : 0));
+        g = L.cglob[r * ncols + c] + (t - L.cpos[e + c]);
         q = left ? 0 : (right ? ncols - 1 : cell[g] - (r == 0 ? f0 : (r == 1 ? f1 : f2)));
       } else {
         q = cell[g] - (r == 0 ? f0 : (r == 1 ? f1 : f2));
       }
       v[p] = snap[g];
-      if (W == 5) om[p] = omega[g];
+      if (W == kMOmega) om[p] = omega[g];
       v[p].x = __builtin_fmaf(v[p].x, unit, kMUnit * ((float)q - 0.5f * (float)(cb - ca + 1)));
       v[p].y = __builtin_fmaf(v[p].y, unit, kMUnit * (float)(r - 1));
       const float big = __builtin_fabsf(v[p].x) + __builtin_fabsf(v[p].y) + __builtin_fabsf(v[p].z) +
                         __builtin_fabsf(v[p].w) + __builtin_fabsf(om[p]);
-      most = __builtin_fmaxf(most, big < 0x1p100f ? __builtin_fabsf(om[p]) : __builtin_inff());
+      most[0] = __builtin_fmaxf(most[0], big < 0x1p100f ? __builtin_fabsf(om[p]) : __builtin_inff());
+      most[1] = __builtin_fmaxf(most[1], __builtin_fabsf(v[p].z));
+      most[2] = __builtin_fmaxf(most[2], __builtin_fabsf(v[p].w));
     }
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) most = __builtin_fmaxf(most, __shfl_xor(most, o, 64));
-  if (lane == 0) Ls.most[wave] = most;
-  if ((int)threadIdx.x < ntile) Ls.col[threadIdx.x] = (unsigned short)(cell[gtb + threadIdx.x] - row * A.ncv - ca + 1);
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) most[k] = __builtin_fmaxf(most[k], __shfl_xor(most[k], o, 64));
+  if (lane == 0)
+#pragma unroll
+    for (int k = 0; k < 3; ++k) Ls.most[wave][k] = most[k];
+  if ((int)threadIdx.x < ntile) Ls.col[threadIdx.x] = (unsigned char)(cell[gtb + threadIdx.x] - row * A.ncv - ca + 1);
   m_init(Ls.M);
   __syncthreads();
-  most = __builtin_fmaxf(__builtin_fmaxf(Ls.most[0], Ls.most[1]), __builtin_fmaxf(Ls.most[2], Ls.most[3]));
-  if (!(most < 0x1p100f)) return false;
-  const int scale = most > 0x1p-90f ? ilogbf(most) + 1 : -89;
-  const float s30 = ldexpf(1.f, 30 - scale);
+  MScale scale[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const float m = __builtin_fmaxf(__builtin_fmaxf(Ls.most[0][k], Ls.most[1][k]), __builtin_fmaxf(Ls.most[2][k], Ls.most[3][k]));
+    if (k == 0 && !(m < 0x1p100f)) return false;
+    scale[k] = m_scale(m, kMMark);
+  }
+  const float uo = ldexpf(1.f, scale[0].up), uc = ldexpf(1.f, scale[1].up), us = ldexpf(1.f, scale[2].up);
 #pragma unroll
   for (int p = 0; p < kPasses; ++p)
     if (lane < ((to[p] + 15) & ~15))
-      m_write<W>(Ls.M, at[p] + lane, lane < to[p], v[p].x, v[p].y, v[p].z, v[p].w, om[p] * s30);
+      m_write<W>(Ls.M, at[p] + lane, lane < to[p], v[p].x, v[p].y, v[p].z * uc, v[p].w * us, om[p] * uo, scale[1],
+                 scale[2]);
   __syncthreads();
-  const int first = b1 + L.cpos[ncols + 1] + 64 * wave, count = min(max(ntile - 64 * wave, 0), 64);
+  const int first = b1 + L.cpos[ncols + 2] + 64 * wave, count = min(max(ntile - 64 * wave, 0), 64);
   if (count == 0) return true;
   const int p = gtb + 64 * wave + lane;
   const float4 me = lane < count ? snap[p] : make_float4(0.f, 0.f, 0.f, 0.f);
-  const float mo = W == 5 && lane < count ? omega[p] : 0.f;
+  const float mo = W == kMOmega && lane < count ? omega[p] : 0.f;
   sum = m_sums<W>(
-      Ls.M, first, count, 3, r2, band, me.z, me.w, mo * s30, scale,
+      Ls.M, first, count, 3, r2, band, me.z * uc, me.w * us, mo * uo, scale[1], scale[2], scale[0],
       [&](int i, int r, int &a, int &b) {
-        const int q0 = r * ncols + Ls.col[64 * wave + i] - 1;
-        const int q1 = r * ncols + Ls.col[64 * wave + min(i + 15, count - 1)] + 1;
-        const int base = r == 0 ? 0 : (r == 1 ? b1 : b2);
-        a = base + L.cpos[q0];
-        b = base + L.cpos[q1] + L.ccnt[q1];
+        const int e = r * (ncols + 1), base = r == 0 ? 0 : (r == 1 ? b1 : b2);
+        a = base + L.cpos[e + Ls.col[64 * wave + i] - 1];
+        b = base + L.cpos[e + Ls.col[64 * wave + min(i + 15, count - 1)] + 2];
       },
       [&](int i, int e) {
         // differences of the staged positions first: their band is narrower
@@ -737,12 +769,14 @@ __device__ __forceinline__ bool vt_sums(const DevParams &P, const VArgs &A, int 
         if (__builtin_fabsf(dd) > tight) return dd < 0.f;
         // the reference's FP64 test (x_i as stored, rhs_verlet's :566-581)
         const int r = e < b1 ? 0 : (e < b2 ? 1 : 2), t = e - (r == 0 ? 0 : (r == 1 ? b1 : b2));
-        int q = r * ncols, hi = q + ncols - 1;  // the last cell that starts at or before t holds it
+        const unsigned short *cpos = L.cpos + r * (ncols + 1);
+        int q = 0, hi = ncols - 1;  // the last cell that starts at or before t holds it
         while (q < hi) {
           const int mid = (q + hi + 1) >> 1;
-          if (L.cpos[mid] <= t) q = mid; else hi = mid - 1;
+          if (cpos[mid] <= t) q = mid; else hi = mid - 1;
         }
-        const double *pi = state + (long)(gtb + 64 * wave + i) * S, *pj = state + (long)(L.cglob[q] + t - L.cpos[q]) * S;
+        const double *pi = state + (long)(gtb + 64 * wave + i) * S;
+        const double *pj = state + (long)(L.cglob[r * ncols + q] + t - cpos[q]) * S;
         double ddx, ddy;
         class_c_unsigned(P, pi[0], pi[1], pj[0], pj[1], ddx, ddy);
         return ddx * ddx + ddy * ddy <= P.rho2;
@@ -878,7 +912,7 @@ __global__ __launch_bounds__(kVB, 3) void vt_step(DevParams P, VArgs A, StepArgs
                                                const float *__restrict__ omega, double *__restrict__ nstate,
                                                float4 *__restrict__ nsnap, float *__restrict__ nomega,
                                                double *__restrict__ compl_out) {
-  constexpr int W = SRK ? 5 : 2;
+  constexpr int W = SRK ? kMOmega : kMPlain;
   __shared__ VtLds<W> Ls;
   const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
   const int4 td = tile < ntiles ? tiles[tile] : make_int4(0, 0, 0, 0);
@@ -893,8 +927,9 @@ __global__ __launch_bounds__(kVB, 3) void vt_step(DevParams P, VArgs A, StepArgs
     const bool have = staged && vt_sums<S, W>(P, A, row, ca, cb, gtb, ntile, cell, state, snap, omega, Ls, sum);
     const int u = threadIdx.x, p = gtb + u;
     if (u < ntile) {
-      // (rare) staged values that are not finite: the cells; an overflowing stage: the list
-      if (!have) sum = vt_walk<S, SRK>(P, A, list, start, cell, state, snap, omega, p, staged ? -1 : len[p]);
+      // (rare) staged values that are not finite, or small ones beside a large one out of range: the cells; an
+      // overflowing stage: the list
+      if (!have || sum.n == kMOpen) sum = vt_walk<S, SRK>(P, A, list, start, cell, state, snap, omega, p, staged ? -1 : len[p]);
       d2 = vt_particle<S, SRK>(P, A, U, vt_coef(P, U), U.step_dev ? (uint64_t)*U.step_dev : U.step, state, id, nat,
                                nstate, nsnap, nomega, compl_out, sum, p, cell[p] - row * A.ncv, row);
     }
@@ -1068,12 +1103,14 @@ int vf_create(VerletFast **out, hipStream_t st, const DevParams &P, double rho, 
   A(hipMalloc(&v->bmax, sizeof(int)));
   v->tiled = ncv <= kRowTileCols;
   if (v->tiled) {
-    // slots per row: the greedy spans of a row 1.5x the mean at about 94% of a tile each, plus 2,
-    // and at least enough spans of vt_wcap columns to cover a row
+    // slots per row: the greedy spans of a row 1.5x the mean at about 94% of a tile each (or 80% of what
+    // the mean density leaves them of the stage, vt_tiles), plus 2, and at least enough spans of vt_wcap
+    // columns to cover a row
     v->vt_wcap = kVCols - 2;
-    const double row_mean = (double)n / (double)ncv;
+    const double row_mean = (double)n / (double)ncv, cell_mean = row_mean / (double)ncv;
+    const double cols = std::max(1.0, std::floor((kMStage - 24) / (3.0 * cell_mean)) - 2.0);
     v->vt_cmax = std::max((ncv + v->vt_wcap - 1) / v->vt_wcap,
-                          std::min(ncv, (int)std::ceil(1.5 * row_mean / (0.94 * kTileCap)) + 2));
+                          (int)std::min((double)ncv, std::ceil(1.5 * row_mean / std::min(0.94 * kTileCap, 0.8 * cols * cell_mean)) + 2));
     A(hipMalloc(&v->local, sizeof(int) * (size_t)v->cells));
     A(hipMalloc(&v->vtiles, sizeof(int4) * (size_t)ncv * v->vt_cmax));
   }
