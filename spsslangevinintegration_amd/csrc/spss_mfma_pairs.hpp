@@ -14,9 +14,9 @@
 // sixteen particles by sixteen planes by 64 candidates in a v_mfma_i32_16x16x64_i8: whole numbers, exact in
 // any order and grouping.  An FP32 phasor is kept whole from 2^-13 of the scale on, and beside one of 2^-9
 // in range what smaller ones lose (2^-38) is below that one's own rounding to FP32 (2^-34): these sums
-// are closer to the exact ones than FP32 partial sums are.  Marks tell whether there is one in range; where
-// there is none (beside a particle far off its neighbours in the same tile) the caller takes the sums
-// itself.
+// are closer to the exact ones than FP32 partial sums are; so for the weighted ones beside one of 2^-18 (the
+// bulk of a Lorentzian clipped at 200 of its widths is at 2^-8).  Marks tell whether there is one in range; where there is none
+// (beside a particle far off its neighbours in the same tile) the caller takes the sums itself.
 //
 // Bound: the vector units, 46 operations per 1,024 pairs where a walk over candidates takes 180, and
 // what comes before and after.  Cycles of a SIMD per 1,024 pairs, measured alone: this product 71 (by
@@ -104,7 +104,7 @@ __device__ __forceinline__ MScale m_scale(float most, float mark) {
   const bool none = !(most > 0x1p-90f);  // such values may as well be zeros: they lose 2^-127 at most
   return {none ? 119 : 29 - ilogbf(most), none ? 0.f : mark};
 }
-constexpr float kMMark = 0x1p21f;
+constexpr float kMMark = 0x1p21f, kMMarkOmega = 0x1p12f;
 
 // v = hi + 2^-LOW lo for |v| <= 2^30
 template <int LOW>
@@ -122,7 +122,7 @@ __device__ __forceinline__ unsigned m_digits16(int q) { return (((unsigned)q + 0
 // of one unit and come here together; x, y in cells / kMUnit; c, s, om: scaled
 template <int W>
 __device__ __forceinline__ void m_write(MStage<W> &L, int e, bool valid, float x, float y, float c, float s,
-                                        float om, MScale kc, MScale ks) {
+                                        float om, MScale kc, MScale ks, MScale ko) {
   const int lane = threadIdx.x & 63;
   const unsigned s1 = lane & 1 ? 0x03070105u : 0x06020400u, s2 = lane & 2 ? 0x03020706u : 0x05040100u;
   const uint2 xy = make_uint2(m_halves(x), m_halves(y));
@@ -132,16 +132,19 @@ __device__ __forceinline__ void m_write(MStage<W> &L, int e, bool valid, float x
   constexpr int kNext = 4 * kMDigits;  // the same digit of the next word
   int lc, ls;
   const int hc = m_fixed<7>(c, lc), hs = m_fixed<7>(s, ls);
-  const unsigned marks = (m_marked(c, kc) ? 1u : 0u) | (m_marked(s, ks) ? 2u : 0u);
+  unsigned marks = (m_marked(c, kc) ? 1u : 0u) | (m_marked(s, ks) ? 2u : 0u);
   d[0] = quad_transpose(m_digits(hc), s1, s2);
   d[kNext] = quad_transpose(m_digits(hs), s1, s2);
-  d[2 * kNext] = quad_transpose((lc & 0xff) | (ls & 0xff) << 8 | marks << 16, s1, s2);
+  const unsigned low = (lc & 0xff) | (ls & 0xff) << 8;
   if (W == kMOmega) {
-    const int hx = m_fixed<15>(om * (c * 0x1p-30f), lc), hy = m_fixed<15>(om * (s * 0x1p-30f), ls);
+    const float vx = om * (c * 0x1p-30f), vy = om * (s * 0x1p-30f);
+    marks |= (m_marked(vx, ko) ? 4u : 0u) | (m_marked(vy, ko) ? 8u : 0u);
+    const int hx = m_fixed<15>(vx, lc), hy = m_fixed<15>(vy, ls);
     d[3 * kNext] = quad_transpose(m_digits(hx), s1, s2);
     d[4 * kNext] = quad_transpose(m_digits(hy), s1, s2);
     d[5 * kNext] = quad_transpose(m_digits16(lc) | m_digits16(ls) << 16, s1, s2);
   }
+  d[2 * kNext] = quad_transpose(low | marks << 16, s1, s2);
 }
 
 struct MSums {
@@ -302,7 +305,8 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
     out.tx = ldexp(-(whole(tx) + (double)hx + 0x1p-15 * (double)(lx + lc)), 30 - ko.up - kc.up);
     out.ty = ldexp(-(whole(ty) + (double)hy + 0x1p-15 * (double)(ly + ls)), 30 - ko.up - ks.up);
   }
-  if (out.n > 1 && (marked & 3) != 3) {
+  constexpr unsigned kAll = W == kMOmega ? 15u : 3u;
+  if (out.n > 1 && (marked & kAll) != kAll) {
     out.n = kMOpen;
     return out;
   }

@@ -740,14 +740,14 @@ __device__ __forceinline__ bool vt_sums(const DevParams &P, const VArgs &A, int 
   for (int k = 0; k < 3; ++k) {
     const float m = __builtin_fmaxf(__builtin_fmaxf(Ls.most[0][k], Ls.most[1][k]), __builtin_fmaxf(Ls.most[2][k], Ls.most[3][k]));
     if (k == 0 && !(m < 0x1p100f)) return false;
-    scale[k] = m_scale(m, kMMark);
+    scale[k] = m_scale(m, k == 0 ? kMMarkOmega : kMMark);
   }
   const float uo = ldexpf(1.f, scale[0].up), uc = ldexpf(1.f, scale[1].up), us = ldexpf(1.f, scale[2].up);
 #pragma unroll
   for (int p = 0; p < kPasses; ++p)
     if (lane < ((to[p] + 15) & ~15))
       m_write<W>(Ls.M, at[p] + lane, lane < to[p], v[p].x, v[p].y, v[p].z * uc, v[p].w * us, om[p] * uo, scale[1],
-                 scale[2]);
+                 scale[2], scale[0]);
   __syncthreads();
   const int first = b1 + L.cpos[ncols + 2] + 64 * wave, count = min(max(ntile - 64 * wave, 0), 64);
   if (count == 0) return true;

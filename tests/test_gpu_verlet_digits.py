@@ -1,5 +1,5 @@
-"""What the FP32C Verlet steps keep of small phasors: states synchronised near a phase at which sines or cosines
-are small, with and without a particle far off the rest in the same tile; and densities at which the stage,
+"""What the FP32C Verlet steps keep of small phasors and omegas: states synchronised near a phase at which sines or cosines
+are small, with and without a particle far off the rest in the same tile; an omega that diverges; and densities at which the stage,
 not the workgroup, bounds a tile.  Reference: the oracle's FP64 steps.
 
 Bounds: a phasor's component is rounded once to FP32 (2^-25 of itself), its sum over the neighbours is taken
@@ -62,6 +62,23 @@ def test_synchronised_phases(spss, phase, spread, stray):
     tol = SIGMA * DT * 2.0 ** -24 * (np.abs(c) * _most(xy, rho, s) + np.abs(s) * _most(xy, rho, c))
     # the oracle's own roundings: of the phases' differences, and of the sums
     tol += SIGMA * DT * 2.0 ** -50 * (phase + _most(xy, rho, phi - phase))
+    assert np.all(d <= tol), (d.max(), np.max(d / tol))
+
+
+@pytest.mark.parametrize("size", [1e5, 1e8, 1e12, 1e16, 1e25, 1e35])
+def test_an_omega_that_diverges(spss, size):
+    """the complementary force's terms err by three roundings of 2^-24 of (|omega_j| + |omega_i|) at most, of those
+    in range alone"""
+    n, rho = 3000, 0.06
+    print(f"[gpu] verlet digits omega={size}", flush=True)
+    xy = np.random.default_rng(8).random((n, 2))
+    g, o, st = tiles._systems(spss, xy, rho, v0=0.0)
+    st[7, 3] = size
+    g.set_state(st.reshape(-1))
+    tiles._step(spss, g, o, st, "srk")
+    om = np.abs(st[:, 3])
+    d = np.abs(g.complementary_force() - o.complementary_force())
+    tol = SIGMA * 3 * 2.0 ** -24 * (_most(xy, rho, om) + om) + 1e-12
     assert np.all(d <= tol), (d.max(), np.max(d / tol))
 
 
