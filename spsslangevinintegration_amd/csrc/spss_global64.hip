@@ -8,8 +8,8 @@
 // stage, no stage pass, no launch for the reduction.  A small system stays in the registers of one
 // workgroup for whole steps.
 //
-// What bounds it: small systems the chain phasor - sums - derivative (n = 1,000: 1.1 us per stage; a
-// Runge-Kutta step took 55 us in 17 launches and takes 4.4), systems up to about 100,000 the latency of a
+// What bounds it: small systems the chain phasor - sums - derivative (n = 1,000: 1.2 us per stage; a
+// Runge-Kutta step took 55 us in 17 launches and takes 4.7), systems up to about 100,000 the latency of a
 // launch (4 us; a step of 16,384: 56 -> 17 us), large ones memory: a Dormand-Prince trial of 1,048,576 470 ->
 // 214 us, an Euler step 75 -> 25 us.
 //
@@ -568,17 +568,23 @@ __device__ __forceinline__ double swap_add(double a, double b) {
   return u.d + v.d;
 }
 
-__device__ __forceinline__ double row_sum(double x) {  // lane 15 of each row
-  x += dpp<0x111, 0xf>(x);
+// the sums of a, b, c, d over a wave: in lane 15 of the rows of 16 lanes that column_of names
+__device__ __forceinline__ double four_sums(double a, double b, double c, double d) {
+  double x = swap_add<true>(swap_add<false>(a, b), swap_add<false>(c, d));
+  x += dpp<0x111, 0xf>(x);  // row_shr:1
   x += dpp<0x112, 0xf>(x);
   x += dpp<0x114, 0xf>(x);
   x += dpp<0x118, 0xf>(x);
   return x;
 }
+__device__ __forceinline__ int column_of(int lane) { return ((lane >> 4) & 1) * 2 + (lane >> 5); }
 
 // Up to 256 * PPT particles: one workgroup, the particles in registers, nsteps steps.  The chain of a
 // stage is a phasor, the sums over the workgroup (register moves, one LDS exchange) and the
-// derivative.  The four waves have a SIMD each, and one wave of independent particles issues nearly
+// derivative.  Cosines and sines are added in two parts, multiples of 2^-40, whose sums are exact in any order,
+// and the rest, whose sums err by 2^-80; the omega-weighted ones, which have no such bound, carry their rounding
+// errors over a thread's particles and over the waves, as the block sums of larger systems do over their blocks
+// (all of them that way: n = 1,000 20 us more for 80 stages).  The four waves have a SIMD each, and one wave of independent particles issues nearly
 // every cycle it is given, so the particles are split over registers before they are split over more
 // waves, whose reductions would only add instructions.
 enum GfStepper { kSmallRk4, kSmallEuler, kSmallSrk };
@@ -590,7 +596,8 @@ __global__ __launch_bounds__(256) void gf_small(DevParams P, int nsteps, double 
                                                 double *__restrict__ k4, double *__restrict__ compl_out, GfNoise Z) {
   constexpr bool HO = STEPPER == kSmallSrk;
   constexpr int COLS = HO ? 4 : 2;
-  __shared__ double sh[2][COLS][4];
+  constexpr bool kOne = PPT == 1;  // a block's sums alone, plain
+  __shared__ double sh[2][HO && !kOne ? 8 : 4][4];  // the waves' sums
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   double y[PPT][S], st[PPT][S], w[PPT], sn[PPT], cs[PPT];
 #pragma unroll
@@ -618,32 +625,49 @@ __global__ __launch_bounds__(256) void gf_small(DevParams P, int nsteps, double 
       for (int p = 0; p < PPT; ++p)
         if (!(fabs(st[p][2]) <= 0x1p30)) sincos(st[p][2], &sn[p], &cs[p]);
     }
-    double s[COLS] = {};
+    double s[4] = {}, m[2] = {}, e[2] = {};  // the parts of the cosines and of the sines; the weighted ones
 #pragma unroll
     for (int p = 0; p < PPT; ++p) {
       const bool in = p * 256 + (int)threadIdx.x < P.n;
       const double c1 = in ? cs[p] : 0.0, s1 = in ? sn[p] : 0.0;
-      s[0] += c1;
-      s[1] += s1;
-      if (HO) {
-        s[COLS - 2] += in ? st[p][S - 1] * c1 : 0.0;
-        s[COLS - 1] += in ? st[p][S - 1] * s1 : 0.0;
+      constexpr double kSplit = 6144.0;  // 1.5 2^12: of up to 2^11 terms
+      const double ch = kOne ? c1 : (c1 + kSplit) - kSplit, sh1 = kOne ? s1 : (s1 + kSplit) - kSplit;
+      const double w[2] = {HO && in ? st[p][S - 1] * c1 : 0.0, HO && in ? st[p][S - 1] * s1 : 0.0};
+      if (kOne) {
+        s[0] = c1, s[1] = s1, s[2] = w[0], s[3] = w[1];
+        continue;
       }
+      s[0] += ch;
+      s[1] += sh1;
+      s[2] += c1 - ch;
+      s[3] += s1 - sh1;
+      if (HO) add_terms<2>(w, m, e);
     }
-    double t = swap_add<false>(s[0], s[1]);
-    if (HO) {
-      t = row_sum(swap_add<true>(t, swap_add<false>(s[COLS - 2], s[COLS - 1])));
-      if ((lane & 15) == 15) sh[flip][((lane >> 4) & 1) * 2 + (lane >> 5)][wv] = t;
-    } else {
-      t = row_sum(t);
-      t += dpp<0x142, 0xa>(t);  // row_bcast:15
-      if ((lane & 31) == 31) sh[flip][lane >> 5][wv] = t;
+    double t = four_sums(s[0], s[1], s[2], s[3]);
+    if ((lane & 15) == 15) sh[flip][column_of(lane)][wv] = t;
+    if (HO && !kOne) {
+      t = four_sums(m[0], m[1], e[0], e[1]);
+      if ((lane & 15) == 15) sh[flip][(HO && !kOne ? 4 : 0) + column_of(lane)][wv] = t;
     }
     __syncthreads();
+    const auto four = [](const double *x) { return (x[0] + x[1]) + (x[2] + x[3]); };
     double v[COLS];
 #pragma unroll
-    for (int q = 0; q < COLS; ++q)
-      v[q] = ((sh[flip][q][0] + sh[flip][q][1]) + (sh[flip][q][2] + sh[flip][q][3])) / (double)P.n;
+    for (int q = 0; q < 2; ++q) v[q] = (kOne ? four(sh[flip][q]) : four(sh[flip][q]) + four(sh[flip][2 + q])) / (double)P.n;
+    if (HO)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        if (kOne) {
+          v[COLS - 2 + q] = four(sh[flip][2 + q]) / (double)P.n;
+          continue;
+        }
+        const double *x = sh[flip][HO && !kOne ? 4 + q : 0];
+        double r, u, z, d0, d1, d2;
+        two_sum(x[0], x[1], r, d0);
+        two_sum(x[2], x[3], u, d1);
+        two_sum(r, u, z, d2);
+        v[COLS - 2 + q] = (z + (((d0 + d1) + d2) + four(sh[flip][HO && !kOne ? 6 + q : 0]))) / (double)P.n;
+      }
     flip ^= 1;  // the other half is free: every wave had read it before this barrier
     F.zx = v[0];
     F.zy = v[1];
@@ -795,9 +819,9 @@ void stochastic(hipStream_t st, const DevParams &P, long nsteps, double dt, doub
   }
 }
 
-// Largest systems of one workgroup.  A step there, in launches: Runge-Kutta n = 2,048: 8.9, 17 us (twice
-// as many do not fit its registers); Euler n = 1,024: 3.5, 5.4 us, 2,048: 6.6, 5.4 us; stochastic
-// Runge-Kutta 4.3, 6.5 and 7.8, 6.5 us.
+// Largest systems of one workgroup.  A step there, in launches: Runge-Kutta n = 2,048: 10, 17 us (twice
+// as many do not fit its registers); Euler n = 1,024: 3.4, 5.4 us, 2,048: 6.6, 5.4 us; stochastic
+// Runge-Kutta 4.5, 6.5 and 7.8, 6.5 us.
 constexpr int kSmallRk4N = 2048, kSmallStochasticN = 1024;
 constexpr int kSmallSteps = 1024;  // steps of one launch
 
