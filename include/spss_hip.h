@@ -148,8 +148,8 @@ int spss_run(spss_system *sys, int stepper, int method, long nsteps, double dt, 
 /* No reference counterpart (the reference has no graphs): readies spss_run of the FP32C linked-list
  * Euler/SRK steps with Philox noise -- enters the cell-ordered resident copy of the state and
  * captures the HIP graphs every later run of this stepper and dt replays, from both buffer
- * parities, without taking a step.  A no-op for runs that step eagerly (other precisions, methods
- * or noise).  spss_run then replays every step from graphs (the first step of a run enters the
+ * parities, without taking a step.  For runs that step eagerly (other precisions, methods or
+ * noise) it allocates the workspace of the FP64 all-pairs sums and does nothing else.  spss_run then replays every step from graphs (the first step of a run enters the
  * resident order eagerly when it is not there yet). */
 int spss_prepare_run(spss_system *sys, int stepper, int method, double dt, int noise_mode);
 /* No reference counterpart: steps launched one by one and steps replayed from graphs since the

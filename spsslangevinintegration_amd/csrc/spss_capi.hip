@@ -207,11 +207,18 @@ int ensure_scan(spss_system *h) {
   return dalloc_n(&h->scan_blk, scan_blocks(h->n) + 1);
 }
 
+// With the handle where the reference's dispatch on rho takes all pairs, otherwise at the first evaluation:
+// 2.6 kB a particle at n = 4,099, 80 bytes of a million's, that other systems do without.  The stream may be
+// captured then: relaxed, this thread may allocate meanwhile.
 int ensure_all_pairs(spss_system *h) {
   if (h->ap.rec) return SPSS_OK;
   const size_t n = h->n;
   h->ap.nseg = all_pairs_segments(h->n);
-  TRY(dalloc_n(&h->ap.rec, (5 + (size_t)h->ap.nseg * 5) * n));  // one allocation for the three arrays
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  HIPCHECK(hipThreadExchangeStreamCaptureMode(&mode));
+  const int rc = dalloc_n(&h->ap.rec, (5 + (size_t)h->ap.nseg * 5) * n);  // one allocation for the three arrays
+  HIPCHECK(hipThreadExchangeStreamCaptureMode(&mode));
+  TRY(rc);
   h->ap.om = h->ap.rec + 4 * n;
   h->ap.part = h->ap.om + n;
   return SPSS_OK;
@@ -309,9 +316,10 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
   if (tiled) {
     TRY(ensure_cells64(h));
     launch_cells64_build(st, h->P, d_state, d_kprev, k_coef * dt, h->ncx, h->cells64);
-  } else if (m == SPSS_METHOD_ALL_PAIRS)
+  } else if (m == SPSS_METHOD_ALL_PAIRS) {
+    TRY(ensure_all_pairs(h));
     launch_all_pairs_stage(st, h->P, d_state, d_kprev, k_coef * dt, h->stage, h->ap);
-  else if (m != SPSS_METHOD_GLOBAL_FIELD && (!verlet || h->should_update))  // the Verlet pair sums stage in the order of their lists
+  } else if (m != SPSS_METHOD_GLOBAL_FIELD && (!verlet || h->should_update))  // the Verlet pair sums stage in the order of their lists
     launch_stage(st, (long)h->s * h->n, d_state, d_kprev, k_coef * dt, h->stage);
   switch (m) {
     case SPSS_METHOD_GLOBAL_FIELD:
@@ -692,8 +700,8 @@ int spss_create(const spss_params *p, spss_system **out) {
   step(dalloc_n(&h->noise, (size_t)3 * h->n));
   step(dalloc_n(&h->partial, std::max((size_t)(nb * 4 + 64), gf_part_doubles(p->n))));
   step(dalloc_n(&h->scal, 64));
-  // with the handle, so that an all-pairs evaluation allocates nothing (a caller may capture it)
-  if (p->precision != SPSS_PRECISION_FP32C) step(ensure_all_pairs(h));
+  if (p->precision != SPSS_PRECISION_FP32C && resolve_method(h, SPSS_METHOD_AUTO) == SPSS_METHOD_ALL_PAIRS)
+    step(ensure_all_pairs(h));
   if (rc != SPSS_OK) {
     spss_destroy(h);
     return rc;
@@ -922,7 +930,10 @@ int spss_run(spss_system *h, int stepper, int method, long nsteps, double dt, in
 int spss_prepare_run(spss_system *h, int stepper, int method, double dt, int noise_mode) {
   if (!h) return fail(SPSS_ERR_INVALID, "NULL handle");
   const int kind = graph_run_kind(h, stepper, method, noise_mode);
-  if (!kind) return SPSS_OK;  // spss_run steps eagerly here
+  if (!kind)  // spss_run steps eagerly here
+    return h->p.precision != SPSS_PRECISION_FP32C && resolve_method(h, method) == SPSS_METHOD_ALL_PAIRS
+               ? ensure_all_pairs(h)
+               : SPSS_OK;
   const bool srk = stepper == SPSS_STEPPER_SRK && h->s == 4;
   const double *nat = h->have_nat ? h->nat : nullptr;
   if (kind == 2) TRY(ensure_vfast(h));
