@@ -231,7 +231,6 @@ int spss_batch_create(const spss_batch_params *bp, int nrep, const spss_replica 
     return fast_fail(rc);
   }
   launch_fill_double(b->st, (long)b->s * b->n, b->state, 0.0);
-  (void)b->copy.reserve(sizeof(double) * (size_t)b->s * b->n);  // with the other workspaces: 0.4 ms less at the first read
   launch_fill_double(b->st, b->n, b->nat, 0.0);
   rc = fast_batch_reset(b->fast, b->st, 0);
   if (rc != SPSS_OK) {

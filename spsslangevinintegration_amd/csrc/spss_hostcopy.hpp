@@ -1,11 +1,13 @@
 // spss_hostcopy.hpp -- copies from device memory to a caller's ordinary (pageable) memory.
 //
-// The runtime stages such a copy through its own pinned memory with one thread: 21 MB take 1.2 ms, of
-// which the transfer is 0.4, and 5.1 ms into memory that has no pages yet.  Here the transfer goes to a
-// pinned buffer of the handle in pieces, and up to kCopyThreads threads move them on as they arrive: 0.68
-// and 1.3 ms (two threads 0.68 and 3.0).  Below 16 MB the runtime does it: a handle's first copy of 10 MB took
-// 1.3 ms here (new pinned pages, threads) and 0.65 there, a later one 0.55 and 0.62.  So it does for memory that
-// is pinned already, and for copies to the device, where it is no slower.
+// The runtime stages such a copy through its own pinned memory with one thread: 20 MB take 1.16 ms, of
+// which the transfer is 0.4, and 4.8 ms into memory that has no pages yet.  Here the transfer goes to a
+// pinned buffer of the handle in pieces, and up to kCopyThreads threads move them on as they arrive: 0.73
+// and 1.24 ms (two threads 0.68 and 3.0 at 21 MB).  Into memory that has its pages both take as long at 8 MB (0.47;
+// 4 MB 0.24 and 0.37, 12 MB 0.70 and 0.55, 16 MB 0.93 and 0.62): the runtime copies less than that.  It
+// also makes a handle's first copy, for which the pinned pages (1 ms) would come on top and which for
+// many handles is the only one; and it copies to memory that is pinned already, and to the device, where this is
+// no faster.
 // Every call returns with the copy done, as before.
 #pragma once
 
@@ -20,7 +22,7 @@
 
 namespace spss {
 
-constexpr size_t kCopyMin = 16u << 20, kCopyBuffer = 32u << 20;  // bytes
+constexpr size_t kCopyMin = 8u << 20, kCopyBuffer = 32u << 20;  // bytes
 constexpr int kCopyPieces = 16, kCopyThreads = 8;
 
 // the pinned buffer (at most kCopyBuffer bytes) and the pieces' events, kept by a handle and given back
@@ -31,23 +33,6 @@ class HostCopy {
   HostCopy(const HostCopy &) = delete;
   HostCopy &operator=(const HostCopy &) = delete;
   ~HostCopy() { drop(); }
-
-  // the buffer for copies of that much; false if there is none (they go to the runtime then)
-  bool reserve(size_t bytes) {
-    if (bytes < kCopyMin) return false;
-    const size_t want = std::min(kCopyBuffer, piece_of(bytes) * kCopyPieces);
-    if (cap_ >= want) return true;
-    drop();
-    bool ok = hipHostMalloc(reinterpret_cast<void **>(&pin_), want, hipHostMallocDefault) == hipSuccess;
-    for (hipEvent_t &e : ev_) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-    if (!ok) {
-      (void)hipGetLastError();
-      drop();
-      return false;
-    }
-    cap_ = want;
-    return true;
-  }
 
   hipError_t to_host(void *dst, const void *src, size_t bytes, hipStream_t st) {
     if (!staged(dst, bytes)) return direct(dst, src, bytes, hipMemcpyDeviceToHost, st);
@@ -77,6 +62,7 @@ class HostCopy {
  private:
   char *pin_ = nullptr;
   size_t cap_ = 0;
+  bool again_ = false;  // there has been a copy of kCopyMin bytes or more
   hipEvent_t ev_[kCopyPieces] = {};
 
   static size_t piece_of(size_t m) { return ((m + kCopyPieces - 1) / kCopyPieces + 4095) / 4096 * 4096; }
@@ -96,6 +82,22 @@ class HostCopy {
     cap_ = 0;
   }
 
+  // the buffer for copies of that much; false if there is none (they go to the runtime then)
+  bool reserve(size_t bytes) {
+    const size_t want = std::min(kCopyBuffer, piece_of(bytes) * kCopyPieces);
+    if (cap_ >= want) return true;
+    drop();
+    bool ok = hipHostMalloc(reinterpret_cast<void **>(&pin_), want, hipHostMallocDefault) == hipSuccess;
+    for (hipEvent_t &e : ev_) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+      (void)hipGetLastError();
+      drop();
+      return false;
+    }
+    cap_ = want;
+    return true;
+  }
+
   // whether a copy of that much to `host` is staged here; allocates the buffer
   bool staged(const void *host, size_t bytes) {
     if (bytes < kCopyMin) return false;
@@ -104,6 +106,10 @@ class HostCopy {
       if (a.type != hipMemoryTypeUnregistered) return false;
     } else {
       (void)hipGetLastError();  // memory that the runtime does not know
+    }
+    if (!again_) {
+      again_ = true;
+      return false;
     }
     return reserve(bytes);
   }
