@@ -36,7 +36,7 @@ constexpr int kMaxLayers = 8;
 constexpr int kMaxDim = 4096;
 constexpr int kLossCap = 1 << 16;
 constexpr long kPredictPiece = 32768;   // rows copied and launched together
-constexpr long kPredictCap = 1L << 20;  // rows on the device at a time: 4 MB per column
+constexpr long kPredictBytes = 64L << 20;  // of rows and outputs on the device at a time, kept by the network
 
 int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
@@ -61,7 +61,7 @@ struct spss_mlp {
   bool narrow = false;    // all layers in LDS, one launch for all of them (ml_rows, ml_grad, ml_predict)
   Net net{};
   float *dzl[kMaxLayers] = {};  // narrow: gradients w.r.t. every Z [max_batch x d_{l+1}]
-  float *px = nullptr, *py = nullptr;  // rows and outputs of one predict call (at most kPredictCap rows)
+  float *px = nullptr, *py = nullptr;  // rows and outputs of one predict call
   long prows = 0;
 };
 
@@ -276,7 +276,8 @@ int spss_mlp_predict(spss_mlp *m, const float *x, long n, float *y) {
   if (n < 0) return set_error(SPSS_ERR_INVALID, "n must be >= 0");
   const int din = m->dims[0], dout = m->dims[m->L];
   if (m->narrow) {
-    const long cap = std::min(n, kPredictCap);
+    // at least kPredictPiece rows: a narrow network's row has at most kNarrow inputs and as many outputs
+    const long cap = std::min(n, kPredictBytes / (long)(sizeof(float) * (din + dout)));
     if (cap > m->prows) {
       if (m->px) hipFree(m->px), m->px = nullptr;
       if (m->py) hipFree(m->py), m->py = nullptr;

@@ -1,0 +1,28 @@
+"""Tables of more rows than a network keeps on the device at a time (64 MB of rows and outputs): the same outputs as
+row by row chunks of the table, and no more memory held."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def test_table_beyond_the_workspace():
+    import spsslangevinintegration_amd as spss
+    dims, rows = (128, 16, 128), 200003
+    print(f"[gpu] predict rows={rows} dims={dims}", flush=True)
+    net = spss.MLP(dims, max_batch=64, seed=3)
+    x = np.random.default_rng(1).uniform(-1, 1, (rows, dims[0])).astype(np.float32)
+    few = net.predict(x[:100])
+    hip = C.CDLL("libamdhip64.so.7")  # the runtime that the library is linked against
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    before = free.value
+    y = net.predict(x)
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    print(f"  {(before - free.value) / 1e6:.1f} MB held", flush=True)
+    assert before - free.value <= 80e6
+    assert np.array_equal(y[:100], few)
+    for a in (65500, 131000, 199900):
+        assert np.array_equal(y[a:a + 103], net.predict(x[a:a + 103]))
