@@ -522,7 +522,8 @@ __global__ __launch_bounds__(kTB, 4) void ml_predict(Net N, const float *__restr
           const int row = 16 * q + 4 * g + r;
           const float z = acc[t][q][r] + bo[t];
           if (!last)
-            a[row * kPP + o] = gelu(z);  // zeros past the last output: the next layer's padding
+            a[row * kPP + o] = o < out ? gelu(z) : 0.f;  // zeros past the last output: the next layer's padding (an
+                                                         // infinite input times its zero weights is none)
           else if (row < R && o < out)
             Y[(long)(b0 + row) * out + o] = z;
         }

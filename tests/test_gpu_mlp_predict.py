@@ -26,3 +26,22 @@ def test_table_beyond_the_workspace():
     assert np.array_equal(y[:100], few)
     for a in (65500, 131000, 199900):
         assert np.array_equal(y[a:a + 103], net.predict(x[a:a + 103]))
+
+
+@pytest.mark.parametrize("width", [1, 3, 5, 6, 17, 18, 64, 127])
+def test_activations_that_overflow(width):
+    """a hidden unit of the first layer overflows, all of the second and the output with it: infinite, as the sums
+    of the real units are, whatever the widths leave of a tile"""
+    import spsslangevinintegration_amd as spss
+    dims = (1, width, width, 2)
+    print(f"[gpu] predict overflow width={width}", flush=True)
+    net = spss.MLP(dims, max_batch=64, seed=3)
+    w1 = np.zeros((width, 1))
+    w1[0] = 1e38
+    w2 = np.full((width, width), 0.5)
+    w3 = np.full((2, width), 0.25)
+    w3[1] = -0.25
+    parts = [w1, np.zeros(width), w2, np.zeros(width), w3, np.zeros(2)]
+    net.params = np.concatenate([p.ravel() for p in parts]).astype(np.float32)
+    y = net.predict(np.array([[10.0], [0.0], [20.0]], dtype=np.float32))
+    assert np.all(np.isposinf(y[[0, 2], 0])) and np.all(np.isneginf(y[[0, 2], 1])) and np.all(y[1] == 0)
