@@ -27,13 +27,6 @@ namespace {
 // outside it at all, ClassA is no minimum image there), or a phase without a finite phasor
 constexpr double kExactMark = __builtin_huge_val();
 
-__device__ __forceinline__ void phasor_any(double phi, double ref, double &sn, double &cs) {
-  if (fabs(phi) <= kPhase64)
-    frame_phasor(phi, ref, sn, cs);
-  else
-    sincos(phi - ref, &sn, &cs);
-}
-
 template <int S>
 __global__ __launch_bounds__(256) void ap_stage(DevParams P, const double *__restrict__ state,
                                                 const double *__restrict__ kprev,
@@ -52,7 +45,7 @@ __global__ __launch_bounds__(256) void ap_stage(DevParams P, const double *__res
   }
   double x, y, sn, cs;
   apply_pbc(P, st[0], st[1], x, y);
-  phasor_any(st[kPhi], ref, sn, cs);
+  frame_phasor_any(st[kPhi], ref, sn, cs);
   bool fine = fabs(sn) <= 1.5 && fabs(st[0]) <= kFar64 * P.xs && fabs(st[1]) <= kFar64 * P.ys;
   if (S == 6) fine = fine && st[0] >= 0.0 && st[0] < P.xs && st[1] >= 0.0 && st[1] < P.ys;
   if (S == 4 && P.higher_order) {
@@ -240,7 +233,7 @@ __global__ __launch_bounds__(256) void ap_finish(DevParams P, int nseg, const do
   for (int q = 0; q < S; ++q) st[q] = stage[(long)i * S + q];
   const double om_i = HO ? st[Slots<S>::omega] - frame_ref(stage[Slots<S>::omega]) : 0.0;
   double s_i, c_i;
-  phasor_any(st[Slots<S>::phi], frame_ref(stage[Slots<S>::phi]), s_i, c_i);
+  frame_phasor_any(st[Slots<S>::phi], frame_ref(stage[Slots<S>::phi]), s_i, c_i);
   const PairAcc pa = pair_acc<S>(P, a, s_i, c_i, om_i);
   write_k<S>(P, st, i, pa, nat ? nat[i] : 0.0, k_next, compl_out);
 }

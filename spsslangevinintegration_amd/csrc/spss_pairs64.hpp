@@ -26,15 +26,17 @@ struct PhasorSums {
   double S = 0.0, C = 0.0, card = 0.0, TS = 0.0, TC = 0.0;
 };
 
-// sin and cos of x + e for |x| <= 2^30 and a correction |e| far below one: reduction to |r| <= pi/4 by
+// sin and cos of x + e for |x| <= 2^30 and a correction |e| <= 2^-22: reduction to |r| <= pi/4 by
 // multiples of pi/2 (pi/2 in two parts, Cody and Waite, Software Manual for the Elementary Functions;
-// the first difference is exact, the multiples' low bits are 2^-52), then the Taylor polynomials to r^17 and r^16, whose next
-// terms are below 2^-60.  Branch-free and about a fifth of the instructions of the general sincos.
+// the first difference is exact, the multiples' low bits are 2^-52; the second part and the correction go into r
+// together, which leaves 2^-54 for what r lacks: that much may be taken to first order), then the Taylor
+// polynomials to r^17 and r^16, whose next terms are below 2^-60.  Branch-free and about a fifth of the instructions of the general sincos.
 __device__ __forceinline__ void small_sincos(double x, double e, double &sn, double &cs) {
   const double k = rint(x * 0x1.45f306dc9c883p-1);  // 2 / pi
   const double r0 = __builtin_fma(-k, 0x1.921fb54442d18p+0, x);
-  const double r = __builtin_fma(-k, 0x1.1a62633145c07p-54, r0);
-  e = __builtin_fma(-k, 0x1.1a62633145c07p-54, r0 - r) + e;  // what r lacks
+  const double t = __builtin_fma(-k, 0x1.1a62633145c07p-54, e);
+  const double r = r0 + t;
+  e = (r0 - r) + t;  // what r lacks
   const double z = r * r;
   double p = __builtin_fma(z, 1.0 / 355687428096000.0, -1.0 / 1307674368000.0);
   p = __builtin_fma(z, p, 1.0 / 6227020800.0);
@@ -91,10 +93,11 @@ __device__ __forceinline__ void frame_phasor_any(double phi, double ref, double 
   if (fabs(d) <= 0x1p30) {
     small_sincos(d, err, sn, cs);
   } else {
-    double s, c;
+    double s, c, se, ce;  // the error is of order one from 2^53 on
     sincos(d, &s, &c);
-    sn = __builtin_fma(err, c, s);
-    cs = __builtin_fma(-err, s, c);
+    sincos(err, &se, &ce);
+    sn = __builtin_fma(se, c, ce * s);
+    cs = __builtin_fma(-se, s, ce * c);
   }
 }
 
