@@ -129,80 +129,70 @@ __global__ __launch_bounds__(256) void c64_rank(DevParams P, int nc, const int *
 
 constexpr int kCols = 64;   // staged columns of a tile at most
 
-template <bool HO, int CAP, int NP>
+template <bool HO, int CAP, int TB>
 struct Stage64 {
   double4 rec[CAP];  // x, y (the periodic image next to the tile), sin psi, cos psi
   double om[HO ? CAP : 1];
   int offs[3][kCols + 1];  // staged entries before each staged column of a row of cells
   int first[3][kCols];     // its first sorted position
-  int col[NP];             // cell column of each particle of the workgroup
+  int col[TB];             // cell column of each particle of the workgroup
   int cut;                 // particles of the tile (past it: beyond kCols columns)
 };
 
-// the sums over the candidates [u, u + 4) (MASKED: only those before e) of a staged window for the
-// PPL particles of a lane: an entry read from LDS serves PPL pairs
-template <int S, bool HO, int PPL, bool MASKED, class LDS, class EXACT>
+// the sums over the candidates [u, u + 4) (MASKED: only those before e) of a staged window
+template <int S, bool HO, bool MASKED, class LDS, class EXACT>
 __device__ __forceinline__ void four_pairs(const DevParams &P, double band, double neg_slope, const LDS &L, int u, int e,
-                                           const double (&x_i)[PPL], const double (&y_i)[PPL], PhasorSums (&a)[PPL],
-                                           const EXACT &exact) {
-  double w[PPL][4], near = 1e300;
+                                           double x_i, double y_i, PhasorSums &a, const EXACT &exact) {
+  double w[4], near = 1e300;
   double4 r[4];
 #pragma unroll
   for (int q = 0; q < 4; ++q) r[q] = L.rec[MASKED ? min(u + q, e - 1) : u + q];
 #pragma unroll
-  for (int p = 0; p < PPL; ++p)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const double dx = r[q].x - x_i[p], dy = r[q].y - y_i[p];
-      const double t = __builtin_fma(dx, dx, __builtin_fma(dy, dy, -P.rho2));
-      near = fmin(near, fabs(t));
-      w[p][q] = pair_weight(t, neg_slope);
-      if (MASKED && u + q >= e) w[p][q] = 0.0;
-    }
+  for (int q = 0; q < 4; ++q) {
+    const double dx = r[q].x - x_i, dy = r[q].y - y_i;
+    const double t = __builtin_fma(dx, dx, __builtin_fma(dy, dy, -P.rho2));
+    near = fmin(near, fabs(t));
+    w[q] = pair_weight(t, neg_slope);
+    if (MASKED && u + q >= e) w[q] = 0.0;
+  }
   if (near <= band) {  // rare: the reference's own test decides
 #pragma unroll
-    for (int p = 0; p < PPL; ++p)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) w[p][q] = (!MASKED || u + q < e) && exact(p, u + q) ? 1.0 : 0.0;
+    for (int q = 0; q < 4; ++q) w[q] = (!MASKED || u + q < e) && exact(u + q) ? 1.0 : 0.0;
   }
 #pragma unroll
-  for (int p = 0; p < PPL; ++p)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      a[p].S = __builtin_fma(w[p][q], r[q].z, a[p].S);
-      a[p].C = __builtin_fma(w[p][q], r[q].w, a[p].C);
-      a[p].card += w[p][q];
-      if (HO) {
-        const double wo = w[p][q] * L.om[MASKED ? min(u + q, e - 1) : u + q];
-        a[p].TS = __builtin_fma(wo, r[q].z, a[p].TS);
-        a[p].TC = __builtin_fma(wo, r[q].w, a[p].TC);
-      }
+  for (int q = 0; q < 4; ++q) {
+    a.S = __builtin_fma(w[q], r[q].z, a.S);
+    a.C = __builtin_fma(w[q], r[q].w, a.C);
+    a.card += w[q];
+    if (HO) {
+      const double wo = w[q] * L.om[MASKED ? min(u + q, e - 1) : u + q];
+      a.TS = __builtin_fma(wo, r[q].z, a.TS);
+      a.TC = __builtin_fma(wo, r[q].w, a.TC);
     }
+  }
 }
 
-// One workgroup per TB * PPL particles of a row of cells (chunk k of row r, then chunk k +
-// gridDim.y, ...), PPL neighbours of the cell order per lane: the three rows of cells around them are
-// staged into LDS, positions as the periodic image next to the tile, so that a separation is a plain
+// One workgroup per TB particles of a row of cells (chunk k of row r, then chunk k + gridDim.y, ...), one per
+// lane in cell order: the three rows of cells around them are staged into LDS, positions as the periodic image next to the tile, so that a separation is a plain
 // difference; dense cells pass through the stage in windows of CAP entries.  A lane walks the three
-// column ranges of its particles, contiguous in the stage, in the reference's stencil order
-// (ParticleSystemFirstOrderPtr.cpp:83-88); a candidate past a particle's own columns is at least a
-// cell width away, so that only the exact test has to look at the columns.
-template <int S, bool HO, int TB, int PPL, int CAP>
+// column ranges of its particle, contiguous in the stage, in the reference's stencil order
+// (ParticleSystemFirstOrderPtr.cpp:83-88).
+template <int S, bool HO, int TB, int CAP>
 __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double band, double neg_slope, int nc, int rows8,
                                                 const int *__restrict__ start, const int *__restrict__ order,
                                                 const double *__restrict__ snap, const int *__restrict__ bad,
                                                 const double *__restrict__ nat, double *__restrict__ k_next,
                                                 double *__restrict__ compl_out) {
-  constexpr int kPhi = Slots<S>::phi, kOm = S == 3 ? 2 : Slots<S>::omega, NP = TB * PPL;
-  __shared__ Stage64<HO, CAP, NP> L;
+  constexpr int kPhi = Slots<S>::phi, kOm = S == 3 ? 2 : Slots<S>::omega;
+  __shared__ Stage64<HO, CAP, TB> L;
   // workgroups go round the eight XCDs: each takes an eighth of the rows, so that neighbouring rows
   // share an L2
   const int row = (blockIdx.x & 7) * rows8 + (blockIdx.x >> 3);
   if (row >= nc) return;
   const int r0 = start[row * nc], r1 = start[(row + 1) * nc];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int base = r0 + blockIdx.y * NP; base < r1; base += gridDim.y * NP) {
-    const int last = min(r1, base + NP);
+  for (int base = r0 + blockIdx.y * TB; base < r1; base += gridDim.y * TB) {
+    const int last = min(r1, base + TB);
     if (*bad) {  // pair by pair, the reference's expressions
       for (int g = base + threadIdx.x; g < last; g += TB) {
         double st[S], x_i, y_i;
@@ -227,21 +217,14 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
       }
       continue;
     }
-    const int g0 = base + threadIdx.x * PPL;
-    int cx[PPL];
-    double x_i[PPL], y_i[PPL], phi_i[PPL];
-#pragma unroll
-    for (int p = 0; p < PPL; ++p) {
-      const int g = min(g0 + p, last - 1);  // a lane past the end repeats the last particle
-      key_wrap<S>(P, snap[(long)g * S], snap[(long)g * S + 1], x_i[p], y_i[p]);
-      phi_i[p] = snap[(long)g * S + kPhi];
-      cx[p] = cell_coord(x_i[p], nc);
-    }
+    const int g = base + threadIdx.x, gi = min(g, last - 1);  // a lane past the end repeats the last particle
+    double x_i, y_i;
+    key_wrap<S>(P, snap[(long)gi * S], snap[(long)gi * S + 1], x_i, y_i);
+    const double phi_i = snap[(long)gi * S + kPhi];
+    const int cx = cell_coord(x_i, nc);
     const double ref = frame_ref(snap[(long)base * S + kPhi]);
     const double om_ref = HO ? frame_ref(snap[(long)base * S + kOm]) : 0.0;
-#pragma unroll
-    for (int p = 0; p < PPL; ++p)
-      if (g0 + p < last) L.col[g0 + p - base] = cx[p];
+    if (g < last) L.col[threadIdx.x] = cx;
     if (threadIdx.x == 0) L.cut = last;
     int done = base;  // particles before it are finished
     while (done < last) {
@@ -250,9 +233,7 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
       const int ca = L.col[done - base];
       int cut = last;
       if (L.col[last - 1 - base] > ca + kCols - 3) {  // a sparse row (the same for all threads)
-#pragma unroll
-        for (int p = PPL - 1; p >= 0; --p)
-          if (g0 + p >= done && g0 + p < last && cx[p] > ca + kCols - 3) atomicMin(&L.cut, g0 + p);
+        if (g >= done && g < last && cx > ca + kCols - 3) atomicMin(&L.cut, g);
         __syncthreads();
         cut = L.cut;
         __syncthreads();
@@ -284,27 +265,20 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
       __syncthreads();
       const int n0 = L.offs[0][ncols], n1 = n0 + L.offs[1][ncols], total = n1 + L.offs[2][ncols];
       const auto rowbase = [n0, n1](int k) { return k == 0 ? 0 : (k == 1 ? n0 : n1); };
-      // a lane takes part with the particles of its that lie in the tile
-      const int pa = max(g0, done) - g0, pe = min(g0 + PPL, cut) - g0;  // [pa, pe) of its PPL
-      const bool mine = pa < pe;
-      PhasorSums a[PPL];
-      double s_i[PPL] = {}, c_i[PPL] = {}, om_i[PPL] = {};
-      int ql = 0, qr = 0;  // staged columns of the lane: those of its first to its last particle in the tile
+      const bool mine = g >= done && g < cut;  // a lane takes part if its particle lies in the tile
+      const int ql = cx - ca;                  // its first staged column
+      PhasorSums a;
+      double s_i = 0.0, c_i = 0.0, om_i = 0.0;
       if (mine) {
-#pragma unroll
-        for (int p = 0; p < PPL; ++p) {
-          if (p == pa) ql = cx[p] - ca;
-          if (p == pe - 1) qr = cx[p] - ca + 3;
-          // a particle meets itself among its candidates: its own term is taken off beforehand
-          frame_phasor(phi_i[p], ref, s_i[p], c_i[p]);
-          a[p].S = -s_i[p];
-          a[p].C = -c_i[p];
-          a[p].card = -1.0;
-          if (HO) {
-            om_i[p] = snap[(long)min(g0 + p, last - 1) * S + kOm] - om_ref;
-            a[p].TS = -(om_i[p] * s_i[p]);
-            a[p].TC = -(om_i[p] * c_i[p]);
-          }
+        // a particle meets itself among its candidates: its own term is taken off beforehand
+        frame_phasor(phi_i, ref, s_i, c_i);
+        a.S = -s_i;
+        a.C = -c_i;
+        a.card = -1.0;
+        if (HO) {
+          om_i = snap[(long)gi * S + kOm] - om_ref;
+          a.TS = -(om_i * s_i);
+          a.TC = -(om_i * c_i);
         }
       }
       for (int w0 = 0; w0 < total; w0 += CAP) {
@@ -337,49 +311,41 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
         __syncthreads();
         if (mine) {
           // the reference's test of the staged entry u: its sorted position from the staging plan
-          const auto exact = [&](int p, int u) {
+          const auto exact = [&](int u) {
             const int v = w0 + u, k = v < n0 ? 0 : (v < n1 ? 1 : 2);
             int q = 0;
             while (rowbase(k) + L.offs[k][q + 1] <= v) ++q;
-            if (q < cx[p] - ca || q > cx[p] - ca + 2) return false;
             const double *sj = snap + ((long)L.first[k][q] + v - rowbase(k) - L.offs[k][q]) * S;
             double x_j = sj[0], y_j = sj[1];
             if (S == 6) key_wrap<6>(P, x_j, y_j, x_j, y_j);
-            return pair_in_range<S>(P, x_i[p], y_i[p], x_j, y_j);
+            return pair_in_range<S>(P, x_i, y_i, x_j, y_j);
           };
 #pragma unroll 1
           for (int k = 0; k < 3; ++k) {
             int u = max(rowbase(k) + L.offs[k][ql], w0) - w0;
-            const int e = min(rowbase(k) + L.offs[k][qr], w1) - w0;
-            PhasorSums r[PPL];  // a sum per row of cells: shorter chains of roundings
-            for (; u + 4 <= e; u += 4) four_pairs<S, HO, PPL, false>(P, band, neg_slope, L, u, e, x_i, y_i, r, exact);
-            if (u < e) four_pairs<S, HO, PPL, true>(P, band, neg_slope, L, u, e, x_i, y_i, r, exact);
-#pragma unroll
-            for (int p = 0; p < PPL; ++p) {
-              a[p].S += r[p].S;
-              a[p].C += r[p].C;
-              a[p].card += r[p].card;
-              if (HO) {
-                a[p].TS += r[p].TS;
-                a[p].TC += r[p].TC;
-              }
+            const int e = min(rowbase(k) + L.offs[k][ql + 3], w1) - w0;
+            PhasorSums r;  // a sum per row of cells: shorter chains of roundings
+            for (; u + 4 <= e; u += 4) four_pairs<S, HO, false>(P, band, neg_slope, L, u, e, x_i, y_i, r, exact);
+            if (u < e) four_pairs<S, HO, true>(P, band, neg_slope, L, u, e, x_i, y_i, r, exact);
+            a.S += r.S;
+            a.C += r.C;
+            a.card += r.card;
+            if (HO) {
+              a.TS += r.TS;
+              a.TC += r.TC;
             }
           }
         }
       }
       if (mine) {
+        const int i = order[g];
+        double st[S];
 #pragma unroll
-        for (int p = 0; p < PPL; ++p) {
-          if (p < pa || p >= pe) continue;
-          const int i = order[g0 + p];
-          double st[S];
-#pragma unroll
-          for (int q = 0; q < S; ++q) st[q] = snap[(long)(g0 + p) * S + q];
-          const PairAcc acc = pair_acc<S>(P, a[p], s_i[p], c_i[p], om_i[p]);
-          double sn, cs;
-          small_sincos(st[kPhi], 0.0, sn, cs);
-          write_k<S>(P, st, i, acc, nat ? nat[i] : 0.0, sn, cs, k_next, compl_out);
-        }
+        for (int q = 0; q < S; ++q) st[q] = snap[(long)g * S + q];
+        const PairAcc acc = pair_acc<S>(P, a, s_i, c_i, om_i);
+        double sn, cs;
+        small_sincos(st[kPhi], 0.0, sn, cs);
+        write_k<S>(P, st, i, acc, nat ? nat[i] : 0.0, sn, cs, k_next, compl_out);
       }
       done = cut;
     }
@@ -403,15 +369,15 @@ void build(hipStream_t st, const DevParams &P, const double *state, const double
   B.cur = next;
 }
 
-template <int S, bool HO, int TB, int PPL, int CAP>
+template <int S, bool HO, int TB, int CAP>
 void pairs_as(hipStream_t st, const DevParams &P, int nc, const Cells64 &B, const double *nat, double *k_next,
               double *compl_out) {
   const int rows8 = (nc + 7) / 8;
   // chunks of a row of mean length, one more for the spread; longer rows loop
   const long per_row = (P.n + nc - 1) / nc;
-  const unsigned chunks = (unsigned)std::min<long>((per_row + per_row / 8) / (TB * PPL) + 1, 65535);
+  const unsigned chunks = (unsigned)std::min<long>((per_row + per_row / 8) / TB + 1, 65535);
   const double band = pair_band(P.rho2, 1.0, 1.0);
-  c64_pairs<S, HO, TB, PPL, CAP><<<dim3((unsigned)rows8 * 8, chunks), dim3(TB), 0, st>>>(
+  c64_pairs<S, HO, TB, CAP><<<dim3((unsigned)rows8 * 8, chunks), dim3(TB), 0, st>>>(
       P, band, pair_neg_slope(band), nc, rows8, B.start, B.order[B.cur], B.snap, B.bad, nat, k_next, compl_out);
 }
 
@@ -422,9 +388,9 @@ void pairs(hipStream_t st, const DevParams &P, int nc, const Cells64 &B, const d
   // particles 128 a workgroup fill the chip better (per evaluation of model 6: 39.6 -> 36 us at
   // n = 20,000 against 42.2 -> 43.6 us at n = 50,000)
   if (P.n >= 40960)
-    pairs_as<S, HO, 256, 1, 1152>(st, P, nc, B, nat, k_next, compl_out);
+    pairs_as<S, HO, 256, 1152>(st, P, nc, B, nat, k_next, compl_out);
   else
-    pairs_as<S, HO, 128, 1, 640>(st, P, nc, B, nat, k_next, compl_out);
+    pairs_as<S, HO, 128, 640>(st, P, nc, B, nat, k_next, compl_out);
 }
 
 }  // namespace
