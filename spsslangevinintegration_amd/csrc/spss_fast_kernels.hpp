@@ -30,8 +30,11 @@ namespace spss {
 
 namespace {
 constexpr int kFB = kTileCap;   // threads per pair workgroup (one particle of a row tile each)
-constexpr int kStageMax = 1120; // staged entries per workgroup (particles + row padding): 1,024 left a step of
-                                // 1M particles a few tiles to redo (fr_far 10.9, now 4.7 us; fr_pairs +0.4)
+// Staged entries per workgroup (particles + row padding).  From 50 neighbours on square cells, and 60 on cells split
+// in x, a stage of 1,024 leaves tiles over to fr_far: an Euler step of 100,000 particles with 80 neighbours 42
+// -> 31 us at 1,120, of 1M with 53, 80, 110 neighbours 87 -> 84, 112 -> 100, 133 -> 127; below, where both
+// hold every tile, the LDS costs 1% at most.
+constexpr int kStageMax = 1120;
 constexpr int kPad = 4;         // padding entries after each staged row (>= the unroll - 1)
 constexpr int kMaxCells = 336;  // staged cells (2ky+1) x (W+2kx) of one workgroup
 constexpr int kMaxSpan = 25;    // stencil columns 2kx+1 (kx = k * xsplit <= 12)

@@ -15,10 +15,11 @@
 // any order and grouping.  An FP32 phasor is kept whole from 2^-13 of the scale on, and beside one of 2^-9
 // in range what smaller ones lose (2^-38) is below that one's own rounding to FP32 (2^-34): these sums
 // are closer to the exact ones than FP32 partial sums are; so for the weighted ones beside one of 2^-18 (the
-// bulk of a Lorentzian clipped at 200 of its widths is at 2^-8).  Marks tell whether there is one in range; where there is none
-// (beside a particle far off its neighbours in the same tile) the caller takes the sums itself.
+// bulk of a Lorentzian clipped at 200 of its widths is at 2^-8).  Planes of marks tell, by the same
+// product, whether there is one in range; where there is none (beside a particle far off its neighbours in the
+// same tile) the caller takes the sums itself.
 //
-// Bound: the vector units, 46 operations per 1,024 pairs where a walk over candidates takes 180, and
+// Bound: the vector units, 42 operations per 1,024 pairs where a walk over candidates takes 180, and
 // what comes before and after.  Cycles of a SIMD per 1,024 pairs, measured alone: this product 71 (by
 // v_mfma_f32_16x16x4_f32 139, and nothing else issues meanwhile), signs to bytes and the band's minimum
 // 85 (by v_cvt_pk_u8_f32, which takes eight cycles, 180), the digit products 34; the loop 244.
@@ -44,7 +45,7 @@ constexpr float kMUnit = 1024.f;      // positions: cells to |x| < 25 in halves,
 constexpr float kMSquare = 0x1p-14f;  // squares in halves
 constexpr float kMFar = 3e4f;         // "|x|^2" of padding at x = 0, in squares: beyond every range
 
-// W: words of digits per entry: the first four digits of cos and of sin, the last one of both with the marks;
+// W: words of digits per entry: the first four digits of cos and of sin, the last one of both and the two marks;
 // the first digits of omega cos and omega sin, their last two in one word
 constexpr int kMPlain = 3, kMOmega = 6;
 template <int W>
@@ -113,7 +114,10 @@ __device__ __forceinline__ int m_fixed(float v, int &lo) {
   lo = (int)__builtin_rintf((v - h) * (float)(1 << LOW));
   return (int)h;
 }
-__device__ __forceinline__ bool m_marked(float v, MScale k) { return __builtin_fabsf(v) >= k.mark; }
+// whether both components of an entry are marked
+__device__ __forceinline__ unsigned m_marked(float x, MScale kx, float y, MScale ky) {
+  return __builtin_fabsf(x) >= kx.mark && __builtin_fabsf(y) >= ky.mark ? 1u : 0u;
+}
 // signed digits of a 32-bit number, and of a smaller one's two
 __device__ __forceinline__ unsigned m_digits(int q) { return ((unsigned)q + 0x80808080u) ^ 0x80808080u; }
 __device__ __forceinline__ unsigned m_digits16(int q) { return (((unsigned)q + 0x8080u) ^ 0x8080u) & 0xffffu; }
@@ -132,19 +136,18 @@ __device__ __forceinline__ void m_write(MStage<W> &L, int e, bool valid, float x
   constexpr int kNext = 4 * kMDigits;  // the same digit of the next word
   int lc, ls;
   const int hc = m_fixed<7>(c, lc), hs = m_fixed<7>(s, ls);
-  unsigned marks = (m_marked(c, kc) ? 1u : 0u) | (m_marked(s, ks) ? 2u : 0u);
   d[0] = quad_transpose(m_digits(hc), s1, s2);
   d[kNext] = quad_transpose(m_digits(hs), s1, s2);
-  const unsigned low = (lc & 0xff) | (ls & 0xff) << 8;
+  unsigned low = (lc & 0xff) | (ls & 0xff) << 8 | m_marked(c, kc, s, ks) << 16;
   if (W == kMOmega) {
     const float vx = om * (c * 0x1p-30f), vy = om * (s * 0x1p-30f);
-    marks |= (m_marked(vx, ko) ? 4u : 0u) | (m_marked(vy, ko) ? 8u : 0u);
+    low |= m_marked(vx, ko, vy, ko) << 24;
     const int hx = m_fixed<15>(vx, lc), hy = m_fixed<15>(vy, ls);
     d[3 * kNext] = quad_transpose(m_digits(hx), s1, s2);
     d[4 * kNext] = quad_transpose(m_digits(hy), s1, s2);
     d[5 * kNext] = quad_transpose(m_digits16(lc) | m_digits16(ls) << 16, s1, s2);
   }
-  d[2 * kNext] = quad_transpose(low | marks << 16, s1, s2);
+  d[2 * kNext] = quad_transpose(low, s1, s2);
 }
 
 struct MSums {
@@ -165,7 +168,7 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), i = lane & 15, g = lane >> 4;
   MSums out;
   int sx[2] = {0, 0}, sy[2] = {0, 0}, kx = 0, ky = 0, tx[2] = {0, 0}, ty[2] = {0, 0}, lx = 0, ly = 0;
-  unsigned marked = 0;
+  int mp = 0, mo = 0;  // marked phasors, weighted ones in range
   // the units of each group's candidates, four groups at once, one row per lane
   int total = 0;
   {
@@ -190,11 +193,10 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
   const char *fb = (g < 2 ? reinterpret_cast<const char *>(L.pos[0]) : reinterpret_cast<const char *>(L.sq)) + 16 * (i & 3);
   constexpr int kSecond = sizeof(L.pos[0]);
   const int second = g < 2 ? kSecond : 0;
-  // the planes: the phasors' ten digits, and ones; the weighted ones' twelve; the marks
-  const char *l1 = i < 10 ? reinterpret_cast<const char *>(L.limb[i]) : reinterpret_cast<const char *>(L.ones);
-  const int m1 = i < 10 ? -1 : 0;
+  // the planes: the phasors' ten digits, the marks, ones; the weighted ones' twelve digits
+  const char *l1 = i < 12 ? reinterpret_cast<const char *>(L.limb[i]) : reinterpret_cast<const char *>(L.ones);
+  const int m1 = i < 12 ? -1 : 0;
   const char *l2 = reinterpret_cast<const char *>(L.limb[W == kMOmega && i < 12 ? 12 + i : 0]);
-  const char *lm = reinterpret_cast<const char *>(L.limb[10]);
   for (int gr = 0; 16 * gr < count; ++gr) {
     const bool real = 16 * gr + i < count;
     const uint2 own = m_pos(L, real ? first + 16 * gr + i : kMStage);
@@ -234,12 +236,10 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
       return r;  // t[q][r]: entry 4r + q of the lane's unit
     };
     const auto bits = [](float t) { return __builtin_bit_cast(unsigned, t); };
-    mint4 any = {0, 0, 0, 0};  // marks in range
     int el = 16 * ul[0], ef = 16 * uf[0];
     for (int u = 0; u < n; u += 4) {
       const Products c = products(features(ef));
       const mint4 d1 = *reinterpret_cast<const mint4 *>(l1 + (el & m1));
-      const mint4 dm = *reinterpret_cast<const mint4 *>(lm + el);
       const int el0 = el;
       el = 16 * ul[u + 4];
       ef = 16 * uf[u + 4];
@@ -267,22 +267,19 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
         }
       }
       s1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(d1, w, s1, 0, 0, 0);
-      any |= w & dm;
       if (W == kMOmega) s2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(*reinterpret_cast<const mint4 *>(l2 + el0), w, s2, 0, 0, 0);
     }
     // lanes i and 16 + i hold the first digits of the cosines' and the sines' sums, lane 32 + i the last ones and
-    // the count; lane 16 gr + i takes them, in pairs
+    // the marks, lane 48 + i the count; lane 16 gr + i takes them, in pairs
     const int p0 = s1[0] + (s1[1] << 8), p1 = s1[2] + (s1[3] << 8);
     const int x0 = __shfl(p0, i), x1 = __shfl(p1, i), y0 = __shfl(p0, 16 + i), y1 = __shfl(p1, 16 + i);
-    const int z0 = __shfl(s1[0], 32 + i), z1 = __shfl(s1[1], 32 + i), cn = __shfl(s1[2], 32 + i);
-    unsigned seen = (unsigned)(any[0] | any[1] | any[2] | any[3]);
-    seen |= __shfl_xor(seen, 16);
-    seen |= __shfl_xor(seen, 32);
+    const int z0 = __shfl(s1[0], 32 + i), z1 = __shfl(s1[1], 32 + i), cn = __shfl(s1[0], 48 + i);
+    const int c0 = __shfl(s1[2], 32 + i), c1 = W == kMOmega ? __shfl(s1[3], 32 + i) : 0;
     if (g == gr) {
       sx[0] = x0, sx[1] = x1, sy[0] = y0, sy[1] = y1, kx = z0, ky = z1;
       out.n = -cn;
-      marked = seen | seen >> 16;
-      marked |= marked >> 8;
+      mp = c0;
+      mo = c1;
     }
     if (W == kMOmega) {
       const int q0 = s2[0] + (s2[1] << 8), q1 = s2[2] + (s2[3] << 8);
@@ -305,8 +302,7 @@ __device__ __forceinline__ MSums m_sums(MStage<W> &L, int first, int count, int 
     out.tx = ldexp(-(whole(tx) + (double)hx + 0x1p-15 * (double)(lx + lc)), 30 - ko.up - kc.up);
     out.ty = ldexp(-(whole(ty) + (double)hy + 0x1p-15 * (double)(ly + ls)), 30 - ko.up - ks.up);
   }
-  constexpr unsigned kAll = W == kMOmega ? 15u : 3u;
-  if (out.n > 1 && (marked & kAll) != kAll) {
+  if (out.n > 1 && (mp == 0 || (W == kMOmega && mo == 0))) {
     out.n = kMOpen;
     return out;
   }
