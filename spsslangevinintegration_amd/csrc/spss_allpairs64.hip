@@ -2,7 +2,7 @@
 // ParticleSystemFirstOrderPtr.cpp:225-316 / ParticleSystemSecondOrderPtr.cpp:155-230.
 //
 //   ap_stage   the stage state, and per particle a 32-byte record {x, y, sin psi, cos psi} (wrapped
-//              position, phasor in the frame of particle 0's phase) and omega - omega_0
+//              position, phasor in the frame of particle 0's phase) and omega
 //   ap_pairs   grid (groups of BLOCK particles) x (segments of the j's): the phasor sums of every
 //              particle over one segment, j ascending
 //   ap_finish  the segments' sums added in ascending order, the derivative
@@ -49,9 +49,8 @@ __global__ __launch_bounds__(256) void ap_stage(DevParams P, const double *__res
   bool fine = fabs(sn) <= 1.5 && fabs(st[0]) <= kFar64 * P.xs && fabs(st[1]) <= kFar64 * P.ys;
   if (S == 6) fine = fine && st[0] >= 0.0 && st[0] < P.xs && st[1] >= 0.0 && st[1] < P.ys;
   if (S == 4 && P.higher_order) {
-    const double o = st[kOm] - frame_ref(state[kOm] + (kprev ? kc_dt * kprev[kOm] : 0.0));
-    fine = fine && fabs(o) < 1e300;
-    om[i] = o;
+    fine = fine && fabs(st[kOm]) < 1e300;
+    om[i] = st[kOm];
   }
   rec[i] = make_double4(fine ? x : kExactMark, y, sn, cs);
 }
@@ -68,7 +67,7 @@ template <int S, bool HO, int PPL, int T, bool MASKED>
 __device__ __forceinline__ void four_j(const DevParams &P, double band, double neg_slope,
                                        const double *__restrict__ stage, const double4 *tile, const double *tom, int i0,
                                        int j0, int t0, int cnt, const double (&x_i)[PPL], const double (&y_i)[PPL],
-                                       PhasorSums (&a)[PPL]) {
+                                       const double (&om_i)[PPL], PhasorSums (&a)[PPL]) {
   double w[PPL][4], near = 1e300;
   double4 r[4];
 #pragma unroll
@@ -101,7 +100,7 @@ __device__ __forceinline__ void four_j(const DevParams &P, double band, double n
     for (int u = 0; u < 4; ++u) {
       add_pair(a[p], w[p][u], r[u].z, r[u].w);
       if (HO) {
-        const double wo = w[p][u] * tom[MASKED ? min(t0 + u, cnt - 1) : t0 + u];
+        const double wo = w[p][u] * (tom[MASKED ? min(t0 + u, cnt - 1) : t0 + u] - om_i[p]);
         a[p].TS = __builtin_fma(wo, r[u].z, a[p].TS);
         a[p].TC = __builtin_fma(wo, r[u].w, a[p].TC);
       }
@@ -121,13 +120,17 @@ __global__ __launch_bounds__(BLOCK / PPL) void ap_pairs(DevParams P, double band
   const int n = P.n;
   const int i0 = blockIdx.x * BLOCK;
   const int jb = blockIdx.y * seglen, je = min(n, jb + seglen);
-  double x_i[PPL], y_i[PPL];
+  double x_i[PPL], y_i[PPL], om_i[PPL];
   bool mine_ok = true;
 #pragma unroll
   for (int p = 0; p < PPL; ++p) {
     const int i = i0 + p * T + threadIdx.x;
-    x_i[p] = y_i[p] = 0.0;
+    x_i[p] = y_i[p] = om_i[p] = 0.0;
     if (i < n) {
+      if (HO) {
+        om_i[p] = stage[(long)i * S + Slots<S>::omega];
+        mine_ok = mine_ok && fabs(om_i[p]) < 1e300;
+      }
       x_i[p] = stage[(long)i * S];
       y_i[p] = stage[(long)i * S + 1];
       if (S == 6)  // model 6 wraps nothing (ParticleSystemSecondOrderPtr.cpp:188-193)
@@ -153,9 +156,9 @@ __global__ __launch_bounds__(BLOCK / PPL) void ap_pairs(DevParams P, double band
       int t0 = 0;
       if (!own)
         for (; t0 + 4 <= cnt; t0 += 4)
-          four_j<S, HO, PPL, T, false>(P, band, neg_slope, stage, tile, tom, i0, j0, t0, cnt, x_i, y_i, a);
+          four_j<S, HO, PPL, T, false>(P, band, neg_slope, stage, tile, tom, i0, j0, t0, cnt, x_i, y_i, om_i, a);
       for (; t0 < cnt; t0 += 4)
-        four_j<S, HO, PPL, T, true>(P, band, neg_slope, stage, tile, tom, i0, j0, t0, cnt, x_i, y_i, a);
+        four_j<S, HO, PPL, T, true>(P, band, neg_slope, stage, tile, tom, i0, j0, t0, cnt, x_i, y_i, om_i, a);
     } else {
       for (int t = 0; t < cnt; ++t) {
         const int j = j0 + t;
@@ -167,8 +170,8 @@ __global__ __launch_bounds__(BLOCK / PPL) void ap_pairs(DevParams P, double band
             const double4 r = tile[t];
             add_pair(a[p], 1.0, r.z, r.w);
             if (HO) {
-              a[p].TS = __builtin_fma(tom[t], r.z, a[p].TS);
-              a[p].TC = __builtin_fma(tom[t], r.w, a[p].TC);
+              a[p].TS = __builtin_fma(tom[t] - om_i[p], r.z, a[p].TS);
+              a[p].TC = __builtin_fma(tom[t] - om_i[p], r.w, a[p].TC);
             }
           }
         }
@@ -231,10 +234,9 @@ __global__ __launch_bounds__(256) void ap_finish(DevParams P, int nseg, const do
   double st[S];
 #pragma unroll
   for (int q = 0; q < S; ++q) st[q] = stage[(long)i * S + q];
-  const double om_i = HO ? st[Slots<S>::omega] - frame_ref(stage[Slots<S>::omega]) : 0.0;
   double s_i, c_i;
   frame_phasor_any(st[Slots<S>::phi], frame_ref(stage[Slots<S>::phi]), s_i, c_i);
-  const PairAcc pa = pair_acc<S>(P, a, s_i, c_i, om_i);
+  const PairAcc pa = pair_acc<S>(P, a, s_i, c_i);
   write_k<S>(P, st, i, pa, nat ? nat[i] : 0.0, k_next, compl_out);
 }
 

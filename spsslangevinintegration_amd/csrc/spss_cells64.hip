@@ -142,7 +142,7 @@ struct Stage64 {
 // the sums over the candidates [u, u + 4) (MASKED: only those before e) of a staged window
 template <int S, bool HO, bool MASKED, class LDS, class EXACT>
 __device__ __forceinline__ void four_pairs(const DevParams &P, double band, double neg_slope, const LDS &L, int u, int e,
-                                           double x_i, double y_i, PhasorSums &a, const EXACT &exact) {
+                                           double x_i, double y_i, double om_i, PhasorSums &a, const EXACT &exact) {
   double w[4], near = 1e300;
   double4 r[4];
 #pragma unroll
@@ -165,7 +165,7 @@ __device__ __forceinline__ void four_pairs(const DevParams &P, double band, doub
     a.C = __builtin_fma(w[q], r[q].w, a.C);
     a.card += w[q];
     if (HO) {
-      const double wo = w[q] * L.om[MASKED ? min(u + q, e - 1) : u + q];
+      const double wo = w[q] * (L.om[MASKED ? min(u + q, e - 1) : u + q] - om_i);
       a.TS = __builtin_fma(wo, r[q].z, a.TS);
       a.TC = __builtin_fma(wo, r[q].w, a.TC);
     }
@@ -223,7 +223,6 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
     const double phi_i = snap[(long)gi * S + kPhi];
     const int cx = cell_coord(x_i, nc);
     const double ref = frame_ref(snap[(long)base * S + kPhi]);
-    const double om_ref = HO ? frame_ref(snap[(long)base * S + kOm]) : 0.0;
     if (g < last) L.col[threadIdx.x] = cx;
     if (threadIdx.x == 0) L.cut = last;
     int done = base;  // particles before it are finished
@@ -270,16 +269,13 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
       PhasorSums a;
       double s_i = 0.0, c_i = 0.0, om_i = 0.0;
       if (mine) {
-        // a particle meets itself among its candidates: its own term is taken off beforehand
+        // a particle meets itself among its candidates: its own term is taken off beforehand (those with omegas are
+        // zeros)
         frame_phasor(phi_i, ref, s_i, c_i);
         a.S = -s_i;
         a.C = -c_i;
         a.card = -1.0;
-        if (HO) {
-          om_i = snap[(long)gi * S + kOm] - om_ref;
-          a.TS = -(om_i * s_i);
-          a.TC = -(om_i * c_i);
-        }
+        if (HO) om_i = snap[(long)gi * S + kOm];
       }
       for (int w0 = 0; w0 < total; w0 += CAP) {
         const int w1 = min(total, w0 + CAP);
@@ -300,7 +296,7 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
           const int jrow = row + k - 1;
           L.rec[v] = make_double4(xw + (left ? -1.0 : (right ? 1.0 : 0.0)),
                                   yw + (jrow < 0 ? -1.0 : (jrow >= nc ? 1.0 : 0.0)), sj[kPhi], 0.0);
-          if (HO) L.om[v] = sj[kOm] - om_ref;
+          if (HO) L.om[v] = sj[kOm];
         }
         for (int v = threadIdx.x; v < w1 - w0; v += TB) {  // a thread's own entries
           double sn, cs;
@@ -325,8 +321,8 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
             int u = max(rowbase(k) + L.offs[k][ql], w0) - w0;
             const int e = min(rowbase(k) + L.offs[k][ql + 3], w1) - w0;
             PhasorSums r;  // a sum per row of cells: shorter chains of roundings
-            for (; u + 4 <= e; u += 4) four_pairs<S, HO, false>(P, band, neg_slope, L, u, e, x_i, y_i, r, exact);
-            if (u < e) four_pairs<S, HO, true>(P, band, neg_slope, L, u, e, x_i, y_i, r, exact);
+            for (; u + 4 <= e; u += 4) four_pairs<S, HO, false>(P, band, neg_slope, L, u, e, x_i, y_i, om_i, r, exact);
+            if (u < e) four_pairs<S, HO, true>(P, band, neg_slope, L, u, e, x_i, y_i, om_i, r, exact);
             a.S += r.S;
             a.C += r.C;
             a.card += r.card;
@@ -342,7 +338,7 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
         double st[S];
 #pragma unroll
         for (int q = 0; q < S; ++q) st[q] = snap[(long)g * S + q];
-        const PairAcc acc = pair_acc<S>(P, a, s_i, c_i, om_i);
+        const PairAcc acc = pair_acc<S>(P, a, s_i, c_i);
         double sn, cs;
         small_sincos(st[kPhi], 0.0, sn, cs);
         write_k<S>(P, st, i, acc, nat ? nat[i] : 0.0, sn, cs, k_next, compl_out);

@@ -211,9 +211,9 @@ __global__ __launch_bounds__(kBlock) void k_verlet_build_cells(DevParams P, cons
 
 // stage state in the order of the lists' build (order null: as it is), and what the pair sums read of
 // it: x, y wrapped into the box (NaN farther out than the guard band covers) and the phasor in the frame
-// of the phase that particle 0's state has; om: omega from that state's
+// of the phase that particle 0's state has; om: omega
 template <int S>
-__device__ __forceinline__ void stage_record(const DevParams &P, const double *v, double ref, double om_ref, int t,
+__device__ __forceinline__ void stage_record(const DevParams &P, const double *v, double ref, int t,
                                              const VerletStage &V) {
 #pragma unroll
   for (int q = 0; q < S; ++q) V.stage[(long)t * S + q] = v[q];
@@ -222,7 +222,7 @@ __device__ __forceinline__ void stage_record(const DevParams &P, const double *v
   apply_pbc(P, v[0], v[1], xw, yw);
   const bool near = fabs(v[0]) <= kFar64 * P.xs && fabs(v[1]) <= kFar64 * P.ys;
   reinterpret_cast<double4 *>(V.rec)[t] = make_double4(near ? xw : __builtin_nan(""), yw, sn, cs);
-  if (S == 4) V.om[t] = v[S - 1] - om_ref;
+  if (S == 4) V.om[t] = v[S - 1];
 }
 
 // vmax: the step's displacement maxima, cleared (may be null)
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(kBlock) void k_stage_order(DevParams P, const doubl
   double v[S];
 #pragma unroll
   for (int q = 0; q < S; ++q) v[q] = state[i * S + q] + (kprev ? kc_dt * kprev[i * S + q] : 0.0);
-  stage_record<S>(P, v, frame_ref(state[2]), S == 4 ? frame_ref(state[S - 1]) : 0.0, t, V);
+  stage_record<S>(P, v, frame_ref(state[2]), t, V);
 }
 
 // Verlet pair loop, ParticleSystemFirstOrderPtr.cpp:553-613 (x_i as stored), through the phasors
@@ -264,6 +264,7 @@ __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double ban
   const int i = t < P.n ? (order ? order[t] : t) : -1;
   PhasorSums q;
   double4 own{};
+  double om_i = 0.0;
   double pre = 0.0, old = 0.0, k4[S] = {};  // THEN 2: component l of k1 + 2 k2 + 2 k3 and of the state
   if (THEN == 2 && i >= 0 && l < S) {
     const long c = (long)i * S + l;
@@ -272,6 +273,7 @@ __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double ban
   }
   if (i >= 0) {
     own = rec[t];
+    if (HO) om_i = om[t];
     int u = vstart[i] + l;
     const int e = vstart[i + 1];
     if (u < e) {
@@ -294,7 +296,7 @@ __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double ban
           q.C += r.w;
           q.card += 1.0;
           if (HO) {
-            const double o = om[j];
+            const double o = om[j] - om_i;
             q.TS += o * r.z;
             q.TC += o * r.w;
           }
@@ -320,14 +322,14 @@ __global__ __launch_bounds__(kBlock) void k_verlet_pairs(DevParams P, double ban
 #pragma unroll
     for (int k = 0; k < S; ++k) st[k] = vstage[(long)t * S + k];
     phasor_of(st[2], sn, cs);
-    write_k<S>(P, st, i, pair_acc<S>(P, q, own.z, own.w, HO ? om[t] : 0.0), nat ? nat[i] : 0.0, sn, cs, k_next,
+    write_k<S>(P, st, i, pair_acc<S>(P, q, own.z, own.w), nat ? nat[i] : 0.0, sn, cs, k_next,
                compl_out);
     const long ii = (long)i * S;
     if (THEN == 1) {
       double v[S];
 #pragma unroll
       for (int k = 0; k < S; ++k) v[k] = N.base[ii + k] + N.kc * k_next[ii + k];  // what k_next holds: see write_k
-      stage_record<S>(P, v, frame_ref(N.base[2]), S == 4 ? frame_ref(N.base[S - 1]) : 0.0, t, N.next);
+      stage_record<S>(P, v, frame_ref(N.base[2]), t, N.next);
     } else if (THEN == 2) {
 #pragma unroll
       for (int k = 0; k < S; ++k) k4[k] = k_next[ii + k];

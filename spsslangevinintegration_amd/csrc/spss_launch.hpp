@@ -109,7 +109,7 @@ constexpr int kAllPairsDefault = 4;
 extern const int kAllPairsConfigs[kAllPairsConfigCount][2];
 struct AllPairsScratch {
   double *rec = nullptr;   // [4 n] {x, y, sin psi, cos psi} per particle
-  double *om = nullptr;    // [n] omega relative to particle 0's
+  double *om = nullptr;    // [n] omega
   double *part = nullptr;  // [nseg][5][n] the segments' sums
   int nseg = 0;
 };
@@ -151,8 +151,8 @@ void launch_verlet_count_cells(hipStream_t st, const DevParams &P, const double 
                                const CellBuffers &cb, double rmax2, int *vcount);
 void launch_verlet_fill_cells(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy,
                               const CellBuffers &cb, double rmax2, const int *vstart, int *vlist, int *vslot);
-// the stage state in the order of the lists' build (null: over all pairs), with the records and relative
-// omegas that the pair sums over it read
+// the stage state in the order of the lists' build (null: over all pairs), with the records and omegas that
+// the pair sums over it read
 struct VerletStage {
   double *stage = nullptr;  // [s n]
   double *rec = nullptr;    // [4 n] {x, y, sin psi, cos psi}

@@ -8,7 +8,9 @@
 // rounds like phi_j - phi_i does, and near synchrony (all psi small) S, s_i and every rounding
 // error scale with the spread of the phases, so the sums keep the relative accuracy of the direct
 // form there as well.  The complementary force's sum of (omega_j - omega_i) cos(phi_j - phi_i -
-// alpha) goes through sum omega' sin psi and sum omega' cos psi with omega' = omega - omega_ref.
+// alpha) goes through the sums of (omega_j - omega_i) sin psi_j and (omega_j - omega_i) cos psi_j: the differences
+// are taken pair by pair (an operation of some twenty), since no frame's omega would do for all, where one is
+// far off the others.
 //
 // Neighbour sets are the reference's bit for bit: the cheap distance test decides only outside a
 // guard band around rho^2 that covers its rounding, pairs inside it go through the reference's own
@@ -23,7 +25,8 @@ namespace spss {
 
 // sums over the neighbours of one particle, in the frame of the reference phase
 struct PhasorSums {
-  double S = 0.0, C = 0.0, card = 0.0, TS = 0.0, TC = 0.0;
+  double S = 0.0, C = 0.0, card = 0.0;
+  double TS = 0.0, TC = 0.0;  // of omega_j - omega_i times the phasors
 };
 
 // sin and cos of x + e for |x| <= 2^30 and a correction |e| <= 2^-22: reduction to |r| <= pi/4 by
@@ -101,7 +104,7 @@ __device__ __forceinline__ void frame_phasor_any(double phi, double ref, double 
   }
 }
 
-// a reference phase or phase velocity: any value of an ordinary size serves
+// a reference phase: any value of an ordinary size serves
 __device__ __forceinline__ double frame_ref(double v) { return fabs(v) <= kPhase64 ? v : 0.0; }
 
 // |t| of a pair below which its distance test goes to pair_in_range.  Coordinates up to
@@ -137,10 +140,9 @@ __device__ __forceinline__ double cross(double a, double b, double c, double d) 
 }
 
 // the coupling sums of the reference (PairAcc) from the phasor sums: s_i, c_i the particle's own
-// phasor, om_i relative to the frame's reference
+// phasor
 template <int S>
-__device__ __forceinline__ PairAcc pair_acc(const DevParams &P, const PhasorSums &q, double s_i, double c_i,
-                                            double om_i) {
+__device__ __forceinline__ PairAcc pair_acc(const DevParams &P, const PhasorSums &q, double s_i, double c_i) {
   PairAcc a{0.0, 0.0, 0.0};
   if (q.card == 0.0) return a;
   // sums of sin, cos (phi_j - phi_i)
@@ -149,7 +151,7 @@ __device__ __forceinline__ PairAcc pair_acc(const DevParams &P, const PhasorSums
   a.card = q.card;
   if (S == 4 && P.higher_order) {
     const double tsn = cross(c_i, q.TS, s_i, q.TC), tcs = __builtin_fma(c_i, q.TC, s_i * q.TS);
-    a.compl_f = (tcs - om_i * cs) * P.cos_a + (tsn - om_i * sn) * P.sin_a;
+    a.compl_f = tcs * P.cos_a + tsn * P.sin_a;
   }
   return a;
 }
