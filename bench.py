@@ -47,12 +47,12 @@ def pair_kernel_bytes(n, cells):
 # HBM bytes per launch of that kernel measured with rocprofv3 FETCH_SIZE / WRITE_SIZE, scaled
 # by the copy-kernel calibration, by cell layout (subdivision, x split)
 # (profiles/fr_pairs_euler_N1M_hbm_traffic.txt)
-PAIR_KERNEL_TRAFFIC = {(1, 1): 4.4389e7, (1, 2): 4.7781e7, (1, 4): 5.4909e7}
+PAIR_KERNEL_TRAFFIC = {(1, 1): 4.44e7, (1, 2): 4.78e7, (1, 4): 5.49e7}
 # HBM bytes of the three kernels of one resident step (fr_pairs, fr_far, fr_scatter), the same way
-STEP_TRAFFIC = {(1, 1): 1.9577e8, (1, 2): 2.0656e8, (1, 4): 2.1588e8}
+STEP_TRAFFIC = {(1, 1): 1.9339e8, (1, 2): 2.0112e8, (1, 4): 2.1680e8}
 # VALU instructions issued per CU-cycle by that kernel (SQ_INSTS_VALU / (256 CUs x cycles),
 # profiles/fr_pairs_euler_N1M_valu.txt), by cell layout: the nominal rate is one per CU-cycle
-PAIR_KERNEL_VALU_PER_CU_CYCLE = {(1, 1): 0.99, (1, 2): 0.91, (1, 4): 0.86}
+PAIR_KERNEL_VALU_PER_CU_CYCLE = {(1, 1): 0.98, (1, 2): 0.91, (1, 4): 0.85}
 # algorithmic HBM bytes per particle-step of the cell-list step (s = 4 state, one RHS): FP64 state
 # read + write 16*s, FP32 snapshot x, y, phi written and read 8*3, cell key and sorted index written
 # and read 16, cell start/count table 8 per cell -- the compulsory traffic of the reference

@@ -73,7 +73,7 @@ __global__ void ob_phasors(const double *__restrict__ state, int n, long npad, i
 // runs of L terms for 64 exponents (a wave per run and component, an exponent per lane), ob_long_runs
 // composes 16 of them, and ob_walk goes through the long runs, into their runs where a long one
 // leaves its binade, and term by term where a run does (n = 1,048,576, random phases: about half of
-// the long runs, a tenth to a third of the runs).  106 + 11 us for the maps, 1.1-1.7 ms for the walk:
+// the long runs, a tenth to a third of the runs).  121 + 11 us for the maps, 1.1-1.7 ms for the walk:
 // 4.5 cycles per addition left (370,000 at most of the million), 340 per map looked up.
 __global__ __launch_bounds__(256) void ob_runs(const float *__restrict__ ph, long npad, int L, int nruns,
                                                SeqMap *__restrict__ runs) {

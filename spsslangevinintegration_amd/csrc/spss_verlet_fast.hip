@@ -20,7 +20,7 @@
 // so no list is read; lists are built for the few tiles that overflow the stage or a workgroup, and
 // for vf_lists, from the state that the last rebuild left in the scratch arrays.  Snapshots of tiled
 // grids hold positions from the centre of the particle's cell.  At N = 1M, 53 neighbours, skin
-// 0.2 rho, stochastic Runge-Kutta: 107 us per step (a third each: staging, sums, update), where walking
+// 0.2 rho, stochastic Runge-Kutta: 113 us per step (about a third each: staging, sums, update), where walking
 // 16-bit lists from LDS took 125, bound by LDS reads, and building them 190 per rebuild.
 //
 // Wider grids keep an ELL list of width K per slot with its length, in blocks of 256 slots and chunks of
