@@ -17,8 +17,8 @@
 // cells of one row, as for the cell-list pair kernel).  The step is one workgroup per tile: the 3 x (W + 2)
 // cells around its W cells go into LDS and the sums over the particles within rho come from the matrix
 // cores (spss_mfma_pairs.hpp).  The cells of the last rebuild hold every candidate until the next one,
-// so no list is read; lists are built for the few tiles that overflow the stage or a workgroup, and
-// for vf_lists, from the state that the last rebuild left in the scratch arrays.  Snapshots of tiled
+// so no list is read; the tiles that overflow the stage or a workgroup walk those cells (vt_rest), and lists
+// are built for vf_lists alone, from the state that the last rebuild left in the scratch arrays.  Snapshots of tiled
 // grids hold positions from the centre of the particle's cell.  At N = 1M, 53 neighbours, skin
 // 0.2 rho, stochastic Runge-Kutta: 113 us per step (about a third each: staging, sums, update), where walking
 // 16-bit lists from LDS took 125, bound by LDS reads, and building them 190 per rebuild.
@@ -31,7 +31,7 @@
 //
 // One step is a rebuild -- launches that return at once unless the device flag asks for one:
 // the flag, cell keys and histogram; the scan's blocks; starts and bucket fill; stable rank and gather into
-// scratch with the row tiles; back into the resident arrays with the new snapshot and the lists -- and the step,
+// scratch with the row tiles; back into the resident arrays with the new snapshot -- and the step,
 // which ends with the Euler/SRK update of step_particle, the new snapshot and the step's largest
 // squared displacement (maxima by group of workgroups), which the next step's first launch turns into its
 // flag on the device.  No host synchronisation: steps replay from HIP graphs.  Seven launches (tiled
@@ -70,7 +70,7 @@ struct VCtl {
   int force;                    // the resident copy was just entered: rebuild
   double acc[2];                // accumulated_displacement_, by the parity of the step that reads it
   unsigned long long step;      // Philox step of graph-replayed steps
-  int big_tiles;                // tiles of the last rebuild holding more particles than a workgroup
+  int nrest;                    // items of vt_rest since the last rebuild
   int pad;
   // the last step's largest |dr|^2 by group of workgroups (workgroup b in group b % kGroups), as the
   // bits of a non-negative double, one word per cache line so that the groups' atomics run apart
@@ -156,7 +156,7 @@ __global__ __launch_bounds__(kVB) void vr_keys(DevParams P, VArgs A, int parity,
     const int flag = A.ctl->force || acc + stepd > A.half_skin;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
       A.ctl->flag = flag;
-      if (flag) A.ctl->big_tiles = 0;  // counted again by vr_settle
+      if (flag) A.ctl->nrest = 0;  // vr_settle adds them again
       A.ctl->acc[1 - parity] = flag ? 0.0 : acc;
       if (step_inc) *step_inc += 1ull;
     }
@@ -579,8 +579,8 @@ __global__ __launch_bounds__(kVB) void vs_step(DevParams P, VArgs A, StepArgs U,
 // per tile -- a span of whole cells of one row, as for the cell-list pair kernel -- stages the
 // snapshots (and omega) of the 3 x (W + 2) cells around its W cells, which hold every candidate until
 // the next rebuild, and takes the sums over them on the matrix cores (spss_mfma_pairs.hpp): a
-// superset of the lists, whose pairs beyond rho count for nothing, with no list read.  So lists are
-// built only for tiles whose cells overflow the stage or whose particles outnumber the workgroup.
+// superset of the lists, whose pairs beyond rho count for nothing, with no list read.  Tiles whose cells
+// overflow the stage or whose particles outnumber the workgroup walk those cells through global memory.
 
 constexpr int kVCols = 48;  // staged columns W + 2
 
@@ -611,6 +611,10 @@ __device__ __forceinline__ int vt_plan(const VArgs &A, const int *__restrict__ s
   return ((L.len[0] + 15) & ~15) + ((L.len[1] + 15) & ~15) + ((L.len[2] + 15) & ~15);
 }
 
+// whether a workgroup of vt_step takes a tile of nt particles and that staged total; the others are cut into items
+constexpr int kRestItem = 64;
+__device__ __forceinline__ bool vt_takes(int total, int nt) { return total <= kMStage && nt <= kVB; }
+
 // back into the resident arrays, with the snapshot of the new order
 template <int S>
 __global__ __launch_bounds__(kVB) void vr_settle(DevParams P, VArgs A, const double *__restrict__ sstate,
@@ -619,8 +623,7 @@ __global__ __launch_bounds__(kVB) void vr_settle(DevParams P, VArgs A, const dou
                                                  int *__restrict__ id, double *__restrict__ nat,
                                                  int *__restrict__ cell, float4 *__restrict__ snap,
                                                  float *__restrict__ omega, const int *__restrict__ start,
-                                                 const int4 *__restrict__ tiles, int ntiles, int *__restrict__ list,
-                                                 int *__restrict__ len) {
+                                                 const int4 *__restrict__ tiles, int ntiles, int2 *__restrict__ rest) {
   if (gate_off(A)) return;
   for (int q = blockIdx.x * kVB + threadIdx.x; q < A.n; q += gridDim.x * kVB) {
     double st[S];
@@ -635,9 +638,10 @@ __global__ __launch_bounds__(kVB) void vr_settle(DevParams P, VArgs A, const dou
     cell[q] = c;
     snap[q] = tiles ? vsnap_cell(P, st, c % A.ncv, c / A.ncv, A.h) : vsnap_of(P, st);
     omega[q] = S == 4 ? (float)st[3] : 0.f;
-  }  // tiled grids: the lists of the tiles that walk theirs, from the scratch copy of the state, in
-  // list_of_slot's order
+  }
+  // tiled grids: the tiles that the workgroups of vt_step cannot take, in items of vt_rest
   __shared__ VtPlan L;
+  __shared__ int at;
   for (int tile = tiles ? blockIdx.x : ntiles; tile < ntiles; tile += gridDim.x) {  // (the same for the whole workgroup)
     const int4 td = tiles[tile];
     const int row = td.y, ca = td.z, cb = td.w;
@@ -645,10 +649,12 @@ __global__ __launch_bounds__(kVB) void vr_settle(DevParams P, VArgs A, const dou
     __syncthreads();  // the previous tile's plan is consumed
     const int total = vt_plan(A, start, row, ca, cb, L);
     const int gtb = start[row * A.ncv + ca], nt = start[row * A.ncv + cb] - gtb;
-    if (nt > kVB && threadIdx.x == 0) atomicAdd(&A.ctl->big_tiles, 1);
-    if (total <= kMStage && nt <= kVB) continue;
-    for (int u = threadIdx.x; u < nt; u += kVB)
-      list_of_slot<S, true>(P, A, start, scell, sstate, nullptr, list, len, gtb + u);
+    if (vt_takes(total, nt)) continue;
+    const int items = (nt + kRestItem - 1) / kRestItem;
+    if (threadIdx.x == 0) at = atomicAdd(&A.ctl->nrest, items);
+    __syncthreads();
+    for (int u = threadIdx.x; u < items; u += kVB)
+      rest[at + u] = make_int2(gtb + u * kRestItem, min(kRestItem, nt - u * kRestItem));
   }
 }
 
@@ -661,7 +667,7 @@ struct VtLds {
   double wmax[kVB / 64];
 };
 
-// The sums of the tile's particles (the workgroup's first kVB) over the staged cells.  Positions are
+// The sums of the tile's particles over the staged cells.  Positions are
 // taken from the tile's centre.  False: a staged value is not finite (the same for every thread).
 template <int S, int W>
 __device__ __forceinline__ bool vt_sums(const DevParams &P, const VArgs &A, int row, int ca, int cb, int gtb, int ntile,
@@ -784,56 +790,65 @@ __device__ __forceinline__ bool vt_sums(const DevParams &P, const VArgs &A, int 
   return true;
 }
 
-// The sums of slot p of a tiled grid through global memory, over its list (L >= 0) or over the cells of
-// the last rebuild, every pair by the reference's FP64 test (x_i as stored, rhs_verlet's :566-581).
-template <int S, bool SRK>
-__device__ __forceinline__ MSums vt_walk(const DevParams &P, const VArgs &A, const int *__restrict__ list,
-                                         const int *__restrict__ start, const int *__restrict__ cell,
-                                         const double *__restrict__ state, const float4 *__restrict__ snap,
-                                         const float *__restrict__ omega, int p, int L) {
+// The sums of slot p of a tiled grid through global memory, over a part of each of the 3 x 3 cells of the last
+// rebuild: FP32 distances between snapshots, which are relative to their cells (their errors are within the
+// guard band that vs_step's have), the band decided by the reference's FP64 test (x_i as stored, rhs_verlet's
+// :566-581); phasor sums in four FP32 partials flushed into FP64 every U candidates.  Neighbouring lanes are
+// particles of one cell and read the same candidates, in order, where lists of a dense cell scatter.
+template <int S, bool SRK, int U>
+__device__ __forceinline__ MSums vt_walk(const DevParams &P, const VArgs &A, const int *__restrict__ start,
+                                         const int *__restrict__ cell, const double *__restrict__ state,
+                                         const float4 *__restrict__ snap, const float *__restrict__ omega, int p,
+                                         int part = 0, int parts = 1) {
+  static_assert(U % 4 == 0 && U <= 16, "partials of four candidates at most");
   MSums m;
-  const double xi = state[(long)p * S], yi = state[(long)p * S + 1];
-  const auto range = [&](int a, int b, auto slot) {  // entries [a, b), four at a time
-    for (int t0 = a; t0 < b; t0 += 4) {
-      double x[4], y[4];
-      float4 o[4];
-      float om[4];
-      int j[4];
+  const float4 me = snap[p];
+  const double *pi = state + (long)p * S;
+  const int c = cell[p], cx = c % A.ncv, cy = c / A.ncv;
+  const float h = (float)A.h;
+  for (int k = 0; k < 9; ++k) {
+    const int dxc = k % 3 - 1, dyc = k / 3 - 1;
+    const int cj = adjust_cell(cy + dyc, A.ncv) * A.ncv + adjust_cell(cx + dxc, A.ncv);
+    const int first = start[cj], count = start[cj + 1] - first;
+    const int b = first + (int)((long)count * (part + 1) / parts);
+    const float xi = me.x - (float)dxc * h, yi = me.y - (float)dyc * h;
+    for (int t0 = first + (int)((long)count * part / parts); t0 < b; t0 += U) {
+      float4 o[U];
+      float om[U], ax[4] = {}, ay[4] = {}, bx[4] = {}, by[4] = {};
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        j[k] = slot(min(t0 + k, b - 1));
-        x[k] = state[(long)j[k] * S];
-        y[k] = state[(long)j[k] * S + 1];
-        o[k] = snap[j[k]];
-        if (SRK) om[k] = omega[j[k]];
+      for (int u = 0; u < U; ++u) {
+        const int j = min(t0 + u, b - 1);
+        o[u] = snap[j];
+        if (SRK) om[u] = omega[j];
       }
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        double dx, dy;
-        class_c_unsigned(P, xi, yi, x[k], y[k], dx, dy);
-        if (t0 + k < b && j[k] != p && dx * dx + dy * dy <= P.rho2) {
-          m.sx += (double)o[k].z;
-          m.sy += (double)o[k].w;
-          ++m.n;
-          if (SRK) {
-            m.tx += (double)om[k] * (double)o[k].z;
-            m.ty += (double)om[k] * (double)o[k].w;
-          }
+      for (int u = 0; u < U; ++u) {
+        const float dx = o[u].x - xi, dy = o[u].y - yi;
+        const float dd = __builtin_fmaf(dy, dy, __builtin_fmaf(dx, dx, -A.r2c));
+        bool in = dd < 0.f;
+        if (__builtin_fabsf(dd) <= A.r2h) {  // rare
+          const double *pj = state + (long)min(t0 + u, b - 1) * S;
+          double ddx, ddy;
+          class_c_unsigned(P, pi[0], pi[1], pj[0], pj[1], ddx, ddy);
+          in = ddx * ddx + ddy * ddy <= P.rho2;
+        }
+        in = in && t0 + u < b && t0 + u != p;
+        m.n += in ? 1 : 0;
+        ax[u & 3] += in ? o[u].z : 0.f;
+        ay[u & 3] += in ? o[u].w : 0.f;
+        if (SRK) {
+          bx[u & 3] += in ? om[u] * o[u].z : 0.f;
+          by[u & 3] += in ? om[u] * o[u].w : 0.f;
         }
       }
+      m.sx += ((double)ax[0] + (double)ax[1]) + ((double)ax[2] + (double)ax[3]);
+      m.sy += ((double)ay[0] + (double)ay[1]) + ((double)ay[2] + (double)ay[3]);
+      if (SRK) {
+        m.tx += ((double)bx[0] + (double)bx[1]) + ((double)bx[2] + (double)bx[3]);
+        m.ty += ((double)by[0] + (double)by[1]) + ((double)by[2] + (double)by[3]);
+      }
     }
-  };
-  if (L >= 0) {
-    range(0, L, [&](int t) { return list[lslot(p, t, A.K)]; });
-    return m;
   }
-  const int c = cell[p];
-  const int cx = c % A.ncv, cy = c / A.ncv;
-  for (int dyc = -1; dyc <= 1; ++dyc)
-    for (int dxc = -1; dxc <= 1; ++dxc) {
-      const int cj = adjust_cell(cy + dyc, A.ncv) * A.ncv + adjust_cell(cx + dxc, A.ncv);
-      range(start[cj], start[cj + 1], [](int t) { return t; });
-    }
   return m;
 }
 
@@ -867,51 +882,72 @@ __device__ __forceinline__ Coef vt_coef(const DevParams &P, const StepArgs &U) {
   return K;
 }
 
-// The particles of an oversized tile past the first kVB (a single cell holding more than a tile's
-// particles: dense clusters), through global memory; launched before vt_step; their displacements
-// join the group maxima too.  (A launch of its own: as extra workgroups of vt_step, its particle
-// loop would raise vt_step's registers.)
+// The particles of the tiles that vt_step's workgroups cannot take (cells of more than a hundred particles:
+// dense clusters), 64 a workgroup, a quarter of the candidates per wave; launched before vt_step; their
+// displacements join the group maxima too.  30,000 particles of 940 neighbours each: 118 us an Euler
+// step (580 by walking lists, 1,267 by FP64 distances along them).
+// (A launch of its own: as extra workgroups of vt_step, its particle loop would raise vt_step's registers.)
 template <int S, bool SRK>
-__global__ __launch_bounds__(kVB) void vt_rest(DevParams P, VArgs A, StepArgs U, const int4 *__restrict__ tiles,
-                                               int ntiles, const int *__restrict__ list, const int *__restrict__ len,
+__global__ __launch_bounds__(kVB) void vt_rest(DevParams P, VArgs A, StepArgs U, const int2 *__restrict__ rest,
                                                const int *__restrict__ start, const int *__restrict__ cell,
                                                const double *__restrict__ state, const int *__restrict__ id,
                                                const double *__restrict__ nat, const float4 *__restrict__ snap,
                                                const float *__restrict__ omega, double *__restrict__ nstate,
                                                float4 *__restrict__ nsnap, float *__restrict__ nomega,
                                                double *__restrict__ compl_out) {
-  __shared__ double wmax[kVB / 64];
-  if (A.ctl->big_tiles == 0) return;  // the usual case: every tile fits its workgroup
+  static_assert(kRestItem == 64, "a lane per particle, in every wave");
+  constexpr int kWaves = kVB / 64;
+  __shared__ double sum[kWaves][SRK ? 4 : 2][64];
+  __shared__ int num[kWaves][64];
+  __shared__ double wmax[kWaves];
+  const int items = A.ctl->nrest;
+  if (items == 0) return;  // the usual case: every tile fits its workgroup
   const Coef K = vt_coef(P, U);
   const uint64_t step = U.step_dev ? (uint64_t)*U.step_dev : U.step;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   double d2 = 0.0;
-  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const int4 td = tiles[t];
-    if (td.z >= td.w) continue;
-    const int g0 = start[td.y * A.ncv + td.z], ntile = start[td.y * A.ncv + td.w] - g0;
-    for (int u = kVB + threadIdx.x; u < ntile; u += kVB) {
-      const int p = g0 + u;
-      const MSums m = vt_walk<S, SRK>(P, A, list, start, cell, state, snap, omega, p, len[p]);
-      d2 = fmax(d2, vt_particle<S, SRK>(P, A, U, K, step, state, id, nat, nstate, nsnap, nomega, compl_out, m, p,
-                                        cell[p] - td.y * A.ncv, td.y));
+  for (int t = blockIdx.x; t < items; t += gridDim.x) {
+    const int2 it = rest[t];
+    const int p = it.x + min(lane, it.y - 1);
+    MSums m = vt_walk<S, SRK, 8>(P, A, start, cell, state, snap, omega, p, w, kWaves);
+    sum[w][0][lane] = m.sx;
+    sum[w][1][lane] = m.sy;
+    if (SRK) {
+      sum[w][SRK ? 2 : 0][lane] = m.tx;
+      sum[w][SRK ? 3 : 0][lane] = m.ty;
     }
+    num[w][lane] = m.n;
+    __syncthreads();
+    if (w == 0 && lane < it.y) {
+      const auto all = [&](int q) { return ((sum[0][q][lane] + sum[1][q][lane]) + sum[2][q][lane]) + sum[3][q][lane]; };
+      m.sx = all(0);
+      m.sy = all(1);
+      if (SRK) {
+        m.tx = all(SRK ? 2 : 0);
+        m.ty = all(SRK ? 3 : 0);
+      }
+      m.n = num[0][lane] + num[1][lane] + num[2][lane] + num[3][lane];
+      const int c = cell[p];
+      d2 = fmax(d2, vt_particle<S, SRK>(P, A, U, K, step, state, id, nat, nstate, nsnap, nomega, compl_out, m, p,
+                                        c % A.ncv, c / A.ncv));
+    }
+    __syncthreads();
   }
   step_max(A, d2, wmax);
 }
 
-// The step of a tile's first kVB particles, one per lane (vt_rest has the others), and the step's
+// The step of a tile's particles, one per lane (vt_rest has the tiles that do not fit), and the step's
 // largest displacement as in vs_step.
 // (three workgroups per CU: no more registers than the vector ones, so that the products' results need
 // not be moved out of the accumulation registers)
 template <int S, bool SRK>
 __global__ __launch_bounds__(kVB, 3) void vt_step(DevParams P, VArgs A, StepArgs U, const int4 *__restrict__ tiles,
-                                               int ntiles, const int *__restrict__ list, const int *__restrict__ len,
-                                               const int *__restrict__ start, const int *__restrict__ cell,
-                                               const double *__restrict__ state, const int *__restrict__ id,
-                                               const double *__restrict__ nat, const float4 *__restrict__ snap,
-                                               const float *__restrict__ omega, double *__restrict__ nstate,
-                                               float4 *__restrict__ nsnap, float *__restrict__ nomega,
-                                               double *__restrict__ compl_out) {
+                                               int ntiles, const int *__restrict__ start,
+                                               const int *__restrict__ cell, const double *__restrict__ state,
+                                               const int *__restrict__ id, const double *__restrict__ nat,
+                                               const float4 *__restrict__ snap, const float *__restrict__ omega,
+                                               double *__restrict__ nstate, float4 *__restrict__ nsnap,
+                                               float *__restrict__ nomega, double *__restrict__ compl_out) {
   constexpr int W = SRK ? kMOmega : kMPlain;
   __shared__ VtLds<W> Ls;
   const int tile = xcd_block((int)blockIdx.x, (int)gridDim.x);
@@ -922,16 +958,16 @@ __global__ __launch_bounds__(kVB, 3) void vt_step(DevParams P, VArgs A, StepArgs
     const int total = vt_plan(A, start, row, ca, cb, Ls.plan);
     const int gtb = Ls.plan.cglob[cb - ca + 3];
     const int ntile = start[row * A.ncv + cb] - gtb;
-    const bool staged = total <= kMStage;
-    MSums sum;
-    const bool have = staged && vt_sums<S, W>(P, A, row, ca, cb, gtb, ntile, cell, state, snap, omega, Ls, sum);
-    const int u = threadIdx.x, p = gtb + u;
-    if (u < ntile) {
-      // (rare) staged values that are not finite, or small ones beside a large one out of range: the cells; an
-      // overflowing stage: the list
-      if (!have || sum.n == kMOpen) sum = vt_walk<S, SRK>(P, A, list, start, cell, state, snap, omega, p, staged ? -1 : len[p]);
-      d2 = vt_particle<S, SRK>(P, A, U, vt_coef(P, U), U.step_dev ? (uint64_t)*U.step_dev : U.step, state, id, nat,
-                               nstate, nsnap, nomega, compl_out, sum, p, cell[p] - row * A.ncv, row);
+    if (vt_takes(total, ntile)) {
+      MSums sum;
+      const bool have = vt_sums<S, W>(P, A, row, ca, cb, gtb, ntile, cell, state, snap, omega, Ls, sum);
+      const int u = threadIdx.x, p = gtb + u;
+      if (u < ntile) {
+        // (rare) staged values that are not finite, or small ones beside a large one out of range
+        if (!have || sum.n == kMOpen) sum = vt_walk<S, SRK, 4>(P, A, start, cell, state, snap, omega, p);
+        d2 = vt_particle<S, SRK>(P, A, U, vt_coef(P, U), U.step_dev ? (uint64_t)*U.step_dev : U.step, state, id, nat,
+                                 nstate, nsnap, nomega, compl_out, sum, p, cell[p] - row * A.ncv, row);
+      }
     }
   }
   step_max(A, d2, Ls.wmax);
@@ -1001,6 +1037,7 @@ struct VerletFast {
   bool tiled = false;
   int vt_wcap = 0, vt_cmax = 0;
   int4 *vtiles = nullptr;
+  int2 *rest = nullptr;  // items of vt_rest
   int *local = nullptr, *key = nullptr, *slotc = nullptr, *count = nullptr, *start = nullptr, *tmp = nullptr, *blocksum = nullptr;
   double *sstate = nullptr, *snat = nullptr;
   int *sid = nullptr, *scell = nullptr;
@@ -1052,7 +1089,7 @@ void vf_destroy(VerletFast *v) {
   void *b[] = {v->vstate[0], v->vstate[1], v->vsnap[0], v->vsnap[1], v->vomega[0], v->vomega[1], v->vid,
                v->vcell,     v->vnat,      v->list,     v->len,      v->key,       v->slotc,     v->count,
                v->start,     v->tmp,       v->blocksum, v->sstate,   v->snat,      v->sid,       v->scell,
-               v->ctl,       v->bmax,      v->vtiles,   v->local};
+               v->ctl,       v->bmax,      v->vtiles,   v->local,  v->rest};
   for (void *p : b) hipFree(p);
   delete v;
 }
@@ -1113,6 +1150,7 @@ int vf_create(VerletFast **out, hipStream_t st, const DevParams &P, double rho, 
                           (int)std::min((double)ncv, std::ceil(1.5 * row_mean / std::min(0.94 * kTileCap, 0.8 * cols * cell_mean)) + 2));
     A(hipMalloc(&v->local, sizeof(int) * (size_t)v->cells));
     A(hipMalloc(&v->vtiles, sizeof(int4) * (size_t)ncv * v->vt_cmax));
+    A(hipMalloc(&v->rest, sizeof(int2) * ((size_t)n / kRestItem + (size_t)ncv * v->vt_cmax)));  // a ragged item per tile
   }
   if (e != hipSuccess) {
     vf_destroy(v);
@@ -1234,15 +1272,15 @@ static void launch_step(VerletFast *v, hipStream_t st, const DevParams &P, const
   const int ntiles = v->tiled ? v->ncv * v->vt_cmax : 0;
   vr_settle<S><<<gg, kVB, 0, st>>>(P, A, v->sstate, v->sid, v->snat, v->scell, v->vstate[c], v->vid,
                                    nat ? v->vnat : nullptr, v->vcell, v->vsnap[c], v->vomega[c], v->start,
-                                   v->tiled ? v->vtiles : nullptr, ntiles, v->list, v->len);
+                                   v->tiled ? v->vtiles : nullptr, ntiles, v->rest);
   if (v->tiled) {
     const unsigned tg = (unsigned)((ntiles + 7) / 8 * 8);  // a multiple of 8 for xcd_block
-    vt_rest<S, SRK><<<std::min(tg, (unsigned)kGateGrid), kVB, 0, st>>>(
-        P, A, U, v->vtiles, ntiles, v->list, v->len, v->start, v->vcell, v->vstate[c], v->vid, nat, v->vsnap[c],
-        v->vomega[c], v->vstate[o], v->vsnap[o], v->vomega[o], SRK ? compl_out : nullptr);
-    vt_step<S, SRK><<<tg, kVB, 0, st>>>(P, A, U, v->vtiles, ntiles, v->list, v->len, v->start, v->vcell, v->vstate[c],
-                                        v->vid, nat, v->vsnap[c], v->vomega[c], v->vstate[o], v->vsnap[o],
-                                        v->vomega[o], SRK ? compl_out : nullptr);
+    vt_rest<S, SRK><<<kGateGrid, kVB, 0, st>>>(P, A, U, v->rest, v->start, v->vcell, v->vstate[c], v->vid, nat,
+                                               v->vsnap[c], v->vomega[c], v->vstate[o], v->vsnap[o], v->vomega[o],
+                                               SRK ? compl_out : nullptr);
+    vt_step<S, SRK><<<tg, kVB, 0, st>>>(P, A, U, v->vtiles, ntiles, v->start, v->vcell, v->vstate[c], v->vid, nat,
+                                        v->vsnap[c], v->vomega[c], v->vstate[o], v->vsnap[o], v->vomega[o],
+                                        SRK ? compl_out : nullptr);
   } else {
     vr_lists<S><<<nb, kVB, 0, st>>>(P, A, v->start, v->vcell, v->vstate[c], v->vsnap[c], v->list, v->len);
     const unsigned nb8 = (nb + 7u) & ~7u;  // a multiple of 8 for xcd_block
