@@ -181,8 +181,10 @@ int ensure_cells64(spss_system *h) {
   if (B.mem) return SPSS_OK;
   const size_t n = h->n, cells = (size_t)h->ncx * h->ncy;
   // one allocation (twelve took 0.4 ms), each array on a boundary of 256 bytes
-  const size_t ints[] = {n, n, n, n, 2 * n, cells, cells + 1, cells + 1, (size_t)scan_blocks(cells) + 1, 1};
-  int **to[] = {&B.order[0], &B.order[1], &B.key, &B.slot, &B.tmp, &B.count, &B.start, &B.local, &B.blocksum, &B.bad};
+  const size_t ints[] = {n, n, n, n, 2 * n, cells, cells + 1, cells + 1, (size_t)scan_blocks(cells) + 1, 2,
+                         2 * (n / 128 + h->ncy)};
+  int **to[] = {&B.order[0], &B.order[1], &B.key, &B.slot, &B.tmp, &B.count, &B.start, &B.local, &B.blocksum, &B.bad,
+                &B.extra};
   const auto padded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
   const size_t state = padded(sizeof(double) * n * h->s);
   size_t all = 2 * state;
@@ -192,7 +194,7 @@ int ensure_cells64(spss_system *h) {
   B.pre = reinterpret_cast<double *>(at);
   B.snap = reinterpret_cast<double *>(at + state);
   at += 2 * state;
-  for (int k = 0; k < 10; ++k) {
+  for (int k = 0; k < 11; ++k) {
     *to[k] = reinterpret_cast<int *>(at);
     at += padded(sizeof(int) * ints[k]);
   }

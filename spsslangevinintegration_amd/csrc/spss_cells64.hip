@@ -30,7 +30,7 @@ __global__ __launch_bounds__(256) void c64_keys(DevParams P, const double *__res
                                                 double *__restrict__ pre, int *__restrict__ key,
                                                 int *__restrict__ slot, int *__restrict__ count, int *__restrict__ bad) {
   const int t = blockIdx.x * 256 + threadIdx.x, lane = threadIdx.x & 63;
-  if (t == 0) *bad = 0;
+  if (t < 2) bad[t] = 0;  // and the number of extra chunks
   int c = -1;
   if (t < P.n) {
     const long i = order[t];
@@ -60,13 +60,16 @@ __global__ __launch_bounds__(256) void c64_keys(DevParams P, const double *__res
 // Bucket fill, and the second half of the scan beside it: `local` holds the starts inside blocks of
 // 256 * kScanItems cells, the blocks' offsets come from their totals (every workgroup sums them
 // itself: one launch less than a kernel that adds them first).  The final starts go to `start`, the
-// histogram is cleared.
+// histogram is cleared.  Rows of more than `cap` particles, what their own workgroups of c64_pairs take, leave the
+// rest in extra chunks of tb particles for all of its workgroups: {row, first position}.
 constexpr int kPlaceBlocks = 1024;  // scan blocks at most (2 million cells)
-__global__ __launch_bounds__(256) void c64_place(int n, int m, int nblk, const int *__restrict__ key,
+__global__ __launch_bounds__(256) void c64_place(int n, int m, int nc, int nblk, int cap, int tb,
+                                                 const int *__restrict__ key,
                                                  const int *__restrict__ slot, const int *__restrict__ local,
                                                  const int *__restrict__ total, const int *__restrict__ order,
                                                  int *__restrict__ start, int *__restrict__ count,
-                                                 int2 *__restrict__ tmp) {
+                                                 int2 *__restrict__ tmp, int *__restrict__ extras,
+                                                 int2 *__restrict__ extra) {
   __shared__ int off[kPlaceBlocks + 1];
   if (threadIdx.x < 64) {
     int run = 0;
@@ -94,6 +97,15 @@ __global__ __launch_bounds__(256) void c64_place(int n, int m, int nblk, const i
       count[t] = 0;
     }
     if (t == m) start[m] = off[nblk];
+    if (t < nc) {
+      const int a = t * nc, b = a + nc;
+      const int r0 = local[a] + off[a / (256 * kScanItems)], r1 = b < m ? local[b] + off[b / (256 * kScanItems)] : off[nblk];
+      const int chunks = (r1 - r0 - cap + tb - 1) / tb;
+      if (r1 - r0 > cap) {
+        int2 *to = extra + atomicAdd(extras, chunks);
+        for (int k = 0; k < chunks; ++k) to[k] = make_int2(t, r0 + cap + k * tb);
+      }
+    }
   }
 }
 
@@ -172,7 +184,8 @@ __device__ __forceinline__ void four_pairs(const DevParams &P, double band, doub
   }
 }
 
-// One workgroup per TB particles of a row of cells (chunk k of row r, then chunk k + gridDim.y, ...), one per
+// One workgroup per TB particles of a row of cells (chunk k of row r; then the extra chunks of rows longer than
+// gridDim.y of them, shared out over all workgroups: 30,000 particles in one row of 33: 3.8 ms with a row left to its own, 0.38), one per
 // lane in cell order: the three rows of cells around them are staged into LDS, positions as the periodic image next to the tile, so that a separation is a plain
 // difference; dense cells pass through the stage in windows of CAP entries.  A lane walks the three
 // column ranges of its particle, contiguous in the stage, in the reference's stencil order
@@ -181,17 +194,27 @@ template <int S, bool HO, int TB, int CAP>
 __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double band, double neg_slope, int nc, int rows8,
                                                 const int *__restrict__ start, const int *__restrict__ order,
                                                 const double *__restrict__ snap, const int *__restrict__ bad,
-                                                const double *__restrict__ nat, double *__restrict__ k_next,
-                                                double *__restrict__ compl_out) {
+                                                const int2 *__restrict__ extra, const double *__restrict__ nat,
+                                                double *__restrict__ k_next, double *__restrict__ compl_out) {
   constexpr int kPhi = Slots<S>::phi, kOm = S == 3 ? 2 : Slots<S>::omega;
   __shared__ Stage64<HO, CAP, TB> L;
   // workgroups go round the eight XCDs: each takes an eighth of the rows, so that neighbouring rows
   // share an L2
-  const int row = (blockIdx.x & 7) * rows8 + (blockIdx.x >> 3);
-  if (row >= nc) return;
-  const int r0 = start[row * nc], r1 = start[(row + 1) * nc];
+  int row = (blockIdx.x & 7) * rows8 + (blockIdx.x >> 3);
+  const int extras = bad[1];
+  int next = blockIdx.y * gridDim.x + blockIdx.x;  // of the extra chunks
+  int base = row < nc ? start[row * nc] + (int)blockIdx.y * TB : 0, r1 = row < nc ? start[(row + 1) * nc] : 0;
+  bool own = base < r1;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int base = r0 + blockIdx.y * TB; base < r1; base += gridDim.y * TB) {
+  for (;; own = false) {
+    if (!own) {
+      if (next >= extras) break;
+      const int2 it = extra[next];
+      next += gridDim.x * gridDim.y;
+      row = it.x;
+      base = it.y;
+      r1 = start[(row + 1) * nc];
+    }
     const int last = min(r1, base + TB);
     if (*bad) {  // pair by pair, the reference's expressions
       for (int g = base + threadIdx.x; g < last; g += TB) {
@@ -348,6 +371,16 @@ __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double 
   }
 }
 
+// 256 particles a workgroup of c64_pairs stage the fewest entries per particle; below some ten thousand
+// particles 128 a workgroup fill the chip better (per evaluation of model 6: 39.6 -> 36 us at
+// n = 20,000 against 42.2 -> 43.6 us at n = 50,000)
+int chunk(int n) { return n >= 40960 ? 256 : 128; }
+// chunks of a row of mean length, one more for the spread
+int row_chunks(int n, int nc) {
+  const long per_row = (n + nc - 1) / nc;
+  return (int)std::min<long>((per_row + per_row / 8) / chunk(n) + 1, 65535);
+}
+
 template <int S>
 void build(hipStream_t st, const DevParams &P, const double *state, const double *kprev, double kc_dt, int nc,
            Cells64 &B) {
@@ -359,8 +392,8 @@ void build(hipStream_t st, const DevParams &P, const double *state, const double
   // by the cells too, of which few particles may have many (200 on 2 million: 2,674 us an evaluation by the
   // particles alone, now 46)
   const dim3 np(std::max(nb.x, std::min((unsigned)(m / 256 + 1), 2048u)));
-  c64_place<<<np, tb, 0, st>>>(P.n, m, nblk, B.key, B.slot, B.local, B.blocksum, B.order[B.cur], B.start, B.count,
-                               (int2 *)B.tmp);
+  c64_place<<<np, tb, 0, st>>>(P.n, m, nc, nblk, row_chunks(P.n, nc) * chunk(P.n), chunk(P.n), B.key, B.slot, B.local,
+                               B.blocksum, B.order[B.cur], B.start, B.count, (int2 *)B.tmp, B.bad + 1, (int2 *)B.extra);
   c64_rank<S><<<nb, tb, 0, st>>>(P, nc, B.key, B.start, (const int2 *)B.tmp, B.pre, B.order[next], B.snap, B.bad);
   B.cur = next;
 }
@@ -369,21 +402,16 @@ template <int S, bool HO, int TB, int CAP>
 void pairs_as(hipStream_t st, const DevParams &P, int nc, const Cells64 &B, const double *nat, double *k_next,
               double *compl_out) {
   const int rows8 = (nc + 7) / 8;
-  // chunks of a row of mean length, one more for the spread; longer rows loop
-  const long per_row = (P.n + nc - 1) / nc;
-  const unsigned chunks = (unsigned)std::min<long>((per_row + per_row / 8) / TB + 1, 65535);
   const double band = pair_band(P.rho2, 1.0, 1.0);
-  c64_pairs<S, HO, TB, CAP><<<dim3((unsigned)rows8 * 8, chunks), dim3(TB), 0, st>>>(
-      P, band, pair_neg_slope(band), nc, rows8, B.start, B.order[B.cur], B.snap, B.bad, nat, k_next, compl_out);
+  c64_pairs<S, HO, TB, CAP><<<dim3((unsigned)rows8 * 8, (unsigned)row_chunks(P.n, nc)), dim3(TB), 0, st>>>(
+      P, band, pair_neg_slope(band), nc, rows8, B.start, B.order[B.cur], B.snap, B.bad, (const int2 *)B.extra, nat,
+      k_next, compl_out);
 }
 
 template <int S, bool HO>
 void pairs(hipStream_t st, const DevParams &P, int nc, const Cells64 &B, const double *nat, double *k_next,
            double *compl_out) {
-  // 256 particles a workgroup stage the fewest entries per particle; below some ten thousand
-  // particles 128 a workgroup fill the chip better (per evaluation of model 6: 39.6 -> 36 us at
-  // n = 20,000 against 42.2 -> 43.6 us at n = 50,000)
-  if (P.n >= 40960)
+  if (chunk(P.n) == 256)
     pairs_as<S, HO, 256, 1152>(st, P, nc, B, nat, k_next, compl_out);
   else
     pairs_as<S, HO, 128, 640>(st, P, nc, B, nat, k_next, compl_out);

@@ -128,7 +128,9 @@ struct Cells64 {
   char *mem = nullptr;                 // the allocation that holds them all
   int *order[2] = {nullptr, nullptr};  // [n] particle of each sorted position: the last build's, the next one's
   int cur = 0;
-  int *key = nullptr, *slot = nullptr, *count = nullptr, *blocksum = nullptr, *bad = nullptr;
+  int *key = nullptr, *slot = nullptr, *count = nullptr, *blocksum = nullptr;
+  int *bad = nullptr;    // [2] some particle is out of the cheap tests' range; extra chunks
+  int *extra = nullptr;  // [2 (n / 128 + rows)] the extra chunks
   int *local = nullptr, *start = nullptr;      // [cells + 1] starts inside a scan block, starts
   int *tmp = nullptr;                          // [2 n]
   double *pre = nullptr, *snap = nullptr;      // [s n] stage state in the last build's and in this one's order
