@@ -36,6 +36,9 @@ constexpr int kMaxLayers = 8;
 constexpr int kMaxDim = 4096;
 constexpr int kLossCap = 1 << 16;
 constexpr long kPredictPiece = 32768;   // rows copied and launched together
+// up to here 16 rows a workgroup still give every one of the 256 units at most one: 4,096 rows of 3 x 128 hidden 57 us a
+// call instead of 69; 6,144 to 8,192 are equal, 16 rows 71 and 74, 64 rows 71 and 73
+constexpr int kPredictFew = 16 * 256;
 constexpr long kPredictBytes = 64L << 20;  // of rows and outputs on the device at a time, kept by the network
 
 int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
@@ -293,8 +296,9 @@ int spss_mlp_predict(spss_mlp *m, const float *x, long n, float *y) {
         const int B = (int)std::min<long>(kPredictPiece, c1 - r0);
         MCHK(hipMemcpyAsync(m->px + (r0 - c0) * din, x + r0 * din, (size_t)B * din * sizeof(float),
                             hipMemcpyHostToDevice, m->st));
-        hipLaunchKernelGGL(ml_predict, dim3(cdiv(B, kPR)), dim3(kTB), 0, m->st, m->net, m->p,
-                           m->px + (r0 - c0) * din, B, m->py + (r0 - c0) * dout);
+        const bool few = B <= kPredictFew;
+        hipLaunchKernelGGL(few ? ml_predict<1> : ml_predict<4>, dim3(cdiv(B, few ? 16 : 64)), dim3(kTB), 0, m->st,
+                           m->net, m->p, m->px + (r0 - c0) * din, B, m->py + (r0 - c0) * dout);
         MCHK(hipGetLastError());
       }
       MCHK(hipMemcpyAsync(y + c0 * dout, m->py, (size_t)(c1 - c0) * dout * sizeof(float), hipMemcpyDeviceToHost, m->st));

@@ -446,20 +446,22 @@ __global__ __launch_bounds__(kTB) void ml_grad(Net N, float *__restrict__ p, flo
   p[e] = pe - A.step_size * mm / (sqrtf(vv) * A.inv_sqrt_bc2 + A.eps);
 }
 
-// Forward pass of 64 rows per workgroup through all layers, on the matrix cores (v_mfma_f32_16x16x4_f32: an
+// Forward pass of 16 Q rows per workgroup through all layers, on the matrix cores (v_mfma_f32_16x16x4_f32: an
 // FP32 multiply-add per term, k ascending, so the sums are those of the kernels above bit for bit): the rows'
 // activations in LDS, a wave's up to 32 outputs of all rows in its registers, the weights straight from
 // the caches with the next sixteen inputs' on their way.  A layer's outputs replace its inputs once
 // every wave has its sums.  100,000 rows of 3 x 128 hidden: 201 us (34 TFLOP/s; the products 60, the error
 // functions of the GELUs 75, neither beside the other), 219 for FMAs of the vector units with the weights
-// through LDS.  The call is bound by the rows' way up: 32,768 of them take 54 us.
-constexpr int kPR = 64;           // rows
+// through LDS.  The call is bound by the rows' way up: 32,768 of them take 54 us.  64 rows a workgroup (Q = 4) read the
+// weights least often; where they leave units idle, 16 (Q = 1): one row of 3 x 128 hidden 50 us a call instead of 62.
 constexpr int kPP = kNarrow + 4;  // pitch of a row's activations: a product's 16 rows x 4 inputs in 64 banks
 
 typedef float mlp4 __attribute__((ext_vector_type(4)));
 
+template <int Q>  // 16 Q rows
 __global__ __launch_bounds__(kTB, 4) void ml_predict(Net N, const float *__restrict__ p, const float *__restrict__ X,
                                                      int n, float *__restrict__ Y) {
+  constexpr int kPR = 16 * Q;
   __shared__ __align__(16) float a[kPR * kPP];
   const int tid = threadIdx.x, b0 = blockIdx.x * kPR, R = min(kPR, n - b0);
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, g = lane >> 4;
@@ -473,7 +475,7 @@ __global__ __launch_bounds__(kTB, 4) void ml_predict(Net N, const float *__restr
     const int in = N.dims[l], out = N.dims[l + 1], tiles = (out + 15) / 16;
     const float *wl = p + N.woff[l], *bias = p + N.boff[l];
     const bool last = l + 1 == N.L, two = wave + 4 < tiles;
-    mlp4 acc[2][4] = {};  // outputs 16 (wave + 4 t) + c of rows 16 q + 4 g ..
+    mlp4 acc[2][Q] = {};  // outputs 16 (wave + 4 t) + c of rows 16 q + 4 g ..
     float bo[2] = {};
     if (wave < tiles) {
       const int o0 = 16 * wave + c, o1 = o0 + 64;
@@ -494,14 +496,14 @@ __global__ __launch_bounds__(kTB, 4) void ml_predict(Net N, const float *__restr
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           if (k0 + 4 * s >= in) break;
-          float x[4];
+          float x[Q];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) x[q] = a[(16 * q + c) * kPP + k0 + 4 * s + g];
+          for (int q = 0; q < Q; ++q) x[q] = a[(16 * q + c) * kPP + k0 + 4 * s + g];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) acc[0][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q], w[0][s], acc[0][q], 0, 0, 0);
+          for (int q = 0; q < Q; ++q) acc[0][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q], w[0][s], acc[0][q], 0, 0, 0);
           if (two)
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int q = 0; q < Q; ++q)
               acc[1][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[q], w[1][s], acc[1][q], 0, 0, 0);
         }
 #pragma unroll
@@ -516,7 +518,7 @@ __global__ __launch_bounds__(kTB, 4) void ml_predict(Net N, const float *__restr
       if (wave + 4 * t >= tiles) continue;
       const int o = 16 * (wave + 4 * t) + c;
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int q = 0; q < Q; ++q)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int row = 16 * q + 4 * g + r;

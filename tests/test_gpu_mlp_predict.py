@@ -45,3 +45,16 @@ def test_activations_that_overflow(width):
     net.params = np.concatenate([p.ravel() for p in parts]).astype(np.float32)
     y = net.predict(np.array([[10.0], [0.0], [20.0]], dtype=np.float32))
     assert np.all(np.isposinf(y[[0, 2], 0])) and np.all(np.isneginf(y[[0, 2], 1])) and np.all(y[1] == 0)
+
+
+@pytest.mark.parametrize("dims", [(6, 128, 128, 128, 2), (128, 128, 128), (5, 17, 3), (1, 1, 1)])
+def test_rows_by_16_and_by_64(dims):
+    """a row's outputs are the same bits in a table of any length: tables up to 4,096 rows go 16 rows a workgroup,
+    longer ones 64"""
+    import spsslangevinintegration_amd as spss
+    net = spss.MLP(dims, max_batch=64, seed=5)
+    x = np.random.default_rng(2).uniform(-1, 1, (4163, dims[0])).astype(np.float32)
+    print(f"[gpu] predict rows dims={dims}", flush=True)
+    y = net.predict(x)
+    for n in (1, 15, 16, 17, 63, 65, 4080, 4095, 4096, 4097):
+        assert np.array_equal(net.predict(x[:n]), y[:n]), n
