@@ -27,3 +27,19 @@ def test_summary(phases):
     wa, warg = OO.summary(st.reshape(-1), 3)
     assert abs(a - wa) <= 2 * np.spacing(np.float32(wa)), (a, wa)
     assert abs(arg - warg) <= 2 * np.spacing(np.float32(abs(warg))), (arg, warg)
+
+
+@pytest.mark.parametrize("n", [2, 255, 8191, 16383, 16384, 16385, 20479, 20480, 20481, 69633])
+def test_summary_counts(n):
+    """sums of one launch (up to 16,384 particles) and of maps of runs (beyond), around their steps"""
+    import spsslangevinintegration_amd as spss
+    print(f"[gpu] summary counts n={n}", flush=True)
+    st = np.zeros((n, 6))
+    st[:, 4] = np.random.default_rng(n).choice(np.linspace(-1.2, 4.5, 17), n)
+    g = spss.ParticleSystem(model=6, n=n, rho=0.8)
+    g.set_state(st.reshape(-1))
+    a, arg = g.summary()
+    g.close()
+    wa, warg = OO.summary(st.reshape(-1), 6)
+    assert abs(a - wa) <= 2 * np.spacing(np.float32(wa)), (a, wa)
+    assert abs(arg - warg) <= 2 * np.spacing(np.float32(abs(warg))), (arg, warg)
