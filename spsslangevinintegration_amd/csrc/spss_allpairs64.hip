@@ -6,6 +6,7 @@
 //   ap_pairs   grid (groups of BLOCK particles) x (segments of the j's): the phasor sums of every
 //              particle over one segment, j ascending
 //   ap_finish  the segments' sums added in ascending order, the derivative
+//   ap_few     all of it, for up to 64 particles
 //
 // What bounds it: VALU issue, 14 instructions per pair (the test, the weight, three sums).  One
 // thread per particle over all j leaves most of the chip idle below some 10^5 particles (17
@@ -27,6 +28,18 @@ namespace {
 // outside it at all, ClassA is no minimum image there), or a phase without a finite phasor
 constexpr double kExactMark = __builtin_huge_val();
 
+// the record of a particle whose stage state is st
+template <int S>
+__device__ __forceinline__ double4 record(const DevParams &P, const double (&st)[S], double ref) {
+  double x, y, sn, cs;
+  apply_pbc(P, st[0], st[1], x, y);
+  frame_phasor_any(st[Slots<S>::phi], ref, sn, cs);
+  bool fine = fabs(sn) <= 1.5 && fabs(st[0]) <= kFar64 * P.xs && fabs(st[1]) <= kFar64 * P.ys;
+  if (S == 6) fine = fine && st[0] >= 0.0 && st[0] < P.xs && st[1] >= 0.0 && st[1] < P.ys;
+  if (S == 4 && P.higher_order) fine = fine && fabs(st[Slots<S>::omega]) < 1e300;
+  return make_double4(fine ? x : kExactMark, y, sn, cs);
+}
+
 template <int S>
 __global__ __launch_bounds__(256) void ap_stage(DevParams P, const double *__restrict__ state,
                                                 const double *__restrict__ kprev,
@@ -34,7 +47,7 @@ __global__ __launch_bounds__(256) void ap_stage(DevParams P, const double *__res
                                                 double *__restrict__ om) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= P.n) return;
-  constexpr int kPhi = Slots<S>::phi, kOm = Slots<S>::omega;
+  constexpr int kPhi = Slots<S>::phi;
   const double ref = frame_ref(state[kPhi] + (kprev ? kc_dt * kprev[kPhi] : 0.0));
   double st[S];
 #pragma unroll
@@ -43,16 +56,8 @@ __global__ __launch_bounds__(256) void ap_stage(DevParams P, const double *__res
     st[q] = state[e] + (kprev ? kc_dt * kprev[e] : 0.0);
     stage[e] = st[q];
   }
-  double x, y, sn, cs;
-  apply_pbc(P, st[0], st[1], x, y);
-  frame_phasor_any(st[kPhi], ref, sn, cs);
-  bool fine = fabs(sn) <= 1.5 && fabs(st[0]) <= kFar64 * P.xs && fabs(st[1]) <= kFar64 * P.ys;
-  if (S == 6) fine = fine && st[0] >= 0.0 && st[0] < P.xs && st[1] >= 0.0 && st[1] < P.ys;
-  if (S == 4 && P.higher_order) {
-    fine = fine && fabs(st[kOm]) < 1e300;
-    om[i] = st[kOm];
-  }
-  rec[i] = make_double4(fine ? x : kExactMark, y, sn, cs);
+  if (S == 4 && P.higher_order) om[i] = st[Slots<S>::omega];
+  rec[i] = record<S>(P, st, ref);
 }
 
 __device__ __forceinline__ void add_pair(PhasorSums &a, double w, double s, double c) {
@@ -105,6 +110,25 @@ __device__ __forceinline__ void four_j(const DevParams &P, double band, double n
         a[p].TC = __builtin_fma(wo, r[u].w, a[p].TC);
       }
     }
+}
+
+// particle j, its record r and omega om_j, by the reference's own test
+template <int S, bool HO, int PPL, int T>
+__device__ __forceinline__ void exact_j(const DevParams &P, const double *__restrict__ stage, const double4 &r,
+                                        double om_j, int i0, int j, const double (&x_i)[PPL], const double (&y_i)[PPL],
+                                        const double (&om_i)[PPL], PhasorSums (&a)[PPL]) {
+  const double x_j = stage[(long)j * S], y_j = stage[(long)j * S + 1];
+#pragma unroll
+  for (int p = 0; p < PPL; ++p) {
+    const int i = i0 + p * T + threadIdx.x;
+    if (i != j && pair_in_range<S>(P, x_i[p], y_i[p], x_j, y_j)) {
+      add_pair(a[p], 1.0, r.z, r.w);
+      if (HO) {
+        a[p].TS = __builtin_fma(om_j - om_i[p], r.z, a[p].TS);
+        a[p].TC = __builtin_fma(om_j - om_i[p], r.w, a[p].TC);
+      }
+    }
+  }
 }
 
 // PPL particles per lane (BLOCK / PPL threads): a tile entry read from LDS serves PPL pairs, which
@@ -160,22 +184,8 @@ __global__ __launch_bounds__(BLOCK / PPL) void ap_pairs(DevParams P, double band
       for (; t0 < cnt; t0 += 4)
         four_j<S, HO, PPL, T, true>(P, band, neg_slope, stage, tile, tom, i0, j0, t0, cnt, x_i, y_i, om_i, a);
     } else {
-      for (int t = 0; t < cnt; ++t) {
-        const int j = j0 + t;
-        const double x_j = stage[(long)j * S], y_j = stage[(long)j * S + 1];
-#pragma unroll
-        for (int p = 0; p < PPL; ++p) {
-          const int i = i0 + p * T + threadIdx.x;
-          if (i != j && pair_in_range<S>(P, x_i[p], y_i[p], x_j, y_j)) {
-            const double4 r = tile[t];
-            add_pair(a[p], 1.0, r.z, r.w);
-            if (HO) {
-              a[p].TS = __builtin_fma(tom[t] - om_i[p], r.z, a[p].TS);
-              a[p].TC = __builtin_fma(tom[t] - om_i[p], r.w, a[p].TC);
-            }
-          }
-        }
-      }
+      for (int t = 0; t < cnt; ++t)
+        exact_j<S, HO, PPL, T>(P, stage, tile[t], HO ? tom[t] : 0.0, i0, j0 + t, x_i, y_i, om_i, a);
     }
   }
   double *out = part + (long)blockIdx.y * (HO ? 5 : 3) * n;
@@ -240,6 +250,55 @@ __global__ __launch_bounds__(256) void ap_finish(DevParams P, int nseg, const do
   write_k<S>(P, st, i, pa, nat ? nat[i] : 0.0, k_next, compl_out);
 }
 
+// Up to 64 particles: stage, pair sums and derivative in one launch of one wave, the stage and its records in LDS.
+// The same sums as by the kernels above (one segment); a Runge-Kutta step of 2 particles in 14 to 18 us for 51, of 64
+// in 28 for 58.  (One wave is the line: 65 particles take 52 by the three launches.)
+// (kprev and k_next may be the same array: every lane has read kprev before the wave writes.)
+constexpr int kFew = kAllPairsFew;
+
+template <int S, bool HO>
+__global__ __launch_bounds__(kFew) void ap_few(DevParams P, double band, double neg_slope,
+                                               const double *__restrict__ state, const double *kprev, double kc_dt,
+                                               const double *__restrict__ nat, double *k_next, double *compl_out) {
+  __shared__ double4 tile[kFew];
+  __shared__ double tom[kFew], stage[kFew * S];
+  const int n = P.n, i = threadIdx.x;
+  constexpr int kPhi = Slots<S>::phi;
+  const double ref = frame_ref(state[kPhi] + (kprev ? kc_dt * kprev[kPhi] : 0.0));
+  double st[S] = {}, x_i[1] = {0.0}, y_i[1] = {0.0}, om_i[1] = {0.0};
+  bool ok = true;
+  double4 mine{};
+  if (i < n) {
+#pragma unroll
+    for (int q = 0; q < S; ++q) {
+      const int e = i * S + q;
+      st[q] = state[e] + (kprev ? kc_dt * kprev[e] : 0.0);
+      stage[e] = st[q];
+    }
+    mine = record<S>(P, st, ref);
+    ok = mine.x != kExactMark;
+    tile[i] = mine;
+    if (S == 6) {
+      x_i[0] = st[0];
+      y_i[0] = st[1];
+    } else {
+      apply_pbc(P, st[0], st[1], x_i[0], y_i[0]);
+    }
+    if (HO) tom[i] = om_i[0] = st[Slots<S>::omega];
+  }
+  PhasorSums a[1];
+  if (__syncthreads_and(ok)) {
+    for (int t0 = 0; t0 < n; t0 += 4)
+      four_j<S, HO, 1, kFew, true>(P, band, neg_slope, stage, tile, tom, 0, 0, t0, n, x_i, y_i, om_i, a);
+  } else {
+    for (int j = 0; j < n; ++j)
+      exact_j<S, HO, 1, kFew>(P, stage, tile[j], tom[j], 0, j, x_i, y_i, om_i, a);
+  }
+  if (i >= n) return;
+  const PairAcc pa = pair_acc<S>(P, a[0], mine.z, mine.w);
+  write_k<S>(P, st, i, pa, nat ? nat[i] : 0.0, k_next, compl_out);
+}
+
 template <int S, bool HO, int BLOCK, int JT>
 void pairs_as(hipStream_t st, const DevParams &P, const AllPairsScratch &W, const double *stage) {
   constexpr int PPL = BLOCK >= 128 ? 2 : 1;
@@ -286,6 +345,23 @@ void launch_all_pairs_stage(hipStream_t st, const DevParams &P, const double *st
     case 3: ap_stage<3><<<nb, dim3(256), 0, st>>>(P, state, kprev, kc_dt, stage, rec, W.om); break;
     case 4: ap_stage<4><<<nb, dim3(256), 0, st>>>(P, state, kprev, kc_dt, stage, rec, W.om); break;
     case 6: ap_stage<6><<<nb, dim3(256), 0, st>>>(P, state, kprev, kc_dt, stage, rec, W.om); break;
+    default: break;
+  }
+}
+
+void launch_all_pairs_few(hipStream_t st, const DevParams &P, const double *state, const double *kprev, double kc_dt,
+                          const double *nat, double *k_next, double *compl_out) {
+  const double band = pair_band(P.rho2, P.xs, P.ys), slope = pair_neg_slope(band);
+  const dim3 wg(kFew);
+  switch (P.s) {
+    case 3: ap_few<3, false><<<1, wg, 0, st>>>(P, band, slope, state, kprev, kc_dt, nat, k_next, compl_out); break;
+    case 4:
+      if (P.higher_order)
+        ap_few<4, true><<<1, wg, 0, st>>>(P, band, slope, state, kprev, kc_dt, nat, k_next, compl_out);
+      else
+        ap_few<4, false><<<1, wg, 0, st>>>(P, band, slope, state, kprev, kc_dt, nat, k_next, compl_out);
+      break;
+    case 6: ap_few<6, false><<<1, wg, 0, st>>>(P, band, slope, state, kprev, kc_dt, nat, k_next, compl_out); break;
     default: break;
   }
 }

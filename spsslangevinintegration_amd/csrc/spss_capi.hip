@@ -319,8 +319,10 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
     TRY(ensure_cells64(h));
     launch_cells64_build(st, h->P, d_state, d_kprev, k_coef * dt, h->ncx, h->cells64);
   } else if (m == SPSS_METHOD_ALL_PAIRS) {
-    TRY(ensure_all_pairs(h));
-    launch_all_pairs_stage(st, h->P, d_state, d_kprev, k_coef * dt, h->stage, h->ap);
+    if (h->n > kAllPairsFew) {
+      TRY(ensure_all_pairs(h));
+      launch_all_pairs_stage(st, h->P, d_state, d_kprev, k_coef * dt, h->stage, h->ap);
+    }
   } else if (m != SPSS_METHOD_GLOBAL_FIELD && (!verlet || h->should_update))  // the Verlet pair sums stage in the order of their lists
     launch_stage(st, (long)h->s * h->n, d_state, d_kprev, k_coef * dt, h->stage);
   switch (m) {
@@ -328,7 +330,10 @@ int rhs_device(spss_system *h, int method, const double *d_state, const double *
       launch_global(st, h->P, d_state, d_kprev, k_coef * dt, h->partial, nat, d_knext, compl_out);
       break;
     case SPSS_METHOD_ALL_PAIRS:
-      launch_all_pairs(st, h->P, h->ap, h->stage, nat, d_knext, compl_out, h->ap_config);
+      if (h->n > kAllPairsFew)
+        launch_all_pairs(st, h->P, h->ap, h->stage, nat, d_knext, compl_out, h->ap_config);
+      else
+        launch_all_pairs_few(st, h->P, d_state, d_kprev, k_coef * dt, nat, d_knext, compl_out);
       break;
     case SPSS_METHOD_LINKED_LIST:
       if (h->p.precision == SPSS_PRECISION_FP32C) {

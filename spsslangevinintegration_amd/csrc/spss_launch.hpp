@@ -118,6 +118,10 @@ void launch_all_pairs_stage(hipStream_t st, const DevParams &P, const double *st
                             double *stage, const AllPairsScratch &W);
 void launch_all_pairs(hipStream_t st, const DevParams &P, const AllPairsScratch &W, const double *stage,
                       const double *nat, double *k_next, double *compl_out, int config = kAllPairsDefault);
+// the same derivative of up to kAllPairsFew particles in one launch, without a workspace
+constexpr int kAllPairsFew = 64;
+void launch_all_pairs_few(hipStream_t st, const DevParams &P, const double *state, const double *kprev, double kc_dt,
+                          const double *nat, double *k_next, double *compl_out);
 void launch_cell_build(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy, CellBuffers &cb);
 void launch_linked_list(hipStream_t st, const DevParams &P, const double *stage, int ncx, int ncy,
                         const CellBuffers &cb, const double *nat, double *k_next, double *compl_out);
