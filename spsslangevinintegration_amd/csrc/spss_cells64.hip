@@ -184,11 +184,12 @@ __device__ __forceinline__ void four_pairs(const DevParams &P, double band, doub
   }
 }
 
-// One workgroup per TB particles of a row of cells (chunk k of row r; then the extra chunks of rows longer than
-// gridDim.y of them, shared out over all workgroups: 30,000 particles in one row of 33: 3.8 ms with a row left to its own, 0.38), one per
-// lane in cell order: the three rows of cells around them are staged into LDS, positions as the periodic image next to the tile, so that a separation is a plain
-// difference; dense cells pass through the stage in windows of CAP entries.  A lane walks the three
-// column ranges of its particle, contiguous in the stage, in the reference's stencil order
+// One workgroup per TB particles of a row of cells (chunk k of row r; then the extra chunks of longer rows, shared
+// out over all workgroups: 30,000 particles in one row of 33 in 0.38 ms, 3.8 with a row left to its own), one per
+// lane in cell order: the three rows of cells around them are staged into LDS, positions as the periodic image next
+// to the tile, so that a separation is a plain difference; dense cells pass through the stage in windows of CAP
+// entries.  A lane walks the three column ranges of its particle, contiguous in the stage, in the reference's
+// stencil order
 // (ParticleSystemFirstOrderPtr.cpp:83-88).
 template <int S, bool HO, int TB, int CAP>
 __global__ __launch_bounds__(TB, HO ? 3 : 4) void c64_pairs(DevParams P, double band, double neg_slope, int nc, int rows8,
